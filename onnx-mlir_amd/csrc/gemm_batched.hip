@@ -1,0 +1,457 @@
+// int8 products of two activations, batched (the attention products of a
+// transformer: scores Q K^T and context P V over batch x heads), in one launch
+// and without a packed copy of the right-hand side.
+//
+// What is computed is what gemm_kernels.hip computes,
+//     Y[i,j] = sum_k (A[i,k] - az[i]) * (B[k,j] - bz[j])        (mod 2^32)
+// as sum A'B' + db*rowsum(A') + da*colsum(B') + K*da*db, once per batch entry.
+//
+// k_gemm_i8_batched
+//   Bound: the int32 results (32 x 12 heads of 128x64x128: 25 MB out, 6 MB in;
+//   4.5 us at the 5.66 TB/s the device stores at) and, with one K step, the
+//   chain load -> LDS -> MFMA -> store of a block.  Measured 7.0 us = 4.5 TB/s.
+//   Why one launch: packing B and multiplying, matrix by matrix, is three
+//   launches of 1.3 to 3.5 us an entry, whatever the entry's size (the same
+//   product: 3.5 ms).
+//   Why B is transposed here: it is used by M / 64 blocks and never again, so
+//   an operand-order copy in memory costs more than it saves.  A thread reads
+//   4 columns x 4 or 8 rows of B as 4-byte words (a wave: whole rows of the
+//   tile), turns 4 x 4 byte blocks around with eight v_perm_b32, and writes the
+//   columns' K bytes into LDS in operand order; column sums are two dot
+//   products of registers it holds anyway.
+//   Why 64 x 128 (64 x 64 for N <= 64): 384 entries of 128 x 128 are 768
+//   blocks, three per CU, so that one block's stores run beside another's
+//   loads.
+//   LDS layout of B: [column tile of 32][16-byte K chunk][column][16 bytes],
+//   the column's place within its group of four XORed with (column / 16) % 4:
+//   the 4- and 8-byte writes of a wave (columns four apart) and the 16-byte
+//   operand reads then both touch every bank equally often.
+//   Loads: buffer loads with a lane offset that never changes (64-bit addresses
+//   per load: 2 x 256x4096x4096 50.4 us, this form 38.4), two K steps in
+//   flight; results written through where row pieces are whole lines (8.6 ->
+//   7.5 us, streaming stores 7.9).  Four blocks a CU where 128 registers suffice
+//   (96 x 512x64x512 22.6 -> 20.3 us against three), three for the 128-wide
+//   unaligned form (156 x 441x64x441 39.4 -> 33.7 us against two).
+#include "gemm_common.h"
+#include "gemm_epilogue.h"
+
+namespace om {
+
+using namespace gemm;
+
+namespace {
+
+constexpr int BM = 64;
+constexpr int kBatchDims = GemmBatch::kDims;
+
+struct BatchParams {
+  const uint8_t *A, *B;
+  int64_t a_total, b_total; // bytes behind A and B
+  int M, N, K;
+  uint32_t a_flip, b_flip; // 0x80808080 for uint8 operands
+  int tiles_m, tiles_n;
+  int first; // batch entry of the launch's first block
+  int dims[kBatchDims];    // sizes of the batch dimensions, outermost first
+  int64_t a_step[kBatchDims], b_step[kBatchDims]; // in matrices; 0 broadcasts
+  bool a_zp_per_matrix, b_zp_per_matrix;
+};
+
+// Bytes at offset `off` of a buffer of `total` bytes, for addresses of any
+// alignment: a load that would run past the buffer's end is moved back to end
+// with it and its bytes shifted down.
+__device__ __forceinline__ uint32_t load4_any(
+    const uint8_t *__restrict__ p, int off, int total) {
+  typedef uint32_t u32_any __attribute__((aligned(1)));
+  const int at = off < total - 4 ? off : total - 4;
+  return *(const u32_any *)(p + at) >> ((off - at) * 8);
+}
+__device__ __forceinline__ v4i load16_any(
+    const uint8_t *__restrict__ p, int off, int total) {
+  const int at = off < total - 16 ? off : total - 16;
+  const int sh = (off - at) * 8;
+  const v4i_any raw = *(const v4i_any *)(p + at);
+  uint64_t lo = (uint32_t)raw.x | ((uint64_t)(uint32_t)raw.y << 32);
+  uint64_t hi = (uint32_t)raw.z | ((uint64_t)(uint32_t)raw.w << 32);
+  if (sh >= 64) {
+    lo = hi;
+    hi = 0;
+  }
+  const int s1 = sh & 63;
+  if (s1) {
+    lo = (lo >> s1) | (hi << (64 - s1));
+    hi >>= s1;
+  }
+  return (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
+      (int)(uint32_t)(hi >> 32)};
+}
+
+// ALIGNED: K % 16 == 0 with A on a 16-byte boundary and N % 4 == 0 with B on a
+// 4-byte one, so that every load is whole and inside its row.
+template <int BN, int EPI, bool ALIGNED>
+__global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_batched(
+    const BatchParams bp, const EpiParams ep) {
+  static_assert(BN == 128 || BN == 64, "tile width");
+  constexpr int TM = BN == 128 ? 2 : 1; // row tiles of 32 per wave
+  constexpr int KPT = BN / 16;          // K rows of B per thread
+  constexpr int CG = BN / 4;            // groups of four columns
+  __shared__ __attribute__((aligned(16))) uint8_t sA[2][BM * BK];
+  __shared__ __attribute__((aligned(16))) uint8_t sB[2][BN * BK];
+  __shared__ int32_t s_rowsum[BM], s_da[BM];
+  __shared__ int32_t s_colsum[BN];
+
+  // The tiles of one batch entry go to one XCD, whose L2 then holds its A and B.
+  int pid = blockIdx.x;
+  {
+    const int per = (int)gridDim.x >> 3;
+    if (per > 0 && pid < per * 8)
+      pid = (pid & 7) * per + (pid >> 3);
+  }
+  const int M = bp.M, N = bp.N, K = bp.K;
+  const int tiles = bp.tiles_m * bp.tiles_n;
+  const int rank = pid / tiles; // among the launch's entries
+  const int entry = bp.first + rank;
+  const int t = pid - rank * tiles;
+  const int tm = t / bp.tiles_n;
+  const int m0 = tm * BM, n0 = (t - tm * bp.tiles_n) * BN;
+  int64_t ai = 0, bi = 0;
+  {
+    int rest = entry;
+#pragma unroll
+    for (int d = kBatchDims - 1; d > 0; --d) {
+      const int q = rest / bp.dims[d];
+      const int c = rest - q * bp.dims[d];
+      rest = q;
+      ai += c * bp.a_step[d];
+      bi += c * bp.b_step[d];
+    }
+    ai += rest * bp.a_step[0];
+    bi += rest * bp.b_step[0];
+  }
+  // The entry's matrices, addressed by 32-bit offsets (gemm_batched_ok).
+  const uint8_t *const Ae = bp.A + ai * M * K, *const Be = bp.B + bi * K * N;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, lh = lane >> 5;
+
+  // A: row tid / 4 of the tile, 16-byte chunk tid % 4 of the K step.
+  const int ar = tid >> 2, ac = tid & 3;
+  const bool a_row = m0 + ar < M;
+  // B: columns 4 cg .. 4 cg + 3, KPT rows from kg * KPT of the K step.
+  const int cg = tid % CG, kg = tid / CG;
+  const bool b_col = n0 + cg * 4 < N;
+
+  // ALIGNED: buffer loads, a lane offset that never changes and the K step as
+  // scalar offset; what lies outside the matrices (rows past M and columns past
+  // N are sent there) reads as 0.  Otherwise global loads at byte addresses.
+  constexpr int kOutside = 0x7FFFFFFF;
+  const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)Ae, 0, M * K, 0x00020000);
+  const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)Be, 0, K * N, 0x00020000);
+  const int a_off = (m0 + ar) * K + ac * 16;
+  const int b_off = kg * KPT * N + n0 + cg * 4;
+  const int a_voff = a_row ? a_off : kOutside, b_voff = b_col ? b_off : kOutside;
+  const int64_t a_left = bp.a_total - ai * M * K, b_left = bp.b_total - bi * K * N;
+  const int a_end = a_left < kOutside ? (int)a_left : kOutside;
+  const int b_end = b_left < kOutside ? (int)b_left : kOutside;
+
+  int32_t rs = 0, cs[4] = {0, 0, 0, 0};
+  // Operands on their way from memory: two K steps, so that a step's loads have
+  // the time of two to arrive.
+  v4i ra0, ra1;
+  uint32_t rb0[KPT], rb1[KPT];
+  // (Steps past the end load nothing, or the first bytes of A and B, which
+  // nobody uses: with no branch around a load its wait is exact.)
+  auto load = [&](int k0, v4i &ra, uint32_t(&rb)[KPT]) {
+    if (ALIGNED) {
+      ra = __builtin_amdgcn_raw_buffer_load_b128(arsrc, a_voff, k0, 0);
+#pragma unroll
+      for (int i = 0; i < KPT; ++i)
+        rb[i] = __builtin_amdgcn_raw_buffer_load_b32(
+            brsrc, b_voff, (k0 + i) * N, 0);
+    } else {
+      ra = load16_any(Ae, a_row && k0 + ac * 16 < K ? a_off + k0 : 0, a_end);
+#pragma unroll
+      for (int i = 0; i < KPT; ++i) {
+        const bool in = b_col && k0 + kg * KPT + i < K;
+        rb[i] = load4_any(Be, in ? b_off + (k0 + i) * N : 0, b_end);
+      }
+    }
+  };
+  // Registers to LDS, as int8 and in operand order; bytes past K become 0 in
+  // both operands (rows past M and columns past N are never stored).
+  auto store = [&](int k0, int buf, const v4i &ra, const uint32_t(&rb)[KPT]) {
+    const int gk = k0 + ac * 16;
+    const int len = a_row ? K - gk : 0; // bytes of the chunk inside the row
+    v4i v = ra ^ (v4i){(int)bp.a_flip, (int)bp.a_flip, (int)bp.a_flip,
+                     (int)bp.a_flip};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int keep = len - w * 4;
+      const uint32_t mask = keep >= 4  ? 0xFFFFFFFFu
+                            : keep > 0 ? (1u << (8 * keep)) - 1
+                                       : 0u;
+      v[w] = (int)((uint32_t)v[w] & mask);
+    }
+    rs += frag_rowsum(v);
+    *(v4i *)(&sA[buf][lds_off(ar, ac)]) = v;
+    uint32_t o[4][KPT / 4];
+#pragma unroll
+    for (int h = 0; h < KPT / 4; ++h) {
+      uint32_t r[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        r[i] = k0 + kg * KPT + h * 4 + i < K ? rb[h * 4 + i] ^ bp.b_flip : 0u;
+      const uint32_t t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);
+      const uint32_t t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
+      const uint32_t t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
+      const uint32_t t3 = __builtin_amdgcn_perm(r[3], r[2], 0x07030602u);
+      o[0][h] = __builtin_amdgcn_perm(t2, t0, 0x05040100u);
+      o[1][h] = __builtin_amdgcn_perm(t2, t0, 0x07060302u);
+      o[2][h] = __builtin_amdgcn_perm(t3, t1, 0x05040100u);
+      o[3][h] = __builtin_amdgcn_perm(t3, t1, 0x07060302u);
+    }
+    const int chunk = (kg * KPT) >> 4, within = (kg * KPT) & 15;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int h = 0; h < KPT / 4; ++h)
+        cs[j] = __builtin_amdgcn_sdot4((int)o[j][h], 0x01010101, cs[j], false);
+      uint8_t *const dst = &sB[buf][((cg >> 3) * 4 + chunk) * 512 +
+                                    ((cg & 7) * 4 + ((j ^ (cg >> 2)) & 3)) * 16 +
+                                    within];
+      if (KPT == 8)
+        *(uint64_t *)dst = o[j][0] | ((uint64_t)o[j][KPT / 4 - 1] << 32);
+      else
+        *(uint32_t *)dst = o[j][0];
+    }
+  };
+
+  const int ct = BN == 128 ? wave : wave & 1;     // the wave's column tile
+  const int rt = BN == 128 ? 0 : (wave >> 1) * 32; // its first row
+  v16i acc[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      acc[i][r] = 0;
+  const int bslot =
+      ((l32 & ~3) | ((l32 ^ (ct * 2 + (l32 >> 4))) & 3)) * 16;
+
+  // What the epilogue needs per row and column, requested before the operands.
+  if (tid < BN)
+    s_colsum[tid] = 0;
+  if (tid < BM) {
+    const int32_t oa = bp.a_flip ? 128 : 0;
+    int32_t az = 0;
+    if (ep.a_zp_len > 0) {
+      const int m = m0 + tid < M ? m0 + tid : 0;
+      az = load_zp_i32(ep.a_zp, bp.a_flip != 0,
+          ep.a_zp_len > 1 ? (bp.a_zp_per_matrix ? ai * M : 0) + m : 0);
+    }
+    s_da[tid] = oa - az;
+  }
+  const int n = n0 + ct * 32 + l32;
+  const int nc = n < N ? n : N - 1;
+  int32_t db = bp.b_flip ? 128 : 0;
+  if (ep.b_zp_len > 0)
+    db -= load_zp_i32(ep.b_zp, bp.b_flip != 0,
+        ep.b_zp_len > 1 ? (bp.b_zp_per_matrix ? bi * N : 0) + nc : 0);
+  float sj = 0.0f;
+  int32_t yz = 0;
+  if (EPI == kEpiQ8) {
+    // (a_scale * b_scale) / y_scale, in this order
+    // (src/Conversion/ONNXToKrnl/Math/QLinearMatMul.cpp:127)
+    sj = (ep.a_scale[0] * ep.b_scale[ep.b_scale_len == 1 ? 0 : nc]) /
+         ep.y_scale[0];
+    yz = load_zp_i32(ep.y_zp, ep.y_unsigned, 0);
+  }
+
+  auto multiply = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const v4i b = *(const v4i *)(&sB[buf][(ct * 4 + s * 2 + lh) * 512 + bslot]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const v4i a =
+            *(const v4i *)(&sA[buf][lds_off(rt + i * 32 + l32, s * 2 + lh)]);
+        acc[i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, acc[i], 0, 0, 0);
+      }
+    }
+  };
+  load(0, ra0, rb0);
+  if (K <= BK) { // one step: nothing to overlap
+    store(0, 0, ra0, rb0);
+    __syncthreads();
+    multiply(0);
+  } else {
+    load(BK, ra1, rb1);
+    store(0, 0, ra0, rb0);
+    lds_barrier();
+    for (int k0 = 0;; k0 += 2 * BK) {
+      load(k0 + 2 * BK, ra0, rb0);
+      multiply(0);
+      if (k0 + BK >= K)
+        break;
+      store(k0 + BK, 1, ra1, rb1);
+      lds_barrier();
+      load(k0 + 3 * BK, ra1, rb1);
+      multiply(1);
+      if (k0 + 2 * BK >= K)
+        break;
+      store(k0 + 2 * BK, 0, ra0, rb0);
+      lds_barrier();
+    }
+  }
+
+  // Row sums: the four threads of a row.  Column sums: the threads of a column
+  // group add theirs up in LDS.
+  rs += __shfl_xor(rs, 1, 64);
+  rs += __shfl_xor(rs, 2, 64);
+  if (ac == 0)
+    s_rowsum[ar] = rs;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    atomicAdd(&s_colsum[cg * 4 + j], cs[j]);
+  __syncthreads();
+
+  // 32x32 accumulator layout: lane holds column lane % 32; register r holds
+  // row 8*(r/4) + 4*(lane/32) + r%4.
+  if (n >= N)
+    return;
+  const uint32_t csn = (uint32_t)s_colsum[ct * 32 + l32];
+  // A descriptor over the tile's rows inside the matrix: stores to rows past M
+  // fall outside and are dropped (gemm_batched_ok keeps 64 rows below 2^31
+  // bytes).
+  constexpr int ES = EPI == kEpiQ8 ? 1 : 4;
+  const int rows = M - m0 < BM ? M - m0 : BM;
+  char *const out = (char *)ep.out +
+                    (((int64_t)entry * M + m0) * N + n0) * (int64_t)ES;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      out, 0, (int)(((int64_t)rows * N - n0) * ES), 0x00020000);
+  const int voff = ((4 * lh) * N + ct * 32 + l32) * ES;
+  auto rows_out = [&](auto aux) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int first = rt + i * 32 + 8 * (r >> 2) + (r & 3); // of lane 0
+        const uint32_t da = (uint32_t)s_da[first + 4 * lh];
+        const uint32_t y =
+            (uint32_t)acc[i][r] + da * csn +
+            (uint32_t)db * ((uint32_t)s_rowsum[first + 4 * lh] + (uint32_t)K * da);
+        if (EPI == kEpiI32)
+          __builtin_amdgcn_raw_buffer_store_b32(
+              (int)y, rsrc, voff, first * N * ES, decltype(aux)::value);
+        else
+          __builtin_amdgcn_raw_buffer_store_b8(
+              (unsigned char)requantize(ep, y, sj, yz), rsrc, voff,
+              first * N * ES, decltype(aux)::value);
+      }
+    }
+  };
+  if (((int64_t)N * ES) % 128 == 0)
+    rows_out(std::integral_constant<int, kAuxThrough>{});
+  else
+    rows_out(std::integral_constant<int, 0>{});
+}
+
+template <int EPI>
+hipError_t launch_epi(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
+    int64_t entries, bool aligned) {
+  const unsigned blocks = (unsigned)(entries * bp.tiles_m * bp.tiles_n);
+  if (bp.N <= 64) {
+    if (aligned)
+      k_gemm_i8_batched<64, EPI, true><<<blocks, 256, 0, s>>>(bp, ep);
+    else
+      k_gemm_i8_batched<64, EPI, false><<<blocks, 256, 0, s>>>(bp, ep);
+  } else {
+    if (aligned)
+      k_gemm_i8_batched<128, EPI, true><<<blocks, 256, 0, s>>>(bp, ep);
+    else
+      k_gemm_i8_batched<128, EPI, false><<<blocks, 256, 0, s>>>(bp, ep);
+  }
+  return hipGetLastError();
+}
+
+constexpr int64_t kMaxBytes = (int64_t)1 << 30; // of one matrix, with a tile's overhang
+constexpr int64_t kMaxBlocks = (int64_t)1 << 22; // of one launch
+
+int64_t tiles_of(int64_t M, int64_t N) {
+  const int64_t bn = N <= 64 ? 64 : 128;
+  return ((M + BM - 1) / BM) * ((N + bn - 1) / bn);
+}
+
+} // namespace
+
+bool gemm_batched_ok(const GemmArgs &g, const GemmBatch &b) {
+  return g.epi != kEpiF32 && g.M > 0 && g.N > 0 && g.K > 0 &&
+         (g.M + BM) * g.K < kMaxBytes && (g.K + 4 * BK) * g.N < kMaxBytes && b.count > 0 && b.count <= INT32_MAX &&
+         g.M * g.K * b.a_mats >= 16 && g.K * g.N * b.b_mats >= 4 &&
+         g.M < kMaxBytes && g.N < ((int64_t)1 << 23) &&
+         tiles_of(g.M, g.N) <= kMaxBlocks;
+}
+
+// One launch wins while an entry's operands are not reused enough to pay for
+// packing B and for launches of its own (this kernel / packing and multiplying
+// entry by entry): 384 x 128x64x128 7.1 us / 3.5 ms, 8 x 1024x1024x1024 29.0 /
+// 79.1, 2 x 1024x4096x1024 40.4 / 52.5, 4 x 2048x2048x2048 89.5 / 93.7; beyond
+// that the tile kernels' 1.5 - 2 POP/s are ahead of the 0.77 reached here.
+bool gemm_batched_pays(const GemmArgs &g) {
+  return g.M * g.N * g.K <= ((int64_t)1 << 33);
+}
+
+hipError_t launch_gemm_batched(
+    hipStream_t s, const GemmArgs &g, const GemmBatch &b) {
+  if (!gemm_batched_ok(g, b))
+    return hipErrorInvalidValue;
+  BatchParams bp = {};
+  bp.A = (const uint8_t *)g.A;
+  bp.B = (const uint8_t *)b.B;
+  bp.a_total = g.M * g.K * b.a_mats;
+  bp.b_total = g.K * g.N * b.b_mats;
+  bp.M = (int)g.M;
+  bp.N = (int)g.N;
+  bp.K = (int)g.K;
+  bp.a_flip = g.a_unsigned ? 0x80808080u : 0u;
+  bp.b_flip = g.b_unsigned ? 0x80808080u : 0u;
+  bp.tiles_m = (int)((g.M + BM - 1) / BM);
+  bp.tiles_n = (int)(tiles_of(g.M, g.N) / bp.tiles_m);
+  for (int d = 0; d < kBatchDims; ++d) {
+    bp.dims[d] = (int)b.dims[d];
+    bp.a_step[d] = b.a_step[d];
+    bp.b_step[d] = b.b_step[d];
+  }
+  bp.a_zp_per_matrix = b.a_zp_per_matrix;
+  bp.b_zp_per_matrix = b.b_zp_per_matrix;
+  EpiParams ep = {};
+  ep.a_zp = g.a_zp;
+  ep.a_zp_len = g.a_zp ? g.a_zp_len : 0;
+  ep.b_zp = g.b_zp;
+  ep.b_zp_len = g.b_zp ? g.b_zp_len : 0;
+  ep.a_scale = g.a_scale;
+  ep.b_scale = g.b_scale;
+  ep.b_scale_len = g.b_scale_len;
+  ep.y_scale = g.y_scale;
+  ep.y_zp = g.y_zp;
+  ep.out = g.out;
+  ep.y_unsigned = g.y_unsigned;
+  ep.narrow = (int)g.narrow;
+  const bool aligned = g.K % 16 == 0 && g.N % 4 == 0 &&
+                       (((uintptr_t)g.A) & 15) == 0 && (((uintptr_t)b.B) & 3) == 0;
+  note_gemm_kernel("k_gemm_i8_batched");
+  const int64_t per_launch = kMaxBlocks / tiles_of(g.M, g.N);
+  for (int64_t e = 0; e < b.count; e += per_launch) {
+    const int64_t entries = b.count - e < per_launch ? b.count - e : per_launch;
+    bp.first = (int)e;
+    const hipError_t rc =
+        g.epi == kEpiI32 ? launch_epi<kEpiI32>(s, bp, ep, entries, aligned)
+                         : launch_epi<kEpiQ8>(s, bp, ep, entries, aligned);
+    if (rc != hipSuccess)
+      return rc;
+  }
+  return hipSuccess;
+}
+
+} // namespace om

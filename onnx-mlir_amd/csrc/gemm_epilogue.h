@@ -20,6 +20,20 @@ namespace gemm {
 // be issued back to back without waiting on one another.
 // bj: the bias of the column, or -0.0f, which leaves every value (both zeros
 // included) as it is.
+// One accumulator to its 8-bit result (kEpiQ8), in the low byte.
+__device__ __forceinline__ uint32_t requantize(
+    const EpiParams &ep, uint32_t y, float sj, int32_t yz) {
+  const float f = (float)(int32_t)y * sj;
+  const int32_t q = (int32_t)__builtin_rintf(f);
+  int32_t v = (int32_t)((uint32_t)q + (uint32_t)yz);
+  if (ep.narrow == kSaturate) {
+    const int32_t lo = ep.y_unsigned ? 0 : -128;
+    const int32_t hi = ep.y_unsigned ? 255 : 127;
+    v = v < lo ? lo : (v > hi ? hi : v);
+  }
+  return (uint32_t)v & 0xFF;
+}
+
 template <int EPI>
 __device__ __forceinline__ void store_one(const EpiParams &ep, int64_t o,
     uint32_t y, float sj, int32_t yz, float bj) {
@@ -29,15 +43,7 @@ __device__ __forceinline__ void store_one(const EpiParams &ep, int64_t o,
     const float f = (float)(int32_t)y * sj + bj;
     ((float *)ep.out)[o] = relu_f32(f, ep.floor);
   } else {
-    const float f = (float)(int32_t)y * sj;
-    const int32_t q = (int32_t)__builtin_rintf(f);
-    int32_t v = (int32_t)((uint32_t)q + (uint32_t)yz);
-    if (ep.narrow == kSaturate) {
-      const int32_t lo = ep.y_unsigned ? 0 : -128;
-      const int32_t hi = ep.y_unsigned ? 255 : 127;
-      v = v < lo ? lo : (v > hi ? hi : v);
-    }
-    ((uint8_t *)ep.out)[o] = (uint8_t)(v & 0xFF);
+    ((uint8_t *)ep.out)[o] = (uint8_t)requantize(ep, y, sj, yz);
   }
 }
 

@@ -1580,6 +1580,7 @@ int gemm_quantizes_rows(int64_t M, int64_t K, int64_t N, const void *x) {
 }
 
 const char *last_gemm_kernel() { return t_last_kernel; }
+void note_gemm_kernel(const char *name) { t_last_kernel = name; }
 
 namespace {
 // onnx.Gelu (gelu_f32) in place over n floats, for the kernels that do not

@@ -164,8 +164,29 @@ struct GemmArgs {
 };
 
 hipError_t launch_gemm(hipStream_t s, const GemmArgs &g);
-// Name of the kernel the calling thread's last launch_gemm chose.
+// Name of the kernel the calling thread's last launch_gemm or
+// launch_gemm_batched chose.
 const char *last_gemm_kernel();
+void note_gemm_kernel(const char *name);
+
+// A batched product in one launch, the right-hand side as it lies in memory
+// (gemm_batched.hip): GemmArgs describes one batch entry (Bp and colsum are not
+// read; kEpiI32 or kEpiQ8), GemmBatch which matrices the entries multiply.
+struct GemmBatch {
+  static constexpr int kDims = 4;
+  const void *B;        // [b_mats, K, N] row-major
+  int64_t count;        // batch entries; out is [count, M, N]
+  int64_t dims[kDims];  // their dimensions, outermost first; product = count
+  int64_t a_step[kDims], b_step[kDims]; // matrices of A / B from one index of
+                        // a dimension to the next (0: broadcast)
+  int64_t a_mats, b_mats;
+  bool a_zp_per_matrix, b_zp_per_matrix; // [a_mats, M] / [b_mats, N]
+};
+bool gemm_batched_ok(const GemmArgs &g, const GemmBatch &b);
+// Whether it is the faster way, against packing each matrix of B and
+// multiplying entry by entry with the kernels of launch_gemm.
+bool gemm_batched_pays(const GemmArgs &g);
+hipError_t launch_gemm_batched(hipStream_t s, const GemmArgs &g, const GemmBatch &b);
 
 // Whether launch_gemm can take an f32 activation of this shape in GemmArgs::X:
 // 0 no; 1 yes, every block quantizes the rows for itself; 2 yes, the blocks

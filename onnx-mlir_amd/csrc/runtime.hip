@@ -1071,13 +1071,29 @@ bool axis_split(const View &x, int64_t scale_numel, int64_t axis,
 //    [.., M, K] are folded into M; one product.
 //  - B [.., K, N] with leading (batch) dimensions: A is [.., M, K] (or [K],
 //    taken as [1, K]), the batch dimensions of A and B are broadcast against
-//    each other, and there is one M x K x N product per batch entry:
-//    a_batch[i] / b_batch[i] are the matrices of A / B that entry i multiplies.
+//    each other, and there is one M x K x N product per batch entry.  The batch
+//    dimensions are kept merged where A and B both step through two of them as
+//    through one (dimensions of 1 are dropped): entry (i0, i1, ..) multiplies
+//    matrix sum(i * a_step) of A and sum(i * b_step) of B.
 struct MatmulShape {
   int64_t M = 0, K = 0, N = 0;
   int64_t batches = 1;
   int64_t a_mats = 1, b_mats = 1; // matrices held by A and by B
-  std::vector<int64_t> a_batch, b_batch;
+  struct Dim {
+    int64_t size, a_step, b_step;
+  };
+  std::vector<Dim> batch; // outermost first
+
+  // The matrices that entry e multiplies.
+  void matrices(int64_t e, int64_t &ai, int64_t &bi) const {
+    ai = bi = 0;
+    for (size_t d = batch.size(); d-- > 0;) {
+      const int64_t c = e % batch[d].size;
+      e /= batch[d].size;
+      ai += c * batch[d].a_step;
+      bi += c * batch[d].b_step;
+    }
+  }
 };
 
 bool matmul_dims(const View &a, const View &b, const char *op, bool allow_batched_b,
@@ -1098,8 +1114,6 @@ bool matmul_dims(const View &a, const View &b, const char *op, bool allow_batche
     sh.M = 1;
     for (int64_t i = 0; i + 1 < a.rank; ++i)
       sh.M *= a.shape[i];
-    sh.a_batch.assign(1, 0);
-    sh.b_batch.assign(1, 0);
     return true;
   }
   if (!allow_batched_b) {
@@ -1109,8 +1123,8 @@ bool matmul_dims(const View &a, const View &b, const char *op, bool allow_batche
   sh.M = a.rank >= 2 ? a.shape[a.rank - 2] : 1;
   const int64_t ar = a.rank >= 2 ? a.rank - 2 : 0, br = b.rank - 2;
   const int64_t r = ar > br ? ar : br;
-  std::vector<int64_t> dims(r), astr(r, 0), bstr(r, 0);
   int64_t am = 1, bm = 1;
+  sh.batches = 1;
   for (int64_t i = r - 1; i >= 0; --i) { // right-aligned, as numpy broadcasts
     const int64_t ai = i - (r - ar), bi = i - (r - br);
     const int64_t ad = ai >= 0 ? a.shape[ai] : 1, bd = bi >= 0 ? b.shape[bi] : 1;
@@ -1119,33 +1133,28 @@ bool matmul_dims(const View &a, const View &b, const char *op, bool allow_batche
           (long long)ad, (long long)bd);
       return false;
     }
-    dims[i] = ad == 1 ? bd : ad;
-    astr[i] = ad == 1 ? 0 : am;
-    bstr[i] = bd == 1 ? 0 : bm;
+    const MatmulShape::Dim d = {
+        ad == 1 ? bd : ad, ad == 1 ? 0 : am, bd == 1 ? 0 : bm};
     am *= ad;
     bm *= bd;
+    sh.batches *= d.size;
+    if (d.size == 1)
+      continue;
+    if (!sh.batch.empty()) {
+      MatmulShape::Dim &in = sh.batch.back(); // the next dimension inwards
+      if (d.a_step == in.a_step * in.size && d.b_step == in.b_step * in.size) {
+        in.size *= d.size;
+        continue;
+      }
+    }
+    sh.batch.push_back(d);
   }
+  std::reverse(sh.batch.begin(), sh.batch.end());
   sh.a_mats = am;
   sh.b_mats = bm;
-  sh.batches = 1;
-  for (int64_t d : dims)
-    sh.batches *= d;
   if (sh.batches > ((int64_t)1 << 20)) {
     fail(EINVAL, "%s: more than 2^20 batch entries", op);
     return false;
-  }
-  sh.a_batch.resize((size_t)sh.batches);
-  sh.b_batch.resize((size_t)sh.batches);
-  for (int64_t e = 0; e < sh.batches; ++e) {
-    int64_t rest = e, ai = 0, bi = 0;
-    for (int64_t i = r - 1; i >= 0; --i) {
-      const int64_t c = rest % dims[i];
-      rest /= dims[i];
-      ai += c * astr[i];
-      bi += c * bstr[i];
-    }
-    sh.a_batch[(size_t)e] = ai;
-    sh.b_batch[(size_t)e] = bi;
   }
   return true;
 }
@@ -1406,30 +1415,21 @@ void run_matmul(const MatmulSpec &sp) {
   g.K = K;
   g.N = N;
   const int32_t *colsum = nullptr;
-  // One right-hand side: packed once (cached for a constant).  Batched: the
-  // matrices of B are packed one after the other into buffers of this call.
+  // One right-hand side: packed once (cached for a constant).  Batched: as it
+  // lies in memory, or packed matrix by matrix below.
   const int64_t Kpad = round_up(K > 0 ? K : 1, kGemmBK);
   const int64_t Npad = round_up(N, kGemmBN);
   const size_t bp_bytes = (size_t)Kpad * Npad;
   int8_t *bp_all = nullptr;
   int32_t *cs_all = nullptr;
+  const uint8_t *db = nullptr;
   if (b.rank <= 2) {
     if (!packed_b(call, b, K, N, g.Bp, colsum)) {
       call.finish();
       return;
     }
   } else {
-    const uint8_t *db = (const uint8_t *)call.in(b);
-    bp_all = (int8_t *)call.temp(bp_bytes * (size_t)sh.b_mats);
-    cs_all = (int32_t *)call.temp((size_t)Npad * 4 * (size_t)sh.b_mats);
-    for (int64_t i = 0; call.ok && i < sh.b_mats; ++i)
-      call.check(launch_pack_b(call.c.stream, db + (size_t)i * K * N, b_uns, K, N,
-                     bp_all + (size_t)i * bp_bytes, cs_all + (size_t)i * Npad),
-          "pack B");
-    if (!call.ok) {
-      call.finish();
-      return;
-    }
+    db = (const uint8_t *)call.in(b);
   }
   g.colsum = colsum;
   const uint8_t *d_azp = sp.a_zp ? (const uint8_t *)call.in(azp) : nullptr;
@@ -1478,12 +1478,43 @@ void run_matmul(const MatmulSpec &sp) {
     call.finish();
     return;
   }
-  // One product per batch entry, queued one after the other.
+  if (call.ok && sh.batch.size() <= (size_t)GemmBatch::kDims) {
+    GemmBatch gb = {};
+    gb.B = db;
+    gb.count = sh.batches;
+    const size_t lead = GemmBatch::kDims - sh.batch.size();
+    for (size_t d = 0; d < (size_t)GemmBatch::kDims; ++d) {
+      gb.dims[d] = d < lead ? 1 : sh.batch[d - lead].size;
+      gb.a_step[d] = d < lead ? 0 : sh.batch[d - lead].a_step;
+      gb.b_step[d] = d < lead ? 0 : sh.batch[d - lead].b_step;
+    }
+    gb.a_mats = sh.a_mats;
+    gb.b_mats = sh.b_mats;
+    // zero points given per matrix ([.., M, 1] / [.., 1, N]) move with it
+    gb.a_zp_per_matrix = azl > M;
+    gb.b_zp_per_matrix = bzl > N;
+    if (gemm_batched_ok(g, gb) && gemm_batched_pays(g)) {
+      call.check(launch_gemm_batched(call.c.stream, g, gb), sp.op);
+      call.finish();
+      return;
+    }
+  }
+  // The matrices of B packed one after the other into buffers of this call,
+  // then one product per batch entry, queued one after the other.
+  if (call.ok) {
+    bp_all = (int8_t *)call.temp(bp_bytes * (size_t)sh.b_mats);
+    cs_all = (int32_t *)call.temp((size_t)Npad * 4 * (size_t)sh.b_mats);
+  }
+  for (int64_t i = 0; call.ok && i < sh.b_mats; ++i)
+    call.check(launch_pack_b(call.c.stream, db + (size_t)i * K * N, b_uns, K, N,
+                   bp_all + (size_t)i * bp_bytes, cs_all + (size_t)i * Npad),
+        "pack B");
   const uint8_t *d_a = (const uint8_t *)g.A;
   char *d_y = (char *)g.out;
   const size_t y_es = sp.epi == kEpiQ8 ? 1 : 4;
   for (int64_t e = 0; call.ok && e < sh.batches; ++e) {
-    const int64_t ai = sh.a_batch[(size_t)e], bi = sh.b_batch[(size_t)e];
+    int64_t ai, bi;
+    sh.matrices(e, ai, bi);
     GemmArgs ge = g;
     ge.A = d_a + (size_t)ai * M * K;
     ge.Bp = bp_all + (size_t)bi * bp_bytes;

@@ -296,3 +296,36 @@ def test_limits_with_nan_infinities_and_the_other_quotient(rt, oracle):
         rt.set_quant_mode(0)
     with pytest.raises(rt.RuntimeError_, match="limits"):
         rt.DynQuantMatMulDequantLimits(h, W2, None, s2, x_limits=np.zeros(3, np.float32))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 16, 4), (5, 1, 9), (63, 15, 63), (64, 64, 64), (65, 65, 65), (64, 16, 128),
+                                   (66, 48, 68), (130, 129, 127), (33, 200, 129), (128, 64, 132), (200, 320, 256)])
+@pytest.mark.parametrize("adt,bdt", [(np.uint8, np.uint8), (np.int8, np.int8), (np.uint8, np.int8)])
+def test_batched_kernel_edges(rt, oracle, M, K, N, adt, bdt):
+    """k_gemm_i8_batched at the edges of its 64-row and 64- / 128-column tiles,
+    one to five K steps, aligned and unaligned rows, zero points of every form,
+    int32 and requantized results, and batch dimensions that broadcast against
+    each other on either side."""
+    rng = np.random.default_rng(M * 1000 + K * 10 + N)
+
+    def rand(dt, shape):
+        i = np.iinfo(dt)
+        return rng.integers(i.min, i.max + 1, shape).astype(dt)
+
+    for alead, blead in (((2, 3), (2, 3)), ((2, 1), (3,)), ((1,), (4,)), ((2, 1, 3), (2, 2, 1))):
+        A, B = rand(adt, alead + (M, K)), rand(bdt, blead + (K, N))
+        forms = ((rand(adt, ()), rand(bdt, ())), (None, None), (rand(adt, alead + (M, 1)), rand(bdt, blead + (1, N))))
+        for az, bz in forms:
+            got = rt.MatMulInteger(A, B, az, bz)
+            a64 = A.astype(np.int64) - (0 if az is None else az.astype(np.int64))
+            b64 = B.astype(np.int64) - (0 if bz is None else bz.astype(np.int64))
+            assert np.array_equal(got, np.matmul(a64, b64)), (alead, blead, az is None)
+        if A.size >= 16:  # (an A below one 16-byte load goes matrix by matrix)
+            assert rt.last_gemm_kernel() == "k_gemm_i8_batched"
+    s, ydt = np.float32(0.01), adt
+    az, bz, yz = rand(adt, ()), rand(bdt, ()), rand(ydt, ())
+    A, B = rand(adt, (3, M, K)), rand(bdt, (3, K, N))
+    for mode in (rt.WRAP, rt.SATURATE):
+        got = rt.QLinearMatMul(A, s, az, B, s, bz, np.float32(0.5), yz, mode)
+        want = oracle.qlinear_matmul(A, s, az, B, s, bz, np.float32(0.5), yz, mode)
+        assert np.array_equal(got, want)
