@@ -141,9 +141,11 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
   const int cg = tid % CG, kg = tid / CG;
   const bool b_col = n0 + cg * 4 < N;
 
-  // ALIGNED: buffer loads, a lane offset that never changes and the K step as
+  // ALIGNED: buffer loads, lane offsets that never change and the K step as
   // scalar offset; what lies outside the matrices (rows past M and columns past
-  // N are sent there) reads as 0.  Otherwise global loads at byte addresses.
+  // N are sent there) reads as 0.  The scalar offset itself stays inside: the
+  // hardware compares the lane offset with the descriptor's size minus it,
+  // unsigned.  Otherwise global loads at byte addresses.
   constexpr int kOutside = 0x7FFFFFFF;
   const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
       (void *)Ae, 0, M * K, 0x00020000);
@@ -151,7 +153,11 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
       (void *)Be, 0, K * N, 0x00020000);
   const int a_off = (m0 + ar) * K + ac * 16;
   const int b_off = kg * KPT * N + n0 + cg * 4;
-  const int a_voff = a_row ? a_off : kOutside, b_voff = b_col ? b_off : kOutside;
+  const int a_voff = a_row ? a_off : kOutside;
+  int b_voff[KPT];
+#pragma unroll
+  for (int i = 0; i < KPT; ++i)
+    b_voff[i] = b_col ? b_off + i * N : kOutside;
   const int64_t a_left = bp.a_total - ai * M * K, b_left = bp.b_total - bi * K * N;
   const int a_end = a_left < kOutside ? (int)a_left : kOutside;
   const int b_end = b_left < kOutside ? (int)b_left : kOutside;
@@ -161,15 +167,16 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
   // the time of two to arrive.
   v4i ra0, ra1;
   uint32_t rb0[KPT], rb1[KPT];
-  // (Steps past the end load nothing, or the first bytes of A and B, which
-  // nobody uses: with no branch around a load its wait is exact.)
-  auto load = [&](int k0, v4i &ra, uint32_t(&rb)[KPT]) {
+  // (Steps past the end load the first step again, which nobody uses: with no
+  // branch around a load its wait is exact.)
+  auto load = [&](int step, v4i &ra, uint32_t(&rb)[KPT]) {
+    const int k0 = step < K ? step : 0;
     if (ALIGNED) {
       ra = __builtin_amdgcn_raw_buffer_load_b128(arsrc, a_voff, k0, 0);
 #pragma unroll
       for (int i = 0; i < KPT; ++i)
         rb[i] = __builtin_amdgcn_raw_buffer_load_b32(
-            brsrc, b_voff, (k0 + i) * N, 0);
+            brsrc, b_voff[i], k0 * N, 0);
     } else {
       ra = load16_any(Ae, a_row && k0 + ac * 16 < K ? a_off + k0 : 0, a_end);
 #pragma unroll
@@ -343,11 +350,11 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
             (uint32_t)db * ((uint32_t)s_rowsum[first + 4 * lh] + (uint32_t)K * da);
         if (EPI == kEpiI32)
           __builtin_amdgcn_raw_buffer_store_b32(
-              (int)y, rsrc, voff, first * N * ES, decltype(aux)::value);
+              (int)y, rsrc, voff + first * N * ES, 0, decltype(aux)::value);
         else
           __builtin_amdgcn_raw_buffer_store_b8(
-              (unsigned char)requantize(ep, y, sj, yz), rsrc, voff,
-              first * N * ES, decltype(aux)::value);
+              (unsigned char)requantize(ep, y, sj, yz), rsrc,
+              voff + first * N * ES, 0, decltype(aux)::value);
       }
     }
   };

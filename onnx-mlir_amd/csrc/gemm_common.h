@@ -245,6 +245,14 @@ bool wreg_pays(int64_t M, int64_t N);
 hipError_t launch_gemm_wreg(hipStream_t st, const GemmArgs &g,
     const EpiParams &ep, int a_mode);
 
+// k_gemm_i8_skinny (gemm_skinny.hip): up to 64 rows.  skinny_quantizes_rows:
+// whether it takes the f32 activation of a fused layer (GemmArgs::X) and
+// quantizes it in every block.
+bool skinny_ok(int64_t M, int64_t K, const void *a);
+bool skinny_quantizes_rows(int64_t M, int64_t K, const void *x);
+hipError_t launch_gemm_skinny(hipStream_t st, const GemmArgs &g,
+    const EpiParams &ep, int a_mode);
+
 // k_gemm_i8_flight (gemm_flight.hip): problems that one round of blocks covers,
 // K a multiple of 256 up to 1024.  The _dq forms take the f32 activation of a dynamically
 // quantized layer (GemmArgs::X) and quantize it in the same launch; the launch

@@ -30,7 +30,8 @@
 //                        into a ring of three LDS stages; up to one tile per CU
 //   k_gemm_i8            tiles staged through registers, LDS double buffered;
 //                        also the general path: any K, any alignment of A
-//   k_gemm_i8_skinny_bp  M <= 32: weight streaming, K split over the waves
+// and, in files of their own, k_gemm_i8_skinny (M <= 64, weight streaming),
+// k_gemm_i8_flight, k_gemm_i8_wreg and k_gemm_i8_batched.
 // A tiles in LDS have 64-byte rows whose 16-byte chunk index is XOR-swizzled
 // with bits 2..3 of the row (bank-conflict free writes and operand reads); Bp
 // tiles in LDS keep their global order.
@@ -893,337 +894,6 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_bs(
       acc, rsp, m0, ncol0, M, N, K, ep);
 }
 
-// ---- skinny GEMM (M <= 64): weight streaming -------------------------------
-// With few rows the product is bound by reading the weights once (32 rows
-// per MFMA row tile, TR = 1 or 2 tiles against the same Bp operands), so
-// the kernel is organised around keeping many KiB of Bp in flight per CU and
-// nothing else: a block owns one 32-column tile, whose operands for all of K
-// are one contiguous run of Bp (2 KiB per K step); its 8 waves take
-// contiguous slices of K, and every Bp load is a fully coalesced KiB.  A (at
-// most 32 rows, zero rows above M) is read from L2 in operand layout.  The
-// eight partial 32x32 results are summed through LDS.  No LDS staging, no
-// barrier in the K loop.
-//
-// DQ: the activation arrives as f32 X[M,K] (at most kSkinnyDqBytes elements)
-// and every block quantizes it itself, exactly as DynamicQuantizeLinear
-// would: minimum and maximum over all of X, scale and zero point from them,
-// the 8-bit values minus 128 into LDS, from where the K loop takes its A
-// operands.  That is 16 KiB of reads from L2 per block for one row of 4096,
-// in place of a launch of its own in front of this one.  Whole layer with
-// 4096 x 11008 weights, this kernel against DynamicQuantizeLinear (5.4 us by
-// itself at these sizes) in front of it: 1 row 8.9 / 10.6 us, 4 rows 10.7 /
-// 12.9, 5 rows 11.7 / 13.5, 6 rows 12.9 / 13.6, 8 rows 15.2 / 13.9: the cost
-// grows with every row that every block reads.  With the four-instruction
-// quotient the same comparison reads 4 rows 9.7 / 12.4, 6 rows 10.4 / 12.5,
-// 8 rows 11.2 / 12.6, 16 rows 14 / 13.2: the limit is eight rows of 4096.
-// Requesting the first Bp operands before the rows are quantized did
-// not shorten it, and neither did rows K + 16 bytes apart in LDS (no two
-// lanes' 16-byte reads in the same banks): 4 rows 10.7 -> 11.7 us, 8 rows
-// 15.2 -> 17.1 us with the index arithmetic that takes.
-//
-// Tried and dropped: one launch in which the first blocks of the grid quantize
-// X between them (8192 elements each), publish the result through global
-// memory, and every block waits for it with all its weights already
-// requested.  While the 45 MB weight stream saturates HBM every dependent
-// memory step of that chain -- the load of X, the exchange of minima and
-// maxima, the acknowledgement of the quantized rows, the "done" exchange, the
-// copy of the rows into LDS, the polling wave's own weights -- takes 1.2 to
-// 2 us: 16 rows 15.0 us (rows seen at 8.0 us, K loop over at 11.4 us), 4 rows
-// 12.5 us, 1 row 11.8 us, all slower than what they would replace.
-constexpr int kSkinnyDqBytes = 32768;
-// Whether k_gemm_i8_skinny_bp can quantize this activation itself (DQ).
-bool skinny_quantizes_rows(int64_t M, int64_t K, const void *x) {
-  return M >= 1 && M <= 32 && K > 0 && K % 16 == 0 &&
-         M * K <= kSkinnyDqBytes && ((((uintptr_t)x) & 15) == 0);
-}
-
-// DQ: 0, or the float4 of X a thread takes when the block quantizes X itself
-// (4, 8 or 16: up to 8192, 16384 or kSkinnyDqBytes elements).
-template <int A_MODE, int EPI, int DQ, int TR, bool STG>
-__global__ __launch_bounds__(512) void k_gemm_i8_skinny_bp(
-    const uint8_t *__restrict__ A, const float *__restrict__ X,
-    const int8_t *__restrict__ Bp, int M, int N, int K, int Kpad,
-    EpiParams ep) {
-  // TR row tiles of 32 (M <= 32 * TR); with two of them a wave keeps half as
-  // many K steps in flight, to stay within the same registers.
-  constexpr int WAVES = 8, U = (TR == 1) ? 4 : 2;
-  static_assert(!DQ || A_MODE == 2, "quantized rows are stored minus 128");
-  static_assert(TR == 1 || (TR == 2 && !DQ), "row tiles");
-  static_assert(!(DQ && STG), "quantized rows are in LDS already");
-  // STG: A rows from global memory pass through a piece of LDS private to
-  // the wave: a load instruction takes whole rows of the batch of U steps (CPR
-  // 16-byte chunks each, so every cache line it touches is used completely),
-  // the MFMA operands -- 32 bytes of each of 32 rows -- are read back from
-  // there.  Loading the operands straight from global memory touches 32
-  // lines per instruction for 32 bytes each, and the eight waves' lines do
-  // not stay in the CU's cache until their other three quarters are wanted
-  // (K=4096 N=11008, 32 rows: 12.6 us that way, 9.1 us with loads of whole
-  // lines).  Rows lie CPR * 16 + 16 bytes apart in LDS, which spreads the
-  // rows of one operand read over the banks.  Up to 4 rows the direct loads
-  // are kept: the lanes of the rows that are not there fetch nothing, and
-  // the way through LDS costs more than it saves (1 row 7.7 against 8.3 us,
-  // 4 rows 8.1 / 8.4, 16 rows 9.4 / 8.7, 32 rows 12.6 / 9.6).
-  constexpr int CPR = U * 4;
-  constexpr int kPitch = CPR * 16 + 16;
-  constexpr int kStageWave = 32 * TR * kPitch;
-  constexpr int kPartBytes = WAVES * 16 * 64 * 4;
-  constexpr int kLdsBytes = (STG && WAVES * kStageWave > kPartBytes)
-                                ? WAVES * kStageWave
-                                : kPartBytes;
-  // The staged rows, and the rows quantized here (DQ), share the memory of
-  // the partial sums, which are not written before every wave has left the
-  // K loop.
-  __shared__ __attribute__((aligned(16))) uint8_t lds_raw[kLdsBytes];
-  int32_t(*const part)[16][64] = (int32_t(*)[16][64])lds_raw;
-  __shared__ int32_t part_rs[WAVES][64];
-  static_assert(kPartBytes >= kSkinnyDqBytes, "quantized rows fit");
-  uint8_t *const aq = lds_raw;
-  __shared__ float s_lo[WAVES], s_hi[WAVES];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31;
-  const int lh = lane >> 5;
-  const int nt = blockIdx.x;
-
-  const int KT = Kpad / BK;
-  const int per = (KT + WAVES - 1) / WAVES;
-  const int kt_begin = wave * per;
-  const int kt_end = (kt_begin + per < KT) ? kt_begin + per : KT;
-
-  float dq_scale = 0.0f;
-  int32_t dq_zp = 0;
-  if (DQ) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    constexpr int NV = DQ > 0 ? DQ : 1; // float4 per thread
-    static_assert(DQ * 4 * WAVES * 64 <= kSkinnyDqBytes, "quantized rows fit");
-    const int nvec = (M * K) >> 2; // K % 16 == 0, M * K <= kSkinnyDqBytes
-    const f4 *__restrict__ x4 = (const f4 *)X;
-    f4 v[NV];
-    float lo = __builtin_inff(), hi = -__builtin_inff();
-    const float nan = __builtin_nanf(""); // neutral for minnum / maxnum
-#pragma unroll
-    for (int j = 0; j < NV; ++j) {
-      const int e = j * (WAVES * 64) + tid;
-      v[j] = e < nvec ? x4[e] : (f4){nan, nan, nan, nan};
-      lo = __builtin_fminf(__builtin_fminf(lo, v[j].x),
-          __builtin_fminf(__builtin_fminf(v[j].y, v[j].z), v[j].w));
-      hi = __builtin_fmaxf(__builtin_fmaxf(hi, v[j].x),
-          __builtin_fmaxf(__builtin_fmaxf(v[j].y, v[j].z), v[j].w));
-    }
-    if (ep.x_limits) { // (the same for every thread) known from the layer before
-      lo = ep.x_limits[0];
-      hi = ep.x_limits[1];
-    } else {
-      lo = wave_min(lo);
-      hi = wave_max(hi);
-      if (lane == 0) {
-        s_lo[wave] = lo;
-        s_hi[wave] = hi;
-      }
-      __syncthreads();
-      lo = s_lo[0];
-      hi = s_hi[0];
-#pragma unroll
-      for (int w = 1; w < WAVES; ++w) {
-        lo = __builtin_fminf(lo, s_lo[w]);
-        hi = __builtin_fmaxf(hi, s_hi[w]);
-      }
-    }
-    float zpf;
-    dynamic_params(lo, hi, dq_scale, zpf);
-    dq_zp = (int32_t)(uint32_t)zpf;
-    const float recip = 1.0f / dq_scale;
-    auto quantize = [&](auto fast_c) {
-      constexpr bool FAST = decltype(fast_c)::value;
-#pragma unroll
-      for (int j = 0; j < NV; ++j) {
-        const int e = j * (WAVES * 64) + tid;
-        if (e < nvec) {
-          const uint32_t q = quant_pack4<false, true, FAST>(v[j].x, v[j].y,
-              v[j].z, v[j].w, dq_scale, dq_scale, dq_scale, dq_scale, recip,
-              recip, recip, recip, zpf, zpf, zpf, zpf);
-          ((uint32_t *)aq)[e] = q ^ 0x80808080u;
-        }
-      }
-    };
-    if (scale_is_tame(dq_scale)) // the same for every thread
-      quantize(std::true_type{});
-    else
-      quantize(std::false_type{});
-    __syncthreads();
-  }
-
-  bool row_ok[TR];
-  const uint8_t *__restrict__ ap[TR];
-#pragma unroll
-  for (int t = 0; t < TR; ++t) {
-    row_ok[t] = t * 32 + l32 < M;
-    ap[t] = (DQ ? (const uint8_t *)aq : A) +
-            (int64_t)(row_ok[t] ? t * 32 + l32 : 0) * K;
-  }
-  const int8_t *__restrict__ bp = Bp + (int64_t)nt * KT * 2048 + lane * 16;
-  constexpr int kFill = (A_MODE == 1) ? (int)0x80808080 : 0;
-
-  v16i acc[TR];
-#pragma unroll
-  for (int t = 0; t < TR; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      acc[t][r] = 0;
-  const bool need_rs = ep.need_rowsum;
-  int32_t rsp[TR]; // this lane's share of rowsum(A') of row t*32 + lane % 32
-#pragma unroll
-  for (int t = 0; t < TR; ++t)
-    rsp[t] = 0;
-  for (int kt = kt_begin; kt < kt_end; kt += U) {
-    v4i a[TR][U][2], b[U][2];
-    constexpr int RPI = 64 / CPR;       // rows per load instruction
-    constexpr int NLD = 32 * TR / RPI;  // load instructions per batch
-    v4i ar[NLD];
-    if (STG) {
-      const int ld_chunk = lane % CPR;
-      const int step = kt + ld_chunk / 4;
-      const int k0 = step * BK + (ld_chunk & 3) * 16;
-      const bool k_in = step < kt_end && k0 < K; // K % 16 == 0: a chunk is in or out
-#pragma unroll
-      for (int j = 0; j < NLD; ++j) {
-        const int row = j * RPI + lane / CPR;
-        const bool in = k_in && row < M;
-        ar[j] = *(const v4i *)(A + (in ? (int64_t)row * K + k0 : 0));
-        if (!in)
-          ar[j] = (v4i){kFill, kFill, kFill, kFill};
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      // steps past this wave's slice reload its last step and are discarded
-      const int s = (kt + u < kt_end) ? kt + u : kt_end - 1;
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) {
-        if (!STG) {
-          const int k0 = s * BK + (sub * 2 + lh) * 16;
-#pragma unroll
-          for (int t = 0; t < TR; ++t) {
-            const bool in = row_ok[t] && k0 < K;
-            a[t][u][sub] = *(const v4i *)(ap[t] + (in ? k0 : 0));
-            if (!in)
-              a[t][u][sub] = (v4i){kFill, kFill, kFill, kFill};
-          }
-        }
-        b[u][sub] = *(const v4i *)(bp + (int64_t)s * 2048 + sub * 1024);
-      }
-    }
-    if (STG) {
-      // Through the wave's own piece of LDS into operand order.  The LDS
-      // instructions of a wave execute in order; the fences keep the compiler
-      // from moving the reads above the writes of other lanes, and the next
-      // batch's writes above these reads.
-      uint8_t *const stg = lds_raw + wave * kStageWave;
-#pragma unroll
-      for (int j = 0; j < NLD; ++j)
-        *(v4i *)(stg + (j * RPI + lane / CPR) * kPitch + (lane % CPR) * 16) =
-            ar[j];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
-#pragma unroll
-          for (int t = 0; t < TR; ++t)
-            a[t][u][sub] = *(const v4i *)(stg + (t * 32 + l32) * kPitch +
-                                          (u * 4 + sub * 2 + lh) * 16);
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (kt + u < kt_end) {
-#pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-#pragma unroll
-          for (int t = 0; t < TR; ++t) {
-            v4i av = a[t][u][sub];
-            if (A_MODE == 1)
-              av ^= (v4i){(int)0x80808080, (int)0x80808080, (int)0x80808080,
-                  (int)0x80808080};
-            if (need_rs)
-              rsp[t] += frag_rowsum(av);
-            acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-                av, b[u][sub], acc[t], 0, 0, 0);
-          }
-        }
-      }
-    }
-  }
-  __syncthreads(); // every wave is done reading its rows from LDS
-
-  // 32x32 accumulator layout: lane holds column (lane & 31); register r holds
-  // row 8*(r/4) + 4*(lane/32) + r%4.  Thread t finishes elements (r, lane)
-  // with r = t / 64 and r + 8.
-  constexpr bool A_OFF = (A_MODE != 0);
-  const int32_t oa = A_OFF ? 128 : 0;
-  const int32_t ob = ep.b_unsigned ? 128 : 0;
-  const int n = nt * 32 + l32;
-  const bool col_ok = n < N;
-  const int nc = col_ok ? n : 0; // columns past N: computed on column 0, not stored
-  int32_t db = ob;
-  if (ep.b_zp_len > 0)
-    db = ob - load_zp_i32(ep.b_zp, ep.b_unsigned, ep.b_zp_len > 1 ? nc : 0);
-  const int32_t cs = ep.colsum[nc];
-  float sj = 0.0f, bj = -0.0f;
-  int32_t yz = 0;
-  if (EPI == kEpiF32 && ep.bias != nullptr)
-    bj = ep.bias[ep.bias_len > 1 ? nc : 0];
-  if (EPI != kEpiI32) {
-    sj = (DQ ? dq_scale : ep.a_scale[0]) *
-         ep.b_scale[ep.b_scale_len == 1 ? 0 : nc];
-    if (EPI == kEpiQ8) {
-      sj = sj / ep.y_scale[0];
-      yz = load_zp_i32(ep.y_zp, ep.y_unsigned, 0);
-    }
-  }
-  // One row tile at a time through the partial-sum buffers.
-#pragma unroll
-  for (int t = 0; t < TR; ++t) {
-    if (t > 0)
-      __syncthreads(); // the sums of the tile before have been read
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-      part[wave][r][lane] = acc[t][r];
-    part_rs[wave][lane] = rsp[t];
-    __syncthreads();
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int r = (tid >> 6) + h * 8;
-      const int ml = 8 * (r >> 2) + 4 * lh + (r & 3); // row within the tile
-      const int m = t * 32 + ml;
-      if (m >= M || !col_ok)
-        continue;
-      uint32_t y = 0;
-#pragma unroll
-      for (int w = 0; w < WAVES; ++w)
-        y += (uint32_t)part[w][r][lane];
-      int32_t da = oa, rs = 0;
-      if (DQ)
-        da = oa - dq_zp;
-      else if (ep.a_zp_len > 0)
-        da = oa - load_zp_i32(ep.a_zp, A_OFF, ep.a_zp_len > 1 ? m : 0);
-      if (need_rs) {
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w)
-          rs += part_rs[w][ml] + part_rs[w][ml + 32];
-      }
-      y += (uint32_t)da * (uint32_t)cs;
-      y += (uint32_t)db * (uint32_t)rs;
-      y += (uint32_t)K * (uint32_t)da * (uint32_t)db;
-      store_one<EPI>(ep, (int64_t)m * N + n, y, sj, yz, bj);
-    }
-  }
-}
-
 // ---- pack B ---------------------------------------------------------------
 // One block transposes a 64(k) x 64(n) tile of B [K,N] through LDS, writes it
 // in MFMA operand order (see the top of the file) and adds the tile's column
@@ -1381,40 +1051,15 @@ hipError_t gemm_launch_cfg(
       t_limits_written = ep.limits.out != nullptr; // and reduces their limits
       return launch_gemm_flight_dq(st, g, ep, *g.dql);
     }
-    if constexpr (A_MODE == 2) {
-      t_last_kernel = "k_gemm_i8_skinny_bp (rows quantized in the kernel)";
-      const dim3 grid((unsigned)((g.N + 31) / 32));
-      const int64_t elements = g.M * g.K;
-      if (elements <= 4 * 4 * 512)
-        k_gemm_i8_skinny_bp<2, EPI, 4, 1, false>
-            <<<grid, 512, 0, st>>>(nullptr, g.X, g.Bp, M, N, K, Kpad, ep);
-      else if (elements <= 8 * 4 * 512)
-        k_gemm_i8_skinny_bp<2, EPI, 8, 1, false>
-            <<<grid, 512, 0, st>>>(nullptr, g.X, g.Bp, M, N, K, Kpad, ep);
-      else
-        k_gemm_i8_skinny_bp<2, EPI, 16, 1, false>
-            <<<grid, 512, 0, st>>>(nullptr, g.X, g.Bp, M, N, K, Kpad, ep);
-    }
-    return hipGetLastError();
+    t_last_kernel = "k_gemm_i8_skinny (rows quantized in the kernel)";
+    return launch_gemm_skinny(st, g, ep, A_MODE);
   }
   // Up to 64 rows the weight-streaming kernel is ahead of every tile kernel
   // (K=4096 N=11008: M=33 11.6 against 17.2 us, M=48 12.3 / 17.7; K=11008
   // N=4096 M=64: 15.0 / 37.7; K=768 N=3072 M=64: 4.2 / 6.0).
-  const bool skinny_rows = g.M <= 64;
-  if (skinny_rows && g.K > 0 && g.K % 16 == 0 && ((((uintptr_t)g.A) & 15) == 0) &&
-      !(force && force[0])) {
-    const dim3 grid((unsigned)((g.N + 31) / 32));
-    t_last_kernel = "k_gemm_i8_skinny_bp";
-    if (g.M <= 4)
-      k_gemm_i8_skinny_bp<A_MODE, EPI, 0, 1, false>
-          <<<grid, 512, 0, st>>>(A, nullptr, g.Bp, M, N, K, Kpad, ep);
-    else if (g.M <= 32)
-      k_gemm_i8_skinny_bp<A_MODE, EPI, 0, 1, true>
-          <<<grid, 512, 0, st>>>(A, nullptr, g.Bp, M, N, K, Kpad, ep);
-    else
-      k_gemm_i8_skinny_bp<A_MODE, EPI, 0, 2, true>
-          <<<grid, 512, 0, st>>>(A, nullptr, g.Bp, M, N, K, Kpad, ep);
-    return hipGetLastError();
+  if (skinny_ok(g.M, g.K, g.A) && !(force && force[0])) {
+    t_last_kernel = "k_gemm_i8_skinny";
+    return launch_gemm_skinny(st, g, ep, A_MODE);
   }
   const int tiles_m = (int)((g.M + 127) / 128);
   const int tiles_n128 = (int)((g.N + 127) / 128);

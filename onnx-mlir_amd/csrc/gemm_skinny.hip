@@ -1,0 +1,522 @@
+// int8 GEMM for few rows (M <= 64): weight streaming.  What is computed, and
+// the layout of Bp, are described at the top of gemm_kernels.hip.
+//
+// Bound: reading the weights once.  K=4096 N=11008 is 45 MB: 6.4 us at the
+// 7.1 TB/s a read-only sweep reaches, plus about 2 us of launch.
+//
+// Split: a block owns 16 columns (or 32), its 8 waves take contiguous slices of
+// K and add their partial sums up in LDS; no barrier in the K loop.  Sixteen
+// columns, on v_mfma_i32_16x16x64_i8, because blocks are what the device is
+// short of: K=11008 N=4096 gives 256 blocks of 16 columns against 128 of 32, and
+// K=4096 N=11008 fills 256 CUs to 2.7 blocks each instead of 1.3.  A wave
+// requests a batch of two K steps, waits for it and multiplies; what hides the
+// wait is the other waves of the CU (up to 32), and registers are kept for them:
+// batches of four steps, or the next batch requested before the wait, leave room
+// for fewer and are slower (1 row, K=4096 N=11008: 8.3 us; four steps 9.1, a
+// second batch on its way 9.3, both 10.3; 16 waves a block 10.7).  Only up to 4
+// rows that arrive quantized are batches of four ahead (9.2 / 9.6 us).
+// Streaming (nontemporal) loads of the weights: 10.6 against 10.3 us.
+// The epilogue's parameters are requested first and without branches (a wait
+// for a zero point in front of the first weights cost 0.5 us).
+// Against one 32-column tile per block, four steps a batch and parameters
+// loaded behind the K loop (whole fused layer, K=4096 N=11008): 1 row 10.9 -> 8.3
+// us, 4 rows 11.5 -> 9.5, 8 rows 13.0 -> 11.5, 16 rows 14.9 -> 13.7, 64 rows
+// 19.2 -> 18.1; K=11008 N=4096: 1 row 11.6 -> 9.5, 16 rows 15.8 -> 14.3; 24 rows of
+// 1024, N=1024: 6.8 -> 5.6.
+//
+// DQ: the activation arrives as f32 X[M,K] (at most kSkinnyDqBytes elements) and
+// every block quantizes it itself, exactly as DynamicQuantizeLinear would:
+// minimum and maximum over all of X, scale and zero point from them, the 8-bit
+// values minus 128 into LDS, from where the K loop takes its A operands; the
+// first weights are requested before that starts.  Up to 32 Ki elements that
+// beats a launch of its own in front (8 rows of 4096: 11.2 us against 12.6; 16
+// rows 14 against 13).
+//
+// Tried and dropped: one launch in which the first blocks of the grid quantize
+// X between them and every block waits for them with its weights already
+// requested.  While the weight stream saturates HBM every dependent memory step
+// of that chain takes 1.2 to 2 us: 16 rows 15.0 us, 4 rows 12.5, 1 row 11.8.
+#include "gemm_common.h"
+#include "gemm_epilogue.h"
+
+namespace om {
+namespace gemm {
+
+namespace {
+
+constexpr int WAVES = 8;
+constexpr int kSkinnyDqBytes = 32768;
+
+// RT row tiles and CT column tiles of T x T, T = 16 or 32 (M <= T * RT).
+// DQ: 0, or the float4 of X a thread takes when the block quantizes X itself.
+// STG: A rows from global memory pass through a piece of LDS private to the
+// wave: a load instruction takes whole rows of the batch (CPR 16-byte chunks
+// each, so every cache line it touches is used completely), the MFMA operands
+// -- 64 bytes of each of 16 rows -- are read back from there, rows CPR * 16 + 16
+// bytes apart to spread them over the banks.  Up to 4 rows the operands are
+// loaded directly: the lanes of the rows that are not there fetch nothing.
+template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG>
+__global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
+    const uint8_t *__restrict__ A, const float *__restrict__ X,
+    const int8_t *__restrict__ Bp, int M, int N, int K, int Kpad,
+    EpiParams ep) {
+  static_assert(!DQ || (A_MODE == 2 && !STG), "quantized rows");
+  static_assert((T == 16 && CT <= 2) || (T == 32 && CT == 1 && !DQ), "tiles");
+  constexpr int U = !DQ && !STG ? 4 : 2;    // K steps of a batch
+  constexpr int CPR = U * 4;                // 16-byte chunks of a row and batch
+  constexpr int RPI = 64 / CPR;             // rows of a load instruction
+  constexpr int NLD = STG ? T * RT / RPI : 1;
+  constexpr int kPitch = CPR * 16 + 16;
+  constexpr int kStageWave = STG ? T * RT * kPitch : 0;
+  constexpr int REGS = T * T / 64; // accumulator registers of a tile
+  constexpr int SUBS = T / 16;     // MFMAs of a tile and K step
+  constexpr int SLOTS = RT * CT * REGS;
+  constexpr int kPartBytes = WAVES * SLOTS * 64 * 4;
+  // The staged rows, and the rows quantized here, share the memory of the
+  // partial sums, which are not written before every wave has left the K loop.
+  constexpr int kOwnBytes = DQ ? kSkinnyDqBytes : WAVES * kStageWave;
+  constexpr int kLdsBytes = kOwnBytes > kPartBytes ? kOwnBytes : kPartBytes;
+  __shared__ __attribute__((aligned(16))) uint8_t lds_raw[kLdsBytes];
+  int32_t(*const part)[SLOTS][64] = (int32_t(*)[SLOTS][64])lds_raw;
+  __shared__ int32_t rowsum[RT * T]; // of A', over all waves
+  __shared__ float s_lo[WAVES], s_hi[WAVES];
+  uint8_t *const aq = lds_raw;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & (T - 1); // row of A, column of B
+  const int lk = lane / T;       // and 16-byte chunk (of each 64 / SUBS bytes)
+  const int KT = Kpad / BK;
+  const int per = (KT + WAVES - 1) / WAVES;
+  const int kt_begin = wave * per < KT ? wave * per : KT;
+  const int kt_end = kt_begin + per < KT ? kt_begin + per : KT;
+
+  // The column this thread finishes, and what it is scaled and corrected by:
+  // requested first, needed last.
+  const int n = blockIdx.x * (T * CT) + (CT == 2 ? ((tid >> 8) & 1) * 16 : 0) + lr;
+  const bool col_ok = n < N;
+  const int nc = col_ok ? n : 0; // columns past N: computed on column 0, not stored
+  constexpr bool A_OFF = (A_MODE != 0);
+  const int32_t oa = A_OFF ? 128 : 0;
+  const int32_t ob = ep.b_unsigned ? 128 : 0;
+  // (No branch around a load: the wait for it would stand there too.  Absent
+  // operands are read from colsum, which is always valid, and masked.)
+  const bool has_bzp = ep.b_zp_len > 0, has_azp = !DQ && ep.a_zp_len > 0;
+  const bool has_bias = EPI == kEpiF32 && ep.bias != nullptr;
+  const int32_t bz = load_zp_i32(has_bzp ? ep.b_zp : (const void *)ep.colsum,
+      ep.b_unsigned, ep.b_zp_len > 1 ? nc : 0);
+  const int32_t az = load_zp_i32(
+      has_azp ? ep.a_zp : (const void *)ep.colsum, A_OFF, 0);
+  const int32_t cs = ep.colsum[nc];
+  const float bias = (has_bias ? ep.bias : (const float *)ep.colsum)
+      [has_bias && ep.bias_len > 1 ? nc : 0];
+  float bs = 0.0f, as = 0.0f, ys = 1.0f;
+  int32_t yz = 0;
+  if (EPI != kEpiI32) {
+    bs = ep.b_scale[ep.b_scale_len == 1 ? 0 : nc];
+    if (!DQ)
+      as = ep.a_scale[0];
+    if (EPI == kEpiQ8) {
+      ys = ep.y_scale[0];
+      yz = load_zp_i32(ep.y_zp, ep.y_unsigned, 0);
+    }
+  }
+
+  if (tid < RT * T)
+    rowsum[tid] = 0; // (before the barriers that the additions come after)
+
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  constexpr int NV = DQ > 0 ? DQ : 1;
+  f4 v[NV];
+  const int nvec = (M * K) >> 2;
+  if (DQ) {
+    const f4 *__restrict__ x4 = (const f4 *)X;
+    const float nan = __builtin_nanf(""); // neutral for minnum / maxnum
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int e = j * (WAVES * 64) + tid;
+      v[j] = e < nvec ? x4[e] : (f4){nan, nan, nan, nan};
+    }
+  }
+
+  // Operands of this wave's K steps.  Steps past its slice are sent outside the
+  // descriptors and read as zeros (no memory traffic): B' = 0 there.
+  constexpr int kOutside = 0x7FFFFFFF;
+  const int tile = T * CT == 32 ? (int)blockIdx.x : (int)blockIdx.x >> 1;
+  const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(Bp + (int64_t)tile * KT * 2048), 0, KT * 2048, 0x00020000);
+  const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)A, 0, DQ ? 0 : M * K, 0x00020000);
+  int bvoff[CT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+    bvoff[c] = T == 32 ? lane * 16
+                       : (lk >> 1) * 1024 +
+                             ((lk & 1) * 32 +
+                                 (CT == 2 ? c : ((int)blockIdx.x & 1)) * 16 + lr) * 16;
+
+  struct Batch {
+    v4i b[U][CT][SUBS];
+    v4i a[STG ? NLD : (DQ ? 1 : U)];
+  };
+  auto request = [&](int kt, Batch &t) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = kt + u;
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int b = 0; b < SUBS; ++b)
+          t.b[u][c][b] = __builtin_amdgcn_raw_buffer_load_b128(brsrc,
+              s < kt_end ? bvoff[c] + b * 1024 : kOutside,
+              s < kt_end ? s * 2048 : 0, 0);
+    }
+    if (STG) {
+      const int s = kt + (lane % CPR) / 4;
+      const int k0 = s * BK + (lane & 3) * 16;
+      const bool k_in = s < kt_end && k0 < K; // K % 16 == 0: in or out
+#pragma unroll
+      for (int j = 0; j < NLD; ++j) {
+        const int row = j * RPI + lane / CPR;
+        t.a[j] = __builtin_amdgcn_raw_buffer_load_b128(
+            arsrc, k_in && row < M ? row * K + k0 : kOutside, 0, 0);
+      }
+    } else if (!DQ) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k0 = (kt + u) * BK + lk * 16;
+        const bool in = lr < M && kt + u < kt_end && k0 < K;
+        t.a[u] = __builtin_amdgcn_raw_buffer_load_b128(
+            arsrc, in ? lr * K + k0 : kOutside, 0, 0);
+      }
+    }
+  };
+  Batch first; // DQ: on its way while the block quantizes its rows
+  if (DQ) {
+    request(kt_begin, first);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  float dq_scale = 0.0f;
+  int32_t dq_zp = 0;
+  if (DQ) {
+    float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      lo = __builtin_fminf(__builtin_fminf(lo, v[j].x),
+          __builtin_fminf(__builtin_fminf(v[j].y, v[j].z), v[j].w));
+      hi = __builtin_fmaxf(__builtin_fmaxf(hi, v[j].x),
+          __builtin_fmaxf(__builtin_fmaxf(v[j].y, v[j].z), v[j].w));
+    }
+    if (ep.x_limits) { // (the same for every thread) known from the layer before
+      lo = ep.x_limits[0];
+      hi = ep.x_limits[1];
+    } else {
+      lo = wave_min(lo);
+      hi = wave_max(hi);
+      if (lane == 0) {
+        s_lo[wave] = lo;
+        s_hi[wave] = hi;
+      }
+      lds_barrier();
+      lo = s_lo[0];
+      hi = s_hi[0];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) {
+        lo = __builtin_fminf(lo, s_lo[w]);
+        hi = __builtin_fmaxf(hi, s_hi[w]);
+      }
+    }
+    float zpf;
+    dynamic_params(lo, hi, dq_scale, zpf);
+    dq_zp = (int32_t)(uint32_t)zpf;
+    const float recip = 1.0f / dq_scale;
+    auto quantize = [&](auto fast_c) {
+      constexpr bool FAST = decltype(fast_c)::value;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        const int e = j * (WAVES * 64) + tid;
+        if (e < nvec) {
+          const uint32_t q = quant_pack4<false, true, FAST>(v[j].x, v[j].y,
+              v[j].z, v[j].w, dq_scale, dq_scale, dq_scale, dq_scale, recip,
+              recip, recip, recip, zpf, zpf, zpf, zpf);
+          ((uint32_t *)aq)[e] = q ^ 0x80808080u;
+        }
+      }
+    };
+    if (scale_is_tame(dq_scale)) // the same for every thread
+      quantize(std::true_type{});
+    else
+      quantize(std::false_type{});
+    lds_barrier();
+  }
+
+  typedef int vacc __attribute__((ext_vector_type(REGS)));
+  vacc acc[RT][CT];
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int r = 0; r < REGS; ++r)
+        acc[t][c][r] = 0;
+  const bool need_rs = ep.need_rowsum;
+  int32_t rsp[RT]; // this lane's share of rowsum(A') of row t*T + lane % T
+#pragma unroll
+  for (int t = 0; t < RT; ++t)
+    rsp[t] = 0;
+  const v4i flip = {(int)0x80808080, (int)0x80808080, (int)0x80808080,
+      (int)0x80808080};
+  const v4i zero = {0, 0, 0, 0};
+
+  // RS: row sums of A are needed, fixed outside the loop so that its body has no
+  // branch.
+  auto consume = [&](int kt, Batch &t, auto RS) {
+    v4i a[RT][U][SUBS];
+    if (STG) {
+      // Through the wave's own piece of LDS into operand order.  The LDS
+      // instructions of a wave execute in order; the fences keep the compiler
+      // from moving the reads above the writes of other lanes, and the next
+      // batch's writes above these reads.
+      uint8_t *const stg = lds_raw + wave * kStageWave;
+#pragma unroll
+      for (int j = 0; j < NLD; ++j)
+        *(v4i *)(stg + (j * RPI + lane / CPR) * kPitch + (lane % CPR) * 16) =
+            A_MODE == 1 ? t.a[j] ^ flip : t.a[j];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int b = 0; b < SUBS; ++b)
+            a[r][u][b] = *(const v4i *)(stg + (r * T + lr) * kPitch +
+                                        (u * 4 + b * 2 + lk) * 16);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k0 = (kt + u) * BK + lk * 16;
+        const bool in = kt + u < kt_end && k0 < K;
+        if (DQ) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            const int row = r * 16 + lr;
+            a[r][u][0] = *(const v4i *)(aq + (row < M ? row : 0) * K + (in ? k0 : 0));
+            if (decltype(RS)::value)
+              a[r][u][0] = in ? a[r][u][0] : zero;
+          }
+        } else {
+          a[0][u][0] = A_MODE == 1 ? t.a[u] ^ flip : t.a[u];
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < RT; ++r) {
+#pragma unroll
+        for (int b = 0; b < SUBS; ++b) {
+          if (decltype(RS)::value)
+            rsp[r] += frag_rowsum(a[r][u][b]);
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            if constexpr (T == 32)
+              acc[r][c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
+                  a[r][u][b], t.b[u][c][b], acc[r][c], 0, 0, 0);
+            else
+              acc[r][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                  a[r][u][b], t.b[u][c][b], acc[r][c], 0, 0, 0);
+          }
+        }
+      }
+  };
+  auto k_loop = [&](auto RS) {
+    int kt = kt_begin;
+    if (DQ) {
+      consume(kt, first, RS);
+      kt += U;
+    }
+    for (; kt < kt_end; kt += U) {
+      Batch t;
+      request(kt, t);
+      consume(kt, t, RS);
+    }
+  };
+  if (need_rs)
+    k_loop(std::true_type{});
+  else
+    k_loop(std::false_type{});
+  if (A_MODE == 1 && need_rs) {
+    // A chunk outside the slice or past K was read as zeros, that is 16 times
+    // -128 behind the flip: taken out of the row sums again.
+    int out = 0;
+    for (int s = kt_begin; s < kt_end + U - 1 && (s < kt_end || (s - kt_begin) % U); ++s)
+#pragma unroll
+      for (int b = 0; b < SUBS; ++b)
+        out += s >= kt_end || s * BK + (b * 2 + lk) * 16 >= K;
+#pragma unroll
+    for (int t = 0; t < RT; ++t)
+      rsp[t] += out * 2048;
+  }
+  __syncthreads(); // every wave is done reading its rows from LDS
+
+  // Accumulator layout: lane holds column lane % T; register r holds row
+  // 4*(lane/16) + r of a 16x16 tile, 8*(r/4) + 4*(lane/32) + r%4 of a 32x32 one.
+  // Slot (tile, r) is finished by wave slot % 8.
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+      for (int r = 0; r < REGS; ++r)
+        part[wave][(t * CT + c) * REGS + r][lane] = acc[t][c][r];
+    if (need_rs) {
+      int32_t rs = rsp[t];
+#pragma unroll
+      for (int off = T; off < 64; off *= 2)
+        rs += __shfl_xor(rs, off, 64);
+      if (lane < T)
+        atomicAdd(&rowsum[t * T + lane], rs);
+    }
+  }
+  __syncthreads();
+  if (!col_ok)
+    return;
+  const int32_t db = ob - (has_bzp ? bz : 0);
+  const float bj = has_bias ? bias : -0.0f;
+  float sj = 0.0f;
+  if (EPI != kEpiI32) {
+    sj = (DQ ? dq_scale : as) * bs;
+    if (EPI == kEpiQ8)
+      sj = sj / ys;
+  }
+#pragma unroll
+  for (int h = 0; h < (SLOTS + WAVES - 1) / WAVES; ++h) {
+    const int e = h * WAVES + wave;
+    const int rt = e / REGS / CT, r = e % REGS;
+    const int row = T == 32 ? 8 * (r >> 2) + 4 * lk + (r & 3) : 4 * lk + r;
+    const int m = rt * T + row;
+    if (e >= SLOTS || m >= M)
+      continue;
+    uint32_t y = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w)
+      y += (uint32_t)part[w][e][lane];
+    int32_t da = oa - (DQ ? dq_zp : has_azp ? az : 0);
+    if (!DQ && ep.a_zp_len > 1)
+      da = oa - load_zp_i32(ep.a_zp, A_OFF, m);
+    y += (uint32_t)da * (uint32_t)cs;
+    if (need_rs)
+      y += (uint32_t)db * (uint32_t)rowsum[m];
+    y += (uint32_t)K * (uint32_t)da * (uint32_t)db;
+    store_one<EPI>(ep, (int64_t)m * N + n, y, sj, yz, bj);
+  }
+}
+
+// One column tile of 16 per block, or two.  Half-width blocks are what fills the
+// device while N / 16 is up to 256 (K=11008 N=4096, 16 rows: 14.2 us, with 32
+// columns a block 14.4 and only half the CUs busy) and still ahead beyond that
+// where a block does little besides streaming weights (1 row, K=4096 N=11008:
+// 8.5 / 8.9 us).  Beyond 256 blocks two tiles win where a block's own work is
+// large against them: it quantizes more than 16 Ki elements (8 rows of 4096,
+// N=5120: 9.2 / 8.4 us, N=11008: 15.0 / 11.6; N=4096: 8.0 / 8.2), it holds more
+// than 32 rows (64 rows, K=4096 N=6144: 16.0 / 13.7; N=4096: 12.7 / 13.1), or K
+// is short (1 row, K=1024 N=11008: 5.2 / 4.8 us).
+template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG>
+void launch_one(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
+  k_gemm_i8_skinny<A_MODE, EPI, DQ, T, RT, CT, STG>
+      <<<(unsigned)((g.N + T * CT - 1) / (T * CT)), WAVES * 64, 0, st>>>(
+          (const uint8_t *)g.A, g.X, g.Bp, (int)g.M, (int)g.N, (int)g.K,
+          (int)round_up(g.K, kGemmBK), ep);
+}
+// One column tile of 16 per block, or two.  Half-width blocks are what fills the
+// device while N / 16 is up to 256 (K=11008 N=4096, 16 rows: with 32 columns a
+// block only half the CUs are busy) and still ahead beyond that where a block
+// does little besides streaming weights (1 row, K=4096 N=11008: 8.5 / 8.9 us).
+// Beyond 256 blocks two tiles win where a block's own work is large against
+// them: it quantizes more than 16 Ki elements (8 rows of 4096, N=5120: 9.2 / 8.4
+// us, N=11008: 15.0 / 11.6; N=4096: 8.0 / 8.2), or K is short (1 row, K=1024
+// N=11008: 5.2 / 4.8 us).
+template <int A_MODE, int EPI, int DQ, int RT, bool STG>
+void launch_16(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
+  if (g.N > 256 * 16 && ((DQ && g.M * g.K > 16384) || g.K <= 1024))
+    launch_one<A_MODE, EPI, DQ, 16, RT, 2, STG>(st, g, ep);
+  else
+    launch_one<A_MODE, EPI, DQ, 16, RT, 1, STG>(st, g, ep);
+}
+
+template <int A_MODE, int EPI>
+void launch_rows(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
+  if (g.M <= 4)
+    launch_16<A_MODE, EPI, 0, 1, false>(st, g, ep);
+  else if (g.M <= 16)
+    launch_16<A_MODE, EPI, 0, 1, true>(st, g, ep);
+  else if (g.M <= 32)
+    launch_16<A_MODE, EPI, 0, 2, true>(st, g, ep);
+  else if (g.N > 256 * 16)
+    // more than 32 rows beyond 256 blocks: one 32-column tile (64 rows, K=4096
+    // N=6144: 16.0 us with 16 columns, 13.2 so; N=4096: 12.7 / 13.1)
+    launch_one<A_MODE, EPI, 0, 32, 2, 1, true>(st, g, ep);
+  else if (g.M <= 48)
+    launch_one<A_MODE, EPI, 0, 16, 3, 1, true>(st, g, ep);
+  else
+    launch_one<A_MODE, EPI, 0, 16, 4, 1, true>(st, g, ep);
+}
+
+template <int A_MODE>
+void launch_epi(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
+  if (g.epi == kEpiI32)
+    launch_rows<A_MODE, kEpiI32>(st, g, ep);
+  else if (g.epi == kEpiF32)
+    launch_rows<A_MODE, kEpiF32>(st, g, ep);
+  else
+    launch_rows<A_MODE, kEpiQ8>(st, g, ep);
+}
+
+} // namespace
+
+// Whether the kernel can quantize this activation itself (DQ).
+bool skinny_quantizes_rows(int64_t M, int64_t K, const void *x) {
+  return M >= 1 && M <= 32 && K > 0 && K % 16 == 0 &&
+         M * K <= kSkinnyDqBytes && ((((uintptr_t)x) & 15) == 0);
+}
+
+// (K: the offsets of 64 rows and of a column tile's operands stay in 31 bits.)
+bool skinny_ok(int64_t M, int64_t K, const void *a) {
+  return M >= 1 && M <= 64 && K > 0 && K % 16 == 0 && K < (1 << 24) &&
+         ((((uintptr_t)a) & 15) == 0);
+}
+
+hipError_t launch_gemm_skinny(hipStream_t st, const GemmArgs &g,
+    const EpiParams &ep, int a_mode) {
+  if (g.X) {
+    if (g.epi != kEpiF32 || !skinny_quantizes_rows(g.M, g.K, g.X))
+      return hipErrorInvalidValue;
+    const int64_t elements = g.M * g.K;
+    if (g.M > 16)
+      launch_16<2, kEpiF32, 16, 2, false>(st, g, ep);
+    else if (elements <= 4 * 4 * 512)
+      launch_16<2, kEpiF32, 4, 1, false>(st, g, ep);
+    else if (elements <= 8 * 4 * 512)
+      launch_16<2, kEpiF32, 8, 1, false>(st, g, ep);
+    else
+      launch_16<2, kEpiF32, 16, 1, false>(st, g, ep);
+    return hipGetLastError();
+  }
+  if (!skinny_ok(g.M, g.K, g.A))
+    return hipErrorInvalidValue;
+  if (a_mode == 0)
+    launch_epi<0>(st, g, ep);
+  else if (a_mode == 1)
+    launch_epi<1>(st, g, ep);
+  else
+    launch_epi<2>(st, g, ep);
+  return hipGetLastError();
+}
+
+} // namespace gemm
+} // namespace om

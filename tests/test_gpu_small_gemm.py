@@ -329,3 +329,26 @@ def test_batched_kernel_edges(rt, oracle, M, K, N, adt, bdt):
         got = rt.QLinearMatMul(A, s, az, B, s, bz, np.float32(0.5), yz, mode)
         want = oracle.qlinear_matmul(A, s, az, B, s, bz, np.float32(0.5), yz, mode)
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 16, 17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("K,N", [(16, 40), (1008, 4096 + 33), (2064, 4097)])
+def test_few_rows_tile_widths(rt, oracle, M, K, N):
+    """The weight-streaming kernel on both sides of its row-tile edges and of the
+    column counts from which a block takes two column tiles (K <= 1024, or rows
+    it quantizes itself) or one of 32 columns (more than 32 rows): unsigned
+    weights with a zero point per column (row sums of A, whose chunks past K are
+    corrected for), and the fused layer, which quantizes up to 32 Ki elements in
+    the kernel."""
+    rng = np.random.default_rng(M * 7 + N)
+    A, B = rng.integers(0, 256, (M, K)).astype(np.uint8), rng.integers(0, 256, (K, N)).astype(np.uint8)
+    az, bz = np.uint8(131), rng.integers(0, 256, (N,)).astype(np.uint8)
+    got = rt.MatMulInteger(A, B, az, bz)
+    assert "skinny" in rt.last_gemm_kernel()
+    assert np.array_equal(got, oracle.matmul_integer(A, B, az, bz))
+    x = rng.standard_normal((M, K), dtype=np.float32)
+    ws = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    q, s, z = oracle.dynamic_quantize_linear(x)
+    want = oracle.dequant_epilogue(oracle.matmul_integer(q, B, z, bz), s, ws)
+    got = rt.DynQuantMatMulDequant(x, B, bz, ws)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
