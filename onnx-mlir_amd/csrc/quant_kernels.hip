@@ -1702,8 +1702,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_dql_small(
     store(std::integral_constant<int, 0>{});
 }
 
-// Mid-sized tensors (up to 32 float4 per thread of a grid that fills the
-// device once, 16 Mi elements): the whole op in one launch.  Every thread keeps
+// Tensors of up to 56 float4 per thread of a grid that fills the device once
+// (28 Mi elements): the whole op in one launch.  Larger ones keep that much.  Every thread keeps
 // its elements in registers while the blocks exchange their minima and maxima,
 // so x is read once, nothing but the result is written, and there is one
 // launch instead of two.  The grid is one block per CU, and the launcher keeps
@@ -1727,32 +1727,83 @@ __global__ __launch_bounds__(kSmallThreads) void k_dql_small(
 // Stores written through (store_through_u32): with plain stores the kernel
 // ends with the write-back of its 12 MB result (15.4 against 13.9 us), and
 // streaming stores slow down the GEMM that reads the result next by 3 us.
+// Buffer accesses whose offsets are one lane register and a scalar: with 64-bit
+// indices 32 float4 took 220 registers and 48 spilled.
+// Against two launches that read x twice: 22.5 Mi elements 40.0 -> 25.8 us,
+// 28 Mi 48.3 -> 31.5; beyond, where all but the last 28 Mi are still read twice,
+// 32 Mi 53.3 -> 40.6, 64 Mi 95 -> 87.7, 256 Mi 372 -> 360.
 constexpr int kGridThreads = 512;
-constexpr int kGridMaxPerThread = 32; // float4
+// 56 float4 are 224 of the 256 registers that two waves per SIMD leave a lane.
+constexpr int kGridMaxPerThread = 56; // float4
 
-template <int NV>
+// PREFIX: tensors beyond that.  The first `prefix` float4 are only reduced, the
+// ones after them (NV per thread of the grid) are kept and quantized as above;
+// the launcher quantizes the prefix with a launch of its own.
+template <int NV, bool PREFIX>
 __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
-    const float *__restrict__ x, int64_t n, uint8_t *__restrict__ y,
+    const float *__restrict__ x, int64_t n, int64_t prefix, uint8_t *__restrict__ y,
     float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, uint32_t flip,
     unsigned long long *slots, unsigned epoch, unsigned *failed,
     unsigned spin_limit) {
   constexpr int kWaves = kGridThreads / 64;
   __shared__ float s_lo[kWaves], s_hi[kWaves];
   __shared__ int s_ok;
+  float lo = __builtin_inff(), hi = -__builtin_inff();
+  if (PREFIX) {
+    // Streamed past the caches, three loads in flight per lane (256 Mi elements:
+    // 2 loads 385 us, 3 360, 4 366, 8 368, 16 379; the same loads without the
+    // streaming hint 389; 64 Mi: 91.2, 87.7, 87.8, 88.9, 96.2).
+    constexpr int kMU = 3;
+    const f4a *__restrict__ x4 = (const f4a *)x;
+    for (int64_t base = (int64_t)blockIdx.x * (kGridThreads * kMU); base < prefix;
+         base += (int64_t)gridDim.x * (kGridThreads * kMU)) {
+      f4a q[kMU];
+#pragma unroll
+      for (int j = 0; j < kMU; ++j) {
+        // (one past the end is the last one again)
+        const int64_t idx = base + j * kGridThreads + threadIdx.x;
+        q[j] = __builtin_nontemporal_load(&x4[idx < prefix ? idx : prefix - 1]);
+      }
+#pragma unroll
+      for (int j = 0; j < kMU; ++j) {
+        lo = __builtin_fminf(lo, __builtin_fminf(__builtin_fminf(q[j].x, q[j].y),
+                                     __builtin_fminf(q[j].z, q[j].w)));
+        hi = __builtin_fmaxf(hi, __builtin_fmaxf(__builtin_fmaxf(q[j].x, q[j].y),
+                                     __builtin_fmaxf(q[j].z, q[j].w)));
+      }
+    }
+    x += prefix * 4;
+    y += prefix * 4;
+    n -= prefix * 4;
+  }
   const int64_t nvec = n >> 2;
-  const int64_t total = (int64_t)gridDim.x * kGridThreads;
-  const int64_t gtid = (int64_t)blockIdx.x * kGridThreads + threadIdx.x;
-  const f4a *__restrict__ x4 = (const f4a *)x;
-  const f4a nan4 = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""),
-      __builtin_nanf("")};
+  // Whole float4 j of this thread: at bytes 16 * (j * total + gtid) of x, and
+  // bytes 4 * (..) of y.  Buffer accesses with 32-bit offsets: what lies past the
+  // last whole float4 is not read (zeros, which are neutral: the range that
+  // DynamicQuantizeLinear takes always includes 0) and not written, and no
+  // register holds an address or an index.
+  const unsigned total = gridDim.x * kGridThreads;
+  const unsigned gtid = blockIdx.x * kGridThreads + threadIdx.x;
+  const unsigned xbytes = (unsigned)(nvec * 16);
+  // (The scalar offset is kept within the descriptor's size, from which the
+  // hardware subtracts it, unsigned, before it compares the lane offset.)
+  auto at = [&](int j) {
+    const unsigned o = (unsigned)j * total * 16u;
+    return (int)(o < xbytes ? o : xbytes);
+  };
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)x, 0, (int)xbytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+      y, 0, (int)(nvec * 4), 0x00020000);
 
   f4a v[NV];
-  float lo = __builtin_inff(), hi = -__builtin_inff();
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const int64_t idx = (int64_t)j * total + gtid;
-    // NaN is neutral for minnum / maxnum
-    v[j] = idx < nvec ? x4[idx] : nan4;
+    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+    const u4 q = __builtin_amdgcn_raw_buffer_load_b128(
+        xr, (int)(gtid * 16u), at(j), 0);
+    v[j] = (f4a){__uint_as_float(q.x), __uint_as_float(q.y),
+        __uint_as_float(q.z), __uint_as_float(q.w)};
   }
   // the up to three elements after the last whole float4
   const int64_t te = (nvec << 2) + gtid;
@@ -1862,19 +1913,16 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
     scale_out[0] = scale;
     zp_out[0] = (uint8_t)(uint32_t)zpf;
   }
-  uint32_t *__restrict__ y4 = (uint32_t *)y;
   const float recip = 1.0f / scale;
   auto store = [&](auto fast_c) {
     constexpr bool FAST = decltype(fast_c)::value;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      const int64_t idx = (int64_t)j * total + gtid;
-      if (idx < nvec) {
-        const uint32_t q = quant_four<false, true, FAST>(v[j], scale, recip, zpf, flip);
-        // written through (see store_through_u32): 15.4 -> 13.9 us at
-        // [4096, 3072], and the GEMM that reads the result next gains too
-        store_through_u32(y4 + idx, q);
-      }
+      const uint32_t q = quant_four<false, true, FAST>(v[j], scale, recip, zpf, flip);
+      // written through (see store_through_u32): 15.4 -> 13.9 us at
+      // [4096, 3072], and the GEMM that reads the result next gains too
+      __builtin_amdgcn_raw_buffer_store_b32(
+          (int)q, yr, (int)(gtid * 4u), at(j) / 4, 16 /* sc1 */);
     }
   };
   if (scale_is_tame(scale)) // the same for every thread
@@ -2421,7 +2469,7 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
       ((((uintptr_t)y) & 3) == 0)) {
     const int64_t total = (int64_t)scratch.grid_blocks * kGridThreads;
     const int64_t nvec = n >> 2;
-    void (*fn_launch)(const float *, int64_t, uint8_t *, float *, uint8_t *,
+    void (*fn_launch)(const float *, int64_t, int64_t, uint8_t *, float *, uint8_t *,
         uint32_t, unsigned long long *, unsigned, unsigned *, unsigned) =
         nullptr;
     // Up to two float4 per thread of the whole grid the launch takes only as
@@ -2430,13 +2478,22 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
     // the two launches of the general path 8.1; 512 Ki: 128 blocks 7.2
     // against 8.2 for 256 blocks of 4 per thread; 96 Ki: 6.1 against 8.1).
     int64_t blocks = scratch.grid_blocks; // <= scratch.max_blocks
+    int64_t prefix = 0;
     if (nvec <= 2 * total) {
-      fn_launch = k_dql_grid<2>;
+      fn_launch = k_dql_grid<2, false>;
       blocks = (nvec + 2 * kGridThreads - 1) / (2 * kGridThreads);
     } else if (nvec <= 8 * total)
-      fn_launch = k_dql_grid<8>;
+      fn_launch = k_dql_grid<8, false>;
+    else if (nvec <= 16 * total)
+      fn_launch = k_dql_grid<16, false>;
+    else if (nvec <= 32 * total)
+      fn_launch = k_dql_grid<32, false>;
     else if (nvec <= kGridMaxPerThread * total)
-      fn_launch = k_dql_grid<kGridMaxPerThread>;
+      fn_launch = k_dql_grid<kGridMaxPerThread, false>;
+    else {
+      fn_launch = k_dql_grid<kGridMaxPerThread, true>;
+      prefix = nvec - kGridMaxPerThread * total;
+    }
     if (fn_launch) {
       const uint32_t flip = y_shift ? 0x80808080u : 0u;
       // If the previous kernel of this kind was launched on another stream and
@@ -2444,11 +2501,14 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
       GridExchange ex;
       if (dql_exchange_begin(s, scratch, ex)) {
         hipLaunchKernelGGL(fn_launch, dim3((unsigned)blocks),
-            dim3(kGridThreads), 0, s, x, n, y, scale, zp, flip, ex.slots,
+            dim3(kGridThreads), 0, s, x, n, prefix, y, scale, zp, flip, ex.slots,
             ex.epoch, ex.failed, ex.spin_limit);
         const hipError_t e = hipGetLastError();
         dql_exchange_end(s, e == hipSuccess);
-        return e;
+        if (e != hipSuccess || prefix == 0)
+          return e;
+        return quantize_dispatch<false>(
+            s, x, 1, 1, prefix * 4, scale, zp, y, flip);
       }
     }
   }
@@ -2544,7 +2604,7 @@ int dql_grid_blocks() {
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
           hipSuccess ||
       hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &per, k_dql_grid<kGridMaxPerThread>, kGridThreads, 0) != hipSuccess)
+          &per, k_dql_grid<kGridMaxPerThread, true>, kGridThreads, 0) != hipSuccess)
     return 0;
   if (per < 1 || cus < 1)
     return 0;

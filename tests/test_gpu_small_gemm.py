@@ -352,3 +352,24 @@ def test_few_rows_tile_widths(rt, oracle, M, K, N):
     want = oracle.dequant_epilogue(oracle.matmul_integer(q, B, z, bz), s, ws)
     got = rt.DynQuantMatMulDequant(x, B, bz, ws)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("per_thread", [2, 8, 16, 32, 56])
+@pytest.mark.parametrize("extra", [-1, 0, 1, 7])
+def test_dynamic_quantize_register_edges(rt, oracle, per_thread, extra):
+    """DynamicQuantizeLinear around the tensor sizes where one launch keeps
+    another number of float4 per thread (512 threads on each of the CUs), and
+    beyond the largest, where the elements in front of the kept ones are reduced
+    first and quantized by a second launch; the extremes lie at the first
+    element, in the middle and at the last one."""
+    n = rt.device_info()["cus"] * 512 * 4 * per_thread + extra
+    rng = np.random.default_rng(per_thread)
+    x = rng.standard_normal(n, dtype=np.float32)
+    for at in (0, n // 2, n - 1):
+        x[at], x[(at + 1) % n] = 11.0 + at % 3, -9.0
+        wy, ws, wz = oracle.dynamic_quantize_linear(x)
+        dy, ds, dz = rt.DynamicQuantizeLinear(rt.DeviceArray.from_numpy(x))
+        rt.synchronize()
+        assert ds.numpy().view(np.uint32) == np.float32(ws).view(np.uint32) and int(dz.numpy()) == int(wz)
+        assert np.array_equal(dy.numpy(), wy)
+        x[at] = x[(at + 1) % n] = 0.5
