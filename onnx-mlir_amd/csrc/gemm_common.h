@@ -218,11 +218,12 @@ __device__ __forceinline__ int32_t load_zp_i32(
 // Sum of the 16 int8 values of an MFMA A operand register group (one lane:
 // one row, 16 consecutive K bytes).  Kernels add these up over K when the
 // epilogue needs rowsum(A'), i.e. when B carries an offset.
-__device__ __forceinline__ int32_t frag_rowsum(v4i f) {
-  int32_t s = __builtin_amdgcn_sdot4(f.x, 0x01010101, 0, false);
-  s = __builtin_amdgcn_sdot4(f.y, 0x01010101, s, false);
-  s = __builtin_amdgcn_sdot4(f.z, 0x01010101, s, false);
-  return __builtin_amdgcn_sdot4(f.w, 0x01010101, s, false);
+// (`ones`: 0x01010101, or 0 to leave the group out.)
+__device__ __forceinline__ int32_t frag_rowsum(v4i f, int ones = 0x01010101) {
+  int32_t s = __builtin_amdgcn_sdot4(f.x, ones, 0, false);
+  s = __builtin_amdgcn_sdot4(f.y, ones, s, false);
+  s = __builtin_amdgcn_sdot4(f.z, ones, s, false);
+  return __builtin_amdgcn_sdot4(f.w, ones, s, false);
 }
 
 

@@ -27,9 +27,9 @@
 //                        the A tile goes through LDS (copied there without
 //                        passing through registers); more than one tile per CU
 //   k_gemm_i8_dma        A and Bp tiles copied from global memory straight
-//                        into a ring of three LDS stages; up to one tile per CU
-//   k_gemm_i8            tiles staged through registers, LDS double buffered;
-//                        also the general path: any K, any alignment of A
+//                        into a ring of three LDS stages; K a multiple of 16
+//   k_gemm_i8            tiles staged through registers, LDS double buffered:
+//                        the general path, any K, any alignment of A
 // and, in files of their own, k_gemm_i8_skinny (M <= 64, weight streaming),
 // k_gemm_i8_flight, k_gemm_i8_wreg and k_gemm_i8_batched.
 // A tiles in LDS have 64-byte rows whose 16-byte chunk index is XOR-swizzled
@@ -101,9 +101,23 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   constexpr int kFill = (A_MODE == 1) ? (int)0x80808080 : 0;
   const int KTs = Kpad / BK; // K steps: stride between column tiles of Bp
 
+  // kLoadAny: this thread's chunks in K step 0 (rows past M clamped to the
+  // last row, as below) and the last address a 16-byte load may have.
+  const uint8_t *arow[CH_A];
+  const uint8_t *alast = nullptr;
+  if (A_LOAD == kLoadAny) {
+#pragma unroll
+    for (int h = 0; h < CH_A; ++h) {
+      const int q = tid + h * THREADS;
+      const int gm = m0 + (q >> 2) < M ? m0 + (q >> 2) : M - 1;
+      arow[h] = A + (int64_t)gm * K + (q & 3) * 16;
+    }
+    alast = A + ((int64_t)M * K - 16);
+  }
+
   // Global loads only fetch; uint8 data is shifted to int8 after it is read
-  // back from LDS.  In the general paths bytes outside [M,K] are replaced by
-  // the byte that the shift maps to 0.
+  // back from LDS.  In the general paths bytes past the end of a row are
+  // replaced by the byte that the shift maps to 0.
   auto load_global = [&](int k0, v4i(&ra)[CH_A], v4i(&rb)[CH_B]) {
 #pragma unroll
     for (int h = 0; h < CH_A; ++h) {
@@ -121,40 +135,15 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
         const int gmc = gm < M ? gm : M - 1;
         v = *(const v4i *)(A + (int64_t)gmc * K + gk);
       } else if (A_LOAD == kLoadAny) {
-        // One 16-byte load per chunk at whatever address the chunk has.  The
-        // chunk at the end of a row holds K - gk < 16 of its bytes; the rest
-        // (the next row's, or nothing: the load is moved back to end with the
-        // buffer and its bytes shifted down) become the fill byte.  Chunks
-        // outside [M, K] load the first 16 bytes and keep none of them.
-        const bool valid = gm < M && gk < K;
-        const int64_t total = (int64_t)M * K;
-        const int64_t off = valid ? (int64_t)gm * K + gk : 0;
-        const int len = valid ? (K - gk < 16 ? K - gk : 16) : 0;
-        const int64_t off2 = off + 16 <= total ? off : total - 16;
-        const int sh = (int)(off - off2) * 8; // bits to shift down, < 128
-        const v4i_any raw = *(const v4i_any *)(A + off2);
-        uint64_t lo = (uint32_t)raw.x | ((uint64_t)(uint32_t)raw.y << 32);
-        uint64_t hi = (uint32_t)raw.z | ((uint64_t)(uint32_t)raw.w << 32);
-        if (sh >= 64) {
-          lo = hi;
-          hi = 0;
-        }
-        const int s1 = sh & 63;
-        if (s1) {
-          lo = (lo >> s1) | (hi << (64 - s1));
-          hi >>= s1;
-        }
-        const uint64_t fill64 =
-            (uint32_t)kFill | ((uint64_t)(uint32_t)kFill << 32);
-        const uint64_t mlo =
-            len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
-        const uint64_t mhi =
-            len >= 16 ? ~(uint64_t)0
-                      : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
-        lo = (lo & mlo) | (fill64 & ~mlo);
-        hi = (hi & mhi) | (fill64 & ~mhi);
-        v = (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32),
-            (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+        // One 16-byte load per chunk at whatever address the chunk has, moved
+        // back to end with the buffer where it would run past it.  What does
+        // not belong to the row is taken out when the chunk goes to LDS
+        // (mask_tail), one step in K: nothing here waits for the load.  (With
+        // the masking here, in every step, each step paid the latency of its
+        // own loads: 4099 x 777 x 1001 19.7 us against 16.0, the fused layer
+        // 100 x 11000 x 4000 128 against 84.)
+        const uint8_t *const p = arow[h] + k0;
+        v = *(const v4i_any *)(p < alast ? p : alast);
       } else {
         uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -182,7 +171,48 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
                              (ci & 1) * 1024 + (q & 63) * 16);
     }
   };
-  auto store_lds = [&](int buf, const v4i(&ra)[CH_A], const v4i(&rb)[CH_B]) {
+  // kLoadAny, the last K step when it is not a whole one: a chunk keeps the
+  // K - gk bytes that are the row's, shifted down by as much as its load was
+  // moved back; the rest (the next row's, or a whole chunk past the row)
+  // becomes the fill byte.  The weights are zero there, but the row sums count
+  // what these bytes hold.
+  auto mask_tail = [&](v4i(&ra)[CH_A]) {
+    const int k0 = Kpad - BK;
+#pragma unroll
+    for (int h = 0; h < CH_A; ++h) {
+      const int gk = k0 + ((tid + h * THREADS) & 3) * 16;
+      const int len = K - gk < 0 ? 0 : K - gk < 16 ? K - gk : 16;
+      const uint8_t *const p = arow[h] + k0;
+      // bits to shift down: < 128 whenever the chunk holds a byte of the row
+      const int sh = p < alast ? 0 : (int)(p - alast) * 8;
+      uint64_t lo = (uint32_t)ra[h].x | ((uint64_t)(uint32_t)ra[h].y << 32);
+      uint64_t hi = (uint32_t)ra[h].z | ((uint64_t)(uint32_t)ra[h].w << 32);
+      if (sh >= 64) {
+        lo = hi;
+        hi = 0;
+      }
+      const int s1 = sh & 63;
+      if (s1) {
+        lo = (lo >> s1) | (hi << (64 - s1));
+        hi >>= s1;
+      }
+      const uint64_t fill64 =
+          (uint32_t)kFill | ((uint64_t)(uint32_t)kFill << 32);
+      const uint64_t mlo =
+          len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
+      const uint64_t mhi =
+          len >= 16 ? ~(uint64_t)0
+                    : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
+      lo = (lo & mlo) | (fill64 & ~mlo);
+      hi = (hi & mhi) | (fill64 & ~mhi);
+      ra[h] = (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32),
+          (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+    }
+  };
+  // (`tail`: these are the registers of the last K step and that is not whole)
+  auto store_lds = [&](int buf, v4i(&ra)[CH_A], const v4i(&rb)[CH_B], bool tail) {
+    if (A_LOAD == kLoadAny && tail)
+      mask_tail(ra);
 #pragma unroll
     for (int h = 0; h < CH_A; ++h) {
       const int q = tid + h * THREADS;
@@ -231,10 +261,13 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   const int KT = Kpad / BK;
   const int klast = (KT - 1) * BK;
   auto kclamp = [&](int step) { return step < KT ? step * BK : klast; };
+  // (The registers of a step past the last one hold that step again, and may
+  // be masked again or not: nobody reads them.)
+  const int ktail = (A_LOAD == kLoadAny && (K & (BK - 1)) != 0) ? KT - 1 : -1;
   v4i ra0[CH_A], rb0[CH_B], ra1[CH_A], rb1[CH_B];
   load_global(0, ra0, rb0);
   load_global(kclamp(1), ra1, rb1);
-  store_lds(0, ra0, rb0);
+  store_lds(0, ra0, rb0, ktail == 0);
   load_global(kclamp(2), ra0, rb0);
   lds_barrier();
 
@@ -244,14 +277,14 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   // registers two steps ahead, then run the MFMAs of both half steps.  RS is
   // whether row sums of A are needed, fixed outside the loop so that the loop
   // body has no branch.
-  auto k_step = [&](int buf, v4i(&ra)[CH_A], v4i(&rb)[CH_B], int knext,
+  auto k_step = [&](int buf, v4i(&ra)[CH_A], v4i(&rb)[CH_B], int kt,
                     auto RS) {
     v4i fa0[TM], fb0[TN], fa1[TM], fb1[TN];
     read_frags(buf, 0, fa0, fb0);
     read_frags(buf, 1, fa1, fb1);
     __builtin_amdgcn_sched_barrier(0);
-    store_lds(buf ^ 1, ra, rb);
-    load_global(knext, ra, rb);
+    store_lds(buf ^ 1, ra, rb, kt + 1 == ktail);
+    load_global(kclamp(kt + 3), ra, rb);
     __builtin_amdgcn_sched_barrier(0);
     const v4i flip = {(int)0x80808080, (int)0x80808080, (int)0x80808080,
         (int)0x80808080};
@@ -289,10 +322,10 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   auto k_loop = [&](auto RS) {
     int kt = 0;
     while (true) {
-      k_step(0, ra1, rb1, kclamp(kt + 3), RS);
+      k_step(0, ra1, rb1, kt, RS);
       if (++kt >= KT)
         break;
-      k_step(1, ra0, rb0, kclamp(kt + 3), RS);
+      k_step(1, ra0, rb0, kt, RS);
       if (++kt >= KT)
         break;
     }
@@ -369,6 +402,12 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   const int KT = Kpad / BK;
   const int crow = lane >> 2;
   const int cchunk = (lane & 3) ^ ((lane >> 4) & 3);
+  // K is a multiple of 16 (in k_gemm_i8, which takes any K, 512 x 784 x 1001 is
+  // 11.8 us against 7.4 here), so a 16-byte chunk lies wholly inside its row or
+  // wholly past it.  In a last step that is not whole, the chunks past the row
+  // take its last chunk again (klim): the weights are zero there, and the row
+  // sums leave them out.
+  const int klim = K - 16 - cchunk * 16;
   const uint8_t *ga[2];
   const int8_t *gb[CB];
 #pragma unroll
@@ -387,9 +426,10 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   typedef const __attribute__((address_space(1))) void *glb_ptr;
   auto copy_step = [&](int k0, int stage) {
     uint8_t *base = sm + stage * STAGE;
+    const int ka = k0 < klim ? k0 : klim;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      __builtin_amdgcn_global_load_lds((glb_ptr)(ga[h] + k0),
+      __builtin_amdgcn_global_load_lds((glb_ptr)(ga[h] + ka),
           (lds_ptr)(base + (wave * 2 + h) * 1024), 16, 0, 0);
 #pragma unroll
     for (int h = 0; h < CB; ++h)
@@ -438,6 +478,11 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   for (int i = 0; i < TM; ++i)
     rsp[i] = 0;
 
+  // Weights of a row sum: none for a chunk past the end of the row.
+  auto ones = [&](int kt, int s2) {
+    return kt * BK + (s2 * 2 + lh) * 16 < K ? 0x01010101 : 0;
+  };
+
   int stage = 0; // kt % NSTAGE
   // Whether row sums of A are needed is fixed here, outside the loop, so that
   // the loop body has no branch.
@@ -484,7 +529,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
       if (decltype(RS)::value) {
   #pragma unroll
         for (int i = 0; i < TM; ++i)
-          rsp[i] += frag_rowsum(fa0[i]);
+          rsp[i] += frag_rowsum(fa0[i], ones(kt, 0));
       }
   #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -511,7 +556,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
       if (decltype(RS)::value) {
   #pragma unroll
         for (int i = 0; i < TM; ++i)
-          rsp[i] += frag_rowsum(fa1[i]);
+          rsp[i] += frag_rowsum(fa1[i], ones(kt, 1));
       }
   #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -982,8 +1027,9 @@ enum TileCfg : int {
   kNumCfg = 6
 };
 
-// Kernel choice for problems with more than 32 rows, K % 64 == 0 and a
-// 16-byte aligned A (anything else takes the general path of k_gemm_i8).
+// Kernel choice for problems with more than 64 rows, K % 64 == 0 and a
+// 16-byte aligned A (K % 16 == 0: k_gemm_i8_dma, its tile chosen here too;
+// anything else takes the general path of k_gemm_i8).
 // Measured on MI355X over the BERT-base and Llama-7B layer shapes and square
 // problems up to 8192: a 128 x 256 tile of k_gemm_i8_bs costs about 1.7 times
 // a 128 x 128 tile of k_gemm_i8_dma, so it wins when it needs at most half as
@@ -1018,7 +1064,7 @@ int choose_tile(int64_t M, int64_t N, int64_t K) {
 bool gemm_fast_path(int64_t M, int64_t K, const void *A) {
   // K == 0 (an empty sum) has no bytes of A to read: only the general path
   // checks every address against K.
-  return M > 16 && K > 0 && K % 64 == 0 && ((((uintptr_t)A) & 15) == 0);
+  return M > 16 && K > 0 && K % 16 == 0 && ((((uintptr_t)A) & 15) == 0);
 }
 
 // Name of the kernel the calling thread's last launch_gemm chose (for tests
@@ -1030,6 +1076,29 @@ thread_local bool t_gelu_applied = false;
 // Whether that kernel wrote GemmArgs::y_limits itself (launch_gemm runs the
 // reduction over the output when it did not).
 thread_local bool t_limits_written = false;
+
+// k_gemm_i8_dma in tiles of 128 columns or, for cfg = kD128x64, of 64.
+template <int A_MODE, int EPI>
+hipError_t launch_dma(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
+    int Kpad, int cfg) {
+  const int tiles_m = (int)((g.M + 127) / 128);
+  const uint8_t *A = (const uint8_t *)g.A;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  if (cfg == kD128x64) {
+    const int tiles_n = (int)((g.N + 63) / 64);
+    t_last_kernel = "k_gemm_i8_dma (128x64 tiles)";
+    k_gemm_i8_dma<64, 3, 3, A_MODE, EPI>
+        <<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
+            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
+  } else {
+    const int tiles_n = (int)((g.N + 127) / 128);
+    t_last_kernel = "k_gemm_i8_dma (128x128 tiles)";
+    k_gemm_i8_dma<128, 3, 3, A_MODE, EPI>
+        <<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
+            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
+  }
+  return hipGetLastError();
+}
 
 template <int A_MODE, int EPI>
 hipError_t gemm_launch_cfg(
@@ -1078,6 +1147,9 @@ hipError_t gemm_launch_cfg(
     return hipGetLastError();
   }
   const int cfg = choose_tile(g.M, g.N, g.K);
+  if (g.K % 64 != 0)
+    return launch_dma<A_MODE, EPI>(st, g, ep, Kpad,
+        cfg == kD128x64 || cfg == kD128x128 ? cfg : (int)kD128x128);
   // One round of blocks with everything requested at once: small problems,
   // where a pipelined K loop would pay the memory latency step after step
   // (512 x 1024 x 4096 QLinearMatMul: 8.2 us in 128 x 64 tiles of
@@ -1112,22 +1184,12 @@ hipError_t gemm_launch_cfg(
               A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
     break;
   }
-  case kD128x64: {
-    const int tiles_n64 = (int)((g.N + 63) / 64);
-    t_last_kernel = "k_gemm_i8_dma (128x64 tiles)";
-    k_gemm_i8_dma<64, 3, 3, A_MODE, EPI>
-        <<<dim3((unsigned)(tiles_m * tiles_n64)), 256, 0, st>>>(
-            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n64);
-    break;
-  }
+  case kD128x64:
+    return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x64);
   case kW128x384: // (forced, on a shape that kernel does not take)
   case kFlight:
   case kD128x128:
-    t_last_kernel = "k_gemm_i8_dma (128x128 tiles)";
-    k_gemm_i8_dma<128, 3, 3, A_MODE, EPI>
-        <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(
-            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n128);
-    break;
+    return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x128);
   default:
     t_last_kernel = "k_gemm_i8 (128x128 tiles through registers)";
     k_gemm_i8<128, 128, 2, 2, 3, A_MODE, EPI, kLoadAligned>

@@ -373,3 +373,38 @@ def test_dynamic_quantize_register_edges(rt, oracle, per_thread, extra):
         assert ds.numpy().view(np.uint32) == np.float32(ws).view(np.uint32) and int(dz.numpy()) == int(wz)
         assert np.array_equal(dy.numpy(), wy)
         x[at] = x[(at + 1) % n] = 0.5
+
+
+@pytest.mark.parametrize("K", [16, 48, 80, 784, 1008, 17, 63, 65, 127, 777])
+def test_products_whose_rows_end_inside_a_k_step(rt, oracle, K):
+    """K no multiple of 64: the last K step of k_gemm_i8_dma (K % 16 == 0) and
+    of k_gemm_i8 (any K) covers chunks that are partly or wholly past the row,
+    which must count neither in the products nor in the row sums; rows and
+    columns past the edge of the result are dropped by its store descriptor.
+    All operand types, zero points per tensor and per row / column, the three
+    epilogues, results next to memory that must stay as it is."""
+    rng = np.random.default_rng(K)
+    for M, N in ((65, 33), (129, 100), (300, 1001)):
+        for adt, bdt in ((np.uint8, np.int8), (np.int8, np.uint8), (np.uint8, np.uint8), (np.int8, np.int8)):
+            A, B = _rand_q(rng, adt, (M, K)), _rand_q(rng, bdt, (K, N))
+            az, bz = _rand_q(rng, adt, (M,)), _rand_q(rng, bdt, (N,))
+            for a_zp, b_zp in ((None, None), (az[:1], bz), (az, bz[:1])):
+                assert np.array_equal(rt.MatMulInteger(A, B, a_zp, b_zp), mm(oracle, A, B, a_zp, b_zp)), (M, N, adt, bdt)
+            assert ("dma" in rt.last_gemm_kernel()) == (K % 16 == 0), rt.last_gemm_kernel()
+            if adt == bdt:
+                s = [np.float32(v) for v in (0.0173, 0.005, 0.37)]
+                want = oracle.qlinear_matmul(A, s[0], az[:1], B, s[1], bz[:1], s[2], az[1], oracle_lib.WRAP)
+                assert np.array_equal(rt.QLinearMatMul(A, s[0], az[:1], B, s[1], bz[:1], s[2], az[1], rt.WRAP), want)
+        x = rng.normal(0, 1, (M, K)).astype(np.float32)
+        ws, bias = rng.uniform(1e-3, 1e-2, N).astype(np.float32), rng.normal(0, 1, N).astype(np.float32)
+        aq, a_s, a_zp = oracle.dynamic_quantize_linear(x)
+        want = oracle.dequant_epilogue(mm(oracle, aq, B, a_zp, bz), a_s, ws) + bias
+        assert same_f32(rt.DynQuantMatMulDequant(x, B, bz, ws, bias), want)
+        # the result between two guards in one buffer
+        guard = np.full(2 * 512 + M * N, 0x5A5A5A5A, np.int32)
+        whole, dA, dB = (rt.DeviceArray.from_numpy(v) for v in (guard, A, B))
+        rt.MatMulInteger(dA, dB, None, None, out=rt.DeviceArray.view_of(whole, 512, (M, N)))
+        rt.synchronize()
+        got = whole.numpy()
+        assert np.array_equal(got[512:-512].reshape(M, N), mm(oracle, A, B, None, None))
+        assert np.all(got[:512] == 0x5A5A5A5A) and np.all(got[-512:] == 0x5A5A5A5A)
