@@ -47,10 +47,12 @@ __device__ __forceinline__ void store_one(const EpiParams &ep, int64_t o,
   }
 }
 
+// with_colsum (and K = 0 with false): all blocks but the first of a product that
+// is split along K (KSplit in gemm_kernels.hip) leave the terms of the whole K out.
 template <int TM, int TN, int A_MODE, int EPI, int AUX32 = kAuxStream>
 __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
     const int32_t (&rsp)[TM], int mrow0, int ncol0, int M, int N, int K,
-    const EpiParams &ep) {
+    const EpiParams &ep, bool with_colsum = true) {
   const int lane = threadIdx.x & 63;
   const int l32 = lane & 31;
   const int lh = lane >> 5;
@@ -98,7 +100,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
     const int32_t bz =
         load_zp_i32(bzp_ptr, B_UNSIGNED, ep.b_zp_len > 1 ? nc : 0);
     db[j] = ob - (has_bzp ? bz : 0);
-    cs[j] = ep.colsum[nc];
+    cs[j] = with_colsum ? ep.colsum[nc] : 0;
     sj[j] = 0.0f;
     // a_scale * b_scale[j] first, then one multiply per element; for the
     // requantize (a_scale * b_scale) / y_scale, in this order

@@ -31,7 +31,9 @@
 //   k_gemm_i8            tiles staged through registers, LDS double buffered:
 //                        the general path, any K, any alignment of A
 // and, in files of their own, k_gemm_i8_skinny (M <= 64, weight streaming),
-// k_gemm_i8_flight, k_gemm_i8_wreg and k_gemm_i8_batched.
+// k_gemm_i8_flight, k_gemm_i8_wreg and k_gemm_i8_batched.  k_gemm_i8_dma and
+// k_gemm_i8 also multiply parts of K, which k_sum_parts adds up, where a product
+// has few tiles and many K steps (split_plan).
 // A tiles in LDS have 64-byte rows whose 16-byte chunk index is XOR-swizzled
 // with bits 2..3 of the row (bank-conflict free writes and operand reads); Bp
 // tiles in LDS keep their global order.
@@ -47,6 +49,26 @@ using namespace gemm;
 
 namespace {
 
+// Products of few tiles and many K steps are split along K (gemm_k_splits): the
+// blocks of one blockIdx.y multiply `steps` steps of K and write their int32
+// sums as if they were the whole result, to an array of their own `stride`
+// elements after the previous one's; k_sum_parts adds these up, mod 2^32 as all
+// sums here, and does the epilogue.  Per column and whole-K terms of the
+// zero-point algebra go into the first array only; a block's row sums cover its
+// own K.  The arrays are stored plainly: the next kernel reads them at once
+// (u8 results 127 x 2880 x 768 8.3 us, with streaming stores 9.2; larger ones
+// the same).
+struct KSplit {
+  int steps;
+  int64_t stride;
+};
+// SPLIT: the output of this block's part of K.
+__device__ __forceinline__ EpiParams part_of(const EpiParams &ep, const KSplit &ks) {
+  EpiParams e = ep;
+  e.out = (int32_t *)ep.out + (int64_t)blockIdx.y * ks.stride;
+  return e;
+}
+
 // BM x BN block tile, WGM x WGN waves, each wave a (BM/WGM) x (BN/WGN) tile
 // made of 32x32 MFMA tiles.
 // A_MODE: 0 = int8 as is, 1 = uint8 (XOR 0x80 while staging), 2 = already
@@ -56,10 +78,10 @@ namespace {
 // loads at byte addresses, the bytes past the end of a row replaced); kLoadBytes
 // = byte loads (an A of fewer than 16 bytes, K = 0).
 template <int BM, int BN, int WGM, int WGN, int MINB, int A_MODE, int EPI,
-    int A_LOAD>
+    int A_LOAD, bool SPLIT = false>
 __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
     const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n) {
+    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n, KSplit ks = {}) {
   constexpr int THREADS = WGM * WGN * 64;
   constexpr int WTM = BM / WGM, WTN = BN / WGN; // wave tile
   constexpr int TM = WTM / 32, TN = WTN / 32;   // MFMA tiles per wave
@@ -258,14 +280,17 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   // clamped to the last step and their data is never consumed): with no
   // branch around a load the compiler can wait for exactly the register set
   // it is about to store and leave the other set's loads in flight.
-  const int KT = Kpad / BK;
-  const int klast = (KT - 1) * BK;
-  auto kclamp = [&](int step) { return step < KT ? step * BK : klast; };
+  const int kfirst = SPLIT ? (int)blockIdx.y * ks.steps : 0; // in steps
+  const int KT = SPLIT && ks.steps < KTs - kfirst ? ks.steps : KTs - kfirst;
+  auto kclamp = [&](int step) {
+    return (kfirst + (step < KT ? step : KT - 1)) * BK;
+  };
   // (The registers of a step past the last one hold that step again, and may
   // be masked again or not: nobody reads them.)
-  const int ktail = (A_LOAD == kLoadAny && (K & (BK - 1)) != 0) ? KT - 1 : -1;
+  const int ktail =
+      (A_LOAD == kLoadAny && (K & (BK - 1)) != 0 && kfirst + KT == KTs) ? KT - 1 : -1;
   v4i ra0[CH_A], rb0[CH_B], ra1[CH_A], rb1[CH_B];
-  load_global(0, ra0, rb0);
+  load_global(kclamp(0), ra0, rb0);
   load_global(kclamp(1), ra1, rb1);
   store_lds(0, ra0, rb0, ktail == 0);
   load_global(kclamp(2), ra0, rb0);
@@ -334,8 +359,12 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
     k_loop(std::true_type{});
   else
     k_loop(std::false_type{});
-  gemm_epilogue<TM, TN, A_MODE, EPI>(
-      acc, rsp, m0 + wm * WTM, n0 + wn * WTN, M, N, K, ep);
+  if constexpr (SPLIT)
+    gemm_epilogue<TM, TN, A_MODE, EPI, 0>(acc, rsp, m0 + wm * WTM, n0 + wn * WTN,
+        M, N, blockIdx.y == 0 ? K : 0, part_of(ep, ks), blockIdx.y == 0);
+  else
+    gemm_epilogue<TM, TN, A_MODE, EPI>(
+        acc, rsp, m0 + wm * WTM, n0 + wn * WTN, M, N, K, ep);
 }
 
 // ---- GEMM, tiles copied from global memory straight into LDS --------------
@@ -358,10 +387,10 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
 // The operand reads are written as inline assembly: the compiler would make
 // every LDS read wait for all outstanding copies into LDS, whichever stage
 // they target.  The counts waited for below are therefore explicit.
-template <int BN, int NSTAGE, int MINB, int A_MODE, int EPI>
+template <int BN, int NSTAGE, int MINB, int A_MODE, int EPI, bool SPLIT = false>
 __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
     const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n) {
+    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n, KSplit ks = {}) {
   // 2 x 2 waves, each a 64 x (BN/2) tile.
   constexpr int BM = 128, WTM = 64, WTN = BN / 2, TM = 2, TN = WTN / 32;
   static_assert(BN == 128 || BN == 64, "tile width");
@@ -399,7 +428,9 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   // row.  Copy instruction c of the Bp tile moves KiB c of the stage, which
   // is (column tile c/2, half step c%2), unchanged.  A wave issues copies
   // 2*wave, 2*wave+1 of A and CB consecutive copies of Bp.
-  const int KT = Kpad / BK;
+  const int KTs = Kpad / BK; // K steps of the operands, and of this block
+  const int kfirst = SPLIT ? (int)blockIdx.y * ks.steps : 0;
+  const int KT = SPLIT && ks.steps < KTs - kfirst ? ks.steps : KTs - kfirst;
   const int crow = lane >> 2;
   const int cchunk = (lane & 3) ^ ((lane >> 4) & 3);
   // K is a multiple of 16 (in k_gemm_i8, which takes any K, 512 x 784 x 1001 is
@@ -419,7 +450,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
 #pragma unroll
   for (int h = 0; h < CB; ++h) {
     const int c = wave * CB + h;
-    gb[h] = Bp + (int64_t)((n0 >> 5) + (c >> 1)) * KT * 2048 + (c & 1) * 1024 +
+    gb[h] = Bp + (int64_t)((n0 >> 5) + (c >> 1)) * KTs * 2048 + (c & 1) * 1024 +
             lane * 16;
   }
   typedef __attribute__((address_space(3))) void *lds_ptr;
@@ -456,8 +487,9 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
       for (int r = 0; r < 16; ++r)
         acc[i][j][r] = 0;
 
-  const int klast = (KT - 1) * BK;
-  auto kclamp = [&](int step) { return step < KT ? step * BK : klast; };
+  auto kclamp = [&](int step) {
+    return (kfirst + (step < KT ? step : KT - 1)) * BK;
+  };
 #pragma unroll
   for (int p = 0; p < NSTAGE - 1; ++p)
     copy_step(kclamp(p), p);
@@ -480,7 +512,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
 
   // Weights of a row sum: none for a chunk past the end of the row.
   auto ones = [&](int kt, int s2) {
-    return kt * BK + (s2 * 2 + lh) * 16 < K ? 0x01010101 : 0;
+    return (kfirst + kt) * BK + (s2 * 2 + lh) * 16 < K ? 0x01010101 : 0;
   };
 
   int stage = 0; // kt % NSTAGE
@@ -575,8 +607,12 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   // but the block must not release its LDS before they are done.
   __builtin_amdgcn_s_waitcnt(0x0F70);
 
-  gemm_epilogue<TM, TN, A_MODE, EPI>(
-      acc, rsp, m0 + wm * WTM, n0 + wn * WTN, M, N, K, ep);
+  if constexpr (SPLIT)
+    gemm_epilogue<TM, TN, A_MODE, EPI, 0>(acc, rsp, m0 + wm * WTM, n0 + wn * WTN,
+        M, N, blockIdx.y == 0 ? K : 0, part_of(ep, ks), blockIdx.y == 0);
+  else
+    gemm_epilogue<TM, TN, A_MODE, EPI>(
+        acc, rsp, m0 + wm * WTM, n0 + wn * WTN, M, N, K, ep);
 }
 
 // ---- GEMM, Bp streamed to registers -----------------------------------------
@@ -1077,6 +1113,176 @@ thread_local bool t_gelu_applied = false;
 // reduction over the output when it did not).
 thread_local bool t_limits_written = false;
 
+// The sums of `parts` int32 arrays, each `stride` elements (a multiple of 4)
+// after the one before, with the epilogue of a product: 4 consecutive elements
+// of the result per thread.  Bound by the launch and by reading the arrays,
+// which were written a moment ago (at most 256 tiles of 64 KB).
+template <int EPI>
+__global__ __launch_bounds__(256) void k_sum_parts(
+    const int32_t *__restrict__ in, int parts, int64_t stride, unsigned n,
+    unsigned N, EpiParams ep, bool gelu, bool vector_out) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  const unsigned o = (blockIdx.x * 256 + threadIdx.x) * 4;
+  if (o >= n)
+    return;
+  float sj[4] = {}, bj[4] = {};
+  int32_t yz = 0;
+  if (EPI != kEpiI32) {
+    const float as = ep.a_scale[0];
+    const float ys = EPI == kEpiQ8 ? ep.y_scale[0] : 1.0f;
+    if (EPI == kEpiQ8)
+      yz = load_zp_i32(ep.y_zp, ep.y_unsigned, 0);
+    const bool has_bias = EPI == kEpiF32 && ep.bias != nullptr;
+    const float *const bias = has_bias ? ep.bias : ep.b_scale; // always readable
+    unsigned c = o % N;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sj[e] = as * ep.b_scale[ep.b_scale_len == 1 ? 0 : c];
+      if (EPI == kEpiQ8)
+        sj[e] = sj[e] / ys;
+      const float bv = bias[has_bias && ep.bias_len > 1 ? c : 0];
+      bj[e] = has_bias ? bv : -0.0f;
+      c = c + 1 == N ? 0 : c + 1;
+    }
+  }
+  // (the elements past n of the last four lie inside their array's stride)
+  u4 y = {0, 0, 0, 0};
+  int s = 0;
+  for (; s + 4 <= parts; s += 4) {
+    u4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      v[q] = *(const u4 *)(in + (int64_t)(s + q) * stride + o);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      y += v[q];
+  }
+  for (; s < parts; ++s)
+    y += *(const u4 *)(in + (int64_t)s * stride + o);
+  uint32_t r[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (EPI == kEpiI32) {
+      r[e] = y[e];
+    } else if (EPI == kEpiF32) {
+      const float f = relu_f32((float)(int32_t)y[e] * sj[e] + bj[e], ep.floor);
+      r[e] = __float_as_uint(gelu ? gelu_f32(f) : f);
+    } else {
+      r[e] = requantize(ep, y[e], sj[e], yz);
+    }
+  }
+  if (vector_out && o + 4 <= n) {
+    if (EPI == kEpiQ8)
+      *(uint32_t *)((uint8_t *)ep.out + o) =
+          r[0] | (r[1] << 8) | (r[2] << 16) | (r[3] << 24);
+    else
+      *(u4 *)((uint32_t *)ep.out + o) = (u4){r[0], r[1], r[2], r[3]};
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (o + e < n) {
+      if (EPI == kEpiQ8)
+        ((uint8_t *)ep.out)[o + e] = (uint8_t)r[e];
+      else
+        ((uint32_t *)ep.out)[o + e] = r[e];
+    }
+}
+
+// How a product is split along K (KSplit): the tile, the number of parts.
+struct SplitPlan {
+  int parts = 1; // 1: not at all
+  int steps = 0; // K steps of a part
+  bool any = false, narrow = false; // k_gemm_i8; 64-column tiles of k_gemm_i8_dma
+};
+
+int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
+
+// What bounds a product whose tiles cover a part of the CUs is the chain of its
+// K steps, each the time its operands take into one CU: 0.22 us in 128 x 64
+// tiles of k_gemm_i8_dma, 0.28 in 128 x 128 ones, 0.5 in k_gemm_i8 (u8 rows a
+// little more).  Splitting shortens the chain and costs the launch of
+// k_sum_parts, 2.5 us, and the arrays' way through memory, 1.8 us per million
+// elements.  Taken where that comes out a tenth ahead; more than one block per
+// CU gains nothing.  Measured without / with (fused layers with their
+// quantization): layer 102 x 3072 x 734 20.8 / 13.8 us, 65 x 11008 x 4096 43.6 /
+// 21.1, 128 x 4096 x 4096 21.4 / 19.3, 100 x 11000 x 4000 70.0 / 24.4, u8
+// results 517 x 8960 x 576 33.1 / 14.6, int32 600 x 5000 x 2000 43.7 / 24.1,
+// 2048 x 11008 x 768 48.1 / 37.6, 128 x 1536 x 300 9.5 / 7.8; left alone by the
+// rule: int32 2048 x 1280 x 1024 9.5 / 18.5, layer 512 x 1536 x 1536 14.1 /
+// 17.5, 128 x 4096 x 11008 23.3 / 23.7.
+SplitPlan split_plan(const GemmArgs &g, int a_mode) {
+  SplitPlan best;
+  const char *force = getenv("OM_MI355X_GEMM_TILE");
+  if (g.X || (force && force[0]) || g.M <= 0 || g.N <= 0 || g.K <= 0 ||
+      g.M * g.K < 16 || g.M * g.N > ((int64_t)1 << 22) ||
+      skinny_ok(g.M, g.K, g.A))
+    return best;
+  const bool any = !gemm_fast_path(g.M, g.K, g.A);
+  const int64_t KT = round_up(g.K, kGemmBK) / kGemmBK;
+  const int64_t tm = (g.M + 127) / 128, t128 = tm * ((g.N + 127) / 128);
+  if (KT < 8 || t128 > 128 ||
+      (!any && g.K % 64 == 0 &&
+          (flight_ok(g, a_mode) || (wreg_ok(g) && wreg_pays(g.M, g.N)))))
+    return best;
+  const double kWide = 0.28, kNarrow = 0.22, kAny = 0.5;
+  double least = 0.9 * (double)KT * (any ? kAny : g.N > 64 ? kNarrow : kWide);
+  for (int narrow = 0; narrow <= (any || g.N <= 64 ? 0 : 1); ++narrow) {
+    const int64_t tiles = narrow ? tm * ((g.N + 63) / 64) : t128;
+    const int64_t most = 256 / tiles < KT / 4 ? 256 / tiles : KT / 4;
+    for (int64_t parts = 2; parts <= most; ++parts) {
+      const int64_t steps = (KT + parts - 1) / parts;
+      if ((KT + steps - 1) / steps != parts)
+        continue; // (a part without a step)
+      const double us = (double)steps * (any ? kAny : narrow ? kNarrow : kWide) +
+                        2.5 + 1.8e-6 * (double)(parts * g.M * g.N);
+      if (us < least) {
+        least = us;
+        best.parts = (int)parts;
+        best.steps = (int)steps;
+        best.any = any;
+        best.narrow = narrow != 0;
+      }
+    }
+  }
+  return best;
+}
+
+template <int A_MODE, int EPI>
+hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
+    int Kpad, const SplitPlan &p) {
+  const uint8_t *A = (const uint8_t *)g.A;
+  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int tiles_m = (M + 127) / 128;
+  const int tiles_n = p.narrow ? (N + 63) / 64 : (N + 127) / 128;
+  const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)p.parts);
+  const KSplit ks = {p.steps, part_stride(g)};
+  EpiParams pe = ep;
+  pe.out = g.parts;
+  if (p.any) {
+    t_last_kernel = "k_gemm_i8 (any K, any alignment; split along K)";
+    k_gemm_i8<128, 128, 2, 2, 2, A_MODE, kEpiI32, kLoadAny, true>
+        <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+  } else if (p.narrow) {
+    t_last_kernel = "k_gemm_i8_dma (128x64 tiles, split along K)";
+    k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, true>
+        <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+  } else {
+    t_last_kernel = "k_gemm_i8_dma (128x128 tiles, split along K)";
+    k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, true>
+        <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess)
+    return e;
+  const unsigned n = (unsigned)(g.M * g.N);
+  const bool vec = (((uintptr_t)g.out) & (EPI == kEpiQ8 ? 3 : 15)) == 0;
+  k_sum_parts<EPI><<<(n + 1023) / 1024, 256, 0, st>>>(
+      g.parts, p.parts, ks.stride, n, (unsigned)N, ep, g.gelu, vec);
+  t_gelu_applied = EPI == kEpiF32 && g.gelu;
+  return hipGetLastError();
+}
+
 // k_gemm_i8_dma in tiles of 128 columns or, for cfg = kD128x64, of 64.
 template <int A_MODE, int EPI>
 hipError_t launch_dma(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
@@ -1129,6 +1335,11 @@ hipError_t gemm_launch_cfg(
   if (skinny_ok(g.M, g.K, g.A) && !(force && force[0])) {
     t_last_kernel = "k_gemm_i8_skinny";
     return launch_gemm_skinny(st, g, ep, A_MODE);
+  }
+  if (g.parts) {
+    const SplitPlan plan = split_plan(g, A_MODE);
+    if (plan.parts > 1)
+      return launch_split<A_MODE, EPI>(st, g, ep, Kpad, plan);
   }
   const int tiles_m = (int)((g.M + 127) / 128);
   const int tiles_n128 = (int)((g.N + 127) / 128);
@@ -1284,6 +1495,12 @@ int gemm_quantizes_rows(int64_t M, int64_t K, int64_t N, const void *x) {
   if (skinny_quantizes_rows(M, K, x))
     return 1;
   return flight_quantizes_rows(M, K, N, x) ? 2 : 0;
+}
+
+size_t gemm_parts_bytes(const GemmArgs &g) {
+  const SplitPlan p =
+      split_plan(g, (g.X || g.a_preshifted) ? 2 : (g.a_unsigned ? 1 : 0));
+  return p.parts > 1 ? (size_t)p.parts * part_stride(g) * 4 : 0;
 }
 
 const char *last_gemm_kernel() { return t_last_kernel; }

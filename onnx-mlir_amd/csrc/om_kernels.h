@@ -161,8 +161,14 @@ struct GemmArgs {
   // With X, optional: minimum and maximum of X as an earlier product's
   // y_limits gave them; the kernel then does not look for them.
   const float *x_limits;
+  // Optional: gemm_parts_bytes() bytes of scratch, 16-byte aligned, with which
+  // a product of few tiles is split along K.
+  int32_t *parts;
 };
 
+// Scratch with which launch_gemm is faster (the arguments as it will get them);
+// 0: none.
+size_t gemm_parts_bytes(const GemmArgs &g);
 hipError_t launch_gemm(hipStream_t s, const GemmArgs &g);
 // Name of the kernel the calling thread's last launch_gemm or
 // launch_gemm_batched chose.

@@ -538,7 +538,8 @@ struct Ctx {
     return e;
   }
 
-  void *take(size_t bytes) {
+  // optional: null without an error if there is no memory for it.
+  void *take(size_t bytes, bool optional = false) {
     if (bytes == 0)
       bytes = 16;
     bytes = (bytes + 255) & ~(size_t)255;
@@ -551,6 +552,20 @@ struct Ctx {
       return p;
     }
     void *p = nullptr;
+    if (optional) {
+      // (relaxed: a capture that the program has open on a stream of its own
+      // is not disturbed by an allocation that the call could do without)
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      const hipError_t e = hipMalloc(&p, bytes);
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      taken[p] = bytes;
+      return p;
+    }
     hipError_t e = hipMalloc(&p, bytes);
     if (e != hipSuccess) {
       // Give cached buffers back to the driver and retry once.
@@ -840,6 +855,20 @@ struct Call {
     else
       temps.push_back(p);
     return p;
+  }
+
+  // launch_gemm, with the scratch that makes it faster unless the stream is
+  // being captured (a replay would share the scratch with later calls).
+  hipError_t gemm(GemmArgs &g) {
+    const size_t bytes = gemm_parts_bytes(g);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (bytes && hipStreamIsCapturing(c.stream, &capture) == hipSuccess &&
+        capture == hipStreamCaptureStatusNone) {
+      g.parts = (int32_t *)c.take(bytes, /*optional=*/true);
+      if (g.parts)
+        temps.push_back(g.parts);
+    }
+    return launch_gemm(c.stream, g);
   }
 
   // keep_constant: a host buffer declared constant gets a GPU copy that stays
@@ -1474,7 +1503,7 @@ void run_matmul(const MatmulSpec &sp) {
       g.K = round_up(K, 16);
     }
     if (call.ok)
-      call.check(launch_gemm(call.c.stream, g), sp.op);
+      call.check(call.gemm(g), sp.op);
     call.finish();
     return;
   }
@@ -1973,7 +2002,7 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
     g.bias_len = bias_t ? bias.numel : 0;
     g.relu = relu;
     g.gelu = gelu;
-    return launch_gemm(call.c.stream, g);
+    return call.gemm(g);
   };
   const int kind = (call.ok && t_quant_mode == 0 && call.c.dql.grid_blocks >= 0)
                        ? gemm_quantizes_rows(M, K, N, dx)

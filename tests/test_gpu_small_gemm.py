@@ -408,3 +408,49 @@ def test_products_whose_rows_end_inside_a_k_step(rt, oracle, K):
         got = whole.numpy()
         assert np.array_equal(got[512:-512].reshape(M, N), mm(oracle, A, B, None, None))
         assert np.all(got[:512] == 0x5A5A5A5A) and np.all(got[-512:] == 0x5A5A5A5A)
+
+
+@pytest.mark.parametrize("M,K,N", [(65, 2112, 65), (70, 2048, 33), (129, 4096, 258), (130, 2064, 257), (300, 4112, 130),
+                                   (65, 1537, 66), (129, 2001, 129), (257, 4097, 33)])
+def test_products_split_along_k(rt, oracle, monkeypatch, M, K, N):
+    """Few tiles and many K steps: parts of K multiplied by blocks of their own
+    and added up by k_sum_parts.  K of whole steps, of whole 16-byte chunks and
+    odd, a last part shorter than the others, results whose length is no
+    multiple of four and one that does not start on a 16-byte boundary; all
+    operand types, zero points per tensor and per row / column (row sums of each
+    part; whole-K terms once), the three epilogues, bias and activations, the
+    latter against the same product in one piece."""
+    rng = np.random.default_rng(K)
+    for adt, bdt in ((np.uint8, np.int8), (np.int8, np.uint8), (np.uint8, np.uint8), (np.int8, np.int8)):
+        A, B = _rand_q(rng, adt, (M, K)), _rand_q(rng, bdt, (K, N))
+        az, bz = _rand_q(rng, adt, (M,)), _rand_q(rng, bdt, (N,))
+        for a_zp, b_zp in ((None, None), (az[:1], bz), (az, bz[:1])):
+            assert np.array_equal(rt.MatMulInteger(A, B, a_zp, b_zp), mm(oracle, A, B, a_zp, b_zp)), (adt, bdt)
+            assert "split" in rt.last_gemm_kernel(), rt.last_gemm_kernel()
+        if adt == bdt:
+            s = [np.float32(v) for v in (0.0173, 0.005, 2.37)]
+            for mode, rt_mode in ((oracle_lib.WRAP, rt.WRAP), (oracle_lib.SATURATE, rt.SATURATE)):
+                want = oracle.qlinear_matmul(A, s[0], az[:1], B, s[1], bz[:1], s[2], az[1], mode)
+                assert np.array_equal(rt.QLinearMatMul(A, s[0], az[:1], B, s[1], bz[:1], s[2], az[1], rt_mode), want)
+                assert "split" in rt.last_gemm_kernel()
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    ws, bias = rng.uniform(1e-3, 1e-2, N).astype(np.float32), rng.normal(0, 1, N).astype(np.float32)
+    aq, a_s, a_zp = oracle.dynamic_quantize_linear(x)
+    plain = oracle.dequant_epilogue(mm(oracle, aq, B, a_zp, bz), a_s, ws)
+    assert same_f32(rt.DynQuantMatMulDequant(x, B, bz, ws), plain)
+    assert same_f32(rt.DynQuantMatMulDequant(x, B, bz, ws, bias), plain + bias)
+    acts = [rt.DynQuantMatMulDequant(x, B, bz, ws, b, activation=a) for b in (None, bias) for a in (1, rt.ACTIVATION_GELU)]
+    assert "split" in rt.last_gemm_kernel()
+    monkeypatch.setenv("OM_MI355X_GEMM_TILE", "1")
+    want = [rt.DynQuantMatMulDequant(x, B, bz, ws, b, activation=a) for b in (None, bias) for a in (1, rt.ACTIVATION_GELU)]
+    assert "split" not in rt.last_gemm_kernel()
+    monkeypatch.delenv("OM_MI355X_GEMM_TILE")
+    assert all(same_f32(g, w) for g, w in zip(acts, want))
+    # the result one element into a buffer, between guards
+    whole, dA, dB = (rt.DeviceArray.from_numpy(v) for v in (np.full(1026 + M * N, 0x5A5A5A5A, np.int32), A, B))
+    rt.MatMulInteger(dA, dB, None, None, out=rt.DeviceArray.view_of(whole, 513, (M, N)))
+    assert "split" in rt.last_gemm_kernel()
+    rt.synchronize()
+    got = whole.numpy()
+    assert np.array_equal(got[513:-513].reshape(M, N), mm(oracle, A, B, None, None))
+    assert np.all(got[:513] == 0x5A5A5A5A) and np.all(got[-513:] == 0x5A5A5A5A)
