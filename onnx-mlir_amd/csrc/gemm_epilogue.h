@@ -228,10 +228,18 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
     // that is what the range check looks at.  (A bounds test and a 64-bit
     // address per element instead: 512 x 777 x 1001 12.2 us against 11.8, the
     // fused layer 100 x 1001 x 4096 16.7 against 15.5.)
+    // Not where the registers are all taken: with int32 results this form raised
+    // the spilled registers of k_gemm_i8_dma's 128 x 128 tiles with int8 A from 42
+    // to 68 and of k_gemm_i8_bs from 9 to 12, and every tile paid for it, whole
+    // ones too (int8 A: 2048 x 256 x 4096 8.7 -> 9.4 us, 2048 x 768 x 4096 12.3 ->
+    // 13.0).  Those test every element.  (Parts of K, AUX32 = 0, spill fewer
+    // registers with it: 46 against 50.)
+    constexpr bool kEdge = EPI != kEpiI32 ||
+                           TM * TN <= (A_MODE == 0 && AUX32 != 0 ? 2 : 4);
     const int rows = M - mrow0, cols = N - ncol0;
-    if (rows <= 0 || cols <= 0)
+    if (kEdge && (rows <= 0 || cols <= 0))
       return;
-    if ((int64_t)N * (32 * TM + 8) * 4 < ((int64_t)1 << 30)) {
+    if (kEdge && (int64_t)N * (32 * TM + 8) * 4 < ((int64_t)1 << 30)) {
       const int nr = rows < 32 * TM ? rows : 32 * TM;
       const int nc = cols < 32 * TN ? cols : 32 * TN;
       const __amdgpu_buffer_rsrc_t ersrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -276,6 +284,27 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
         edge(std::true_type{});
       else
         edge(std::false_type{});
+      return;
+    }
+    if (!kEdge) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int mbase = mrow0 + i * 32 + 4 * lh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int rr = 8 * (r >> 2) + 4 * lh + (r & 3);
+          const int m = mbase + 8 * (r >> 2) + (r & 3);
+          const int32_t rs_row = __shfl(rsf[i], rr, 64);
+          const int64_t orow = (int64_t)m * N;
+#pragma unroll
+          for (int j = 0; j < TN; ++j) {
+            const uint32_t y = (uint32_t)acc[i][j][r] + cj[j] +
+                               (uint32_t)db[j] * (uint32_t)rs_row;
+            if (m < M && n_[j] < N)
+              store_one<EPI>(ep, orow + n_[j], y, sj[j], yz, bj[j]);
+          }
+        }
+      }
       return;
     }
   }
