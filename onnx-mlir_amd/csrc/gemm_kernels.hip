@@ -387,7 +387,15 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
 // The operand reads are written as inline assembly: the compiler would make
 // every LDS read wait for all outstanding copies into LDS, whichever stage
 // they target.  The counts waited for below are therefore explicit.
-template <int BN, int NSTAGE, int MINB, int A_MODE, int EPI, bool SPLIT = false>
+//
+// RAGGED: K is a multiple of 16 but not of the K step, 64 (in k_gemm_i8, which
+// takes any K, 512 x 784 x 1001 is 11.8 us against 7.4 here).  A form of its own,
+// because what its last step takes costs vector operations in every step: whole
+// steps through it were 2 to 7 % slower (4096 x 6656 x 768 with 8-bit results 36.4
+// us against 38.8, int32 results 1000 x 6656 x 4096 39.8 / 42.6, 4096 x 4096 x 768
+// with 8-bit results 24.5 / 25.8).
+template <int BN, int NSTAGE, int MINB, int A_MODE, int EPI, bool RAGGED,
+    bool SPLIT = false>
 __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
     const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
     int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n, KSplit ks = {}) {
@@ -433,8 +441,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   const int KT = SPLIT && ks.steps < KTs - kfirst ? ks.steps : KTs - kfirst;
   const int crow = lane >> 2;
   const int cchunk = (lane & 3) ^ ((lane >> 4) & 3);
-  // K is a multiple of 16 (in k_gemm_i8, which takes any K, 512 x 784 x 1001 is
-  // 11.8 us against 7.4 here), so a 16-byte chunk lies wholly inside its row or
+  // K is a multiple of 16, so a 16-byte chunk lies wholly inside its row or
   // wholly past it.  In a last step that is not whole, the chunks past the row
   // take its last chunk again (klim): the weights are zero there, and the row
   // sums leave them out.
@@ -457,7 +464,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
   typedef const __attribute__((address_space(1))) void *glb_ptr;
   auto copy_step = [&](int k0, int stage) {
     uint8_t *base = sm + stage * STAGE;
-    const int ka = k0 < klim ? k0 : klim;
+    const int ka = !RAGGED || k0 < klim ? k0 : klim;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       __builtin_amdgcn_global_load_lds((glb_ptr)(ga[h] + ka),
@@ -512,7 +519,8 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
 
   // Weights of a row sum: none for a chunk past the end of the row.
   auto ones = [&](int kt, int s2) {
-    return (kfirst + kt) * BK + (s2 * 2 + lh) * 16 < K ? 0x01010101 : 0;
+    return !RAGGED || (kfirst + kt) * BK + (s2 * 2 + lh) * 16 < K ? 0x01010101
+                                                                  : 0;
   };
 
   int stage = 0; // kt % NSTAGE
@@ -1248,6 +1256,19 @@ SplitPlan split_plan(const GemmArgs &g, int a_mode) {
   return best;
 }
 
+const char *dma_name(bool narrow, bool ragged, bool split) {
+  static const char *const names[2][2][2] = {
+      {{"k_gemm_i8_dma (128x128 tiles)",
+           "k_gemm_i8_dma (128x128 tiles, split along K)"},
+          {"k_gemm_i8_dma (128x128 tiles, ragged K)",
+              "k_gemm_i8_dma (128x128 tiles, ragged K, split along K)"}},
+      {{"k_gemm_i8_dma (128x64 tiles)",
+           "k_gemm_i8_dma (128x64 tiles, split along K)"},
+          {"k_gemm_i8_dma (128x64 tiles, ragged K)",
+              "k_gemm_i8_dma (128x64 tiles, ragged K, split along K)"}}};
+  return names[narrow][ragged][split];
+}
+
 template <int A_MODE, int EPI>
 hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
     int Kpad, const SplitPlan &p) {
@@ -1263,14 +1284,16 @@ hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
     t_last_kernel = "k_gemm_i8 (any K, any alignment; split along K)";
     k_gemm_i8<128, 128, 2, 2, 2, A_MODE, kEpiI32, kLoadAny, true>
         <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
-  } else if (p.narrow) {
-    t_last_kernel = "k_gemm_i8_dma (128x64 tiles, split along K)";
-    k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, true>
-        <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
   } else {
-    t_last_kernel = "k_gemm_i8_dma (128x128 tiles, split along K)";
-    k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, true>
-        <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+    const bool ragged = K % BK != 0;
+    t_last_kernel = dma_name(p.narrow, ragged, true);
+    auto *const kernel =
+        p.narrow ? (ragged ? k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, true, true>
+                           : k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, false, true>)
+                 : (ragged ? k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, true, true>
+                           : k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, false, true>);
+    kernel<<<grid, 256, 0, st>>>(
+        A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess)
@@ -1290,19 +1313,16 @@ hipError_t launch_dma(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
   const int tiles_m = (int)((g.M + 127) / 128);
   const uint8_t *A = (const uint8_t *)g.A;
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
-  if (cfg == kD128x64) {
-    const int tiles_n = (int)((g.N + 63) / 64);
-    t_last_kernel = "k_gemm_i8_dma (128x64 tiles)";
-    k_gemm_i8_dma<64, 3, 3, A_MODE, EPI>
-        <<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
-            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
-  } else {
-    const int tiles_n = (int)((g.N + 127) / 128);
-    t_last_kernel = "k_gemm_i8_dma (128x128 tiles)";
-    k_gemm_i8_dma<128, 3, 3, A_MODE, EPI>
-        <<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
-            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
-  }
+  const bool narrow = cfg == kD128x64, ragged = K % BK != 0;
+  const int tiles_n = narrow ? (N + 63) / 64 : (N + 127) / 128;
+  t_last_kernel = dma_name(narrow, ragged, false);
+  auto *const kernel =
+      narrow ? (ragged ? k_gemm_i8_dma<64, 3, 3, A_MODE, EPI, true>
+                       : k_gemm_i8_dma<64, 3, 3, A_MODE, EPI, false>)
+             : (ragged ? k_gemm_i8_dma<128, 3, 3, A_MODE, EPI, true>
+                       : k_gemm_i8_dma<128, 3, 3, A_MODE, EPI, false>);
+  kernel<<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
+      A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n, KSplit{});
   return hipGetLastError();
 }
 

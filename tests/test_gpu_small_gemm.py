@@ -454,3 +454,16 @@ def test_products_split_along_k(rt, oracle, monkeypatch, M, K, N):
     got = whole.numpy()
     assert np.array_equal(got[513:-513].reshape(M, N), mm(oracle, A, B, None, None))
     assert np.all(got[:513] == 0x5A5A5A5A) and np.all(got[-513:] == 0x5A5A5A5A)
+
+
+@pytest.mark.parametrize("M,K,N,split", [(300, 1152, 260, False), (4096, 1280, 768, False), (300, 2048, 130, True)])
+def test_whole_k_steps_take_the_form_without_a_tail(rt, oracle, M, K, N, split):
+    """k_gemm_i8_dma: only a K that ends inside a step takes the form that looks
+    for the end of the row in every step; both against the oracle, with row sums."""
+    rng = np.random.default_rng(K)
+    for k, ragged in ((K, False), (K + 16, True), (K + 48, True), (K + 64, False)):
+        A, B = _rand_q(rng, np.uint8, (M, k)), _rand_q(rng, np.int8, (k, N))
+        az, bz = _rand_q(rng, np.uint8, (1,)), _rand_q(rng, np.int8, (N,))
+        assert np.array_equal(rt.MatMulInteger(A, B, az, bz), mm(oracle, A, B, az, bz))
+        name = rt.last_gemm_kernel()
+        assert "dma" in name and ("ragged" in name) == ragged and ("split" in name) == split, name
