@@ -352,12 +352,16 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
     k_loop(std::false_type{});
   if (A_MODE == 1 && need_rs) {
     // A chunk outside the slice or past K was read as zeros, that is 16 times
-    // -128 behind the flip: taken out of the row sums again.
-    int out = 0;
-    for (int s = kt_begin; s < kt_end + U - 1 && (s < kt_end || (s - kt_begin) % U); ++s)
+    // -128 behind the flip: taken out of the row sums again.  Those are the
+    // steps that fill the last batch up, and chunks of the very last step of K.
+    // (Counted, not looked for step by step: 4 rows, K=11008 N=4608 13.9 -> 11.9
+    // us, 24 rows 14.8 -> 13.1.)
+    const int steps = kt_end - kt_begin;
+    int out = (U - 1 - (steps + U - 1) % U) * SUBS;
+    if (steps > 0 && kt_end == KT)
 #pragma unroll
       for (int b = 0; b < SUBS; ++b)
-        out += s >= kt_end || s * BK + (b * 2 + lk) * 16 >= K;
+        out += (KT - 1) * BK + (b * 2 + lk) * 16 >= K;
 #pragma unroll
     for (int t = 0; t < RT; ++t)
       rsp[t] += out * 2048;

@@ -467,3 +467,15 @@ def test_whole_k_steps_take_the_form_without_a_tail(rt, oracle, M, K, N, split):
         assert np.array_equal(rt.MatMulInteger(A, B, az, bz), mm(oracle, A, B, az, bz))
         name = rt.last_gemm_kernel()
         assert "dma" in name and ("ragged" in name) == ragged and ("split" in name) == split, name
+
+
+@pytest.mark.parametrize("M", [3, 9, 20, 40, 60])
+def test_few_rows_row_sums_of_padded_steps(rt, oracle, M):
+    """The weight-streaming kernel's row sums leave out the chunks it reads as
+    zeros: steps that fill up a wave's last batch, and chunks past K.  Every K of
+    whole chunks up to three steps a wave, and some beyond."""
+    rng = np.random.default_rng(M)
+    for K in list(range(16, 1600, 80)) + [1536, 2064, 2688, 5520]:
+        A, B = rng.integers(0, 256, (M, K)).astype(np.uint8), rng.integers(0, 256, (K, 24)).astype(np.uint8)
+        az, bz = np.uint8(121), rng.integers(0, 256, (24,)).astype(np.uint8)
+        assert np.array_equal(rt.MatMulInteger(A, B, az, bz), oracle.matmul_integer(A, B, az, bz)), K
