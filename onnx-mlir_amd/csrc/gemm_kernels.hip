@@ -1346,16 +1346,13 @@ hipError_t gemm_launch_cfg(
       t_limits_written = ep.limits.out != nullptr; // and reduces their limits
       return launch_gemm_flight_dq(st, g, ep, *g.dql);
     }
-    t_last_kernel = "k_gemm_i8_skinny (rows quantized in the kernel)";
     return launch_gemm_skinny(st, g, ep, A_MODE);
   }
   // Up to 64 rows the weight-streaming kernel is ahead of every tile kernel
   // (K=4096 N=11008: M=33 11.6 against 17.2 us, M=48 12.3 / 17.7; K=11008
   // N=4096 M=64: 15.0 / 37.7; K=768 N=3072 M=64: 4.2 / 6.0).
-  if (skinny_ok(g.M, g.K, g.A) && !(force && force[0])) {
-    t_last_kernel = "k_gemm_i8_skinny";
+  if (skinny_ok(g.M, g.K, g.A) && !(force && force[0]))
     return launch_gemm_skinny(st, g, ep, A_MODE);
-  }
   if (g.parts) {
     const SplitPlan plan = split_plan(g, A_MODE);
     if (plan.parts > 1)

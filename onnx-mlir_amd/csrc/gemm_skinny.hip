@@ -421,33 +421,35 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
   }
 }
 
-// One column tile of 16 per block, or two.  Half-width blocks are what fills the
-// device while N / 16 is up to 256 (K=11008 N=4096, 16 rows: 14.2 us, with 32
-// columns a block 14.4 and only half the CUs busy) and still ahead beyond that
-// where a block does little besides streaming weights (1 row, K=4096 N=11008:
-// 8.5 / 8.9 us).  Beyond 256 blocks two tiles win where a block's own work is
-// large against them: it quantizes more than 16 Ki elements (8 rows of 4096,
-// N=5120: 9.2 / 8.4 us, N=11008: 15.0 / 11.6; N=4096: 8.0 / 8.2), it holds more
-// than 32 rows (64 rows, K=4096 N=6144: 16.0 / 13.7; N=4096: 12.7 / 13.1), or K
-// is short (1 row, K=1024 N=11008: 5.2 / 4.8 us).
 template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG>
 void launch_one(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
+  note_gemm_kernel(
+      DQ ? (CT == 2 ? "k_gemm_i8_skinny (rows quantized in the kernel, 2 x 16 columns)"
+                    : "k_gemm_i8_skinny (rows quantized in the kernel, 16 columns)")
+      : T == 32 ? "k_gemm_i8_skinny (32 columns)"
+      : CT == 2 ? "k_gemm_i8_skinny (2 x 16 columns)"
+      : STG     ? "k_gemm_i8_skinny (16 columns)"
+                : "k_gemm_i8_skinny (16 columns, rows loaded directly)");
   k_gemm_i8_skinny<A_MODE, EPI, DQ, T, RT, CT, STG>
       <<<(unsigned)((g.N + T * CT - 1) / (T * CT)), WAVES * 64, 0, st>>>(
           (const uint8_t *)g.A, g.X, g.Bp, (int)g.M, (int)g.N, (int)g.K,
           (int)round_up(g.K, kGemmBK), ep);
 }
-// One column tile of 16 per block, or two.  Half-width blocks are what fills the
-// device while N / 16 is up to 256 (K=11008 N=4096, 16 rows: with 32 columns a
-// block only half the CUs are busy) and still ahead beyond that where a block
-// does little besides streaming weights (1 row, K=4096 N=11008: 8.5 / 8.9 us).
-// Beyond 256 blocks two tiles win where a block's own work is large against
-// them: it quantizes more than 16 Ki elements (8 rows of 4096, N=5120: 9.2 / 8.4
-// us, N=11008: 15.0 / 11.6; N=4096: 8.0 / 8.2), or K is short (1 row, K=1024
-// N=11008: 5.2 / 4.8 us).
+// Blocks of 16 columns are what fills the device while N / 16 is up to 256.
+constexpr int64_t kOneRound = 256 * 16;
+
+// One column tile of 16 per block, or two.  Beyond one round of blocks one is
+// still ahead where a block does little besides streaming weights (1 row it
+// quantizes, K=4096 N=4608: 4.6 / 5.2 us, N=11008: 6.6 / 7.1), and two where its own
+// work is large against them: K is short (1 row, K=1024 N=11008: 5.2 / 4.8 us; 5
+// rows it quantizes, K=2048 N=5120: 5.1 / 4.4, K=2688 N=11008: 7.3 / 6.9), or it
+// quantizes more than 16 Ki elements of more than four rows (8 rows of 4096,
+// N=6144: 8.2 / 7.4, N=11008: 13.5 / 10.1; but 4 rows of 8192, N=6144: 12.1 / 13.6).
 template <int A_MODE, int EPI, int DQ, int RT, bool STG>
 void launch_16(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
-  if (g.N > 256 * 16 && ((DQ && g.M * g.K > 16384) || g.K <= 1024))
+  const bool two = DQ ? g.K <= 3072 || (g.M > 4 && g.M * g.K > 16384)
+                      : g.K <= 1024;
+  if (g.N > kOneRound && two)
     launch_one<A_MODE, EPI, DQ, 16, RT, 2, STG>(st, g, ep);
   else
     launch_one<A_MODE, EPI, DQ, 16, RT, 1, STG>(st, g, ep);
@@ -455,20 +457,36 @@ void launch_16(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
 
 template <int A_MODE, int EPI>
 void launch_rows(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
-  if (g.M <= 4)
-    launch_16<A_MODE, EPI, 0, 1, false>(st, g, ep);
-  else if (g.M <= 16)
+  const bool rounds = g.N > kOneRound;
+  if (g.M <= 4) {
+    // Rows loaded directly, with four steps of weights on their way, up to one
+    // round of blocks and for short K (4 rows, K=8192 N=4096: 4.9 us against 5.9
+    // through LDS, K=1536 N=11008 4.1 / 4.2); beyond, other blocks' waves hide the
+    // loads better (K=11008 N=5120: 12.1 / 9.9, K=2688 N=7808: 4.6 / 4.0).
+    if (!rounds || g.K <= 2048)
+      launch_16<A_MODE, EPI, 0, 1, false>(st, g, ep);
+    else
+      launch_one<A_MODE, EPI, 0, 16, 1, 1, true>(st, g, ep);
+  } else if (g.M <= 16) {
     launch_16<A_MODE, EPI, 0, 1, true>(st, g, ep);
-  else if (g.M <= 32)
-    launch_16<A_MODE, EPI, 0, 2, true>(st, g, ep);
-  else if (g.N > 256 * 16)
-    // more than 32 rows beyond 256 blocks: one 32-column tile (64 rows, K=4096
+  } else if (g.M <= 32) {
+    // Beyond one round one 32 x 32 tile beats two of 16 x 16 (24 rows, K=2688
+    // N=5120: 4.9 / 3.9 us, K=11008 N=4608: 13.1 / 12.0), unless the column tiles
+    // lie a multiple of 128 KiB apart: as many streams at one distance hit the
+    // same channels (K=8192 N=4608: 9.7 / 11.0).
+    if (rounds && g.K % 4096 != 0)
+      launch_one<A_MODE, EPI, 0, 32, 1, 1, true>(st, g, ep);
+    else
+      launch_one<A_MODE, EPI, 0, 16, 2, 1, true>(st, g, ep);
+  } else if (rounds) {
+    // more than 32 rows beyond one round: one 32-column tile (64 rows, K=4096
     // N=6144: 16.0 us with 16 columns, 13.2 so; N=4096: 12.7 / 13.1)
     launch_one<A_MODE, EPI, 0, 32, 2, 1, true>(st, g, ep);
-  else if (g.M <= 48)
+  } else if (g.M <= 48) {
     launch_one<A_MODE, EPI, 0, 16, 3, 1, true>(st, g, ep);
-  else
+  } else {
     launch_one<A_MODE, EPI, 0, 16, 4, 1, true>(st, g, ep);
+  }
 }
 
 template <int A_MODE>
@@ -501,14 +519,21 @@ hipError_t launch_gemm_skinny(hipStream_t st, const GemmArgs &g,
     if (g.epi != kEpiF32 || !skinny_quantizes_rows(g.M, g.K, g.X))
       return hipErrorInvalidValue;
     const int64_t elements = g.M * g.K;
+    // As few float4 per thread as the rows need: 32 x 256, N=3072 in the form for
+    // 32 Ki elements 5.1 us against 4.4.
+    auto launch_dq = [&](auto rt) {
+      constexpr int RT = decltype(rt)::value;
+      if (elements <= 4 * 4 * 512)
+        launch_16<2, kEpiF32, 4, RT, false>(st, g, ep);
+      else if (elements <= 8 * 4 * 512)
+        launch_16<2, kEpiF32, 8, RT, false>(st, g, ep);
+      else
+        launch_16<2, kEpiF32, 16, RT, false>(st, g, ep);
+    };
     if (g.M > 16)
-      launch_16<2, kEpiF32, 16, 2, false>(st, g, ep);
-    else if (elements <= 4 * 4 * 512)
-      launch_16<2, kEpiF32, 4, 1, false>(st, g, ep);
-    else if (elements <= 8 * 4 * 512)
-      launch_16<2, kEpiF32, 8, 1, false>(st, g, ep);
+      launch_dq(std::integral_constant<int, 2>{});
     else
-      launch_16<2, kEpiF32, 16, 1, false>(st, g, ep);
+      launch_dq(std::integral_constant<int, 1>{});
     return hipGetLastError();
   }
   if (!skinny_ok(g.M, g.K, g.A))
