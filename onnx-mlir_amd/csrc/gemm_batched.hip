@@ -400,13 +400,43 @@ bool gemm_batched_ok(const GemmArgs &g, const GemmBatch &b) {
          tiles_of(g.M, g.N) <= kMaxBlocks;
 }
 
-// One launch wins while an entry's operands are not reused enough to pay for
-// packing B and for launches of its own (this kernel / packing and multiplying
-// entry by entry): 384 x 128x64x128 7.1 us / 3.5 ms, 8 x 1024x1024x1024 29.0 /
-// 79.1, 2 x 1024x4096x1024 40.4 / 52.5, 4 x 2048x2048x2048 89.5 / 93.7; beyond
-// that the tile kernels' 1.5 - 2 POP/s are ahead of the 0.77 reached here.
-bool gemm_batched_pays(const GemmArgs &g) {
-  return g.M * g.N * g.K <= ((int64_t)1 << 33);
+// One launch against packing each matrix of B and multiplying entry by entry,
+// both by a cost model in microseconds, fitted to 3600 products (1 to 32 entries,
+// 1 to 2048 rows, K 32 to 11008, N 32 to 4096, odd sizes among them): its choice is
+// more than 4 % behind the other for 21 of them, at most 15 %.
+//   One launch: the chain of a block's K steps, or where there are more blocks
+//   than the device holds what the CUs have to do in sum.  It does not split K, so
+//   few entries with a long K are a few blocks: 1 x 8192 x 128 70 us against 14
+//   packed, 16 x 4096 x 4096 37 / 18, four of 1 x 8192 x 128 71 / 54.
+//   Packed: the kernels of launch_gemm, two launches and a pass over each matrix of
+//   B in front, and the launches' own time on the host: 384 x 128x64x128 7.1 us /
+//   3.5 ms, 8 x 1024x1024x1024 29.0 / 79.1, 2 x 1024x4096x1024 40.4 / 52.5.
+// Entries above 2^33 multiply-adds go to the tile kernels (1.5 - 2 POP/s against
+// the 0.77 reached here; 4 x 2048x2048x2048 89.5 / 93.7).
+bool gemm_batched_pays(const GemmArgs &g, const GemmBatch &b) {
+  if (g.M * g.N * g.K > ((int64_t)1 << 33))
+    return false;
+  const double steps = (double)((g.K + BK - 1) / BK);
+  const double out_mb = 4e-6 * (double)(g.M * g.N), b_mb = 1e-6 * (double)(g.K * g.N);
+  const double count = (double)b.count, mats = (double)b.b_mats;
+  const bool narrow = g.N <= 64, chunks = g.K % 16 == 0;
+  const double cus = (double)tiles_of(g.M, g.N) * count / 256;
+  const double chain = narrow ? 0.34 : 0.54, share = (narrow ? 0.2 : 0.23) * cus;
+  const double one = 2.1 + 0.014 * out_mb * count +
+                     steps * (chain > share ? chain : share) *
+                         (chunks && g.N % 4 == 0 ? 1.0 : 1.57);
+  double gemm;
+  if (g.M <= 64 && chunks) {
+    gemm = 2.7 + steps * (0.036 + 0.0009 * (double)g.M) + 0.088 * b_mb;
+  } else if (g.K <= 1024 && g.K % 256 == 0 && g.M * g.N <= ((int64_t)1 << 21)) {
+    gemm = 2.4 + 0.06 * steps;
+  } else {
+    const double tiles = (double)(((g.M + 127) / 128) * ((g.N + 127) / 128)) / 400;
+    gemm = 2.7 + (chunks ? 0.28 : 0.7) * steps * (tiles > 1 ? tiles : 1) + 0.12 * out_mb;
+  }
+  const double device = mats * (3.5 + 0.44 * b_mb) + count * gemm;
+  const double host = 2.5 * (2 * mats + count);
+  return one <= (device > host ? device : host);
 }
 
 hipError_t launch_gemm_batched(

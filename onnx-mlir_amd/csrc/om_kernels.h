@@ -191,7 +191,7 @@ struct GemmBatch {
 bool gemm_batched_ok(const GemmArgs &g, const GemmBatch &b);
 // Whether it is the faster way, against packing each matrix of B and
 // multiplying entry by entry with the kernels of launch_gemm.
-bool gemm_batched_pays(const GemmArgs &g);
+bool gemm_batched_pays(const GemmArgs &g, const GemmBatch &b);
 hipError_t launch_gemm_batched(hipStream_t s, const GemmArgs &g, const GemmBatch &b);
 
 // Whether launch_gemm can take an f32 activation of this shape in GemmArgs::X:

@@ -1522,7 +1522,7 @@ void run_matmul(const MatmulSpec &sp) {
     // zero points given per matrix ([.., M, 1] / [.., 1, N]) move with it
     gb.a_zp_per_matrix = azl > M;
     gb.b_zp_per_matrix = bzl > N;
-    if (gemm_batched_ok(g, gb) && gemm_batched_pays(g)) {
+    if (gemm_batched_ok(g, gb) && gemm_batched_pays(g, gb)) {
       call.check(launch_gemm_batched(call.c.stream, g, gb), sp.op);
       call.finish();
       return;

@@ -503,3 +503,52 @@ def test_few_rows_tile_choice(rt, oracle, M, K, N, layer, product):
     got = rt.MatMulInteger(q, B, z, bz)
     assert product in rt.last_gemm_kernel(), rt.last_gemm_kernel()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("count,M,K,N,shared,one_launch", [
+    (1, 1, 8192, 128, False, False), (1, 16, 4096, 1024, False, False), (1, 64, 2048, 128, False, False), (4, 1, 8192, 128, False, False),
+    (2, 33, 8192, 100, True, False), (1, 130, 4096, 128, False, False), (3, 8, 4099, 130, False, True), (8, 1, 4096, 128, False, True),
+    (1, 16, 128, 1024, False, True), (32, 33, 1024, 64, True, True), (3, 130, 512, 130, False, True)])
+def test_batched_products_of_few_entries(rt, oracle, count, M, K, N, shared, one_launch):
+    """A batched right-hand side with few entries and a long K goes to the kernels
+    that split K over waves (one launch of few blocks took up to five times as
+    long); either way the products are the oracle's, zero points per tensor and
+    per matrix."""
+    rng = np.random.default_rng(K + N + count)
+    A, B = _rand_q(rng, np.uint8, (count, M, K)), _rand_q(rng, np.int8, (1 if shared else count, K, N))
+    for az, bz in ((_rand_q(rng, np.uint8, ()), _rand_q(rng, np.int8, ())),
+                   (_rand_q(rng, np.uint8, A.shape[:2] + (1,)), _rand_q(rng, np.int8, B.shape[:1] + (1, N)))):
+        got = rt.MatMulInteger(A, B, az, bz)
+        assert (rt.last_gemm_kernel() == "k_gemm_i8_batched") == one_launch, rt.last_gemm_kernel()
+        for e in range(count):
+            eb = 0 if shared else e
+            za, zb = (az, bz) if az.ndim == 0 else (az[e].reshape(M), bz[eb].reshape(N))
+            assert np.array_equal(got[e], mm(oracle, A[e], B[eb], np.atleast_1d(za), np.atleast_1d(zb))), e
+
+
+def test_batched_products_matrix_by_matrix(rt):
+    """More batch dimensions that alternate between the operands than one launch
+    addresses: packed and multiplied matrix by matrix, the operands' matrices and
+    zero points found through every dimension's stride."""
+    rng = np.random.default_rng(5)
+    M, K, N = 5, 48, 20
+    A, B = _rand_q(rng, np.uint8, (2, 1, 2, 1, 3, M, K)), _rand_q(rng, np.int8, (1, 2, 1, 3, 1, K, N))
+    az, bz = _rand_q(rng, np.uint8, A.shape[:-1] + (1,)), _rand_q(rng, np.int8, B.shape[:-2] + (1, N))
+    for za, zb in ((None, None), (az, bz)):
+        got = rt.MatMulInteger(A, B, za, zb)
+        assert rt.last_gemm_kernel() != "k_gemm_i8_batched"
+        a64, b64 = (v.astype(np.int64) - (0 if z is None else z.astype(np.int64)) for v, z in ((A, za), (B, zb)))
+        assert np.array_equal(got, np.matmul(a64, b64))
+
+
+def test_batched_products_in_two_launches(rt):
+    """More blocks than one launch takes (2^20 entries of 5 tiles): the second
+    launch's entries start where the first one's end."""
+    rng = np.random.default_rng(6)
+    E, M = 1 << 20, 257
+    A, B = rng.integers(0, 256, (E, M, 1), np.uint8), rng.integers(-128, 128, (E, 1, 1), np.int8)
+    got = rt.MatMulInteger(A, B, np.uint8(7), np.int8(-3))
+    assert rt.last_gemm_kernel() == "k_gemm_i8_batched"
+    for at in range(0, E, 1 << 17):
+        part = slice(at, at + (1 << 17))
+        assert np.array_equal(got[part], (A[part].astype(np.int32) - 7) * (B[part].astype(np.int32) + 3)), at
