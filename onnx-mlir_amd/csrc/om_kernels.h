@@ -32,7 +32,8 @@ struct DqlScratch {
   float *partial_min; // [max_blocks]
   float *partial_max; // [max_blocks]
   unsigned *counter;  // [16], zeroed once: [0] two-pass arrivals, [8] set if
-                      // the exchange of the one-launch kernel ever timed out
+                      // the exchange of the one-launch kernel ever timed out,
+                      // [9] if it did and the op was redone on the GPU
   int grid_blocks;    // dql_grid_blocks(), or 0 to disable the one-launch path
   unsigned spin_limit; // polls a thread of the one-launch kernel waits for
                        // another block's result before giving up
@@ -93,7 +94,8 @@ hipError_t launch_minmax_limits(hipStream_t s, DqlScratch &scratch,
 struct GridExchange {
   unsigned long long *slots;
   unsigned epoch;
-  unsigned *failed;
+  unsigned *failed;   // non-zero: a launch wrote nothing
+  unsigned *repaired; // non-zero: one wrote nothing and was redone behind it
   unsigned spin_limit;
 };
 bool dql_exchange_begin(hipStream_t s, DqlScratch &scratch, GridExchange &x);

@@ -1710,8 +1710,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_dql_small(
 // at most one such kernel in flight, so its blocks become resident together
 // as soon as older work has drained (a cooperative launch would guarantee
 // that, but costs about 30 us per launch on this platform).  The wait for the
-// other blocks is bounded all the same: a block that gives up raises `failed`
-// and writes nothing.
+// other blocks is bounded all the same: a block that gives up stores its launch
+// number to `failed` and writes nothing.
 //
 // Where the time goes, [4096, 768] / [4096, 3072] on MI355X, microseconds
 // since the first block started (median block): own minimum and maximum known
@@ -1897,7 +1897,7 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
   if (!s_ok) {
     if (threadIdx.x == 0)
       __hip_atomic_store(
-          failed, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          failed, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return;
   }
   lo = s_lo[0];
@@ -1930,6 +1930,73 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
   else
     store(std::false_type{});
   if (gtid < 3 && te < n)
+    y[te] = (uint8_t)(quant_one<false, true>(tail, scale, zpf) ^ (flip & 0xFFu));
+}
+
+// Up to this many float4 per thread a give-up is the host's to report or to redo.
+// Larger tensors have only ever been two launches that depend on nothing, and are
+// redone here.  The launch in which nothing is to be done takes 1.5 us: 17 Mi
+// elements 18.8 -> 20.4 us (two passes over x 31.2), 64 Mi 75.0 -> 76.5 (94.6).
+constexpr int kGridReported = 32;
+
+// Behind k_dql_grid for those: nothing at all unless one of its blocks gave up in
+// launch `epoch`.  Then every block looks for the minimum and maximum of the whole
+// tensor itself (no exchange that could fail again) and quantizes its share.
+__global__ __launch_bounds__(kGridThreads) void k_dql_repair(
+    const float *__restrict__ x, int64_t n, uint8_t *__restrict__ y,
+    float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, uint32_t flip,
+    const unsigned *failed, unsigned epoch) {
+  if (*failed != epoch)
+    return;
+  constexpr int kWaves = kGridThreads / 64, kUnroll = 8;
+  __shared__ float s_lo[kWaves], s_hi[kWaves];
+  const int64_t nvec = n >> 2;
+  const f4a *__restrict__ x4 = (const f4a *)x;
+  float lo = __builtin_inff(), hi = -__builtin_inff();
+  for (int64_t base = 0; base < nvec; base += kGridThreads * kUnroll) {
+    f4a q[kUnroll];
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) {
+      // (one past the end is the last one again)
+      const int64_t i = base + j * kGridThreads + threadIdx.x;
+      q[j] = x4[i < nvec ? i : nvec - 1];
+    }
+#pragma unroll
+    for (int j = 0; j < kUnroll; ++j) {
+      lo = __builtin_fminf(lo, __builtin_fminf(__builtin_fminf(q[j].x, q[j].y),
+                                   __builtin_fminf(q[j].z, q[j].w)));
+      hi = __builtin_fmaxf(hi, __builtin_fmaxf(__builtin_fmaxf(q[j].x, q[j].y),
+                                   __builtin_fmaxf(q[j].z, q[j].w)));
+    }
+  }
+  const int64_t te = (nvec << 2) + threadIdx.x;
+  const float tail = te < n ? x[te] : __builtin_nanf("");
+  lo = wave_min(__builtin_fminf(lo, tail));
+  hi = wave_max(__builtin_fmaxf(hi, tail));
+  if ((threadIdx.x & 63) == 0) {
+    s_lo[threadIdx.x >> 6] = lo;
+    s_hi[threadIdx.x >> 6] = hi;
+  }
+  __syncthreads();
+  lo = s_lo[0];
+  hi = s_hi[0];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w) {
+    lo = __builtin_fminf(lo, s_lo[w]);
+    hi = __builtin_fmaxf(hi, s_hi[w]);
+  }
+  float scale, zpf;
+  dynamic_params(lo, hi, scale, zpf);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scale_out[0] = scale;
+    zp_out[0] = (uint8_t)(uint32_t)zpf;
+  }
+  const float recip = 1.0f / scale;
+  for (int64_t i = (int64_t)blockIdx.x * kGridThreads + threadIdx.x; i < nvec;
+       i += (int64_t)gridDim.x * kGridThreads)
+    ((uint32_t *)y)[i] =
+        quant_four<false, true, false>(x4[i], scale, recip, zpf, flip);
+  if (blockIdx.x == 0 && te < n)
     y[te] = (uint8_t)(quant_one<false, true>(tail, scale, zpf) ^ (flip & 0xFFu));
 }
 
@@ -2500,15 +2567,25 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
       // that stream is still busy, this call takes the two-launch path.
       GridExchange ex;
       if (dql_exchange_begin(s, scratch, ex)) {
+        const bool repaired = nvec > kGridReported * total;
+        unsigned *const failed = repaired ? ex.repaired : ex.failed;
         hipLaunchKernelGGL(fn_launch, dim3((unsigned)blocks),
             dim3(kGridThreads), 0, s, x, n, prefix, y, scale, zp, flip, ex.slots,
-            ex.epoch, ex.failed, ex.spin_limit);
-        const hipError_t e = hipGetLastError();
-        dql_exchange_end(s, e == hipSuccess);
-        if (e != hipSuccess || prefix == 0)
-          return e;
-        return quantize_dispatch<false>(
-            s, x, 1, 1, prefix * 4, scale, zp, y, flip);
+            ex.epoch, failed, ex.spin_limit);
+        hipError_t e = hipGetLastError();
+        const bool launched = e == hipSuccess;
+        // (If a block gave up, the front is quantized with parameters that were
+        // not written, and k_dql_repair writes all of y again.)
+        if (e == hipSuccess && prefix)
+          e = quantize_dispatch<false>(
+              s, x, 1, 1, prefix * 4, scale, zp, y, flip);
+        if (e == hipSuccess && repaired) {
+          k_dql_repair<<<scratch.grid_blocks, kGridThreads, 0, s>>>(
+              x, n, y, scale, zp, flip, failed, ex.epoch);
+          e = hipGetLastError();
+        }
+        dql_exchange_end(s, launched);
+        return e;
       }
     }
   }
@@ -2573,6 +2650,7 @@ bool dql_exchange_begin(hipStream_t s, DqlScratch &scratch, GridExchange &x) {
   x.slots = scratch.grid_slots; // 16-byte aligned
   x.epoch = scratch.epoch;
   x.failed = scratch.counter + 8;
+  x.repaired = scratch.counter + 9;
   x.spin_limit = scratch.spin_limit;
   return true;
 }

@@ -447,29 +447,26 @@ struct Ctx {
     return true;
   }
 
-  // Call after the stream has been synchronised.  The one-launch
-  // DynamicQuantizeLinear kernel raises a flag if its grid barrier ever timed
-  // out (its output is then missing); report that and stop using the kernel.
-  // Whether a one-launch kernel of this thread gave up since the last check
-  // (call after the stream has been synchronised).  If so the flag is
-  // cleared and the one-launch kernel is not used again by this thread.
-  // Whether the one-launch kernel raised its flag since the last look.  The
-  // flag is only fetched (a blocking 4-byte copy, tens of microseconds) when
-  // such a kernel has been launched since.
+  // Whether the output of a one-launch kernel of this thread is missing, because
+  // its blocks gave up waiting for one another since the last look (call after
+  // the stream has been synchronised).  If any gave up, also one whose op was
+  // then redone on the GPU, the flags are cleared and the one-launch kernels are
+  // not used again by this thread.  The flags are only fetched (a blocking copy,
+  // tens of microseconds) when such a kernel has been launched since.
   bool dql_unchecked = false;
   bool dql_gave_up() {
     if (!ready || dql.grid_blocks == 0 || !dql_unchecked)
       return false;
     dql_unchecked = false;
-    unsigned flag = 0;
-    if (hipMemcpy(&flag, dql.counter + 8, sizeof(flag),
+    unsigned flag[2] = {0, 0};
+    if (hipMemcpy(flag, dql.counter + 8, sizeof(flag),
             hipMemcpyDeviceToHost) != hipSuccess)
       return false;
-    if (!flag)
+    if (!flag[0] && !flag[1])
       return false;
     (void)hipMemset(dql.counter, 0, 256);
     dql.grid_blocks = 0;
-    return true;
+    return flag[0] != 0;
   }
   bool dql_barrier_ok() {
     if (!dql_gave_up())
@@ -1048,16 +1045,18 @@ bool noalloc_barrier_ok() {
     sp = g_scratch_ptr[dev];
   }
   unsigned *counter = (unsigned *)((char *)sp + sizeof(float) * 2 * kNoAllocBlocks);
-  unsigned flag = 0;
-  if (hipMemcpy(&flag, counter + 8, sizeof(flag), hipMemcpyDeviceToHost) !=
+  unsigned flag[2] = {0, 0};
+  if (hipMemcpy(flag, counter + 8, sizeof(flag), hipMemcpyDeviceToHost) !=
           hipSuccess ||
-      !flag)
+      (!flag[0] && !flag[1]))
     return true;
   (void)hipMemset(counter, 0, 256);
   {
     std::lock_guard<std::mutex> lk(g_scratch_mutex);
     g_scratch_no_grid[dev] = true;
   }
+  if (!flag[0]) // redone on the GPU
+    return true;
   fail(EIO, "DynamicQuantizeLinearNoAlloc: the blocks of the one-launch "
             "kernel timed out waiting for one another (grid barrier); its "
             "output was not written");

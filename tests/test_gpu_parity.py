@@ -533,6 +533,56 @@ def test_dynamic_quantize_barrier_timeout_is_reported():
     assert "ERROR-OK" in out.stdout and "RECOVERED" in out.stdout, out.stdout + out.stderr
 
 
+def test_dynamic_quantize_of_large_tensors_survives_a_barrier_timeout():
+    """Beyond 16 Mi elements (32 float4 for each of 512 threads on every CU) a call
+    on GPU tensors must not depend on the grid barrier: with the bound forced to
+    zero the op is redone behind the kernel that gave up, on the GPU.  Kept whole,
+    with a front that is reduced first, ragged; the fused layer (stored minus
+    128); the entry point that allocates nothing; no error at the synchronisation."""
+    import subprocess, sys, textwrap
+    code = textwrap.dedent("""
+        import sys, numpy as np
+        sys.path.insert(0, %r)
+        import om_mi355x as rt
+        unit = rt.device_info()["cus"] * 512 * 4
+        big = np.random.default_rng(0).normal(0, 1, 60 * unit).astype(np.float32)
+        def want(x):
+            lo, hi = np.float32(min(x.min(), 0)), np.float32(max(x.max(), 0))
+            s = (hi - lo) / np.float32(255)
+            z = np.float32(np.rint(np.clip(np.float32(0) - lo / s, 0, 255)))
+            return np.clip(np.rint(x / s) + z, 0, 255).astype(np.uint8), s, z
+        def check(what, got, x):
+            y, s, z = want(x)
+            print(what, np.array_equal(got[0].numpy(), y) and np.float32(got[1].numpy()) == s and int(got[2].numpy()) == int(z))
+        mode = sys.argv[1]
+        if mode == "fused":
+            x = big[:34 * unit].reshape(-1, 1024)
+            b = np.ones((1024, 8), np.int8)
+            dx, db, ds = (rt.DeviceArray.from_numpy(v) for v in (x, b, np.float32([1.0])))
+            out = rt.DynQuantMatMulDequant(dx, db, None, ds)
+            rt.synchronize()
+            y, s, z = want(x)
+            ref = (y.astype(np.int32).sum(1) - 1024 * np.int32(z)).astype(np.float32) * (s * np.float32(1.0))
+            print("layer", np.array_equal(out.numpy(), np.repeat(ref[:, None], 8, 1)))
+        else:
+            rt.synchronize()
+            inputs = [big[:33 * unit], big[:59 * unit + 3], big[:56 * unit + 1]]
+            arrays = [rt.DeviceArray.from_numpy(x) for x in inputs]
+            if mode == "noalloc":
+                outs = [(rt.DeviceArray(x.shape, np.uint8), rt.DeviceArray((), np.float32), rt.DeviceArray((), np.uint8)) for x in inputs]
+                got = [rt.DynamicQuantizeLinearNoAlloc(a, o) for a, o in zip(arrays, outs)]
+            else:
+                got = [rt.DynamicQuantizeLinear(a) for a in arrays]
+            rt.synchronize()
+            for x, g in zip(inputs, got):
+                check(x.size, g, x)
+    """ % os.path.join(os.path.dirname(HERE), "onnx-mlir_amd"))
+    env = dict(os.environ, OM_MI355X_DQL_SPIN_LIMIT="0")
+    for mode, lines in (("device", 3), ("noalloc", 3), ("fused", 1)):
+        out = subprocess.run([sys.executable, "-c", code, mode], env=env, capture_output=True, text=True, timeout=110)
+        assert out.stdout.count("True") == lines and "False" not in out.stdout, mode + out.stdout + out.stderr
+
+
 def test_perf_report_lines_have_the_reference_format(tmp_path):
     """OM_MI355X_PERF_REPORT=1 makes every entry point synchronous and prints a
     before / after pair per call in the format of src/Runtime/OMInstrument.c:164
