@@ -1703,8 +1703,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_dql_small(
 }
 
 // Tensors of up to 56 float4 per thread of a grid that fills the device once
-// (28 Mi elements): the whole op in one launch.  Larger ones keep that much.  Every thread keeps
-// its elements in registers while the blocks exchange their minima and maxima,
+// (28 Mi elements): the whole op in one launch; up to kGridPrefixMost elements that
+// much of the tensor.  Every thread keeps its elements in registers while the blocks exchange their minima and maxima,
 // so x is read once, nothing but the result is written, and there is one
 // launch instead of two.  The grid is one block per CU, and the launcher keeps
 // at most one such kernel in flight, so its blocks become resident together
@@ -1729,14 +1729,20 @@ __global__ __launch_bounds__(kSmallThreads) void k_dql_small(
 // streaming stores slow down the GEMM that reads the result next by 3 us.
 // Buffer accesses whose offsets are one lane register and a scalar: with 64-bit
 // indices 32 float4 took 220 registers and 48 spilled.
-// Against two launches that read x twice: 22.5 Mi elements 40.0 -> 25.8 us,
-// 28 Mi 48.3 -> 31.5; beyond, where all but the last 28 Mi are still read twice,
-// 32 Mi 53.3 -> 40.6, 64 Mi 95 -> 87.7, 256 Mi 372 -> 360.
+// Against two launches that read x twice (k_dql_repair included; the same tensor
+// again / one of three in turn): 22 Mi elements 38.0 -> 23.1 us / 41.3 -> 29.0, 28 Mi
+// 45.2 -> 26.5 / 48.8 -> 33.3; beyond, where all but the last 28 Mi are still read
+// twice, 32 Mi 50.6 -> 35.3 / 53.8 -> 43.4, 64 Mi 94.6 -> 76.5 / 96.5 -> 89.8.
 constexpr int kGridThreads = 512;
 // 56 float4 are 224 of the 256 registers that two waves per SIMD leave a lane.
 constexpr int kGridMaxPerThread = 56; // float4
+// What stays on chip becomes a small part: 160 Mi elements 224 -> 211 us / 239 -> 225,
+// 192 Mi 272 -> 264 / 287 -> 274, but 224 Mi 316 -> 322 / 332 -> 323 and 256 Mi 360 ->
+// 371 / 379 -> 372.  Larger tensors take two launches, and hold up nobody's
+// exchange meanwhile.
+constexpr int64_t kGridPrefixMost = (int64_t)192 << 20;
 
-// PREFIX: tensors beyond that.  The first `prefix` float4 are only reduced, the
+// PREFIX: tensors beyond kGridMaxPerThread.  The first `prefix` float4 are only reduced, the
 // ones after them (NV per thread of the grid) are kept and quantized as above;
 // the launcher quantizes the prefix with a launch of its own.
 template <int NV, bool PREFIX>
@@ -2557,7 +2563,7 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
       fn_launch = k_dql_grid<32, false>;
     else if (nvec <= kGridMaxPerThread * total)
       fn_launch = k_dql_grid<kGridMaxPerThread, false>;
-    else {
+    else if (n <= kGridPrefixMost) {
       fn_launch = k_dql_grid<kGridMaxPerThread, true>;
       prefix = nvec - kGridMaxPerThread * total;
     }
@@ -2676,7 +2682,7 @@ hipError_t launch_fill_u32(hipStream_t s, uint32_t *p, int64_t n, uint32_t v) {
 
 int dql_grid_blocks() {
   // Blocks of k_dql_grid that are resident at once: one per CU if the
-  // occupancy calculator agrees that one fits (32 float4 per thread).
+  // occupancy calculator agrees that one fits (kGridMaxPerThread float4 per thread).
   int dev = 0, cus = 0, per = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=

@@ -583,6 +583,31 @@ def test_dynamic_quantize_of_large_tensors_survives_a_barrier_timeout():
         assert out.stdout.count("True") == lines and "False" not in out.stdout, mode + out.stdout + out.stderr
 
 
+def test_dynamic_quantize_beyond_192_mi_elements_takes_two_launches():
+    """What stays on chip is too small a part of such tensors: no grid barrier is
+    involved, so with its bound forced to zero one leaves the thread's one-launch
+    kernel switched on, and the next small tensor runs into it."""
+    import subprocess, sys, textwrap
+    code = textwrap.dedent("""
+        import sys
+        sys.path.insert(0, %r)
+        import om_mi355x as rt
+        for n in ((192 << 20) + 4, 192 << 20):
+            rt.DynamicQuantizeLinear(rt.DeviceArray((n,), "float32"))
+            rt.synchronize()
+            rt.DynamicQuantizeLinear(rt.DeviceArray((4096, 768), "float32"))
+            try:
+                rt.synchronize()
+                print("NO-ERROR")
+            except rt.RuntimeError_:
+                print("ERROR")
+                break
+    """ % os.path.join(os.path.dirname(HERE), "onnx-mlir_amd"))
+    env = dict(os.environ, OM_MI355X_DQL_SPIN_LIMIT="0")
+    out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=110)
+    assert out.stdout.split() == ["ERROR"], out.stdout + out.stderr
+
+
 def test_perf_report_lines_have_the_reference_format(tmp_path):
     """OM_MI355X_PERF_REPORT=1 makes every entry point synchronous and prints a
     before / after pair per call in the format of src/Runtime/OMInstrument.c:164
