@@ -552,3 +552,37 @@ def test_batched_products_in_two_launches(rt):
     for at in range(0, E, 1 << 17):
         part = slice(at, at + (1 << 17))
         assert np.array_equal(got[part], (A[part].astype(np.int32) - 7) * (B[part].astype(np.int32) + 3)), at
+
+
+@pytest.mark.parametrize("front", ["one short of a trip", "a trip", "one more", "two trips and a part"])
+def test_dynamic_quantize_with_a_front_that_is_reduced_first(rt, oracle, front):
+    """Tensors whose front does not fit on chip: 56 float4 for each of 512 threads
+    per CU are kept, what lies in front is reduced in trips of three float4 a
+    thread and quantized by a second launch.  The extremes lie in turn at the last
+    element of the front, at the first kept one and in the front's last trip."""
+    threads = rt.device_info()["cus"] * 512
+    trip = 3 * threads
+    n_front = {"one short of a trip": trip - 1, "a trip": trip, "one more": trip + 1, "two trips and a part": 2 * trip + 777}[front]
+    n = (56 * threads + n_front) * 4 + n_front % 4
+    rng = np.random.default_rng(n_front)
+    x = rng.standard_normal(n, dtype=np.float32)
+    for at in (4 * n_front - 1, 4 * n_front, 4 * (n_front - n_front % trip) - 5 if n_front > 2 * trip else 4 * n_front - 9):
+        x[at], x[at + 2] = 11.0 + at % 3, -9.0
+        wy, ws, wz = oracle.dynamic_quantize_linear(x)
+        dy, ds, dz = rt.DynamicQuantizeLinear(rt.DeviceArray.from_numpy(x))
+        rt.synchronize()
+        assert ds.numpy().view(np.uint32) == np.float32(ws).view(np.uint32) and int(dz.numpy()) == int(wz)
+        assert np.array_equal(dy.numpy(), wy), at
+        x[at] = x[at + 2] = 0.5
+
+
+def test_layer_whose_rows_do_not_fit_on_chip(rt, oracle):
+    """The fused layer's rows, stored minus 128, when their front is quantized by a
+    launch of its own."""
+    rng = np.random.default_rng(3)
+    K, N = 1024, 24
+    M = (rt.device_info()["cus"] * 512 * 4 * 56) // K + 1111
+    x, B = rng.standard_normal((M, K), dtype=np.float32), _rand_q(rng, np.int8, (K, N))
+    ws = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    q, s, z = oracle.dynamic_quantize_linear(x)
+    assert same_f32(rt.DynQuantMatMulDequant(x, B, None, ws), oracle.dequant_epilogue(mm(oracle, q, B, z, None), s, ws))
