@@ -38,6 +38,8 @@
 // with bits 2..3 of the row (bank-conflict free writes and operand reads); Bp
 // tiles in LDS keep their global order.
 
+#include <math.h>
+
 #include "gemm_common.h"
 #include "gemm_epilogue.h"
 
@@ -49,7 +51,7 @@ using namespace gemm;
 
 namespace {
 
-// Products of few tiles and many K steps are split along K (gemm_k_splits): the
+// Products of few tiles and many K steps are split along K (split_plan): the
 // blocks of one blockIdx.y multiply `steps` steps of K and write their int32
 // sums as if they were the whole result, to an array of their own `stride`
 // elements after the previous one's; k_sum_parts adds these up, mod 2^32 as all
@@ -1197,13 +1199,6 @@ __global__ __launch_bounds__(256) void k_sum_parts(
     }
 }
 
-// How a product is split along K (KSplit): the tile, the number of parts.
-struct SplitPlan {
-  int parts = 1; // 1: not at all
-  int steps = 0; // K steps of a part
-  bool any = false, narrow = false; // k_gemm_i8; 64-column tiles of k_gemm_i8_dma
-};
-
 int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
 
 // What bounds a product whose tiles cover a part of the CUs is the chain of its
@@ -1219,31 +1214,37 @@ int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
 // 2048 x 11008 x 768 48.1 / 37.6, 128 x 1536 x 300 9.5 / 7.8; left alone by the
 // rule: int32 2048 x 1280 x 1024 9.5 / 18.5, layer 512 x 1536 x 1536 14.1 /
 // 17.5, 128 x 4096 x 11008 23.3 / 23.7.
-SplitPlan split_plan(const GemmArgs &g, int a_mode) {
-  SplitPlan best;
-  const char *force = getenv("OM_MI355X_GEMM_TILE");
-  if (g.X || (force && force[0]) || g.M <= 0 || g.N <= 0 || g.K <= 0 ||
-      g.M * g.K < 16 || g.M * g.N > ((int64_t)1 << 22) ||
+// The plan is made once per product (GemmArgs::split), after the tests that turn
+// most products away; parts are looked for around the minimum of the model.
+GemmSplit split_plan(const GemmArgs &g, int a_mode) {
+  GemmSplit best;
+  const int64_t KT = round_up(g.K, kGemmBK) / kGemmBK;
+  const int64_t tm = (g.M + 127) / 128, t128 = tm * ((g.N + 127) / 128);
+  if (KT < 8 || t128 > 128 || t128 <= 0 || g.X ||
+      g.M * g.N > ((int64_t)1 << 22) || g.M * g.K < 16 ||
       skinny_ok(g.M, g.K, g.A))
     return best;
   const bool any = !gemm_fast_path(g.M, g.K, g.A);
-  const int64_t KT = round_up(g.K, kGemmBK) / kGemmBK;
-  const int64_t tm = (g.M + 127) / 128, t128 = tm * ((g.N + 127) / 128);
-  if (KT < 8 || t128 > 128 ||
-      (!any && g.K % 64 == 0 &&
-          (flight_ok(g, a_mode) || (wreg_ok(g) && wreg_pays(g.M, g.N)))))
+  if (!any && g.K % 64 == 0 &&
+      (flight_ok(g, a_mode) || (wreg_ok(g) && wreg_pays(g.M, g.N))))
+    return best;
+  const char *force = getenv("OM_MI355X_GEMM_TILE");
+  if (force && force[0])
     return best;
   const double kWide = 0.28, kNarrow = 0.22, kAny = 0.5;
+  const double us_part = 1.8e-6 * (double)(g.M * g.N);
   double least = 0.9 * (double)KT * (any ? kAny : g.N > 64 ? kNarrow : kWide);
   for (int narrow = 0; narrow <= (any || g.N <= 64 ? 0 : 1); ++narrow) {
     const int64_t tiles = narrow ? tm * ((g.N + 63) / 64) : t128;
     const int64_t most = 256 / tiles < KT / 4 ? 256 / tiles : KT / 4;
-    for (int64_t parts = 2; parts <= most; ++parts) {
-      const int64_t steps = (KT + parts - 1) / parts;
-      if ((KT + steps - 1) / steps != parts)
-        continue; // (a part without a step)
-      const double us = (double)steps * (any ? kAny : narrow ? kNarrow : kWide) +
-                        2.5 + 1.8e-6 * (double)(parts * g.M * g.N);
+    const double us_step = any ? kAny : narrow ? kNarrow : kWide;
+    // steps * us_step + parts * us_part is least where both are equal
+    const int64_t around = (int64_t)sqrt((double)KT * us_step / us_part);
+    const int64_t low = around - 2 < most - 4 ? around - 2 : most - 4;
+    for (int64_t p = low < 2 ? 2 : low; p <= most && p <= around + 3; ++p) {
+      const int64_t steps = (KT + p - 1) / p;
+      const int64_t parts = (KT + steps - 1) / steps; // (none without a step)
+      const double us = (double)steps * us_step + 2.5 + us_part * (double)parts;
       if (us < least) {
         least = us;
         best.parts = (int)parts;
@@ -1271,7 +1272,8 @@ const char *dma_name(bool narrow, bool ragged, bool split) {
 
 template <int A_MODE, int EPI>
 hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
-    int Kpad, const SplitPlan &p) {
+    int Kpad) {
+  const GemmSplit &p = g.split;
   const uint8_t *A = (const uint8_t *)g.A;
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
   const int tiles_m = (M + 127) / 128;
@@ -1353,11 +1355,8 @@ hipError_t gemm_launch_cfg(
   // N=4096 M=64: 15.0 / 37.7; K=768 N=3072 M=64: 4.2 / 6.0).
   if (skinny_ok(g.M, g.K, g.A) && !(force && force[0]))
     return launch_gemm_skinny(st, g, ep, A_MODE);
-  if (g.parts) {
-    const SplitPlan plan = split_plan(g, A_MODE);
-    if (plan.parts > 1)
-      return launch_split<A_MODE, EPI>(st, g, ep, Kpad, plan);
-  }
+  if (g.parts && g.split.parts > 1)
+    return launch_split<A_MODE, EPI>(st, g, ep, Kpad);
   const int tiles_m = (int)((g.M + 127) / 128);
   const int tiles_n128 = (int)((g.N + 127) / 128);
   if (!gemm_fast_path(g.M, g.K, g.A)) {
@@ -1514,10 +1513,9 @@ int gemm_quantizes_rows(int64_t M, int64_t K, int64_t N, const void *x) {
   return flight_quantizes_rows(M, K, N, x) ? 2 : 0;
 }
 
-size_t gemm_parts_bytes(const GemmArgs &g) {
-  const SplitPlan p =
-      split_plan(g, (g.X || g.a_preshifted) ? 2 : (g.a_unsigned ? 1 : 0));
-  return p.parts > 1 ? (size_t)p.parts * part_stride(g) * 4 : 0;
+size_t gemm_plan_split(GemmArgs &g) {
+  g.split = split_plan(g, (g.X || g.a_preshifted) ? 2 : (g.a_unsigned ? 1 : 0));
+  return g.split.parts > 1 ? (size_t)g.split.parts * part_stride(g) * 4 : 0;
 }
 
 const char *last_gemm_kernel() { return t_last_kernel; }

@@ -116,6 +116,13 @@ inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 hipError_t launch_pack_b(hipStream_t s, const void *B, bool b_unsigned,
     int64_t K, int64_t N, int8_t *Bp, int32_t *colsum);
 
+// How a product is split along K: into `parts` (1: not at all) of `steps` K steps
+// each, in k_gemm_i8 (any) or k_gemm_i8_dma, there in 64-column tiles (narrow).
+struct GemmSplit {
+  int parts = 1, steps = 0;
+  bool any = false, narrow = false;
+};
+
 struct GemmArgs {
   // If set (see gemm_quantizes_rows): the activation as f32 [M,K]; the kernel
   // quantizes it itself as DynamicQuantizeLinear would (A, a_zp and a_scale
@@ -163,14 +170,15 @@ struct GemmArgs {
   // With X, optional: minimum and maximum of X as an earlier product's
   // y_limits gave them; the kernel then does not look for them.
   const float *x_limits;
-  // Optional: gemm_parts_bytes() bytes of scratch, 16-byte aligned, with which
-  // a product of few tiles is split along K.
+  // Optional: gemm_plan_split() bytes of scratch, 16-byte aligned, with which a
+  // product of few tiles is split along K as planned.
   int32_t *parts;
+  GemmSplit split;
 };
 
-// Scratch with which launch_gemm is faster (the arguments as it will get them);
-// 0: none.
-size_t gemm_parts_bytes(const GemmArgs &g);
+// Fills in g.split for the arguments as launch_gemm will get them: the bytes of
+// scratch with which it is faster; 0: none.
+size_t gemm_plan_split(GemmArgs &g);
 hipError_t launch_gemm(hipStream_t s, const GemmArgs &g);
 // Name of the kernel the calling thread's last launch_gemm or
 // launch_gemm_batched chose.

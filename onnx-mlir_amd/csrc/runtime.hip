@@ -857,7 +857,7 @@ struct Call {
   // launch_gemm, with the scratch that makes it faster unless the stream is
   // being captured (a replay would share the scratch with later calls).
   hipError_t gemm(GemmArgs &g) {
-    const size_t bytes = gemm_parts_bytes(g);
+    const size_t bytes = gemm_plan_split(g);
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (bytes && hipStreamIsCapturing(c.stream, &capture) == hipSuccess &&
         capture == hipStreamCaptureStatusNone) {
