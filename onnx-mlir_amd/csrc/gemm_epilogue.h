@@ -18,8 +18,7 @@ namespace gemm {
 // unconditional (indices clamped, absent operands redirected to valid memory
 // and masked afterwards) and all loads precede the stores, so the stores can
 // be issued back to back without waiting on one another.
-// bj: the bias of the column, or -0.0f, which leaves every value (both zeros
-// included) as it is.
+
 // One accumulator to its 8-bit result (kEpiQ8), in the low byte.
 __device__ __forceinline__ uint32_t requantize(
     const EpiParams &ep, uint32_t y, float sj, int32_t yz) {
@@ -34,6 +33,9 @@ __device__ __forceinline__ uint32_t requantize(
   return (uint32_t)v & 0xFF;
 }
 
+// One result, converted and stored at element o of the output.
+// bj: the bias of the column, or -0.0f, which leaves every value (both zeros
+// included) as it is.
 template <int EPI>
 __device__ __forceinline__ void store_one(const EpiParams &ep, int64_t o,
     uint32_t y, float sj, int32_t yz, float bj) {

@@ -14,7 +14,8 @@
 // batches of four steps, or the next batch requested before the wait, leave room
 // for fewer and are slower (1 row, K=4096 N=11008: 8.3 us; four steps 9.1, a
 // second batch on its way 9.3, both 10.3; 16 waves a block 10.7).  Only up to 4
-// rows that arrive quantized are batches of four ahead (9.2 / 9.6 us).
+// rows that arrive quantized, up to 256 blocks, are batches of four ahead
+// (launch_rows).
 // Streaming (nontemporal) loads of the weights: 10.6 against 10.3 us.
 // The epilogue's parameters are requested first and without branches (a wait
 // for a zero point in front of the first weights cost 0.5 us).
@@ -29,8 +30,10 @@
 // minimum and maximum over all of X, scale and zero point from them, the 8-bit
 // values minus 128 into LDS, from where the K loop takes its A operands; the
 // first weights are requested before that starts.  Up to 32 Ki elements that
-// beats a launch of its own in front (8 rows of 4096: 11.2 us against 12.6; 16
-// rows 14 against 13).
+// beats a launch of its own in front (8 rows of 4096: N=4096 6.6 us against 8.1,
+// N=11008 10.2 / 11.3; 16 rows of 2048: N=4096 5.8 / 7.3, N=11008 8.6 / 8.2), except
+// 17 rows and more of K up to 1024, a multiple of 256, which k_gemm_i8_flight_dq
+// could take (32 rows of 1024, N=4096 6.0 / 5.0).
 //
 // Tried and dropped: one launch in which the first blocks of the grid quantize
 // X between them and every block waits for them with its weights already
@@ -53,8 +56,8 @@ constexpr int kSkinnyDqBytes = 32768;
 // wave: a load instruction takes whole rows of the batch (CPR 16-byte chunks
 // each, so every cache line it touches is used completely), the MFMA operands
 // -- 64 bytes of each of 16 rows -- are read back from there, rows CPR * 16 + 16
-// bytes apart to spread them over the banks.  Up to 4 rows the operands are
-// loaded directly: the lanes of the rows that are not there fetch nothing.
+// bytes apart to spread them over the banks.  Otherwise the operands are loaded
+// directly: the lanes of the rows that are not there fetch nothing.
 template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG>
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
     const uint8_t *__restrict__ A, const float *__restrict__ X,

@@ -1738,7 +1738,8 @@ constexpr int kGridThreads = 512;
 constexpr int kGridMaxPerThread = 56; // float4
 // What stays on chip becomes a small part: 160 Mi elements 224 -> 211 us / 239 -> 225,
 // 192 Mi 272 -> 264 / 287 -> 274, but 224 Mi 316 -> 322 / 332 -> 323 and 256 Mi 360 ->
-// 371 / 379 -> 372.  Larger tensors take two launches, and hold up nobody's
+// 371 / 379 -> 372 (256 Mi behind the DequantizeLinear that writes x: both together
+// 556 -> 568).  Larger tensors take two launches, and hold up nobody's
 // exchange meanwhile.
 constexpr int64_t kGridPrefixMost = (int64_t)192 << 20;
 
