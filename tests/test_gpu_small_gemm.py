@@ -586,3 +586,21 @@ def test_layer_whose_rows_do_not_fit_on_chip(rt, oracle):
     ws = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
     q, s, z = oracle.dynamic_quantize_linear(x)
     assert same_f32(rt.DynQuantMatMulDequant(x, B, None, ws), oracle.dequant_epilogue(mm(oracle, q, B, z, None), s, ws))
+
+
+@pytest.mark.parametrize("M,K,N", [(129, 4096, 258), (65, 1537, 66)])
+def test_gelu_of_a_product_split_along_k(rt, oracle, M, K, N):
+    """k_sum_parts applies onnx.Gelu itself: against the oracle's Gelu of the
+    exact product.  Tolerance: 4 units in the last place of erf (2^-22) times
+    |0.5 x|, plus one rounding of the result."""
+    rng = np.random.default_rng(K)
+    x, B = rng.normal(0, 1, (M, K)).astype(np.float32), _rand_q(rng, np.int8, (K, N))
+    ws, bias = rng.uniform(1e-5, 1e-3, N).astype(np.float32), rng.normal(0, 1, N).astype(np.float32)
+    q, s, z = oracle.dynamic_quantize_linear(x)
+    plain = oracle.dequant_epilogue(mm(oracle, q, B, z, None), s, ws)
+    for b, p in ((None, plain), (bias, plain + bias)):
+        got = rt.DynQuantMatMulDequant(x, B, None, ws, b, activation=rt.ACTIVATION_GELU)
+        assert "split" in rt.last_gemm_kernel(), rt.last_gemm_kernel()
+        want = oracle.gelu(p).astype(np.float64)
+        tol = np.abs(0.5 * p.astype(np.float64)) * 2.0 ** -22 + np.abs(want) * 2.0 ** -23 + 1e-45
+        assert (np.abs(got - want) <= tol).all()
