@@ -230,14 +230,11 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
     // that is what the range check looks at.  (A bounds test and a 64-bit
     // address per element instead: 512 x 777 x 1001 12.2 us against 11.8, the
     // fused layer 100 x 1001 x 4096 16.7 against 15.5.)
-    // Not where the registers are all taken: with int32 results this form raised
-    // the spilled registers of k_gemm_i8_dma's 128 x 128 tiles with int8 A from 42
-    // to 68 and of k_gemm_i8_bs from 9 to 12, and every tile paid for it, whole
-    // ones too (int8 A: 2048 x 256 x 4096 8.7 -> 9.4 us, 2048 x 768 x 4096 12.3 ->
-    // 13.0).  Those test every element.  (Parts of K, AUX32 = 0, spill fewer
-    // registers with it: 46 against 50.)
-    constexpr bool kEdge = EPI != kEpiI32 ||
-                           TM * TN <= (A_MODE == 0 && AUX32 != 0 ? 2 : 4);
+    // Not for int32 results of k_gemm_i8_bs, whose registers are all taken: there
+    // this form raised the spilled ones from 9 to 12, and every tile paid for it,
+    // whole ones too (int8 A: 2048 x 256 x 4096 8.7 -> 9.4 us, 2048 x 768 x 4096 12.3
+    // -> 13.0).  Its tiles test every element.
+    constexpr bool kEdge = EPI != kEpiI32 || TM * TN <= 4;
     const int rows = M - mrow0, cols = N - ncol0;
     if (kEdge && (rows <= 0 || cols <= 0))
       return;

@@ -60,10 +60,14 @@ def spills():
 
 
 @pytest.mark.parametrize("kernel,most", [
-    (r"k_gemm_i8_dmaILi128ELi3ELi3ELi0ELi0E", 46),   # int8 A, int32 results: 42, and up to 46 for parts of K
+    # int8 A, int32 results: the epilogue's, behind the K loop.  68 with the edge
+    # stores by descriptor against 42 with a test per element: whole tiles take the
+    # same time either way (4096 x 768 x 768 7.25 / 7.26 us, 4096 x 3072 x 768 16.2 /
+    # 16.2), cut ones less (4096 x 768 x 1001 9.7 / 10.2)
+    (r"k_gemm_i8_dmaILi128ELi3ELi3ELi0ELi0E", 68),
     (r"k_gemm_i8_dmaILi(64|128)ELi3ELi3ELi[12]ELi\dE", 0),
     (r"k_gemm_i8_bsILi4ELi2ELi4ELi4ELi2ELb1ELi\dELi0ELb0E", 9),
-    (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi3ELi0ELi0ELi1E", 46),
+    (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi2E", 0),  # any K, any alignment
     (r"k_gemm_i8_(skinny|batched|flight)I", 0),
 ])
 def test_kernels_spill_no_more_registers(spills, kernel, most):
