@@ -156,9 +156,9 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
     // 28.0 us streaming, 19.4 us plain).
     const __amdgpu_buffer_rsrc_t orsrc =
         __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7FFFFFFF, 0x00020000);
-    auto emit = [&](auto rs_c, auto stream_c, int i, int r, int j,
+    auto emit = [&](auto rs_c, auto stream_c, int i, int r, int j, uint32_t c,
                     int32_t rs_row, int32_t rowb) {
-      uint32_t y = (uint32_t)acc[i][j][r] + cj[j];
+      uint32_t y = (uint32_t)acc[i][j][r] + c;
       if (decltype(rs_c)::value)
         y += (uint32_t)db[j] * (uint32_t)rs_row;
       const int voff = (int)(loff + (uint32_t)(j * 32 * ES));
@@ -193,6 +193,16 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
       // Whole grid inside the matrix: no bounds tests, and every address is
       // (scalar row base) + (one 32-bit lane offset) + constant, so a store
       // costs the few vector instructions that produce its value.
+      // (The corrections pass through an empty statement: the compiler would
+      // otherwise see the same sums in both forms and form them in front of the
+      // branch, all accumulators once more in registers of their own, of which
+      // k_gemm_i8_dma with int32 results spilled 68 and k_gemm_i8_bs 12.)
+      uint32_t c[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        c[j] = cj[j];
+        asm volatile("" : "+v"(c[j]));
+      }
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -204,7 +214,7 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
               (int32_t)((i * 32 + 8 * (r >> 2) + (r & 3)) * N * ES);
 #pragma unroll
           for (int j = 0; j < TN; ++j)
-            emit(rs_c, stream_c, i, r, j, rs_row, rowb);
+            emit(rs_c, stream_c, i, r, j, c[j], rs_row, rowb);
         }
       }
     };
@@ -230,15 +240,10 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
     // that is what the range check looks at.  (A bounds test and a 64-bit
     // address per element instead: 512 x 777 x 1001 12.2 us against 11.8, the
     // fused layer 100 x 1001 x 4096 16.7 against 15.5.)
-    // Not for int32 results of k_gemm_i8_bs, whose registers are all taken: there
-    // this form raised the spilled ones from 9 to 12, and every tile paid for it,
-    // whole ones too (int8 A: 2048 x 256 x 4096 8.7 -> 9.4 us, 2048 x 768 x 4096 12.3
-    // -> 13.0).  Its tiles test every element.
-    constexpr bool kEdge = EPI != kEpiI32 || TM * TN <= 4;
     const int rows = M - mrow0, cols = N - ncol0;
-    if (kEdge && (rows <= 0 || cols <= 0))
+    if (rows <= 0 || cols <= 0)
       return;
-    if (kEdge && (int64_t)N * (32 * TM + 8) * 4 < ((int64_t)1 << 30)) {
+    if ((int64_t)N * (32 * TM + 8) * 4 < ((int64_t)1 << 30)) {
       const int nr = rows < 32 * TM ? rows : 32 * TM;
       const int nc = cols < 32 * TN ? cols : 32 * TN;
       const __amdgpu_buffer_rsrc_t ersrc = __builtin_amdgcn_make_buffer_rsrc(
@@ -283,27 +288,6 @@ __device__ __forceinline__ void gemm_epilogue(v16i (&acc)[TM][TN],
         edge(std::true_type{});
       else
         edge(std::false_type{});
-      return;
-    }
-    if (!kEdge) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int mbase = mrow0 + i * 32 + 4 * lh;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int rr = 8 * (r >> 2) + 4 * lh + (r & 3);
-          const int m = mbase + 8 * (r >> 2) + (r & 3);
-          const int32_t rs_row = __shfl(rsf[i], rr, 64);
-          const int64_t orow = (int64_t)m * N;
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            const uint32_t y = (uint32_t)acc[i][j][r] + cj[j] +
-                               (uint32_t)db[j] * (uint32_t)rs_row;
-            if (m < M && n_[j] < N)
-              store_one<EPI>(ep, orow + n_[j], y, sj[j], yz, bj[j]);
-          }
-        }
-      }
       return;
     }
   }
