@@ -1,0 +1,101 @@
+"""Host model of k_gemm_i8_bs with A copied in stages of two K steps
+(onnx-mlir_amd/csrc/gemm_kernels.hip): where its copies and operand reads go,
+and whether its explicit waits cover what each step reads.  Index arithmetic
+restated for the CPU; and the kernel itself on the GPU, forced, at its edges."""
+import numpy as np
+import pytest
+
+TM, TN, D, NST = 4, 2, 4, 4
+BM, ROW, BK = 32 * TM, 128, 64
+CA, CB = BM // 32, 2 * TN
+LANE = np.arange(64)
+
+
+def slot_of(row, chunk):
+    return row * ROW + ((chunk ^ ((row >> 1) & 7)) << 4)
+
+
+@pytest.mark.parametrize("M,K", [(128, 256), (1, 256), (300, 512), (2048, 11008), (129, 4096)])
+def test_copies_are_in_bounds_and_lie_where_operands_are_read(M, K):
+    pairs = np.arange(K // 128)  # past the last one the descriptor is empty
+    for m0 in {0, (M - 1) // BM * BM}:
+        a_bytes = min(M - m0, BM) * K
+        filled = np.zeros(BM * ROW, bool)
+        for wave in range(4):
+            for h in range(CA):
+                r = (wave * CA + h) * 8 + (LANE >> 3)
+                chunk = (LANE & 7) ^ ((r >> 1) & 7)
+                rc = np.where(m0 + r < M, r, M - 1 - m0)
+                at = pairs[:, None] * ROW + (rc * K + chunk * 16)[None]
+                assert at.min() >= 0 and at.max() + 16 <= a_bytes
+                dst = (wave * CA + h) * 1024 + LANE * 16
+                assert (dst == slot_of(r, chunk)).all()
+                filled[dst[:, None] + np.arange(16)] = True
+        assert filled.all()
+    l32, lh = LANE & 31, LANE >> 5
+    ra = l32 * ROW + ((lh ^ ((l32 >> 1) & 7)) << 4)
+    for h in range(4):
+        for i in range(TM):
+            at = (ra ^ (h << 5)) + i * 32 * ROW
+            assert (at == slot_of(i * 32 + l32, h * 2 + lh)).all()
+            # 16 lanes at a time over the 64 banks: no two in one place
+            for g in range(4):
+                assert len(set((at[g * 16:g * 16 + 16] % 256) // 16)) == 16
+
+
+@pytest.mark.parametrize("KT", [4, 8, 12, 64, 172])
+def test_waits_cover_what_each_step_reads(KT):
+    ops = []  # (kind, asked for, register set or stage), in issue order
+
+    def copy(pair):
+        ops.extend([("a", pair, pair % NST)] * CA)
+
+    def weights(step):
+        ops.extend([("b", step, step % D)] * CB)
+
+    def landed(kind, what, where, young):
+        at = [i for i, o in enumerate(ops) if o[0] == kind and o[2] == where]
+        assert ops[at[-1]][1] == what and at[-1] < len(ops) - young, (kind, what, young)
+
+    young = 2 * CB + CA
+    copy(0)
+    for u in range(D - 1):
+        weights(u)
+        if u == 0:
+            copy(1)
+    landed("a", 0, 0, 3 * CB + CA)
+    for p in range(KT // 2):
+        landed("b", 2 * p, 2 * p % D, young)
+        # overwrites the stage before the last one, which the barrier has freed
+        assert (p + 2) % NST == (p - 2) % NST
+        copy(p + 2)
+        weights(2 * p + 3)
+        landed("b", 2 * p + 1, (2 * p + 1) % D, young)
+        landed("a", p + 1, (p + 1) % NST, young)
+        weights(2 * p + 4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(128, 256, 256), (1, 256, 7), (127, 512, 255), (129, 768, 257), (300, 1280, 513),
+                                   (1024, 512, 768)])
+def test_bs_kernel_at_its_edges(M, K, N, monkeypatch):
+    import oracle_lib
+    import om_mi355x as rt
+    oracle = oracle_lib.load()
+    rng = np.random.default_rng(M + K + N)
+    monkeypatch.setenv("OM_MI355X_GEMM_TILE", "2")
+    for adt, bdt, per in ((np.uint8, np.int8, False), (np.uint8, np.uint8, False), (np.int8, np.uint8, True),
+                          (np.int8, np.int8, True)):
+        def draw(dt, shape):
+            i = np.iinfo(dt)
+            return rng.integers(i.min, i.max + 1, shape, dtype=dt)
+        a, b = draw(adt, (M, K)), draw(bdt, (K, N))
+        az, bz = draw(adt, (M,) if per else ()), draw(bdt, (N,) if per else ())
+        want = oracle.matmul_integer(a, b, az, bz)
+        assert np.array_equal(rt.MatMulInteger(a, b, az, bz), want)
+        if M > 16:
+            assert "k_gemm_i8_bs" in rt.last_gemm_kernel()
+        if not per:
+            s = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+            got = rt.MatMulIntegerDequant(a, b, az, bz, np.float32(0.01), s)
+            assert np.array_equal(got, oracle.dequant_epilogue(want, np.float32(0.01), s))
