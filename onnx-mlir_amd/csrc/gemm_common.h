@@ -246,6 +246,19 @@ bool wreg_pays(int64_t M, int64_t N);
 hipError_t launch_gemm_wreg(hipStream_t st, const GemmArgs &g,
     const EpiParams &ep, int a_mode);
 
+// Elements between the arrays of the parts of a product split along K.
+inline int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
+
+// k_gemm_i8_bs and k_gemm_i8_dma_bs (gemm_bs.hip): Bp streamed into registers, K
+// a multiple of 16 (128 x 256 tiles: of 256) and A 16-byte aligned; split: one
+// of the parts of GemmArgs::split, in 64 x 128 tiles, int32 sums to ep.out.
+enum BsTile : int { kBs128x256, kBs64x256, kBs64x128 };
+bool bs_ok(const GemmArgs &g, BsTile tile);
+hipError_t launch_gemm_bs(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
+    int a_mode, BsTile tile);
+hipError_t launch_gemm_bs_split(hipStream_t st, const GemmArgs &g,
+    const EpiParams &ep, int a_mode);
+
 // k_gemm_i8_skinny (gemm_skinny.hip): up to 64 rows.  skinny_quantizes_rows:
 // whether it takes the f32 activation of a fused layer (GemmArgs::X) and
 // quantizes it in every block.

@@ -23,22 +23,22 @@
 // into registers or copied into LDS.
 //
 // Kernels (all walk K in steps of 64 bytes):
-//   k_gemm_i8_bs         Bp read straight into MFMA operand registers, only
-//                        the A tile goes through LDS (copied there without
-//                        passing through registers); more than one tile per CU
 //   k_gemm_i8_dma        A and Bp tiles copied from global memory straight
 //                        into a ring of three LDS stages; K a multiple of 16
 //   k_gemm_i8            tiles staged through registers, LDS double buffered:
 //                        the general path, any K, any alignment of A
-// and, in files of their own, k_gemm_i8_skinny (M <= 64, weight streaming),
-// k_gemm_i8_flight, k_gemm_i8_wreg and k_gemm_i8_batched.  k_gemm_i8_dma and
-// k_gemm_i8 also multiply parts of K, which k_sum_parts adds up, where a product
-// has few tiles and many K steps (split_plan).
+// and, in files of their own, k_gemm_i8_bs and k_gemm_i8_dma_bs (Bp read straight
+// into MFMA operand registers, only A through LDS), k_gemm_i8_skinny (M <= 64,
+// weight streaming), k_gemm_i8_flight, k_gemm_i8_wreg and k_gemm_i8_batched.
+// k_gemm_i8_dma, k_gemm_i8_dma_bs and k_gemm_i8 also multiply parts of K, which
+// k_sum_parts adds up, where a product has few tiles and many K steps (split_plan).
 // A tiles in LDS have 64-byte rows whose 16-byte chunk index is XOR-swizzled
 // with bits 2..3 of the row (bank-conflict free writes and operand reads); Bp
 // tiles in LDS keep their global order.
 
 #include <math.h>
+
+#include <algorithm>
 
 #include "gemm_common.h"
 #include "gemm_epilogue.h"
@@ -50,26 +50,6 @@ namespace om {
 using namespace gemm;
 
 namespace {
-
-// Products of few tiles and many K steps are split along K (split_plan): the
-// blocks of one blockIdx.y multiply `steps` steps of K and write their int32
-// sums as if they were the whole result, to an array of their own `stride`
-// elements after the previous one's; k_sum_parts adds these up, mod 2^32 as all
-// sums here, and does the epilogue.  Per column and whole-K terms of the
-// zero-point algebra go into the first array only; a block's row sums cover its
-// own K.  The arrays are stored plainly: the next kernel reads them at once
-// (u8 results 127 x 2880 x 768 8.3 us, with streaming stores 9.2; larger ones
-// the same).
-struct KSplit {
-  int steps;
-  int64_t stride;
-};
-// SPLIT: the output of this block's part of K.
-__device__ __forceinline__ EpiParams part_of(const EpiParams &ep, const KSplit &ks) {
-  EpiParams e = ep;
-  e.out = (int32_t *)ep.out + (int64_t)blockIdx.y * ks.stride;
-  return e;
-}
 
 // BM x BN block tile, WGM x WGN waves, each wave a (BM/WGM) x (BN/WGN) tile
 // made of 32x32 MFMA tiles.
@@ -625,295 +605,6 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
         acc, rsp, m0 + wm * WTM, n0 + wn * WTN, M, N, K, ep);
 }
 
-// ---- GEMM, Bp streamed to registers -----------------------------------------
-// The right-hand side is stored in exactly the order the matrix cores consume
-// it: the operand of column tile nt, K step ks, half step sub is one
-// contiguous KiB, 16 bytes per lane.  The four waves of a block sit side by
-// side along N; each owns 32*TN columns that no other wave needs and loads
-// their operands from Bp straight into registers, D steps ahead.  Only the A
-// tile, which all four waves share, goes through LDS, and it gets there
-// without passing through registers (see k_gemm_i8_dma).  Per K step a block
-// therefore moves half as many bytes into LDS as that kernel.
-//
-// A is copied in stages of two K steps, so that a row's piece is one whole
-// 128-byte line: with pieces of 64 bytes every line went into the CU twice.
-// PIPE: the operands of each half step are read one half step early, see the
-// loop.
-template <int TM, int TN, int D, int NST, int MINB, bool PIPE, int A_MODE,
-    int EPI, bool RS>
-__global__ __launch_bounds__(256, MINB) void k_gemm_i8_bs(
-    const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n) {
-  constexpr int BM = 32 * TM, BN = 4 * 32 * TN;
-  constexpr int ROW = 2 * BK;         // bytes of a row in a stage: two K steps
-  constexpr int STAGE = BM * ROW;
-  constexpr int CA = BM / 32; // A copies (1 KiB each) per wave and stage
-  static_assert(BM % 64 == 0, "tile height");
-  // The wait counts below are written for this depth.
-  static_assert(NST == 4 && D == 4 && PIPE, "stages");
-  __shared__ __attribute__((aligned(1024))) uint8_t sm[NST * STAGE];
-
-  int pid = blockIdx.x;
-  {
-    const int nb = gridDim.x;
-    const int per = nb >> 3;
-    if (per > 0 && pid < per * 8)
-      pid = (pid & 7) * per + (pid >> 3);
-  }
-  constexpr int GROUP = 8;
-  const int in_group = GROUP * tiles_n;
-  const int group = pid / in_group;
-  const int first_m = group * GROUP;
-  const int gsize = (tiles_m - first_m < GROUP) ? tiles_m - first_m : GROUP;
-  const int tm = first_m + (pid % in_group) % gsize;
-  const int tn = (pid % in_group) / gsize;
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31;
-  const int lh = lane >> 5;
-  const int ncol0 = n0 + wave * 32 * TN;
-
-  const int KT = Kpad / BK; // a multiple of D
-
-  // A copies: copy j of a stage fills LDS bytes [j*1024, (j+1)*1024) of it,
-  // lane -> row j*8 + lane/8, holding chunk (lane%8) ^ ((row/2)%8) of the row's
-  // 128 bytes: sixteen consecutive rows (two to each turn of the 64 banks) then
-  // hold any one chunk in sixteen different places, which is what an operand
-  // read needs.
-  const int crow = lane >> 3;
-  // By descriptor (tile origin), a 32-bit lane offset that does not change from
-  // stage to stage and the stage as scalar offset: no vector address arithmetic
-  // in the loop, and a stage past the last one is asked for with an empty
-  // descriptor, which moves nothing and counts like any other load.
-  uint32_t ga[CA];
-#pragma unroll
-  for (int h = 0; h < CA; ++h) {
-    const int r = (wave * CA + h) * 8 + crow;
-    const int rc = (m0 + r < M) ? r : M - 1 - m0; // rows past M: never stored
-    ga[h] = (uint32_t)rc * (uint32_t)K +
-            (uint32_t)((lane & 7) ^ ((r >> 1) & 7)) * 16u;
-  }
-  typedef __attribute__((address_space(3))) void *lds_ptr;
-  const int a_bytes = (M - m0 < BM ? M - m0 : BM) * K;
-  const uint8_t *const a_tile = scalar_ptr(A + (int64_t)m0 * K);
-  auto copy_a = [&](int pair, int stage) {
-    uint8_t *base = sm + stage * STAGE + wave * CA * 1024;
-    const bool in = pair < (KT >> 1);
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)a_tile, 0, in ? a_bytes : 0, 0x00020000);
-    const int soff = in ? pair * ROW : 0;
-#pragma unroll
-    for (int h = 0; h < CA; ++h)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc, (lds_ptr)(base + h * 1024), 16, (int)ga[h], soff, 0, 0);
-  };
-
-  // Bp operands of this wave's column tiles, by buffer addressing: one
-  // descriptor in scalar registers, a 32-bit lane offset, and the step as a
-  // scalar offset.  The loads are written as inline assembly because the
-  // compiler, which cannot count memory operations across the loop's back
-  // edge, would otherwise wait for every outstanding one (vmcnt(0)) before
-  // the first use of these registers in each trip, draining the prefetch.
-  v4i brsrc;
-  {
-    const uint64_t a = (uint64_t)(Bp + (int64_t)(ncol0 >> 5) * KT * 2048);
-    brsrc.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)a);
-    brsrc.y = __builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu));
-    brsrc.z = 0;          // bytes covered: set per trip
-    brsrc.w = 0x00020000; // raw buffer, 32-bit elements
-  }
-  int boff[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j)
-    boff[j] = j * KT * 2048 + lane * 16;
-  // step0: first of the D steps that the trip asks for; past the last one the
-  // descriptor is empty.
-  int bfirst = 0;
-  auto weights_of = [&](int step0) {
-    brsrc.z = step0 < KT ? TN * KT * 2048 : 0;
-    bfirst = step0 < KT ? step0 * 2048 : 0;
-  };
-  auto load_b = [&](int u, int sub, v4i(&fb)[TN]) {
-    const int soff = bfirst + u * 2048 + sub * 1024;
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"
-                   : "=v"(fb[j])
-                   : "v"(boff[j]), "s"(brsrc), "s"(soff)
-                   : "memory");
-  };
-
-  // A operand reads: half step h (0 .. 3) of a stage uses chunk 2*h + lane/32
-  // of row lane%32 of MFMA row tile i (32 * ROW bytes apart).
-  const unsigned sm_base = (unsigned)(uintptr_t)(lds_ptr)sm;
-  // (sm_base is a multiple of 128: bits 4 .. 6 are the chunk's)
-  const unsigned ra = sm_base + l32 * ROW + ((lh ^ ((l32 >> 1) & 7)) << 4);
-  auto lds_read = [](v4i &f, unsigned addr, auto off) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2"
-                 : "=v"(f)
-                 : "v"(addr), "n"(decltype(off)::value)
-                 : "memory");
-  };
-  auto read_a = [&](v4i(&f)[TM], int h, unsigned soff) {
-    const unsigned at = (ra ^ (unsigned)(h << 5)) + soff;
-    static_for<TM>([&](auto i) {
-      lds_read(f[decltype(i)::value], at,
-          std::integral_constant<int, decltype(i)::value * 32 * ROW>{});
-    });
-  };
-
-  v16i acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        acc[i][j][r] = 0;
-
-  // Vector memory operations of a wave, in issue order, for every pair of
-  // steps p (CB = 2 * TN weights loads a step):
-  //   step 2p:     CA copies of pair p+2, CB weights of step 2p+3
-  //   step 2p+1:   CB weights of step 2p+4
-  // and, before the loop, what pairs -2 and -1 would have asked for.  They
-  // complete in order, so a wait for "all but the youngest n" is exact:
-  //   top of step 2p: its weights were asked for in step 2p-3; younger: those
-  //     of 2p+1 and 2p+2 and the copies of pair p+1 (2 * CB + CA)
-  //   top of step 2p+1: its weights were asked for in step 2p-2, behind the
-  //     copies of pair p+1, which are read from the second half of this step
-  //     on; younger: the weights of 2p+2 and 2p+3 and the copies of pair p+2
-  // What lies past the last step is asked for too, with empty descriptors (as
-  // the last step once more it cost a tile 112 KiB).  No more than this on its
-  // way: a wave cannot start before it has issued everything in front of the
-  // loop, and the path into the CU takes a load in 64 clocks (weights four steps
-  // ahead and copies half a pair earlier: 2048 x 768 x 4096 12.9 us).
-  // The barrier is at the top of step 2p+1 only: behind it every wave's copies
-  // of pair p+1 are in LDS, and every wave is done with pair p-1 (its last
-  // operands were waited for in step 2p-1), whose stage the copies issued in
-  // step 2p+2, of pair p+3, overwrite.
-  constexpr int CB = 2 * TN;
-  constexpr int kYoung = 2 * CB + CA;
-  static_assert(3 * CB + 2 * CA < 64, "wait count");
-  v4i bs[D][2][TN];
-  weights_of(0);
-  copy_a(0, 0);
-#pragma unroll
-  for (int u = 0; u < D - 1; ++u) {
-    load_b(u, 0, bs[u][0]);
-    load_b(u, 1, bs[u][1]);
-    if (u == 0)
-      copy_a(1, 1);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-  const v4i flip = {(int)0x80808080, (int)0x80808080, (int)0x80808080,
-      (int)0x80808080};
-
-  // RS: row sums of A are needed (B carries an offset); a template argument
-  // so that the loop body has no branch.
-  constexpr bool need_rs = RS;
-  int32_t rsp[TM];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-    rsp[i] = 0;
-  auto wait_vm = [](auto n) {
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (decltype(n)::value & 15) |
-                               ((decltype(n)::value >> 4) << 14));
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto mfmas = [&](v4i(&fa)[TM], v4i(&fb)[TN]) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-      asm volatile("" : "+v"(fa[i])); // written here, behind the wait
-    if (A_MODE == 1) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        fa[i] ^= flip;
-    }
-    if (need_rs) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-        rsp[i] += frag_rowsum(fa[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
-            fa[i], fb[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  // The copies of pair 0 (the oldest) have landed, of every wave.
-  wait_vm(std::integral_constant<int, 3 * CB + CA>{});
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_sched_barrier(0);
-  v4i fa0[TM];
-  read_a(fa0, 0, 0);
-  int stage = 0;
-  for (int kt = 0; kt < KT; kt += D) {
-#pragma unroll
-    for (int u = 0; u < D; u += 2) {
-      // Operands are read one half step early: those of the second half while
-      // the first half's MFMAs run, and those of the next step's first half
-      // while the second half's do, so that no MFMA waits for an LDS read
-      // issued just before it.
-      const unsigned soff = (unsigned)(stage * STAGE);
-      const int nstage = (stage + 1) & (NST - 1);
-      const int v = (u + D - 1) % D; // set of the weights asked for in step u
-      v4i fa1[TM], fb0[TM], fb1[TM];
-      wait_vm(std::integral_constant<int, kYoung>{});
-      read_a(fa1, 1, soff);
-      copy_a(((kt + u) >> 1) + NST - 2, (stage + NST - 2) & (NST - 1));
-      load_b(v, 0, bs[v][0]);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(TM) : "memory");
-      mfmas(fa0, bs[u][0]);
-      read_a(fb0, 2, soff);
-      load_b(v, 1, bs[v][1]);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(TM) : "memory");
-      mfmas(fa1, bs[u][1]);
-      if (u == 0)
-        weights_of(kt + D);
-
-      wait_vm(std::integral_constant<int, kYoung>{});
-      __builtin_amdgcn_s_barrier();
-      __builtin_amdgcn_sched_barrier(0);
-      read_a(fb1, 3, soff);
-      load_b(u, 0, bs[u][0]);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(TM) : "memory");
-      mfmas(fb0, bs[u + 1][0]);
-      read_a(fa0, 0, (unsigned)(nstage * STAGE));
-      load_b(u, 1, bs[u][1]);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(%0)" : : "n"(TM) : "memory");
-      mfmas(fb1, bs[u + 1][1]);
-      stage = nstage;
-    }
-  }
-  // What was asked for past the last step has still to come back; its
-  // registers count as used here, so that nothing else is put there before.
-  __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0)
-#pragma unroll
-  for (int u = 0; u < D; ++u)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-      asm volatile("" : : "v"(bs[u][0][j]), "v"(bs[u][1][j]) : "memory");
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-    asm volatile("" : : "v"(fa0[i]) : "memory");
-  __builtin_amdgcn_sched_barrier(0);
-
-  EpiParams e = ep;
-  e.need_rowsum = RS; // known here: the other form's code goes
-  gemm_epilogue<TM, TN, A_MODE, EPI, kAuxThrough>(
-      acc, rsp, m0, ncol0, M, N, K, e);
-}
-
 // ---- pack B ---------------------------------------------------------------
 // One block transposes a 64(k) x 64(n) tile of B [K,N] through LDS, writes it
 // in MFMA operand order (see the top of the file) and adds the tile's column
@@ -999,41 +690,68 @@ enum TileCfg : int {
   kD128x64 = 3,  // k_gemm_i8_dma with 128 x 64 tiles
   kW128x384 = 4, // k_gemm_i8_wreg: weights in registers, 12 waves of 32 columns
   kFlight = 5,   // k_gemm_i8_flight: one round of blocks, all operands requested at once
-  kNumCfg = 6
+  kB64x256 = 6,  // k_gemm_i8_dma_bs, the same with 64 x 256 tiles
+  kB64x128 = 7,  // and with 64 x 128 tiles
+  kNumCfg = 8
 };
 
-// Kernel choice for problems with more than 64 rows, K % 64 == 0 and a
-// 16-byte aligned A (K % 16 == 0: k_gemm_i8_dma, its tile chosen here too;
-// anything else takes the general path of k_gemm_i8).
-// Measured on MI355X over the BERT-base and Llama-7B layer shapes and square
-// problems up to 8192: a 128 x 256 tile of k_gemm_i8_bs costs about 1.7 times
-// a 128 x 128 tile of k_gemm_i8_dma, so it wins when it needs at most half as
-// many rounds over the 256 CUs and fills at least one round.  When 128 x 128
-// tiles cover at most half the CUs, 128 x 64 tiles spread the work over twice
-// as many (512x1024x4096: 10.1 -> 8.8 us); with 192 tiles for 256 CUs the
-// half-width tiles lose (4096x768x768 7.2 -> 7.6 us, 4096x3072x768 18.6 ->
-// 19.4 us).
+// Kernel choice for problems with more than 64 rows, K a multiple of 16 and a
+// 16-byte aligned A (anything else takes the general path of k_gemm_i8).
+// A tile kernel's time on MI355X, by what the fullest CU has to do:
+//   base + steps * max(lone, step * b) + block * b   microseconds,
+// b the blocks it gets: partly the next whole number, partly the mean, since
+// CUs that are done early leave the others the way to memory (`round`).  Fitted
+// to 150 products of 65 .. 4096 rows, K and N of 256 .. 11008 (a multiple of 16
+// and any number), int32 and f32 results, each timed with every kernel; the
+// choice by it is within 1 % of always taking the fastest, 4 % ahead of the rule
+// it replaced (128 x 128 tiles unless few or many; 4096 x 1024 x 1024 9.3 -> 8.8
+// us, 512 x 4096 x 4096 18.4 -> 15.4, 1235 x 6656 x 2005 31.4 -> 28.8, 1500 x
+// 5120 x 5120 49.7 -> 43.1).
+struct TileCost {
+  TileCfg cfg;
+  int bm, bn, trip; // K steps are done in whole trips
+  double lone, step, block, base, round;
+};
+constexpr TileCost kTileCosts[] = {
+    {kD128x128, 128, 128, 1, 0.0, 0.248, 2.67, 2.24, 0.52},
+    {kD128x64, 128, 64, 1, 0.0, 0.203, 0.77, 2.37, 0.43},
+    {kB128x256, 128, 256, 4, 0.0, 0.314, 5.08, 0.22, 1.0},
+    {kB64x256, 64, 256, 4, 0.0, 0.223, 2.24, 2.78, 0.68},
+    {kB64x128, 64, 128, 4, 0.132, 0.163, 0.75, 2.76, 0.64},
+};
+double tile_us(const TileCost &t, int64_t M, int64_t N, int64_t K) {
+  const int64_t blocks = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+  const double whole = (double)((blocks + 255) / 256);
+  const double b = std::max(
+      1.0, t.round * whole + (1.0 - t.round) * (double)blocks / 256.0);
+  const double steps = (double)(round_up(K, kGemmBK * t.trip) / kGemmBK);
+  return t.base + steps * std::max(t.lone, t.step * b) + t.block * b;
+}
+// Its time, too, where wanted.
 // Override for tests and tuning: OM_MI355X_GEMM_TILE=<TileCfg value>.
-int choose_tile(int64_t M, int64_t N, int64_t K) {
+int choose_tile(int64_t M, int64_t N, int64_t K, double *us = nullptr) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
   if (force && force[0]) {
     const int c = atoi(force);
     if (c >= 0 && c < kNumCfg)
       return c;
   }
-  const int64_t tm = (M + 127) / 128;
-  const int64_t t128 = tm * ((N + 127) / 128);
-  const int64_t t256 = tm * ((N + 255) / 256);
-  const int64_t r128 = (t128 + 255) / 256, r256 = (t256 + 255) / 256;
-  // (k_gemm_i8_bs only with whole trips of its four-step loop body, K % 256
-  // == 0: the step counts it runs with in production -- K = 2048, 4096, 11008
-  // -- and is validated at.  Other K take the 128 x 128 tiles, a few percent
-  // slower on such shapes.)
-  if (t256 >= 256 && r256 * 17 < r128 * 10 && K % (4 * kGemmBK) == 0)
-    return kB128x256;
-  if (N > 64 && t128 <= 128)
-    return kD128x64;
-  return kD128x128;
+  int best = kD128x128;
+  double least = 0.98 * tile_us(kTileCosts[0], M, N, K); // (ties stay with it)
+  for (const TileCost &t : kTileCosts) {
+    // (128 x 256 tiles: K a multiple of 256, the step counts that
+    // instantiation is validated at)
+    if (K >= (1 << 24) ? t.trip != 1 : t.cfg == kB128x256 && K % 256 != 0)
+      continue;
+    const double u = tile_us(t, M, N, K);
+    if (u < least) {
+      least = u;
+      best = t.cfg;
+    }
+  }
+  if (us)
+    *us = least;
+  return best;
 }
 
 bool gemm_fast_path(int64_t M, int64_t K, const void *A) {
@@ -1128,21 +846,20 @@ __global__ __launch_bounds__(256) void k_sum_parts(
     }
 }
 
-int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
-
 // What bounds a product whose tiles cover a part of the CUs is the chain of its
 // K steps, each the time its operands take into one CU: 0.22 us in 128 x 64
-// tiles of k_gemm_i8_dma, 0.28 in 128 x 128 ones, 0.5 in k_gemm_i8 (u8 rows a
-// little more).  Splitting shortens the chain and costs the launch of
-// k_sum_parts, 2.5 us, and the arrays' way through memory, 1.8 us per million
-// elements.  Taken where that comes out a tenth ahead; more than one block per
-// CU gains nothing.  Measured without / with (fused layers with their
-// quantization): layer 102 x 3072 x 734 20.8 / 13.8 us, 65 x 11008 x 4096 43.6 /
-// 21.1, 128 x 4096 x 4096 21.4 / 19.3, 100 x 11000 x 4000 70.0 / 24.4, u8
-// results 517 x 8960 x 576 33.1 / 14.6, int32 600 x 5000 x 2000 43.7 / 24.1,
-// 2048 x 11008 x 768 48.1 / 37.6, 128 x 1536 x 300 9.5 / 7.8; left alone by the
-// rule: int32 2048 x 1280 x 1024 9.5 / 18.5, layer 512 x 1536 x 1536 14.1 /
-// 17.5, 128 x 4096 x 11008 23.3 / 23.7.
+// tiles of k_gemm_i8_dma, 0.28 in 128 x 128 ones, 0.172 in 64 x 128 ones of
+// k_gemm_i8_dma_bs, 0.5 in k_gemm_i8 (u8 rows a little more).  Splitting shortens
+// the chain and costs the launch of k_sum_parts, 2.5 us, and the arrays' way
+// through memory, 1.8 us per million elements.  Taken where that comes out ahead
+// of one piece in the tile chosen for it; more than one block per CU gains nothing.  K of whole steps in the tiles of k_gemm_i8_dma
+// (the others are ahead of them on some shapes and behind on as many: 418 x 7936
+// x 1386 17.1 / 15.8 us, u8 results 517 x 8960 x 576 14.0 / 15.2), other K in
+// those of k_gemm_i8_dma_bs, whose steps do not look for the end of the row
+// (int32 301 x 6384 x 1856 15.4 / 13.8 us, 196 x 5488 x 2688 15.4 / 13.9).
+// Measured in one piece / split: 70 x 8192 x 1024 24.5 / 10.2 us, 118 x 10624 x
+// 1536 31.3 / 12.8, 100 x 4096 x 4096 14.4 / 12.9, 148 x 2304 x 832 9.3 / 8.4; left
+// alone by the rule: 200 x 4096 x 4096 14.3 / 16.3, 128 x 6464 x 9637 21.2 / 21.4.
 // The plan is made once per product (GemmArgs::split), after the tests that turn
 // most products away; parts are looked for around the minimum of the model.
 GemmSplit split_plan(const GemmArgs &g, int a_mode) {
@@ -1150,53 +867,68 @@ GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   const int64_t KT = round_up(g.K, kGemmBK) / kGemmBK;
   const int64_t tm = (g.M + 127) / 128, t128 = tm * ((g.N + 127) / 128);
   if (KT < 8 || t128 > 128 || t128 <= 0 || g.X ||
-      g.M * g.N > ((int64_t)1 << 22) || g.M * g.K < 16 ||
+      g.M * g.N > ((int64_t)1 << 22) || g.M * g.K < 16 || g.K >= (1 << 24) ||
       skinny_ok(g.M, g.K, g.A))
     return best;
   const bool any = !gemm_fast_path(g.M, g.K, g.A);
+  if (!any && KT < 24) // (a second launch for 5 us of steps: within the model's error)
+    return best;
   if (!any && g.K % 64 == 0 &&
       (flight_ok(g, a_mode) || (wreg_ok(g) && wreg_pays(g.M, g.N))))
     return best;
   const char *force = getenv("OM_MI355X_GEMM_TILE");
   if (force && force[0])
     return best;
-  const double kWide = 0.28, kNarrow = 0.22, kAny = 0.5;
+  struct Form {
+    SplitKernel kernel;
+    int64_t tiles, trip;
+    double us_step, us_else; // us_else: beside steps, second launch and arrays
+  };
+  const Form wide = {kSplitDma128, t128, 1, 0.28, 2.3},
+             narrow = {kSplitDma64, tm * ((g.N + 63) / 64), 1, 0.22, 2.3},
+             stream = {kSplitBs, ((g.M + 63) / 64) * ((g.N + 127) / 128), 4, 0.172, 3.5},
+             general = {kSplitAny, t128, 1, 0.5, 0.0};
+  Form forms[2] = {general, general};
+  int count = 1;
+  double least = 0.9 * (double)KT * general.us_step;
+  if (!any) {
+    (void)choose_tile(g.M, g.N, g.K, &least);
+    // (row sums of A cost about a seventh of a step)
+    if (g.b_unsigned || g.b_zp_len > 0)
+      least += 0.15 * std::max(0.0, least - 3.5);
+    least *= 0.98;
+    forms[0] = g.K % kGemmBK != 0 ? stream : wide;
+    if (g.K % kGemmBK == 0 && g.N > 64)
+      forms[count++] = narrow;
+  }
   const double us_part = 1.8e-6 * (double)(g.M * g.N);
-  double least = 0.9 * (double)KT * (any ? kAny : g.N > 64 ? kNarrow : kWide);
-  for (int narrow = 0; narrow <= (any || g.N <= 64 ? 0 : 1); ++narrow) {
-    const int64_t tiles = narrow ? tm * ((g.N + 63) / 64) : t128;
-    const int64_t most = 256 / tiles < KT / 4 ? 256 / tiles : KT / 4;
-    const double us_step = any ? kAny : narrow ? kNarrow : kWide;
+  for (int i = 0; i < count; ++i) {
+    const Form &f = forms[i];
+    const int64_t most = 256 / f.tiles < KT / 4 ? 256 / f.tiles : KT / 4;
     // steps * us_step + parts * us_part is least where both are equal
-    const int64_t around = (int64_t)sqrt((double)KT * us_step / us_part);
+    const int64_t around = (int64_t)sqrt((double)KT * f.us_step / us_part);
     const int64_t low = around - 2 < most - 4 ? around - 2 : most - 4;
     for (int64_t p = low < 2 ? 2 : low; p <= most && p <= around + 3; ++p) {
-      const int64_t steps = (KT + p - 1) / p;
+      const int64_t steps = round_up((KT + p - 1) / p, f.trip);
       const int64_t parts = (KT + steps - 1) / steps; // (none without a step)
-      const double us = (double)steps * us_step + 2.5 + us_part * (double)parts;
-      if (us < least) {
+      const double us = f.us_else + (double)steps * f.us_step + 2.5 +
+                        us_part * (double)parts;
+      if (parts > 1 && us < least) {
         least = us;
         best.parts = (int)parts;
         best.steps = (int)steps;
-        best.any = any;
-        best.narrow = narrow != 0;
+        best.kernel = f.kernel;
       }
     }
   }
   return best;
 }
 
-const char *dma_name(bool narrow, bool ragged, bool split) {
-  static const char *const names[2][2][2] = {
-      {{"k_gemm_i8_dma (128x128 tiles)",
-           "k_gemm_i8_dma (128x128 tiles, split along K)"},
-          {"k_gemm_i8_dma (128x128 tiles, ragged K)",
-              "k_gemm_i8_dma (128x128 tiles, ragged K, split along K)"}},
-      {{"k_gemm_i8_dma (128x64 tiles)",
-           "k_gemm_i8_dma (128x64 tiles, split along K)"},
-          {"k_gemm_i8_dma (128x64 tiles, ragged K)",
-              "k_gemm_i8_dma (128x64 tiles, ragged K, split along K)"}}};
-  return names[narrow][ragged][split];
+const char *dma_name(bool narrow, bool ragged) {
+  return narrow ? (ragged ? "k_gemm_i8_dma (128x64 tiles, ragged K)"
+                          : "k_gemm_i8_dma (128x64 tiles)")
+                : (ragged ? "k_gemm_i8_dma (128x128 tiles, ragged K)"
+                          : "k_gemm_i8_dma (128x128 tiles)");
 }
 
 template <int A_MODE, int EPI>
@@ -1205,28 +937,33 @@ hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
   const GemmSplit &p = g.split;
   const uint8_t *A = (const uint8_t *)g.A;
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
-  const int tiles_m = (M + 127) / 128;
-  const int tiles_n = p.narrow ? (N + 63) / 64 : (N + 127) / 128;
-  const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)p.parts);
   const KSplit ks = {p.steps, part_stride(g)};
   EpiParams pe = ep;
   pe.out = g.parts;
-  if (p.any) {
-    t_last_kernel = "k_gemm_i8 (any K, any alignment; split along K)";
-    k_gemm_i8<128, 128, 2, 2, 2, A_MODE, kEpiI32, kLoadAny, true>
-        <<<grid, 256, 0, st>>>(A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+  hipError_t e;
+  if (p.kernel == kSplitBs) {
+    e = launch_gemm_bs_split(st, g, pe, A_MODE);
   } else {
-    const bool ragged = K % BK != 0;
-    t_last_kernel = dma_name(p.narrow, ragged, true);
-    auto *const kernel =
-        p.narrow ? (ragged ? k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, true, true>
-                           : k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, false, true>)
-                 : (ragged ? k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, true, true>
-                           : k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, false, true>);
-    kernel<<<grid, 256, 0, st>>>(
-        A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+    const bool narrow = p.kernel == kSplitDma64;
+    const int tiles_m = (M + 127) / 128;
+    const int tiles_n = narrow ? (N + 63) / 64 : (N + 127) / 128;
+    const dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)p.parts);
+    t_last_kernel = p.kernel == kSplitAny
+                        ? "k_gemm_i8 (any K, any alignment; split along K)"
+                    : narrow ? "k_gemm_i8_dma (128x64 tiles, split along K)"
+                             : "k_gemm_i8_dma (128x128 tiles, split along K)";
+    if (p.kernel == kSplitAny)
+      k_gemm_i8<128, 128, 2, 2, 2, A_MODE, kEpiI32, kLoadAny, true>
+          <<<grid, 256, 0, st>>>(
+              A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+    else if (narrow)
+      k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, false, true><<<grid, 256, 0, st>>>(
+          A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+    else
+      k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, false, true><<<grid, 256, 0, st>>>(
+          A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+    e = hipGetLastError();
   }
-  const hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return e;
   const unsigned n = (unsigned)(g.M * g.N);
@@ -1246,7 +983,7 @@ hipError_t launch_dma(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
   const bool narrow = cfg == kD128x64, ragged = K % BK != 0;
   const int tiles_n = narrow ? (N + 63) / 64 : (N + 127) / 128;
-  t_last_kernel = dma_name(narrow, ragged, false);
+  t_last_kernel = dma_name(narrow, ragged);
   auto *const kernel =
       narrow ? (ragged ? k_gemm_i8_dma<64, 3, 3, A_MODE, EPI, true>
                        : k_gemm_i8_dma<64, 3, 3, A_MODE, EPI, false>)
@@ -1303,7 +1040,7 @@ hipError_t gemm_launch_cfg(
     return hipGetLastError();
   }
   const int cfg = choose_tile(g.M, g.N, g.K);
-  if (g.K % 64 != 0)
+  if (g.K % 64 != 0 && cfg != kB64x256 && cfg != kB64x128)
     return launch_dma<A_MODE, EPI>(st, g, ep, Kpad,
         cfg == kD128x64 || cfg == kD128x128 ? cfg : (int)kD128x128);
   // One round of blocks with everything requested at once: small problems,
@@ -1327,20 +1064,15 @@ hipError_t gemm_launch_cfg(
     return launch_gemm_wreg(st, g, ep, A_MODE);
   }
   switch (cfg) {
-  case kB128x256: {
-    if (g.K % (4 * kGemmBK) != 0) // (forced, on a K this kernel does not take)
+  case kB128x256:
+  case kB64x256:
+  case kB64x128: {
+    const BsTile tile = cfg == kB128x256  ? kBs128x256
+                        : cfg == kB64x256 ? kBs64x256
+                                          : kBs64x128;
+    if (!bs_ok(g, tile)) // (forced, on a K this kernel does not take)
       return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x128);
-    const int tiles_n = (int)((g.N + 255) / 256);
-    t_last_kernel = "k_gemm_i8_bs (128x256 tiles)";
-    if (ep.need_rowsum)
-      k_gemm_i8_bs<4, 2, 4, 4, 2, true, A_MODE, EPI, true>
-          <<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
-              A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
-    else
-      k_gemm_i8_bs<4, 2, 4, 4, 2, true, A_MODE, EPI, false>
-          <<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
-              A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n);
-    break;
+    return launch_gemm_bs(st, g, ep, A_MODE, tile);
   }
   case kD128x64:
     return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x64);

@@ -117,10 +117,12 @@ hipError_t launch_pack_b(hipStream_t s, const void *B, bool b_unsigned,
     int64_t K, int64_t N, int8_t *Bp, int32_t *colsum);
 
 // How a product is split along K: into `parts` (1: not at all) of `steps` K steps
-// each, in k_gemm_i8 (any) or k_gemm_i8_dma, there in 64-column tiles (narrow).
+// each, and by which kernel: k_gemm_i8_dma in 128 x 128 or 128 x 64 tiles,
+// k_gemm_i8_dma_bs in 64 x 128 ones, k_gemm_i8 (any K and alignment).
+enum SplitKernel : int { kSplitDma128, kSplitDma64, kSplitBs, kSplitAny };
 struct GemmSplit {
   int parts = 1, steps = 0;
-  bool any = false, narrow = false;
+  SplitKernel kernel = kSplitAny;
 };
 
 struct GemmArgs {

@@ -1,23 +1,26 @@
-"""Host model of k_gemm_i8_bs with A copied in stages of two K steps
-(onnx-mlir_amd/csrc/gemm_kernels.hip): where its copies and operand reads go,
+"""Host model of k_gemm_i8_bs and k_gemm_i8_dma_bs, A copied in stages of two K
+steps (onnx-mlir_amd/csrc/gemm_bs.hip): where their copies and operand reads go,
 and whether its explicit waits cover what each step reads.  Index arithmetic
-restated for the CPU; and the kernel itself on the GPU, forced, at its edges."""
+restated for the CPU; and the kernels themselves on the GPU, forced, at their
+edges."""
 import numpy as np
 import pytest
 
-TM, TN, D, NST = 4, 2, 4, 4
-BM, ROW, BK = 32 * TM, 128, 64
-CA, CB = BM // 32, 2 * TN
+D, NST, ROW, BK = 4, 4, 128, 64
 LANE = np.arange(64)
+TILES = [(4, 2), (2, 2), (2, 1)]  # TM, TN
 
 
 def slot_of(row, chunk):
     return row * ROW + ((chunk ^ ((row >> 1) & 7)) << 4)
 
 
-@pytest.mark.parametrize("M,K", [(128, 256), (1, 256), (300, 512), (2048, 11008), (129, 4096)])
-def test_copies_are_in_bounds_and_lie_where_operands_are_read(M, K):
-    pairs = np.arange(K // 128)  # past the last one the descriptor is empty
+@pytest.mark.parametrize("TM", [4, 2])
+@pytest.mark.parametrize("M,K", [(128, 256), (1, 256), (300, 512), (2048, 11008), (129, 4096), (65, 16), (100, 784)])
+def test_copies_are_in_bounds_and_lie_where_operands_are_read(TM, M, K):
+    BM = 32 * TM
+    CA = BM // 32
+    pairs = np.arange(-(-K // 128))  # past the last one the descriptor is empty
     for m0 in {0, (M - 1) // BM * BM}:
         a_bytes = min(M - m0, BM) * K
         filled = np.zeros(BM * ROW, bool)
@@ -27,7 +30,10 @@ def test_copies_are_in_bounds_and_lie_where_operands_are_read(M, K):
                 chunk = (LANE & 7) ^ ((r >> 1) & 7)
                 rc = np.where(m0 + r < M, r, M - 1 - m0)
                 at = pairs[:, None] * ROW + (rc * K + chunk * 16)[None]
-                assert at.min() >= 0 and at.max() + 16 <= a_bytes
+                # a chunk lies wholly inside the tile's rows or the descriptor drops it
+                assert at.min() >= 0 and ((at + 16 <= a_bytes) | (at >= a_bytes)).all()
+                inside = pairs[:, None] * ROW + (chunk * 16)[None] < K
+                assert (at[inside] + 16 <= a_bytes).all()
                 dst = (wave * CA + h) * 1024 + LANE * 16
                 assert (dst == slot_of(r, chunk)).all()
                 filled[dst[:, None] + np.arange(16)] = True
@@ -43,8 +49,10 @@ def test_copies_are_in_bounds_and_lie_where_operands_are_read(M, K):
                 assert len(set((at[g * 16:g * 16 + 16] % 256) // 16)) == 16
 
 
+@pytest.mark.parametrize("TM,TN", TILES)
 @pytest.mark.parametrize("KT", [4, 8, 12, 64, 172])
-def test_waits_cover_what_each_step_reads(KT):
+def test_waits_cover_what_each_step_reads(TM, TN, KT):
+    CA, CB = TM, 2 * TN
     ops = []  # (kind, asked for, register set or stage), in issue order
 
     def copy(pair):
@@ -76,26 +84,46 @@ def test_waits_cover_what_each_step_reads(KT):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,K,N", [(128, 256, 256), (1, 256, 7), (127, 512, 255), (129, 768, 257), (300, 1280, 513),
-                                   (1024, 512, 768)])
-def test_bs_kernel_at_its_edges(M, K, N, monkeypatch):
-    import oracle_lib
-    import om_mi355x as rt
-    oracle = oracle_lib.load()
+@pytest.mark.parametrize("tile,name", [("2", "k_gemm_i8_bs"), ("6", "k_gemm_i8_dma_bs (64x256"), ("7", "k_gemm_i8_dma_bs (64x128")])
+@pytest.mark.parametrize("M,K,N", [(128, 256, 256), (127, 512, 255), (129, 768, 257), (300, 1280, 513), (1024, 512, 768),
+                                   (65, 16, 33), (63, 64, 127), (190, 400, 129), (513, 832, 300), (66, 1136, 260)])
+def test_streaming_kernels_at_their_edges(rt, oracle, monkeypatch, tile, name, M, K, N):
+    """Rows and columns past the result, a K of one chunk up to several trips and
+    any number of steps and chunks past them; row sums, per-row zero points, the
+    three epilogues."""
     rng = np.random.default_rng(M + K + N)
-    monkeypatch.setenv("OM_MI355X_GEMM_TILE", "2")
+    monkeypatch.setenv("OM_MI355X_GEMM_TILE", tile)
+
+    def draw(dt, shape):
+        i = np.iinfo(dt)
+        return rng.integers(i.min, i.max + 1, shape, dtype=dt)
+
     for adt, bdt, per in ((np.uint8, np.int8, False), (np.uint8, np.uint8, False), (np.int8, np.uint8, True),
                           (np.int8, np.int8, True)):
-        def draw(dt, shape):
-            i = np.iinfo(dt)
-            return rng.integers(i.min, i.max + 1, shape, dtype=dt)
         a, b = draw(adt, (M, K)), draw(bdt, (K, N))
         az, bz = draw(adt, (M,) if per else ()), draw(bdt, (N,) if per else ())
         want = oracle.matmul_integer(a, b, az, bz)
         assert np.array_equal(rt.MatMulInteger(a, b, az, bz), want)
-        if M > 16:
-            assert "k_gemm_i8_bs" in rt.last_gemm_kernel()
+        if K % 256 == 0 or tile != "2":
+            assert name in rt.last_gemm_kernel(), rt.last_gemm_kernel()
         if not per:
             s = rng.uniform(1e-3, 1e-2, N).astype(np.float32)
             got = rt.MatMulIntegerDequant(a, b, az, bz, np.float32(0.01), s)
             assert np.array_equal(got, oracle.dequant_epilogue(want, np.float32(0.01), s))
+        if adt == bdt:
+            q = [np.float32(v) for v in (0.0173, 0.005, 0.37)]
+            y = oracle.qlinear_matmul(a, q[0], az.reshape(-1)[:1], b, q[1], bz.reshape(-1)[:1], q[2], az.reshape(-1)[0], 0)
+            assert np.array_equal(rt.QLinearMatMul(a, q[0], az.reshape(-1)[:1], b, q[1], bz.reshape(-1)[:1], q[2],
+                                                   az.reshape(-1)[0], rt.WRAP), y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(65, 2128, 65), (200, 3056, 129), (90, 4176, 300)])
+def test_streaming_kernel_split_along_k(rt, oracle, M, K, N):
+    """Parts of whole trips, the last one of fewer steps and ending inside one."""
+    rng = np.random.default_rng(K)
+    a, b = rng.integers(0, 256, (M, K), dtype=np.uint8), rng.integers(0, 256, (K, N), dtype=np.uint8)
+    az, bz = np.uint8(131), rng.integers(0, 256, N, dtype=np.uint8)
+    assert np.array_equal(rt.MatMulInteger(a, b, az, bz), oracle.matmul_integer(a, b, az, bz))
+    kernel = rt.last_gemm_kernel()
+    assert "dma_bs" in kernel and "split" in kernel and "ragged" in kernel, kernel
