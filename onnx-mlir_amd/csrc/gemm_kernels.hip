@@ -862,16 +862,90 @@ __global__ __launch_bounds__(256) void k_sum_parts(
 // alone by the rule: 200 x 4096 x 4096 14.3 / 16.3, 128 x 6464 x 9637 21.2 / 21.4.
 // The plan is made once per product (GemmArgs::split), after the tests that turn
 // most products away; parts are looked for around the minimum of the model.
+struct SplitForm {
+  SplitKernel kernel;
+  int64_t tiles, trip;
+  double us_step, us_else; // us_else: beside steps, second launch and arrays
+};
+SplitForm split_form(SplitKernel kernel, int64_t M, int64_t N) {
+  const int64_t tm = (M + 127) / 128, t128 = tm * ((N + 127) / 128);
+  switch (kernel) {
+  case kSplitDma128:
+    return {kernel, t128, 1, 0.28, 2.3};
+  case kSplitDma64:
+    return {kernel, tm * ((N + 63) / 64), 1, 0.22, 2.3};
+  case kSplitBs:
+    return {kernel, ((M + 63) / 64) * ((N + 127) / 128), 4, 0.172, 3.5};
+  default:
+    return {kernel, t128, 1, 0.5, 3.5};
+  }
+}
+bool split_possible(int64_t M, int64_t N, int64_t K, bool any) {
+  // (under 24 steps a second launch is within the model's error, unless they
+  // are those of k_gemm_i8)
+  return (K + kGemmBK - 1) / kGemmBK >= (any ? 8 : 24) &&
+         ((M + 127) / 128) * ((N + 127) / 128) <= 128 &&
+         M * N <= ((int64_t)1 << 22) && M * K >= 16 && K < (1 << 24);
+}
+// The split of form f that takes less than `least`, which it lowers.
+void try_split(const SplitForm &f, int64_t M, int64_t N, int64_t K,
+    GemmSplit &best, double &least) {
+  const int64_t KT = (K + kGemmBK - 1) / kGemmBK;
+  const double us_part = 1.8e-6 * (double)(M * N);
+  const int64_t most = 256 / f.tiles < KT / 4 ? 256 / f.tiles : KT / 4;
+  // steps * us_step + parts * us_part is least where both are equal
+  const int64_t around = (int64_t)sqrt((double)KT * f.us_step / us_part);
+  const int64_t low = around - 2 < most - 4 ? around - 2 : most - 4;
+  for (int64_t p = low < 2 ? 2 : low; p <= most && p <= around + 3; ++p) {
+    const int64_t steps = round_up((KT + p - 1) / p, f.trip);
+    const int64_t parts = (KT + steps - 1) / steps; // (none without a step)
+    const double us = f.us_else + (double)steps * f.us_step + 2.5 +
+                      us_part * (double)parts;
+    if (parts > 1 && us < least) {
+      least = us;
+      best.parts = (int)parts;
+      best.steps = (int)steps;
+      best.kernel = f.kernel;
+    }
+  }
+}
+// The time of a product over K, a multiple of 16, and how it is split.
+double product_us(int64_t M, int64_t N, int64_t K, bool rowsums, GemmSplit &best) {
+  double least = 0.0;
+  (void)choose_tile(M, N, K, &least);
+  // (row sums of A cost about a seventh of a step)
+  if (rowsums)
+    least += 0.15 * std::max(0.0, least - 3.5);
+  if (!split_possible(M, N, K, false))
+    return least;
+  double us = 0.98 * least;
+  if (K % kGemmBK != 0) {
+    try_split(split_form(kSplitBs, M, N), M, N, K, best, us);
+  } else {
+    try_split(split_form(kSplitDma128, M, N), M, N, K, best, us);
+    if (N > 64)
+      try_split(split_form(kSplitDma64, M, N), M, N, K, best, us);
+  }
+  return best.parts > 1 ? us : least;
+}
+// And in k_gemm_i8, for any K; the model of kTileCosts, fitted to 30 products.
+double general_us(int64_t M, int64_t N, int64_t K, GemmSplit &best) {
+  const TileCost t = {kT128x128, 128, 128, 1, 0.434, 0.359, 2.33, 2.62, 0.76};
+  double least = tile_us(t, M, N, K);
+  if (split_possible(M, N, K, true)) {
+    // (a tenth off the chain of its steps)
+    double us = 3.5 + 0.45 * (double)((K + kGemmBK - 1) / kGemmBK);
+    try_split(split_form(kSplitAny, M, N), M, N, K, best, us);
+    if (best.parts > 1)
+      least = us;
+  }
+  return least;
+}
 GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   GemmSplit best;
-  const int64_t KT = round_up(g.K, kGemmBK) / kGemmBK;
-  const int64_t tm = (g.M + 127) / 128, t128 = tm * ((g.N + 127) / 128);
-  if (KT < 8 || t128 > 128 || t128 <= 0 || g.X ||
-      g.M * g.N > ((int64_t)1 << 22) || g.M * g.K < 16 || g.K >= (1 << 24) ||
-      skinny_ok(g.M, g.K, g.A))
-    return best;
   const bool any = !gemm_fast_path(g.M, g.K, g.A);
-  if (!any && KT < 24) // (a second launch for 5 us of steps: within the model's error)
+  if (g.X || g.M * g.N <= 0 || !split_possible(g.M, g.N, g.K, any) ||
+      skinny_ok(g.M, g.K, g.A))
     return best;
   if (!any && g.K % 64 == 0 &&
       (flight_ok(g, a_mode) || (wreg_ok(g) && wreg_pays(g.M, g.N))))
@@ -879,48 +953,10 @@ GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
   if (force && force[0])
     return best;
-  struct Form {
-    SplitKernel kernel;
-    int64_t tiles, trip;
-    double us_step, us_else; // us_else: beside steps, second launch and arrays
-  };
-  const Form wide = {kSplitDma128, t128, 1, 0.28, 2.3},
-             narrow = {kSplitDma64, tm * ((g.N + 63) / 64), 1, 0.22, 2.3},
-             stream = {kSplitBs, ((g.M + 63) / 64) * ((g.N + 127) / 128), 4, 0.172, 3.5},
-             general = {kSplitAny, t128, 1, 0.5, 0.0};
-  Form forms[2] = {general, general};
-  int count = 1;
-  double least = 0.9 * (double)KT * general.us_step;
-  if (!any) {
-    (void)choose_tile(g.M, g.N, g.K, &least);
-    // (row sums of A cost about a seventh of a step)
-    if (g.b_unsigned || g.b_zp_len > 0)
-      least += 0.15 * std::max(0.0, least - 3.5);
-    least *= 0.98;
-    forms[0] = g.K % kGemmBK != 0 ? stream : wide;
-    if (g.K % kGemmBK == 0 && g.N > 64)
-      forms[count++] = narrow;
-  }
-  const double us_part = 1.8e-6 * (double)(g.M * g.N);
-  for (int i = 0; i < count; ++i) {
-    const Form &f = forms[i];
-    const int64_t most = 256 / f.tiles < KT / 4 ? 256 / f.tiles : KT / 4;
-    // steps * us_step + parts * us_part is least where both are equal
-    const int64_t around = (int64_t)sqrt((double)KT * f.us_step / us_part);
-    const int64_t low = around - 2 < most - 4 ? around - 2 : most - 4;
-    for (int64_t p = low < 2 ? 2 : low; p <= most && p <= around + 3; ++p) {
-      const int64_t steps = round_up((KT + p - 1) / p, f.trip);
-      const int64_t parts = (KT + steps - 1) / steps; // (none without a step)
-      const double us = f.us_else + (double)steps * f.us_step + 2.5 +
-                        us_part * (double)parts;
-      if (parts > 1 && us < least) {
-        least = us;
-        best.parts = (int)parts;
-        best.steps = (int)steps;
-        best.kernel = f.kernel;
-      }
-    }
-  }
+  if (any)
+    (void)general_us(g.M, g.N, g.K, best);
+  else
+    (void)product_us(g.M, g.N, g.K, g.b_unsigned || g.b_zp_len > 0, best);
   return best;
 }
 
@@ -1103,47 +1139,99 @@ hipError_t gemm_launch_epi(
   }
 }
 
-// Rows of A copied to a pitch of Kp >= K bytes, the bytes past K set to the
-// row's zero point (exclusive-ored with `flip`: 0x80 for rows stored minus
-// 128): an element equal to its zero point stands for the real value 0, so a
-// product over the Kp bytes equals the product over the K (see
-// gemm_pads_rows).  One thread per byte; at most 64 rows.
+// Rows of A copied to a pitch of Kp >= K bytes, a multiple of 16, the bytes past
+// K set to the row's zero point (exclusive-ored with `flip`: 0x80 for rows stored
+// minus 128): an element equal to its zero point stands for the real value 0, so
+// a product over the Kp bytes equals the product over the K (see gemm_padded_k).
+// 16 bytes of the result per thread, read at whatever address they have (M * K
+// >= 16; moved back to end with A where they would run past it).  Bound by the
+// launch and by memory: 4096 x 1000 in 3.4 us.
 __global__ __launch_bounds__(256) void k_pad_rows(const uint8_t *__restrict__ A,
-    int M, int K, int Kp, const uint8_t *__restrict__ zp, int zp_len,
-    uint8_t flip, uint8_t *__restrict__ out) {
-  const int r = blockIdx.y;
-  const uint8_t fill =
-      (uint8_t)((zp && zp_len > 0 ? zp[zp_len > 1 ? r : 0] : 0) ^ flip);
-  for (int c = blockIdx.x * 256 + threadIdx.x; c < Kp; c += gridDim.x * 256)
-    out[(int64_t)r * Kp + c] = c < K ? A[(int64_t)r * K + c] : fill;
+    unsigned M, unsigned K, unsigned chunks, const uint8_t *__restrict__ zp,
+    int zp_len, uint8_t flip, uint8_t *__restrict__ out) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= M * chunks)
+    return;
+  const unsigned r = i / chunks, c = i - r * chunks;
+  const bool has_zp = zp && zp_len > 0;
+  const uint8_t z = (has_zp ? zp : A)[has_zp && zp_len > 1 ? r : 0];
+  const uint8_t *const p = A + (uint64_t)r * K + c * 16;
+  const uint8_t *const last = A + ((uint64_t)M * K - 16);
+  const v4i v = *(const v4i_any *)(p < last ? p : last);
+  const int left = (int)K - (int)(c * 16);
+  const int len = left < 0 ? 0 : left < 16 ? left : 16;
+  uint64_t lo = (uint32_t)v.x | ((uint64_t)(uint32_t)v.y << 32);
+  uint64_t hi = (uint32_t)v.z | ((uint64_t)(uint32_t)v.w << 32);
+  // bits to shift down: < 128 whenever the chunk holds a byte of the row
+  const int sh = p < last ? 0 : (int)(p - last) * 8;
+  if (sh >= 64) {
+    lo = hi;
+    hi = 0;
+  }
+  const int s1 = sh & 63;
+  if (s1) {
+    lo = (lo >> s1) | (hi << (64 - s1));
+    hi >>= s1;
+  }
+  const uint64_t fill =
+      (uint64_t)(uint8_t)((has_zp ? z : 0) ^ flip) * 0x0101010101010101ull;
+  const uint64_t mlo =
+      len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
+  const uint64_t mhi =
+      len >= 16 ? ~(uint64_t)0
+                : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
+  lo = (lo & mlo) | (fill & ~mlo);
+  hi = (hi & mhi) | (fill & ~mhi);
+  *(v4i *)(out + (uint64_t)i * 16) = (v4i){(int)(uint32_t)lo,
+      (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
 }
 
 } // namespace
 
-// Few rows whose length is no multiple of 16 bytes, or that do not start on a
-// 16-byte boundary, would fall to the tile kernels, which take several times
-// as long on such shapes (16 x 4100 x 11008: 41 us against 9 us).  The
-// runtime copies them to an aligned buffer with rows of round_up(K, 16) bytes
-// instead, the tail of each row filled with its zero point, and multiplies
-// with that K: (a - a_zp) is zero there, so the products, the row sums and the
+// A row length that is no multiple of 16 bytes, or an A that does not start on a
+// 16-byte boundary, leaves k_gemm_i8, which takes several times as long as the
+// other kernels (16 x 4100 x 11008: 41 us against 9).  The runtime copies such
+// rows to an aligned buffer first, with as many bytes as this says (0: not), the
+// tail of each row filled with its zero point, and multiplies with that K:
+// (a - a_zp) is zero there, so the products, the row sums and the
 // K * (a offset) * (b offset) term of the zero-point algebra are those of the
-// original rows, bit for bit.
-bool gemm_pads_rows(int64_t M, int64_t K, const void *a) {
+// original rows, bit for bit.  Up to 64 rows: 16-byte chunks, for
+// k_gemm_i8_skinny.  More: whole K steps, where the copy -- 3 us and two ways
+// through memory -- costs clearly less than it saves: f32 results 154 x 1022 x
+// 2258 11.8 -> 7.4 us, int32 932 x 1764 x 746 16.3 -> 12.5, 3711 x 964 x 3580 34.8
+// -> 28.9, u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone by the rule: layer 1674 x
+// 280 x 4123 16.8 / 19.2, int32 4099 x 777 x 1001 16.1 / 18.0.
+int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
+    bool rowsums) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
-  return M >= 1 && M <= 64 && K >= 1 &&
-         (K % 16 != 0 || ((((uintptr_t)a) & 15) != 0)) &&
-         !(force && force[0]);
+  if (M < 1 || K < 1 || N < 1 || (K % 16 == 0 && (((uintptr_t)a) & 15) == 0) ||
+      (force && force[0]) || M * K < 16)
+    return 0;
+  if (M <= 64)
+    return round_up(K, 16);
+  const int64_t Kp = round_up(K, kGemmBK);
+  if (Kp >= (1 << 24) || M * (Kp / 16) > UINT32_MAX || M > INT32_MAX ||
+      N > INT32_MAX)
+    return 0;
+  GemmSplit s1, s2;
+  double us = product_us(M, N, Kp, rowsums, s1);
+  // (k_gemm_i8_flight, one round of 64 x 128 blocks: 4 us)
+  if ((Kp == 512 || Kp == 768 || Kp == 1024) &&
+      ((M + 63) / 64) * ((N + 127) / 128) <= 256)
+    us = std::min(us, 4.0);
+  us += 3.0 + 5e-7 * (double)(M * K);
+  return general_us(M, N, K, s2) > us + std::max(1.5, 0.06 * us) ? Kp : 0;
 }
 
 hipError_t launch_pad_rows(hipStream_t s, const void *a, int64_t M, int64_t K,
-    const void *a_zp, int64_t a_zp_len, bool stored_minus_128, void *out) {
-  const int64_t Kp = round_up(K, 16);
-  if (M < 1 || M > 64 || Kp > INT32_MAX)
+    int64_t Kp, const void *a_zp, int64_t a_zp_len, bool stored_minus_128,
+    void *out) {
+  const int64_t n = M * (Kp / 16);
+  if (M * K < 16 || Kp < K || Kp % 16 != 0 || Kp > INT32_MAX || n > UINT32_MAX)
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)((Kp + 1023) / 1024), (unsigned)M);
-  k_pad_rows<<<grid, 256, 0, s>>>((const uint8_t *)a, (int)M, (int)K, (int)Kp,
-      (const uint8_t *)a_zp, (int)a_zp_len, stored_minus_128 ? 0x80 : 0,
-      (uint8_t *)out);
+  k_pad_rows<<<(unsigned)((n + 255) / 256), 256, 0, s>>>((const uint8_t *)a,
+      (unsigned)M, (unsigned)K, (unsigned)(Kp / 16), (const uint8_t *)a_zp,
+      (int)a_zp_len, stored_minus_128 ? 0x80 : 0, (uint8_t *)out);
   return hipGetLastError();
 }
 

@@ -1490,16 +1490,16 @@ void run_matmul(const MatmulSpec &sp) {
   }
   g.out = call.out(y);
   if (b.rank <= 2) {
-    if (call.ok && gemm_pads_rows(M, K, g.A)) {
-      // few rows of an awkward length or alignment: aligned copies whose tail
+    if (const int64_t Kp = call.ok ? gemm_padded_k(M, K, N, g.A, b_uns || bzl > 0) : 0) {
+      // rows of an awkward length or alignment: aligned copies whose tail
       // holds the zero point, multiplied over the padded length
-      void *padded = call.temp((size_t)M * round_up(K, 16));
+      void *padded = call.temp((size_t)(M * Kp));
       if (call.ok)
-        call.check(launch_pad_rows(call.c.stream, g.A, M, K, d_azp, azl,
+        call.check(launch_pad_rows(call.c.stream, g.A, M, K, Kp, d_azp, azl,
                        /*stored_minus_128=*/false, padded),
             "pad rows");
       g.A = padded;
-      g.K = round_up(K, 16);
+      g.K = Kp;
     }
     if (call.ok)
       call.check(call.gemm(g), sp.op);
@@ -1968,15 +1968,17 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
       else if (call.ok)
         run_dql(call, dx, M * K, aq, call.c.dql_scale, call.c.dql_zp, true);
       g.A = aq;
-      if (call.ok && gemm_pads_rows(M, K, aq)) {
+      padded_k = call.ok ? gemm_padded_k(M, K, N, aq,
+                               b.dtype == OM_MI355X_TYPE_UINT8 || bzl > 0)
+                         : 0;
+      if (padded_k) {
         // (see run_matmul) the quantized rows are stored minus 128
-        void *padded = call.temp((size_t)M * round_up(K, 16));
+        void *padded = call.temp((size_t)(M * padded_k));
         if (call.ok)
-          call.check(launch_pad_rows(call.c.stream, aq, M, K, call.c.dql_zp, 1,
-                         /*stored_minus_128=*/true, padded),
+          call.check(launch_pad_rows(call.c.stream, aq, M, K, padded_k,
+                         call.c.dql_zp, 1, /*stored_minus_128=*/true, padded),
               "pad rows");
         g.A = padded;
-        padded_k = round_up(K, 16);
       }
       if (!call.ok)
         return hipSuccess; // already reported

@@ -127,3 +127,28 @@ def test_streaming_kernel_split_along_k(rt, oracle, M, K, N):
     assert np.array_equal(rt.MatMulInteger(a, b, az, bz), oracle.matmul_integer(a, b, az, bz))
     kernel = rt.last_gemm_kernel()
     assert "dma_bs" in kernel and "split" in kernel and "ragged" in kernel, kernel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,offset", [(154, 1022, 258, 0), (443, 967, 419, 0), (932, 1764, 746, 0), (107, 2009, 620, 0),
+                                          (660, 1020, 474, 0), (154, 1024, 258, 1), (70, 1007, 200, 3), (3, 5, 40, 0), (64, 1001, 70, 0)])
+def test_rows_copied_to_an_aligned_pitch(rt, oracle, M, K, N, offset):
+    """Rows of an awkward length or start, copied in chunks of 16 bytes read at any
+    address (`offset`: bytes in front of A) with tails of zero points."""
+    rng = np.random.default_rng(M + K)
+    for adt, bdt, per in ((np.uint8, np.int8, False), (np.int8, np.uint8, True), (np.uint8, np.uint8, False)):
+        i, j = np.iinfo(adt), np.iinfo(bdt)
+        a, b = rng.integers(i.min, i.max + 1, (M, K), dtype=adt), rng.integers(j.min, j.max + 1, (K, N), dtype=bdt)
+        az, bz = rng.integers(i.min, i.max + 1, M, dtype=adt), rng.integers(j.min, j.max + 1, N, dtype=bdt)
+        az, bz = (az, bz) if per else (az[:1], bz[:1])
+        whole = rt.DeviceArray.from_numpy(np.concatenate([np.full(offset, 77, adt), a.reshape(-1)]))
+        da = rt.DeviceArray.view_of(whole, offset, (M, K))
+        got = rt.MatMulInteger(da, rt.DeviceArray.from_numpy(b), rt.DeviceArray.from_numpy(az), rt.DeviceArray.from_numpy(bz))
+        rt.synchronize()
+        if M * N > 300000 or M <= 64:
+            assert "any K" not in rt.last_gemm_kernel(), rt.last_gemm_kernel()
+        assert np.array_equal(got.numpy(), oracle.matmul_integer(a, b, az, bz))
+    x, s = rng.standard_normal((M, K), dtype=np.float32), rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+    q, qs, qz = oracle.dynamic_quantize_linear(x)
+    got = rt.DynQuantMatMulDequant(x, b, bz, s)
+    assert np.array_equal(got, oracle.dequant_epilogue(oracle.matmul_integer(q, b, qz, bz), qs, s))
