@@ -224,6 +224,26 @@ hipError_t launch_pad_rows(hipStream_t s, const void *a, int64_t M, int64_t K,
     int64_t Kp, const void *a_zp, int64_t a_zp_len, bool stored_minus_128,
     void *out);
 
+// Host tensors of up to a few MiB, between page-locked memory and the GPU
+// (host_copy.hip).  Sizes count up to whole 16-byte vectors on both sides, which
+// have to hold them.
+hipError_t launch_copy_in(hipStream_t s, const void *src, void *dst, size_t bytes);
+struct CopyOut {
+  static constexpr int kTensors = 4;
+  static constexpr unsigned kChunk = 16384;
+  struct {
+    const char *src;      // on the GPU
+    char *dst;            // page-locked
+    unsigned bytes, first_chunk;
+  } t[kTensors];
+  int tensors;
+  unsigned chunks, epoch;
+  unsigned *arrived;      // [chunks], page-locked: epoch once the chunk is there
+  const unsigned *failed; // two words of GPU memory sent along (null: none)
+  unsigned *status;       // where they go, complete with chunk 0
+};
+hipError_t launch_copy_out(hipStream_t s, const CopyOut &a);
+
 // Fill n 32-bit words with v.
 hipError_t launch_fill_u32(hipStream_t s, uint32_t *p, int64_t n, uint32_t v);
 

@@ -477,6 +477,34 @@ struct Ctx {
     return false;
   }
 
+  // Page-locked memory for host tensors that are copied by kernels
+  // (host_copy.hip): words that say which chunks of the results have arrived, the
+  // inputs of the call, its results.  A call that uses it waits before it returns,
+  // so the next one finds it idle.
+  static constexpr size_t kArenaIn = (size_t)2 << 20, kArenaOut = (size_t)4 << 20;
+  static constexpr size_t kArenaWords = 4096; // bytes
+  static constexpr size_t kPieceIn = (size_t)256 << 10;
+  char *arena = nullptr;
+  bool arena_off = false;
+  unsigned arena_epoch = 0;
+  bool arena_ready() {
+    if (arena || arena_off)
+      return arena != nullptr;
+    void *p = nullptr;
+    if (hipHostMalloc(&p, kArenaWords + kArenaIn + kArenaOut,
+            hipHostMallocCoherent) != hipSuccess) {
+      (void)hipGetLastError();
+      arena_off = true;
+      return false;
+    }
+    arena = (char *)p;
+    memset(arena, 0, kArenaWords);
+    return true;
+  }
+  unsigned *arena_words() { return (unsigned *)arena; }
+  char *arena_in() { return arena + kArenaWords; }
+  char *arena_out() { return arena + kArenaWords + kArenaIn; }
+
   bool stage_ready() {
     if (!fork_ev && hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming) !=
                         hipSuccess) {
@@ -643,6 +671,8 @@ struct Ctx {
     taken.clear();
     if (dql.partial_min)
       (void)hipFree(dql.partial_min);
+    if (arena)
+      (void)hipHostFree(arena);
     if (lane.ready) {
       (void)hipHostFree(lane.slot[0]);
       for (int i = 0; i < CopyLane::kSlots; ++i)
@@ -826,6 +856,7 @@ struct Call {
   bool ok = true;
   bool touched_host = false;
   bool used_dql = false; // launched DynamicQuantizeLinear (see dql_barrier_ok)
+  bool one_launch = false; // a kernel of this call may give up (dql_gave_up)
   struct Back {
     void *host;
     void *dev;
@@ -875,8 +906,7 @@ struct Call {
       return v.data;
     if (void *d = backed_lookup(v.data))
       return d;
-    if (is_device_ptr(v.data))
-      return v.data;
+    // (a constant that has a copy is host memory: no need to ask the driver)
     bool constant = false;
     if (keep_constant) {
       std::lock_guard<std::mutex> lk(g_mem_mutex);
@@ -887,6 +917,8 @@ struct Call {
           return it->second.dev;
       }
     }
+    if (is_device_ptr(v.data))
+      return v.data;
     void *d = nullptr;
     if (constant) {
       if (hipMalloc(&d, v.bytes ? v.bytes : 16) != hipSuccess) {
@@ -917,6 +949,8 @@ struct Call {
     hipError_t e;
     if (v.bytes >= Ctx::kStagedIn && c.stage_ready())
       e = c.copy_staged(v.data, d, v.bytes, false);
+    else if (arena_used + v.bytes <= Ctx::kArenaIn && c.arena_ready())
+      e = copy_in(v, d);
     else
       e = hipMemcpyAsync(d, v.data, v.bytes, hipMemcpyHostToDevice, c.stream);
     if (e != hipSuccess) {
@@ -926,6 +960,87 @@ struct Call {
     }
     touched_host = true;
     return d;
+  }
+
+  // Through the arena in pieces: one crosses the bus while the next is copied
+  // into it.
+  size_t arena_used = 0; // of its input side, by this call
+  hipError_t copy_in(const View &v, void *d) {
+    char *const at = c.arena_in() + arena_used;
+    arena_used = (arena_used + v.bytes + 255) & ~(size_t)255;
+    touched_host = true;
+    for (size_t o = 0; o < v.bytes; o += Ctx::kPieceIn) {
+      const size_t n = std::min(Ctx::kPieceIn, v.bytes - o);
+      memcpy(at + o, (const char *)v.data + o, n);
+      const hipError_t e = launch_copy_in(c.stream, at + o, (char *)d + o, n);
+      if (e != hipSuccess)
+        return e;
+    }
+    return hipSuccess;
+  }
+
+  // The results in host memory, by way of the arena, and with them the end of
+  // everything this call has queued.  False: not possible here, or failed (not
+  // `ok`); `failed`: the give-up flags of the one-launch kernels (dql_gave_up).
+  bool bring_back(unsigned (&failed)[2]) {
+    failed[0] = failed[1] = 0;
+    size_t total = 0;
+    CopyOut a = {};
+    for (const Back &b : backs)
+      total += (b.bytes + 255) & ~(size_t)255;
+    if (!ok || backs.empty() || backs.size() > (size_t)CopyOut::kTensors ||
+        total > Ctx::kArenaOut || sync_every_call() || report_enabled() ||
+        !c.arena_ready())
+      return false;
+    char *at = c.arena_out();
+    for (const Back &b : backs) {
+      a.t[a.tensors] = {(const char *)b.dev, at, (unsigned)b.bytes, a.chunks};
+      ++a.tensors;
+      a.chunks += (unsigned)((b.bytes + CopyOut::kChunk - 1) / CopyOut::kChunk);
+      at += (b.bytes + 255) & ~(size_t)255;
+    }
+    constexpr size_t kWords = Ctx::kArenaWords / sizeof(unsigned) - 2;
+    static_assert(Ctx::kArenaOut / CopyOut::kChunk + CopyOut::kTensors <= kWords,
+        "arrival words");
+    a.epoch = ++c.arena_epoch ? c.arena_epoch : ++c.arena_epoch; // (never 0)
+    a.arrived = c.arena_words() + 2;
+    a.status = c.arena_words();
+    a.status[0] = a.status[1] = 0;
+    a.failed = c.dql.counter + 8;
+    const hipError_t e = launch_copy_out(c.stream, a);
+    if (e != hipSuccess) {
+      check(e, "device-to-host copy");
+      return false;
+    }
+    unsigned chunk = 0;
+    for (int t = 0; t < a.tensors; ++t)
+      for (unsigned o = 0; o < a.t[t].bytes; o += CopyOut::kChunk, ++chunk) {
+        if (!arrived(a.arrived + chunk, a.epoch))
+          return false;
+        memcpy((char *)backs[t].host + o, a.t[t].dst + o,
+            std::min(CopyOut::kChunk, a.t[t].bytes - o));
+      }
+    failed[0] = a.status[0];
+    failed[1] = a.status[1];
+    return true;
+  }
+  bool arrived(const unsigned *word, unsigned epoch) {
+    for (unsigned spin = 0;; ++spin) {
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == epoch)
+        return true;
+      __builtin_ia32_pause();
+      if ((spin & 0xFFFF) == 0xFFFF) {
+        // (still running, or something ended the work on this stream)
+        const hipError_t e = hipStreamQuery(c.stream);
+        if (e == hipErrorNotReady)
+          continue;
+        if (e == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) == epoch)
+          return true;
+        fail(EIO, "device-to-host copy failed: %s", hipGetErrorString(e));
+        ok = false;
+        return false;
+      }
+    }
   }
 
   void *out(const View &v) {
@@ -950,8 +1065,30 @@ struct Call {
     }
   }
 
+  // The results are in host memory and nothing of this call runs any more.
+  bool back = false;
+  // Waits for what this call has queued.  True: the output of a one-launch
+  // kernel is missing (Ctx::dql_gave_up); the call has to be redone.
+  bool gave_up(hipError_t &e) {
+    unsigned failed[2];
+    back = bring_back(failed);
+    if (!back) {
+      e = ok ? hipStreamSynchronize(c.stream) : hipErrorUnknown;
+      return e == hipSuccess && c.dql_gave_up();
+    }
+    if (!failed[0] && !failed[1]) {
+      c.dql_unchecked = false; // (the flags of every launch so far)
+      return false;
+    }
+    back = !c.dql_gave_up();
+    return !back;
+  }
+
   void finish() {
-    if (ok) {
+    unsigned failed[2];
+    if (ok && !back && !used_dql)
+      back = bring_back(failed);
+    if (ok && !back) {
       for (const Back &b : backs) {
         hipError_t e;
         if (b.bytes >= Ctx::kStagedOut && c.stage_ready())
@@ -966,7 +1103,7 @@ struct Call {
         }
       }
     }
-    if ((touched_host || sync_every_call() || report_enabled()) && c.ready) {
+    if (!back && (touched_host || sync_every_call() || report_enabled()) && c.ready) {
       hipError_t e = hipStreamSynchronize(c.stream);
       if (e != hipSuccess && ok)
         fail(EIO, "stream synchronisation failed: %s", hipGetErrorString(e));
@@ -992,8 +1129,9 @@ bool is_q8(int dt) {
 // right away: the outputs are correct when the entry point returns.  A call
 // on GPU tensors only returns without waiting; there a give-up is reported
 // (EIO) at the thread's next synchronisation.
+// later: the caller looks after the flag itself, when its results are back.
 void run_dql(Call &call, const float *dx, int64_t n, uint8_t *dy, float *ds,
-    uint8_t *dz, bool y_shift) {
+    uint8_t *dz, bool y_shift, bool later = false) {
   Ctx &c = call.c;
   const int mode = t_quant_mode;
   if (mode != 0) { // never the one-launch kernel: nothing to check afterwards
@@ -1008,16 +1146,20 @@ void run_dql(Call &call, const float *dx, int64_t n, uint8_t *dy, float *ds,
       "DynamicQuantizeLinear");
   if (!call.ok || c.dql.grid_blocks == 0)
     return;
+  call.one_launch = true;
+  if (later)
+    return;
   if (!(call.touched_host || sync_every_call() || report_enabled())) {
     call.used_dql = true;
     return;
   }
-  const hipError_t e = hipStreamSynchronize(c.stream);
+  hipError_t e = hipSuccess;
+  const bool redo = call.gave_up(e);
   if (e != hipSuccess) {
     call.check(e, "stream synchronisation");
     return;
   }
-  if (c.dql_gave_up()) { // grid_blocks is 0 from here on: two launches
+  if (redo) { // grid_blocks is 0 from here on: two launches
     fprintf(stderr,
         "om_mi355x: DynamicQuantizeLinear: the blocks of the one-launch "
         "kernel timed out waiting for one another; redone with two launches, "
@@ -1966,7 +2108,8 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
                        aq, call.c.dql_scale, call.c.dql_zp, true, t_quant_mode),
             "quantize");
       else if (call.ok)
-        run_dql(call, dx, M * K, aq, call.c.dql_scale, call.c.dql_zp, true);
+        run_dql(call, dx, M * K, aq, call.c.dql_scale, call.c.dql_zp, true,
+            /*later=*/true);
       g.A = aq;
       padded_k = call.ok ? gemm_padded_k(M, K, N, aq,
                                b.dtype == OM_MI355X_TYPE_UINT8 || bzl > 0)
@@ -2016,23 +2159,26 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
   const bool in_kernel = kind == 1 || (kind == 2 && (d_xlim || call.c.dql.grid_blocks > 0));
   hipError_t e = hipSuccess;
   if (call.ok) {
+    bool exchanged = in_kernel && exchanges;
     e = run(in_kernel);
-    if (e == hipErrorNotReady && exchanges) // the exchange is taken or off
+    if (e == hipErrorNotReady && exchanges) { // the exchange is taken or off
+      exchanged = false;
       e = run(false);
-    else if (e == hipSuccess && exchanges) {
+    }
+    if (exchanged && e == hipSuccess) {
+      call.one_launch = true;
       call.c.dql_unchecked = true;
+    }
+    if (e == hipSuccess && call.ok && call.one_launch) {
       if (!(call.touched_host || sync_every_call() || report_enabled()))
         call.used_dql = true;
-      else {
-        e = hipStreamSynchronize(call.c.stream);
-        if (e == hipSuccess && call.c.dql_gave_up()) {
-          fprintf(stderr,
-              "om_mi355x: %s: the blocks of the one-launch "
-              "kernel timed out waiting for one another; redone with two launches "
-              "for the quantization and one for the product, which this thread "
-              "uses from now on\n", op);
-          e = run(false);
-        }
+      else if (call.gave_up(e)) {
+        fprintf(stderr,
+            "om_mi355x: %s: the blocks of the one-launch "
+            "kernel timed out waiting for one another; redone with two launches "
+            "for the quantization and one for the product, which this thread "
+            "uses from now on\n", op);
+        e = run(false);
       }
     }
     if (call.ok)
