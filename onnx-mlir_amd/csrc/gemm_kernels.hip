@@ -1188,27 +1188,28 @@ __global__ __launch_bounds__(256) void k_pad_rows(const uint8_t *__restrict__ A,
 
 } // namespace
 
-// A row length that is no multiple of 16 bytes, or an A that does not start on a
-// 16-byte boundary, leaves k_gemm_i8, which takes several times as long as the
-// other kernels (16 x 4100 x 11008: 41 us against 9).  The runtime copies such
-// rows to an aligned buffer first, with as many bytes as this says (0: not), the
-// tail of each row filled with its zero point, and multiplies with that K:
-// (a - a_zp) is zero there, so the products, the row sums and the
-// K * (a offset) * (b offset) term of the zero-point algebra are those of the
-// original rows, bit for bit.  Up to 64 rows: 16-byte chunks, for
-// k_gemm_i8_skinny.  More: whole K steps, where the copy -- 3 us and two ways
-// through memory -- costs clearly less than it saves: f32 results 154 x 1022 x
-// 2258 11.8 -> 7.4 us, int32 932 x 1764 x 746 16.3 -> 12.5, 3711 x 964 x 3580 34.8
-// -> 28.9, u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone by the rule: layer 1674 x
-// 280 x 4123 16.8 / 19.2, int32 4099 x 777 x 1001 16.1 / 18.0.
+// Rows (more than 64) whose length is no multiple of 16 bytes, or that do not start
+// on a 16-byte boundary, leave k_gemm_i8, at half the speed of the other kernels.
+// The runtime copies such rows to an aligned buffer first, with as many bytes as
+// this says (0: not), the tail of each row filled with its zero point, and
+// multiplies with that K: (a - a_zp) is zero there, so the products, the row sums
+// and the K * (a offset) * (b offset) term of the zero-point algebra are those of
+// the original rows, bit for bit.  Where the copy -- 3 us and two ways through
+// memory -- costs clearly less than it saves: f32 results 154 x 1022 x 2258 11.8
+// -> 7.4 us, int32 932 x 1764 x 746 16.3 -> 12.5, 3711 x 964 x 3580 34.8 -> 28.9,
+// u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone by the rule: layer 1674 x 280 x
+// 4123 16.8 / 19.2, int32 4099 x 777 x 1001 16.1 / 18.0.
 int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
     bool rowsums) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
   if (M < 1 || K < 1 || N < 1 || (K % 16 == 0 && (((uintptr_t)a) & 15) == 0) ||
-      (force && force[0]) || M * K < 16)
+      (force && force[0]))
     return 0;
+  // k_gemm_i8_skinny takes such rows as they are; with many long ones the
+  // second line of each piece costs more than the copy (45 x 4981 x 4292 13.1 us,
+  // copied 11.5; layer 37 x 6095 x 612 15.2 / 14.8).
   if (M <= 64)
-    return round_up(K, 16);
+    return M > 32 && K >= 4096 ? round_up(K, 16) : 0;
   const int64_t Kp = round_up(K, kGemmBK);
   if (Kp >= (1 << 24) || M * (Kp / 16) > UINT32_MAX || M > INT32_MAX ||
       N > INT32_MAX)

@@ -58,13 +58,22 @@ constexpr int kSkinnyDqBytes = 32768;
 // -- 64 bytes of each of 16 rows -- are read back from there, rows CPR * 16 + 16
 // bytes apart to spread them over the banks.  Otherwise the operands are loaded
 // directly: the lanes of the rows that are not there fetch nothing.
-template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG>
+// ANY: rows of any length, starting at any address (M * K >= 16).  A chunk is read
+// where it lies, moved back to end with A where it would run past it; what does
+// not belong to the row becomes the byte that stands for 0 behind the shift, in
+// the batches that reach the end of K.  (DQ: rows of any length; those in LDS are
+// round_up(K, 16) bytes apart.)  Without it such rows were copied by a launch in
+// front: layers 13 x 356 x 5568 10.9 -> 3.9 us, 2 x 2380 x 372 10.9 -> 4.1, 15 x
+// 8000 x 871 10.2 (K % 16 == 0, as before); int32 12 x 946 x 734 7.6 -> 3.4, 17 x
+// 4185 x 1633 7.0 -> 7.0.
+template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG, bool ANY>
 __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
     const uint8_t *__restrict__ A, const float *__restrict__ X,
     const int8_t *__restrict__ Bp, int M, int N, int K, int Kpad,
     EpiParams ep) {
   static_assert(!DQ || (A_MODE == 2 && !STG), "quantized rows");
   static_assert((T == 16 && CT <= 2) || (T == 32 && CT == 1 && !DQ), "tiles");
+  static_assert(!ANY || DQ || STG, "rows of any length");
   constexpr int U = !DQ && !STG ? 4 : 2;    // K steps of a batch
   constexpr int CPR = U * 4;                // 16-byte chunks of a row and batch
   constexpr int RPI = 64 / CPR;             // rows of a load instruction
@@ -133,7 +142,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
   constexpr int NV = DQ > 0 ? DQ : 1;
   f4 v[NV];
   const int nvec = (M * K) >> 2;
+  const int P = ANY ? (K + 15) & ~15 : K; // bytes from row to row in LDS (DQ)
+  float odd = __builtin_nanf("");          // ANY: of the last M * K % 4 elements
   if (DQ) {
+    if (ANY && tid < ((M * K) & 3))
+      odd = X[nvec * 4 + tid];
     const f4 *__restrict__ x4 = (const f4 *)X;
     const float nan = __builtin_nanf(""); // neutral for minnum / maxnum
 #pragma unroll
@@ -178,10 +191,16 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
     if (STG) {
       const int s = kt + (lane % CPR) / 4;
       const int k0 = s * BK + (lane & 3) * 16;
-      const bool k_in = s < kt_end && k0 < K; // K % 16 == 0: in or out
+      const bool k_in = s < kt_end && k0 < K; // (K % 16 == 0: in or out)
 #pragma unroll
       for (int j = 0; j < NLD; ++j) {
         const int row = j * RPI + lane / CPR;
+        if (ANY) {
+          const uint8_t *const last = A + (M * K - 16);
+          const uint8_t *const at = A + (row * K + k0);
+          t.a[j] = *(const v4i_any *)(k_in && row < M && at < last ? at : last);
+          continue;
+        }
         t.a[j] = __builtin_amdgcn_raw_buffer_load_b128(
             arsrc, k_in && row < M ? row * K + k0 : kOutside, 0, 0);
       }
@@ -212,6 +231,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
       hi = __builtin_fmaxf(__builtin_fmaxf(hi, v[j].x),
           __builtin_fmaxf(__builtin_fmaxf(v[j].y, v[j].z), v[j].w));
     }
+    lo = __builtin_fminf(lo, odd);
+    hi = __builtin_fmaxf(hi, odd);
     if (ep.x_limits) { // (the same for every thread) known from the layer before
       lo = ep.x_limits[0];
       hi = ep.x_limits[1];
@@ -244,8 +265,37 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
           const uint32_t q = quant_pack4<false, true, FAST>(v[j].x, v[j].y,
               v[j].z, v[j].w, dq_scale, dq_scale, dq_scale, dq_scale, recip,
               recip, recip, recip, zpf, zpf, zpf, zpf);
-          ((uint32_t *)aq)[e] = q ^ 0x80808080u;
+          if (!ANY) {
+            ((uint32_t *)aq)[e] = q ^ 0x80808080u;
+            continue;
+          }
+          uint32_t r = (uint32_t)(e * 4) / (uint32_t)K;
+          uint32_t c = (uint32_t)(e * 4) - r * (uint32_t)K;
+          if ((K & 3) == 0) { // (the same for every thread)
+            *(uint32_t *)(aq + r * P + c) = q ^ 0x80808080u;
+            continue;
+          }
+#pragma unroll
+          for (int b = 0; b < 4; ++b) {
+            aq[r * P + c] = (uint8_t)((q >> (8 * b)) ^ 0x80u);
+            if (++c == (uint32_t)K) {
+              c = 0;
+              ++r;
+            }
+          }
         }
+      }
+      if (ANY) {
+        const int n = M * K;
+        if (tid < (n & 3)) {
+          const uint32_t q = quant_one<false, true, FAST>(odd, dq_scale, zpf, recip);
+          const uint32_t i = (uint32_t)(nvec * 4 + tid), r = i / (uint32_t)K;
+          aq[r * P + (i - r * (uint32_t)K)] = (uint8_t)(q ^ 0x80u);
+        }
+        // what rounds a row up counts as 0 in the row sums
+        const int c = K + (tid & 15);
+        if ((tid >> 4) < M && c < P)
+          aq[(tid >> 4) * P + c] = 0;
       }
     };
     if (scale_is_tame(dq_scale)) // the same for every thread
@@ -283,6 +333,41 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
       // from moving the reads above the writes of other lanes, and the next
       // batch's writes above these reads.
       uint8_t *const stg = lds_raw + wave * kStageWave;
+      // (the same for the whole wave)
+      if (ANY && ((kt + U) * BK > K || kt + U > kt_end)) {
+        const int s = kt + (lane % CPR) / 4;
+        const int k0 = s * BK + (lane & 3) * 16;
+        constexpr uint64_t kFill = A_MODE == 1 ? 0x8080808080808080ull : 0;
+#pragma unroll
+        for (int j = 0; j < NLD; ++j) {
+          const int row = j * RPI + lane / CPR;
+          const int left = s < kt_end && row < M ? K - k0 : 0;
+          const int len = left < 0 ? 0 : left < 16 ? left : 16;
+          // bytes the load was moved back by: < 16 where the chunk has any
+          const int back = row * K + k0 - (M * K - 16);
+          uint64_t lo = (uint32_t)t.a[j].x | ((uint64_t)(uint32_t)t.a[j].y << 32);
+          uint64_t hi = (uint32_t)t.a[j].z | ((uint64_t)(uint32_t)t.a[j].w << 32);
+          const int sh = back > 0 && len > 0 ? back * 8 : 0;
+          if (sh >= 64) {
+            lo = hi;
+            hi = 0;
+          }
+          const int s1 = sh & 63;
+          if (s1) {
+            lo = (lo >> s1) | (hi << (64 - s1));
+            hi >>= s1;
+          }
+          const uint64_t mlo =
+              len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
+          const uint64_t mhi =
+              len >= 16 ? ~(uint64_t)0
+                        : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
+          lo = (lo & mlo) | (kFill & ~mlo);
+          hi = (hi & mhi) | (kFill & ~mhi);
+          t.a[j] = (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32),
+              (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+        }
+      }
 #pragma unroll
       for (int j = 0; j < NLD; ++j)
         *(v4i *)(stg + (j * RPI + lane / CPR) * kPitch + (lane % CPR) * 16) =
@@ -308,7 +393,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
 #pragma unroll
           for (int r = 0; r < RT; ++r) {
             const int row = r * 16 + lr;
-            a[r][u][0] = *(const v4i *)(aq + (row < M ? row : 0) * K + (in ? k0 : 0));
+            a[r][u][0] = *(const v4i *)(aq + (row < M ? row : 0) * P + (in ? k0 : 0));
             if (decltype(RS)::value)
               a[r][u][0] = in ? a[r][u][0] : zero;
           }
@@ -353,7 +438,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
     k_loop(std::true_type{});
   else
     k_loop(std::false_type{});
-  if (A_MODE == 1 && need_rs) {
+  if (A_MODE == 1 && need_rs && !ANY) {
     // A chunk outside the slice or past K was read as zeros, that is 16 times
     // -128 behind the flip: taken out of the row sums again.  Those are the
     // steps that fill the last batch up, and chunks of the very last step of K.
@@ -424,6 +509,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
   }
 }
 
+// Rows that only the ANY form takes.
+bool any_rows(const GemmArgs &g) {
+  return g.K % 16 != 0 || (!g.X && (((uintptr_t)g.A) & 15) != 0);
+}
+
 template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG>
 void launch_one(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   note_gemm_kernel(
@@ -433,10 +523,13 @@ void launch_one(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
       : CT == 2 ? "k_gemm_i8_skinny (2 x 16 columns)"
       : STG     ? "k_gemm_i8_skinny (16 columns)"
                 : "k_gemm_i8_skinny (16 columns, rows loaded directly)");
-  k_gemm_i8_skinny<A_MODE, EPI, DQ, T, RT, CT, STG>
-      <<<(unsigned)((g.N + T * CT - 1) / (T * CT)), WAVES * 64, 0, st>>>(
-          (const uint8_t *)g.A, g.X, g.Bp, (int)g.M, (int)g.N, (int)g.K,
-          (int)round_up(g.K, kGemmBK), ep);
+  auto *kernel = k_gemm_i8_skinny<A_MODE, EPI, DQ, T, RT, CT, STG, false>;
+  if constexpr (DQ || STG)
+    if (any_rows(g))
+      kernel = k_gemm_i8_skinny<A_MODE, EPI, DQ, T, RT, CT, STG, true>;
+  kernel<<<(unsigned)((g.N + T * CT - 1) / (T * CT)), WAVES * 64, 0, st>>>(
+      (const uint8_t *)g.A, g.X, g.Bp, (int)g.M, (int)g.N, (int)g.K,
+      (int)round_up(g.K, kGemmBK), ep);
 }
 // Blocks of 16 columns are what fills the device while N / 16 is up to 256.
 constexpr int64_t kOneRound = 256 * 16;
@@ -466,7 +559,9 @@ void launch_rows(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
     // round of blocks and for short K (4 rows, K=8192 N=4096: 4.9 us against 5.9
     // through LDS, K=1536 N=11008 4.1 / 4.2); beyond, other blocks' waves hide the
     // loads better (K=11008 N=5120: 12.1 / 9.9, K=2688 N=7808: 4.6 / 4.0).
-    if (!rounds || g.K <= 2048)
+    if (any_rows(g))
+      launch_16<A_MODE, EPI, 0, 1, true>(st, g, ep);
+    else if (!rounds || g.K <= 2048)
       launch_16<A_MODE, EPI, 0, 1, false>(st, g, ep);
     else
       launch_one<A_MODE, EPI, 0, 16, 1, 1, true>(st, g, ep);
@@ -506,14 +601,14 @@ void launch_epi(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
 
 // Whether the kernel can quantize this activation itself (DQ).
 bool skinny_quantizes_rows(int64_t M, int64_t K, const void *x) {
-  return M >= 1 && M <= 32 && K > 0 && K % 16 == 0 &&
-         M * K <= kSkinnyDqBytes && ((((uintptr_t)x) & 15) == 0);
+  return M >= 1 && M <= 32 && K > 0 && K <= kSkinnyDqBytes &&
+         M * round_up(K, 16) <= kSkinnyDqBytes && ((((uintptr_t)x) & 15) == 0);
 }
 
 // (K: the offsets of 64 rows and of a column tile's operands stay in 31 bits.)
 bool skinny_ok(int64_t M, int64_t K, const void *a) {
-  return M >= 1 && M <= 64 && K > 0 && K % 16 == 0 && K < (1 << 24) &&
-         ((((uintptr_t)a) & 15) == 0);
+  (void)a;
+  return M >= 1 && M <= 64 && K > 0 && K < (1 << 24) && M * K >= 16;
 }
 
 hipError_t launch_gemm_skinny(hipStream_t st, const GemmArgs &g,

@@ -131,7 +131,7 @@ def test_streaming_kernel_split_along_k(rt, oracle, M, K, N):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N,offset", [(154, 1022, 258, 0), (443, 967, 419, 0), (932, 1764, 746, 0), (107, 2009, 620, 0),
-                                          (660, 1020, 474, 0), (154, 1024, 258, 1), (70, 1007, 200, 3), (3, 5, 40, 0), (64, 1001, 70, 0)])
+                                          (660, 1020, 474, 0), (154, 1024, 258, 1), (70, 1007, 200, 3)])
 def test_rows_copied_to_an_aligned_pitch(rt, oracle, M, K, N, offset):
     """Rows of an awkward length or start, copied in chunks of 16 bytes read at any
     address (`offset`: bytes in front of A) with tails of zero points."""
@@ -145,10 +145,46 @@ def test_rows_copied_to_an_aligned_pitch(rt, oracle, M, K, N, offset):
         da = rt.DeviceArray.view_of(whole, offset, (M, K))
         got = rt.MatMulInteger(da, rt.DeviceArray.from_numpy(b), rt.DeviceArray.from_numpy(az), rt.DeviceArray.from_numpy(bz))
         rt.synchronize()
-        if M * N > 300000 or 16 <= M * K and M <= 64:
+        if M * N > 300000:
             assert "any K" not in rt.last_gemm_kernel(), rt.last_gemm_kernel()
         assert np.array_equal(got.numpy(), oracle.matmul_integer(a, b, az, bz))
     x, s = rng.standard_normal((M, K), dtype=np.float32), rng.uniform(1e-3, 1e-2, N).astype(np.float32)
     q, qs, qz = oracle.dynamic_quantize_linear(x)
     got = rt.DynQuantMatMulDequant(x, b, bz, s)
     assert np.array_equal(got, oracle.dequant_epilogue(oracle.matmul_integer(q, b, qz, bz), qs, s))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,offset", [(1, 17, 5, 0), (16, 1, 40, 0), (7, 3, 33, 0), (7, 1, 20, 0), (2, 9, 64, 0), (4, 255, 100, 0),
+                                          (5, 356, 70, 0), (13, 1001, 4200, 0), (16, 2049, 31, 0), (17, 130, 64, 0), (32, 1021, 100, 0),
+                                          (24, 1537, 4200, 0), (33, 700, 50, 0), (48, 4097, 40, 0), (64, 333, 4200, 0),
+                                          (50, 1031, 5000, 0), (6, 1024, 70, 5), (20, 256, 4200, 1), (60, 128, 30, 15), (3, 64, 9, 8)])
+def test_few_rows_of_any_length(rt, oracle, M, K, N, offset):
+    """The weight-streaming kernel reads rows where they lie: ends inside a chunk, a
+    wave's slice past K, the last chunk of A, starts at any byte; and quantizes
+    rows that float4 do not divide."""
+    rng = np.random.default_rng(M + 7 * K)
+    for adt, bdt, per in ((np.uint8, np.int8, False), (np.int8, np.uint8, True), (np.uint8, np.uint8, False), (np.int8, np.int8, True)):
+        i, j = np.iinfo(adt), np.iinfo(bdt)
+        a, b = rng.integers(i.min, i.max + 1, (M, K), dtype=adt), rng.integers(j.min, j.max + 1, (K, N), dtype=bdt)
+        az, bz = rng.integers(i.min, i.max + 1, M, dtype=adt), rng.integers(j.min, j.max + 1, N, dtype=bdt)
+        az, bz = (az, bz) if per else (az[:1], bz[:1])
+        whole = rt.DeviceArray.from_numpy(np.concatenate([np.full(offset, 77, adt), a.reshape(-1)]))
+        da = rt.DeviceArray.view_of(whole, offset, (M, K))
+        got = rt.MatMulInteger(da, rt.DeviceArray.from_numpy(b), rt.DeviceArray.from_numpy(az), rt.DeviceArray.from_numpy(bz))
+        rt.synchronize()
+        assert "skinny" in rt.last_gemm_kernel() or M * K < 16, rt.last_gemm_kernel()
+        want = oracle.matmul_integer(a, b, az, bz)
+        assert np.array_equal(got.numpy(), want), (adt, bdt)
+        x, s = rng.normal(0.3, 1, (M, K)).astype(np.float32), rng.uniform(1e-3, 1e-2, N).astype(np.float32)
+        x[-1, -1] = 9.5  # the largest element is the very last one
+        q, qs, qz = oracle.dynamic_quantize_linear(x)
+        z = bz if bdt == np.uint8 else None
+        got = rt.DynQuantMatMulDequant(rt.DeviceArray.from_numpy(x), rt.DeviceArray.from_numpy(b),
+                                       None if z is None else rt.DeviceArray.from_numpy(z), rt.DeviceArray.from_numpy(s))
+        rt.synchronize()
+        assert "skinny" in rt.last_gemm_kernel()
+        assert np.array_equal(got.numpy(), oracle.dequant_epilogue(oracle.matmul_integer(q, b, qz, z), qs, s)), (M, K, N)
+        y = [np.float32(v) for v in (0.0173, 0.005, 0.37)]
+        want = oracle.qlinear_matmul(a, y[0], az[:1], b, y[1], bz[:1], y[2], az[0], 1)
+        assert np.array_equal(rt.QLinearMatMul(a, y[0], az[:1], b, y[1], bz[:1], y[2], az[0], rt.SATURATE), want)
