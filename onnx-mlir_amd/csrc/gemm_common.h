@@ -86,6 +86,7 @@ struct EpiParams {
   const float *bias;     // kEpiF32: added after the scaling; null = none
   int64_t bias_len;      // 1 or N
   float floor;           // kEpiF32: relu_floor(whether onnx.Relu follows)
+  bool gelu;             // kEpiF32: onnx.Gelu on the result
   void *out;
   bool b_unsigned;
   bool y_unsigned;

@@ -763,9 +763,6 @@ bool gemm_fast_path(int64_t M, int64_t K, const void *A) {
 // Name of the kernel the calling thread's last launch_gemm chose (for tests
 // and reports).
 thread_local const char *t_last_kernel = "";
-// Whether that kernel applied the onnx.Gelu asked for to its results itself
-// (launch_gemm runs the pass over the output when it did not).
-thread_local bool t_gelu_applied = false;
 // Whether that kernel wrote GemmArgs::y_limits itself (launch_gemm runs the
 // reduction over the output when it did not).
 thread_local bool t_limits_written = false;
@@ -1006,7 +1003,6 @@ hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
   const bool vec = (((uintptr_t)g.out) & (EPI == kEpiQ8 ? 3 : 15)) == 0;
   k_sum_parts<EPI><<<(n + 1023) / 1024, 256, 0, st>>>(
       g.parts, p.parts, ks.stride, n, (unsigned)N, ep, g.gelu, vec);
-  t_gelu_applied = EPI == kEpiF32 && g.gelu;
   return hipGetLastError();
 }
 
@@ -1046,7 +1042,6 @@ hipError_t gemm_launch_cfg(
       if (EPI != kEpiF32 || !g.dql)
         return hipErrorInvalidValue;
       t_last_kernel = "k_gemm_i8_flight (rows quantized in the kernel)";
-      t_gelu_applied = g.gelu; // this kernel applies it to its results
       t_limits_written = ep.limits.out != nullptr; // and reduces their limits
       return launch_gemm_flight_dq(st, g, ep, *g.dql);
     }
@@ -1085,7 +1080,6 @@ hipError_t gemm_launch_cfg(
   // k_gemm_i8_dma; 128 x 768 x 768: 7.0 us).
   if ((cfg == kFlight || !(force && force[0])) && flight_ok(g, A_MODE)) {
     t_last_kernel = "k_gemm_i8_flight (one round, operands requested at once)";
-    t_gelu_applied = EPI == kEpiF32 && g.gelu; // this kernel applies it itself
     t_limits_written = EPI == kEpiF32 && ep.limits.out != nullptr;
     return launch_gemm_flight(st, g, ep, A_MODE);
   }
@@ -1094,7 +1088,6 @@ hipError_t gemm_launch_cfg(
   const bool forced = force && force[0];
   if (wreg_ok(g) && (cfg == kW128x384 || (!forced && wreg_pays(g.M, g.N)))) {
     t_last_kernel = "k_gemm_i8_wreg (weights in registers, 128x384 blocks)";
-    t_gelu_applied = g.epi == kEpiF32 && g.gelu; // this kernel applies it to its results
     // (the limits of y: in the kernel for the f32 results of a fused layer)
     t_limits_written = A_MODE == 2 && EPI == kEpiF32 && ep.limits.out != nullptr;
     return launch_gemm_wreg(st, g, ep, A_MODE);
@@ -1273,49 +1266,6 @@ size_t gemm_plan_split(GemmArgs &g) {
 const char *last_gemm_kernel() { return t_last_kernel; }
 void note_gemm_kernel(const char *name) { t_last_kernel = name; }
 
-namespace {
-// onnx.Gelu (gelu_f32) in place over n floats, for the kernels that do not
-// apply it to their results themselves; y 16-byte aligned or not (the edges
-// go one by one).
-__global__ __launch_bounds__(256) void k_gelu_inplace(float *__restrict__ y,
-    int64_t n) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  const int64_t head = (4 - (int64_t)((((uintptr_t)y) >> 2) & 3)) & 3; // floats before the first aligned vector
-  const int64_t lead = head < n ? head : n;
-  f4 *const y4 = (f4 *)(y + lead);
-  const int64_t nvec = (n - lead) >> 2;
-  const int64_t base = (int64_t)blockIdx.x * 512 + threadIdx.x;
-  f4 v[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t i = base + j * 256;
-    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    v[j] = i < nvec ? y4[i] : zero;
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int64_t i = base + j * 256;
-    if (i < nvec) {
-      f4 o;
-      o.x = gelu_f32(v[j].x);
-      o.y = gelu_f32(v[j].y);
-      o.z = gelu_f32(v[j].z);
-      o.w = gelu_f32(v[j].w);
-      y4[i] = o;
-    }
-  }
-  if (blockIdx.x == 0) {
-    // up to three floats before the first vector and after the last one
-    const int64_t t = threadIdx.x;
-    if (t < lead)
-      y[t] = gelu_f32(y[t]);
-    const int64_t tail = lead + (nvec << 2) + t;
-    if (t < 4 && tail < n)
-      y[tail] = gelu_f32(y[tail]);
-  }
-}
-} // namespace
-
 hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
   if (g.M == 0 || g.N == 0)
     return hipSuccess;
@@ -1343,12 +1293,12 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
     ep.limits = LimitsOut{g.y_limits, g.dql->partial_min, g.dql->partial_max,
         g.dql->counter + 4};
   ep.floor = relu_floor(g.epi == kEpiF32 && g.relu);
+  ep.gelu = g.epi == kEpiF32 && g.gelu;
   ep.out = g.out;
   ep.b_unsigned = g.b_unsigned;
   ep.y_unsigned = g.y_unsigned;
   ep.narrow = (int)g.narrow;
   const int a_mode = (g.X || g.a_preshifted) ? 2 : (g.a_unsigned ? 1 : 0);
-  t_gelu_applied = false;
   t_limits_written = false;
   if (g.y_limits && (g.epi != kEpiF32 || !g.dql))
     return hipErrorInvalidValue;
@@ -1363,14 +1313,6 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
   default:
     e = gemm_launch_epi<2>(s, g, ep, Kpad);
     break;
-  }
-  if (e == hipSuccess && g.epi == kEpiF32 && g.gelu && !t_gelu_applied) {
-    // onnx.Gelu on the result, as a pass of its own over the f32 output
-    const int64_t n = g.M * g.N;
-    const int64_t per_block = 256 * 2 * 4;
-    k_gelu_inplace<<<(unsigned)((n + per_block - 1) / per_block), 256, 0, s>>>(
-        (float *)g.out, n);
-    e = hipGetLastError();
   }
   if (e == hipSuccess && g.y_limits && !t_limits_written)
     e = launch_minmax_limits(s, *g.dql, (const float *)g.out, g.M * g.N, g.y_limits);

@@ -188,3 +188,26 @@ def test_few_rows_of_any_length(rt, oracle, M, K, N, offset):
         y = [np.float32(v) for v in (0.0173, 0.005, 0.37)]
         want = oracle.qlinear_matmul(a, y[0], az[:1], b, y[1], bz[:1], y[2], az[0], 1)
         assert np.array_equal(rt.QLinearMatMul(a, y[0], az[:1], b, y[1], bz[:1], y[2], az[0], rt.SATURATE), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile", ["0", "1", "2", "3", "6", "7", ""])
+@pytest.mark.parametrize("M,K,N", [(129, 256, 260), (256, 512, 256), (70, 1001, 33), (20, 640, 100), (3, 33, 70)])
+def test_gelu_in_every_kernel(rt, oracle, monkeypatch, tile, M, K, N):
+    """onnx.Gelu in the epilogue, whole and cut tiles, rows of whole and of partial
+    lines, with and without row sums.  Tolerance: 4 units in the last place of erf
+    (2^-22) times |0.5 x|, plus one rounding of the result."""
+    if tile:
+        monkeypatch.setenv("OM_MI355X_GEMM_TILE", tile)
+    rng = np.random.default_rng(K)
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    ws, bias = rng.uniform(1e-5, 1e-3, N).astype(np.float32), rng.normal(0, 1, N).astype(np.float32)
+    q, s, z = oracle.dynamic_quantize_linear(x)
+    for bdt, bz in ((np.int8, None), (np.uint8, np.uint8(131))):
+        j = np.iinfo(bdt)
+        b = rng.integers(j.min, j.max + 1, (K, N), dtype=bdt)
+        plain = oracle.dequant_epilogue(oracle.matmul_integer(q, b, z, bz), s, ws) + bias
+        got = rt.DynQuantMatMulDequant(x, b, bz, ws, bias, activation=rt.ACTIVATION_GELU)
+        want = oracle.gelu(plain).astype(np.float64)
+        tol = np.abs(0.5 * plain.astype(np.float64)) * 2.0 ** -22 + np.abs(want) * 2.0 ** -23 + 1e-45
+        assert (np.abs(got - want) <= tol).all(), rt.last_gemm_kernel()
