@@ -1,6 +1,7 @@
-"""Host model of every global and LDS access of k_gemm_i8_bs as it is shipped
-(onnx-mlir_amd/csrc/gemm_kernels.hip, instantiation <TM=4, TN=2, D=4, NST=4,
-PIPE>), of its epilogue's stores (gemm_epilogue.h), of k_pad_rows and of the
+"""Host model of every global and LDS access of k_gemm_i8_bs as it was before A
+was copied in whole lines (gemm_bs.hip; instantiation <TM=4, TN=2, D=4, NST=4,
+PIPE>; the kernel of today: test_bs_line_model.py), of its epilogue's stores
+(gemm_epilogue.h), of k_pad_rows with a byte per thread and of the
 buffer pool's size arithmetic (runtime.hip), checked against the real extents
 of the operands over a grid of shapes; and of the kernel's count of outstanding
 memory operations (its explicit vmcnt waits).  No GPU: this is index arithmetic
@@ -10,9 +11,8 @@ Why it exists: a benchmark loop on 4096 x 1040 x 4096 (rows padded to 1088
 bytes, 17 K steps, this instantiation) once ended with an illegal memory
 access that nothing in the suite shows.  The model finds every access of that
 launch in bounds and every wait sufficient (the assertions below hold for it),
-so the cause is not in what is modelled here; the padding path stays out of
-the library, and the dispatch keeps this kernel to step counts that are
-multiples of four (test_dispatch_keeps_bs_to_whole_trips in the GPU suite).
+so the cause is not in what is modelled here; the dispatch keeps
+k_gemm_i8_bs to step counts that are multiples of four, rows padded or not (test_dispatch_keeps_bs_to_whole_trips in the GPU suite).
 The model of the waits does find the defect of the other development variant
 that failed on the device, the one with six LDS stages (see the last tests of
 the wait model).
