@@ -925,13 +925,31 @@ double product_us(int64_t M, int64_t N, int64_t K, bool rowsums, GemmSplit &best
   }
   return best.parts > 1 ? us : least;
 }
-// And in k_gemm_i8, for any K; the model of kTileCosts, fitted to 30 products.
-double general_us(int64_t M, int64_t N, int64_t K, GemmSplit &best) {
-  const TileCost t = {kT128x128, 128, 128, 1, 0.434, 0.359, 2.33, 2.62, 0.76};
-  double least = tile_us(t, M, N, K);
+// And in k_gemm_i8, for any K: tiles of 128 x 128 and of 64 x 128, four blocks of
+// which run on a CU and are dealt out more evenly; the model of kTileCosts, fitted
+// to 44 products timed with both, row sums dearer to the larger tile.  Int32 4099 x
+// 777 x 1001 16.1 us in the larger, 14.4 in the smaller, 1618 x 653 x 311 8.6 / 6.8,
+// u8 1959 x 1891 x 502 17.2 / 12.5; u8 3694 x 278 x 4295 17.5 / 21.3, int32 2290 x 293 x
+// 8977 25.4 / 28.8.
+double any_us(bool low, int64_t M, int64_t N, int64_t K, bool rowsums) {
+  static constexpr TileCost t128 = {
+      kT128x128, 128, 128, 1, 0.434, 0.359, 2.33, 2.62, 0.76};
+  static constexpr TileCost t64 = {
+      kT128x128, 64, 128, 1, 0.266, 0.191, 1.78, 2.62, 0.95};
+  const double us = tile_us(low ? t64 : t128, M, N, K);
+  return us + (rowsums ? (low ? 0.1 : 0.2) * std::max(0.0, us - 3.5) : 0.0);
+}
+bool any_takes_64_rows(int64_t M, int64_t N, int64_t K, bool rowsums) {
+  return any_us(true, M, N, K, rowsums) < 0.99 * any_us(false, M, N, K, rowsums);
+}
+double general_us(int64_t M, int64_t N, int64_t K, bool rowsums, GemmSplit &best) {
+  double least =
+      std::min(any_us(false, M, N, K, rowsums), any_us(true, M, N, K, rowsums));
   if (split_possible(M, N, K, true)) {
-    // (a tenth off the chain of its steps)
-    double us = 3.5 + 0.45 * (double)((K + kGemmBK - 1) / kGemmBK);
+    // (a long chain is split unless that is clearly worse: 3872 x 10201 x 477 44.4
+    // us in two parts, 48.8 in one piece; a short one where it is ahead: 442 x 1042
+    // x 431 9.9 us in four parts, 9.1 in one piece)
+    double us = K >= 64 * kGemmBK ? 1.15 * least : 0.98 * least - 0.2;
     try_split(split_form(kSplitAny, M, N), M, N, K, best, us);
     if (best.parts > 1)
       least = us;
@@ -951,7 +969,7 @@ GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   if (force && force[0])
     return best;
   if (any)
-    (void)general_us(g.M, g.N, g.K, best);
+    (void)general_us(g.M, g.N, g.K, g.b_unsigned || g.b_zp_len > 0, best);
   else
     (void)product_us(g.M, g.N, g.K, g.b_unsigned || g.b_zp_len > 0, best);
   return best;
@@ -1059,8 +1077,15 @@ hipError_t gemm_launch_cfg(
   if (!gemm_fast_path(g.M, g.K, g.A)) {
     // Any K, any alignment of A (and the forced configurations of the tests
     // when M <= 16); byte loads only for an A of fewer than 16 bytes.
-    t_last_kernel = "k_gemm_i8 (any K, any alignment)";
-    if (g.M * g.K >= 16)
+    const bool low = g.M * g.K >= 16 && any_takes_64_rows(g.M, g.N, g.K, ep.need_rowsum);
+    t_last_kernel = low ? "k_gemm_i8 (any K, any alignment; 64x128 tiles)"
+                        : "k_gemm_i8 (any K, any alignment)";
+    const int tiles_m64 = (int)((g.M + 63) / 64);
+    if (low)
+      k_gemm_i8<64, 128, 2, 2, 4, A_MODE, EPI, kLoadAny>
+          <<<dim3((unsigned)(tiles_m64 * tiles_n128)), 256, 0, st>>>(
+              A, g.Bp, M, N, K, Kpad, ep, tiles_m64, tiles_n128);
+    else if (g.M * g.K >= 16)
       k_gemm_i8<128, 128, 2, 2, 2, A_MODE, EPI, kLoadAny>
           <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(
               A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n128);
@@ -1188,10 +1213,10 @@ __global__ __launch_bounds__(256) void k_pad_rows(const uint8_t *__restrict__ A,
 // multiplies with that K: (a - a_zp) is zero there, so the products, the row sums
 // and the K * (a offset) * (b offset) term of the zero-point algebra are those of
 // the original rows, bit for bit.  Where the copy -- 3 us and two ways through
-// memory -- costs clearly less than it saves: f32 results 154 x 1022 x 2258 11.8
-// -> 7.4 us, int32 932 x 1764 x 746 16.3 -> 12.5, 3711 x 964 x 3580 34.8 -> 28.9,
-// u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone by the rule: layer 1674 x 280 x
-// 4123 16.8 / 19.2, int32 4099 x 777 x 1001 16.1 / 18.0.
+// memory -- costs clearly less than it saves (128 x 128 tiles of k_gemm_i8 at the
+// time of measuring): f32 154 x 1022 x 2258 11.8 -> 7.4 us, 3711 x 964 x 3580 34.8 ->
+// 28.9, u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone: layer 1674 x 280 x 4123 16.8 /
+// 19.2, int32 4099 x 777 x 1001 14.4 / 18.0, u8 1032 x 487 x 6105 12.2 / 13.2.
 int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
     bool rowsums) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
@@ -1214,7 +1239,7 @@ int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
       ((M + 63) / 64) * ((N + 127) / 128) <= 256)
     us = std::min(us, 4.0);
   us += 3.0 + 5e-7 * (double)(M * K);
-  return general_us(M, N, K, s2) > us + std::max(1.5, 0.06 * us) ? Kp : 0;
+  return general_us(M, N, K, rowsums, s2) > us + std::max(1.6, 0.03 * us) ? Kp : 0;
 }
 
 hipError_t launch_pad_rows(hipStream_t s, const void *a, int64_t M, int64_t K,

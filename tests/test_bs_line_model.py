@@ -130,7 +130,7 @@ def test_streaming_kernel_split_along_k(rt, oracle, M, K, N):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,K,N,offset", [(154, 1022, 258, 0), (443, 967, 419, 0), (932, 1764, 746, 0), (107, 2009, 620, 0),
+@pytest.mark.parametrize("M,K,N,offset", [(154, 1022, 258, 0), (443, 967, 419, 0), (900, 1019, 640, 0), (107, 2009, 620, 0),
                                           (660, 1020, 474, 0), (154, 1024, 258, 1), (70, 1007, 200, 3)])
 def test_rows_copied_to_an_aligned_pitch(rt, oracle, M, K, N, offset):
     """Rows of an awkward length or start, copied in chunks of 16 bytes read at any
@@ -211,3 +211,32 @@ def test_gelu_in_every_kernel(rt, oracle, monkeypatch, tile, M, K, N):
         want = oracle.gelu(plain).astype(np.float64)
         tol = np.abs(0.5 * plain.astype(np.float64)) * 2.0 ** -22 + np.abs(want) * 2.0 ** -23 + 1e-45
         assert (np.abs(got - want) <= tol).all(), rt.last_gemm_kernel()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,low", [
+    (65, 257, 129, True), (127, 321, 300, True), (193, 130, 65, True), (1618, 653, 311, True),
+    (300, 272, 200, True),
+    (2637, 787, 995, None), (932, 1764, 746, None), (3694, 78, 4295, False)])
+def test_any_k_in_tiles_of_64_rows(rt, oracle, M, K, N, low):
+    """k_gemm_i8 takes 64 x 128 tiles where they are dealt out better: whole and cut
+    tiles, last steps of every length, A at an odd address, with and without row
+    sums.  Whole numbers: exact."""
+    rng = np.random.default_rng(M + K)
+    for bdt in (np.int8, np.uint8):
+        i = np.iinfo(bdt)
+        b = rng.integers(i.min, i.max + 1, (K, N), dtype=bdt)
+        a = rng.integers(0, 256, (M, K), dtype=np.uint8)
+        azp = np.uint8(77)
+        bzp = np.uint8(131) if bdt == np.uint8 else None
+        want = oracle.matmul_integer(a, b, azp, bzp)
+        got = rt.MatMulInteger(a, b, azp, bzp)
+        kernel = rt.last_gemm_kernel()
+        if "any K" in kernel and "split" not in kernel:
+            assert low is None or ("64x128" in kernel) == low, kernel
+        assert np.array_equal(got, want), kernel
+        whole = rt.DeviceArray.from_numpy(np.concatenate([np.full(3, 77, np.uint8), a.reshape(-1)]))
+        got = rt.MatMulInteger(rt.DeviceArray.view_of(whole, 3, (M, K)), rt.DeviceArray.from_numpy(b),
+                               rt.DeviceArray.from_numpy(np.array(azp)), bzp if bzp is None else rt.DeviceArray.from_numpy(np.array(bzp)))
+        rt.synchronize()
+        assert np.array_equal(got.numpy(), want), rt.last_gemm_kernel()
