@@ -128,13 +128,22 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
     brsrc.z = step < KT ? b_bytes : 0;
     bstep = step < KT ? step * 2048 : 0;
   };
-  auto load_b = [&](int sub, v4i(&fb)[TN]) {
-    const int soff = bstep + sub * 1024;
+  // (The half step is in the instruction: the device compares the other offsets
+  // with the descriptor's size minus the scalar one, unsigned, so that an empty
+  // descriptor asks for nothing only with a scalar offset of 0.)
+  using Half0 = std::integral_constant<int, 0>;
+  using Half1 = std::integral_constant<int, 1>;
+  auto load_b = [&](auto half, v4i(&fb)[TN]) {
+    // (named here: asm operands alone do not capture in a generic lambda)
+    const int soff = bstep;
+    const v4i rsrc = brsrc;
+    const int(&off)[TN] = boff;
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-      asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"
+      asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen offset:%4"
                    : "=v"(fb[j])
-                   : "v"(boff[j]), "s"(brsrc), "s"(soff)
+                   : "v"(off[j]), "s"(rsrc), "s"(soff),
+                   "n"(decltype(half)::value * 1024)
                    : "memory");
   };
 
@@ -193,8 +202,8 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
 #pragma unroll
   for (int u = 0; u < D - 1; ++u) {
     weights_of(u);
-    load_b(0, bs[u][0]);
-    load_b(1, bs[u][1]);
+    load_b(Half0{}, bs[u][0]);
+    load_b(Half1{}, bs[u][1]);
     if (u == 0)
       copy_a(1, 1);
   }
@@ -277,11 +286,11 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
     read_a(fa1, 1, soff);
     copy_a((kt >> 1) + NST - 2, (stage + NST - 2) & (NST - 1));
     weights_of(kt + D - 1);
-    load_b(0, bs[v][0]);
+    load_b(Half0{}, bs[v][0]);
     wait_first();
     mfmas(fa0, bs[u][0], kt, 0, 0);
     read_a(fb0, 2, soff);
-    load_b(1, bs[v][1]);
+    load_b(Half1{}, bs[v][1]);
     wait_first();
     mfmas(fa1, bs[u][1], kt, 0, 1);
 
@@ -290,11 +299,11 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
     __builtin_amdgcn_sched_barrier(0);
     read_a(fb1, 3, soff);
     weights_of(kt + D);
-    load_b(0, bs[u][0]);
+    load_b(Half0{}, bs[u][0]);
     wait_first();
     mfmas(fb0, bs[u + 1][0], kt + 1, 1, 0);
     read_a(fa0, 0, (unsigned)(nstage * STAGE));
-    load_b(1, bs[u][1]);
+    load_b(Half1{}, bs[u][1]);
     wait_first();
     mfmas(fb1, bs[u + 1][1], kt + 1, 1, 1);
     stage = nstage;

@@ -153,6 +153,19 @@ def test_no_register_is_touched_before_its_load_has_landed(kernels, family):
     assert not bad, "\n".join(f"{n}\n    " + "\n    ".join(f"{a:x}: {t}" for a, t in list(b.items())[:5]) for n, b in bad.items())
 
 
+def test_empty_descriptors_come_with_an_offset_of_zero(kernels):
+    """The streaming kernels ask for steps past the last one with a descriptor of
+    size 0.  The device drops what lies past (size - scalar offset), unsigned: the
+    scalar offset is then 0, so a step's second half must lie in the instruction's
+    own offset, for every second load of the weights."""
+    forms = {n: body for n, body in kernels.items() if re.search("k_gemm_i8_(dma_)?bsI", n)}
+    assert forms
+    for name, body in forms.items():
+        loads = [ins.text for ins in body if re.match(r"buffer_load_dwordx4 v\[\d+:\d+\], v\d+, s\[\d+:\d+\], s\d+ offen", ins.text)
+                 and " lds" not in ins.text]
+        assert loads and 2 * sum("offset:1024" in t for t in loads) == len(loads), (name, loads[:4])
+
+
 @pytest.mark.parametrize("wait,touch,seen", [
     ("s_waitcnt vmcnt(0)", "v_mov_b32_e32 v4, 0", False),
     ("s_waitcnt vmcnt(1)", "v_mov_b32_e32 v4, 0", False),    # one younger load may stand
