@@ -885,18 +885,40 @@ struct Call {
     return p;
   }
 
-  // launch_gemm, with the scratch that makes it faster unless the stream is
-  // being captured (a replay would share the scratch with later calls).
-  hipError_t gemm(GemmArgs &g) {
-    const size_t bytes = gemm_plan_split(g);
+  // Scratch that makes a product faster and that it can do without: null if there
+  // is no memory for it, or while the stream is being captured (a replay would
+  // share it with later calls).
+  void *scratch_for(size_t bytes) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (bytes && hipStreamIsCapturing(c.stream, &capture) == hipSuccess &&
-        capture == hipStreamCaptureStatusNone) {
-      g.parts = (int32_t *)c.take(bytes, /*optional=*/true);
-      if (g.parts)
-        temps.push_back(g.parts);
-    }
+    if (hipStreamIsCapturing(c.stream, &capture) != hipSuccess ||
+        capture != hipStreamCaptureStatusNone)
+      return nullptr;
+    void *p = c.take(bytes, /*optional=*/true);
+    if (p)
+      temps.push_back(p);
+    return p;
+  }
+
+  // launch_gemm, with its scratch.
+  hipError_t gemm(GemmArgs &g) {
+    if (const size_t bytes = gemm_plan_split(g))
+      g.parts = (int32_t *)scratch_for(bytes);
     return launch_gemm(c.stream, g);
+  }
+
+  // Rows of an awkward length or alignment, where that pays: aligned copies whose
+  // tail holds the zero point, multiplied over the padded length.
+  // stored_minus_128: 8-bit rows that DynamicQuantizeLinear left so.
+  void pad_rows(GemmArgs &g, bool rowsums, bool stored_minus_128) {
+    const int64_t Kp = ok ? gemm_padded_k(g.M, g.K, g.N, g.A, rowsums) : 0;
+    void *const padded = Kp ? scratch_for((size_t)(g.M * Kp)) : nullptr;
+    if (!padded)
+      return;
+    check(launch_pad_rows(c.stream, g.A, g.M, g.K, Kp, g.a_zp, g.a_zp_len,
+              stored_minus_128, padded),
+        "pad rows");
+    g.A = padded;
+    g.K = Kp;
   }
 
   // keep_constant: a host buffer declared constant gets a GPU copy that stays
@@ -1632,17 +1654,7 @@ void run_matmul(const MatmulSpec &sp) {
   }
   g.out = call.out(y);
   if (b.rank <= 2) {
-    if (const int64_t Kp = call.ok ? gemm_padded_k(M, K, N, g.A, b_uns || bzl > 0) : 0) {
-      // rows of an awkward length or alignment: aligned copies whose tail
-      // holds the zero point, multiplied over the padded length
-      void *padded = call.temp((size_t)(M * Kp));
-      if (call.ok)
-        call.check(launch_pad_rows(call.c.stream, g.A, M, K, Kp, d_azp, azl,
-                       /*stored_minus_128=*/false, padded),
-            "pad rows");
-      g.A = padded;
-      g.K = Kp;
-    }
+    call.pad_rows(g, b_uns || bzl > 0, /*stored_minus_128=*/false);
     if (call.ok)
       call.check(call.gemm(g), sp.op);
     call.finish();
@@ -2092,7 +2104,6 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
   // activations stay on the GPU, stored as (u8 - 128) so that the GEMM stages
   // them without a per-byte fix-up.
   auto run = [&](bool in_kernel) -> hipError_t {
-    int64_t padded_k = 0;
     GemmArgs g = {};
     g.out = dy;
     g.y_limits = d_ylim;
@@ -2111,18 +2122,6 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
         run_dql(call, dx, M * K, aq, call.c.dql_scale, call.c.dql_zp, true,
             /*later=*/true);
       g.A = aq;
-      padded_k = call.ok ? gemm_padded_k(M, K, N, aq,
-                               b.dtype == OM_MI355X_TYPE_UINT8 || bzl > 0)
-                         : 0;
-      if (padded_k) {
-        // (see run_matmul) the quantized rows are stored minus 128
-        void *padded = call.temp((size_t)(M * padded_k));
-        if (call.ok)
-          call.check(launch_pad_rows(call.c.stream, aq, M, K, padded_k,
-                         call.c.dql_zp, 1, /*stored_minus_128=*/true, padded),
-              "pad rows");
-        g.A = padded;
-      }
       if (!call.ok)
         return hipSuccess; // already reported
     }
@@ -2130,7 +2129,7 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
     g.a_preshifted = true;
     g.b_unsigned = b.dtype == OM_MI355X_TYPE_UINT8;
     g.M = M;
-    g.K = padded_k ? padded_k : K;
+    g.K = K;
     g.N = N;
     g.Bp = bp;
     g.colsum = colsum;
@@ -2146,7 +2145,9 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
     g.bias_len = bias_t ? bias.numel : 0;
     g.relu = relu;
     g.gelu = gelu;
-    return call.gemm(g);
+    if (!in_kernel)
+      call.pad_rows(g, g.b_unsigned || bzl > 0, /*stored_minus_128=*/true);
+    return call.ok ? call.gemm(g) : hipSuccess;
   };
   const int kind = (call.ok && t_quant_mode == 0 && call.c.dql.grid_blocks >= 0)
                        ? gemm_quantizes_rows(M, K, N, dx)
