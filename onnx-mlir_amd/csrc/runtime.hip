@@ -512,8 +512,32 @@ struct Ctx {
       fork_ev = nullptr;
       return false;
     }
-    return lane.init(stream);
+    if (!lane.init(stream))
+      return false;
+    if (primed)
+      return true;
+    // Which of the copy engines a stream is given depends on what its first copies
+    // found busy.  With one copy each way on this stream before the lanes' first
+    // ones, the lanes' copies run on two engines side by side; without, all of them
+    // take turns on one (8 MiB of results 362 us, so 332; 4.2 MiB 226 / 195).
+    if (void *p = take(kPrime, /*optional=*/true)) {
+      hipError_t e = hipMemcpyAsync(
+          p, lane.slot[0], kPrime, hipMemcpyHostToDevice, stream);
+      if (e == hipSuccess)
+        e = hipMemcpyAsync(
+            lane.slot[0], p, kPrime, hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess)
+        e = hipStreamSynchronize(stream);
+      give(p);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+      }
+    }
+    return primed = true;
   }
+  bool primed = false;
+  static constexpr size_t kPrime = (size_t)1 << 20; // (bytes; at most a slot's)
 
   // One large buffer (kStagedIn / kStagedOut) between pageable host memory and
   // GPU memory, split into pieces that go round-robin to this thread's lane
@@ -863,6 +887,7 @@ struct Call {
     size_t bytes;
   };
   std::vector<Back> backs;
+  size_t back_bytes = 0; // of all, each rounded up (the arena's layout)
   std::vector<void *> temps;
 
   const char *op;
@@ -971,7 +996,8 @@ struct Call {
     hipError_t e;
     if (v.bytes >= Ctx::kStagedIn && c.stage_ready())
       e = c.copy_staged(v.data, d, v.bytes, false);
-    else if (arena_used + v.bytes <= Ctx::kArenaIn && c.arena_ready())
+    else if (back_bytes <= Ctx::kArenaOut &&
+             arena_used + v.bytes <= Ctx::kArenaIn && c.arena_ready())
       e = copy_in(v, d);
     else
       e = hipMemcpyAsync(d, v.data, v.bytes, hipMemcpyHostToDevice, c.stream);
@@ -985,7 +1011,8 @@ struct Call {
   }
 
   // Through the arena in pieces: one crosses the bus while the next is copied
-  // into it.
+  // into it.  (Not where results follow that are too large for the arena: their
+  // copies, by the copy engine, then start later; see Ctx::stage_ready.)
   size_t arena_used = 0; // of its input side, by this call
   hipError_t copy_in(const View &v, void *d) {
     char *const at = c.arena_in() + arena_used;
@@ -1006,12 +1033,9 @@ struct Call {
   // `ok`); `failed`: the give-up flags of the one-launch kernels (dql_gave_up).
   bool bring_back(unsigned (&failed)[2]) {
     failed[0] = failed[1] = 0;
-    size_t total = 0;
     CopyOut a = {};
-    for (const Back &b : backs)
-      total += (b.bytes + 255) & ~(size_t)255;
     if (!ok || backs.empty() || backs.size() > (size_t)CopyOut::kTensors ||
-        total > Ctx::kArenaOut || sync_every_call() || report_enabled() ||
+        back_bytes > Ctx::kArenaOut || sync_every_call() || report_enabled() ||
         !c.arena_ready())
       return false;
     char *at = c.arena_out();
@@ -1065,6 +1089,8 @@ struct Call {
     }
   }
 
+  // Outputs are named before inputs: where the results go decides how the
+  // operands come.
   void *out(const View &v) {
     if (!ok || v.numel == 0)
       return v.data;
@@ -1076,6 +1102,7 @@ struct Call {
     if (!d)
       return nullptr;
     backs.push_back(Back{v.data, d, v.bytes});
+    back_bytes += (v.bytes + 255) & ~(size_t)255;
     touched_host = true;
     return d;
   }
@@ -1599,6 +1626,7 @@ void run_matmul(const MatmulSpec &sp) {
   const bool a_uns = a.dtype == OM_MI355X_TYPE_UINT8;
   const bool b_uns = b.dtype == OM_MI355X_TYPE_UINT8;
   GemmArgs g = {};
+  g.out = call.out(y);
   g.A = call.in(a);
   g.a_unsigned = a_uns;
   g.a_preshifted = false;
@@ -1652,7 +1680,6 @@ void run_matmul(const MatmulSpec &sp) {
     g.y_unsigned = y.dtype == OM_MI355X_TYPE_UINT8;
     g.narrow = sp.narrow;
   }
-  g.out = call.out(y);
   if (b.rank <= 2) {
     call.pad_rows(g, b_uns || bzl > 0, /*stored_minus_128=*/false);
     if (call.ok)
@@ -1813,6 +1840,7 @@ void om_mi355x_QuantizeLinear(OMTensor *y_t, const OMTensor *x_t,
   if (!call.ok)
     return;
   const int mode = t_quant_mode;
+  void *dy = call.out(y);
   const float *dx = (const float *)call.in(x);
   const float *ds = (const float *)call.in(sc);
   // without zero points the one given only decides the output type
@@ -1820,7 +1848,6 @@ void om_mi355x_QuantizeLinear(OMTensor *y_t, const OMTensor *x_t,
   const void *dz = (zp_t && !(mode & OM_MI355X_QUANT_NO_ZERO_POINT))
                        ? call.in(zp)
                        : nullptr;
-  void *dy = call.out(y);
   if (call.ok)
     call.check(launch_quantize(call.c.stream, dx, outer, channels, inner, ds,
                    dz, y.dtype == OM_MI355X_TYPE_INT8, dy,
@@ -1855,13 +1882,13 @@ void om_mi355x_DequantizeLinear(OMTensor *y_t, const OMTensor *x_t,
   Call call(t_ctx, "DequantizeLinear");
   if (!call.ok)
     return;
+  float *dy = (float *)call.out(y);
   const void *dx = call.in(x);
   const float *ds = (const float *)call.in(sc);
   // (src/Conversion/ONNXToKrnl/Math/Elementwise.cpp:1453)
   const void *dz = (zp_t && !(t_quant_mode & OM_MI355X_QUANT_NO_ZERO_POINT))
                        ? call.in(zp)
                        : nullptr;
-  float *dy = (float *)call.out(y);
   const QKind kind = x.dtype == OM_MI355X_TYPE_UINT8  ? kU8
                      : x.dtype == OM_MI355X_TYPE_INT8 ? kI8
                                                       : kI32;
@@ -1891,10 +1918,10 @@ void om_mi355x_DynamicQuantizeLinear(OMTensor *y_t, OMTensor *scale_t,
   Call call(t_ctx, "DynamicQuantizeLinear");
   if (!call.ok)
     return;
-  const float *dx = (const float *)call.in(x);
   uint8_t *dy = (uint8_t *)call.out(y);
   float *ds = (float *)call.out(sc);
   uint8_t *dz = (uint8_t *)call.out(zp);
+  const float *dx = (const float *)call.in(x);
   if (call.ok)
     run_dql(call, dx, x.numel, dy, ds, dz, false);
   call.finish();
@@ -2084,10 +2111,10 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
   Call call(t_ctx, op);
   if (!call.ok)
     return;
-  const float *dx = (const float *)call.in(x);
-  const float *d_xlim = xlim_t ? (const float *)call.in(xlim, false) : nullptr;
   void *dy = call.out(y); // before the quantization: it decides whether to wait
   float *d_ylim = ylim_t ? (float *)call.out(ylim) : nullptr;
+  const float *dx = (const float *)call.in(x);
+  const float *d_xlim = xlim_t ? (const float *)call.in(xlim, false) : nullptr;
   const int32_t *colsum = nullptr;
   const int8_t *bp = nullptr;
   if (!call.ok || !packed_b(call, b, K, N, bp, colsum)) {
