@@ -695,41 +695,58 @@ enum TileCfg : int {
   kNumCfg = 8
 };
 
+// What the time of a product depends on.
+struct Sizes {
+  int64_t M, N, K;
+  bool bytes;   // 8-bit results
+  bool rowsums; // B carries an offset
+};
+Sizes sizes_of(const GemmArgs &g) {
+  return {g.M, g.N, g.K, g.epi == kEpiQ8, g.b_unsigned || g.b_zp_len > 0};
+}
+
 // Kernel choice for problems with more than 64 rows, K a multiple of 16 and a
 // 16-byte aligned A (anything else takes the general path of k_gemm_i8).
-// A tile kernel's time on MI355X, by what the fullest CU has to do:
-//   base + steps * max(lone, step * b) + block * b   microseconds,
-// b the blocks it gets: partly the next whole number, partly the mean, since
-// CUs that are done early leave the others the way to memory (`round`).  Fitted
-// to 150 products of 65 .. 4096 rows, K and N of 256 .. 11008 (a multiple of 16
-// and any number), int32 and f32 results, each timed with every kernel; the
-// choice by it is within 1 % of always taking the fastest, 4 % ahead of the rule
-// it replaced (128 x 128 tiles unless few or many; 4096 x 1024 x 1024 9.3 -> 8.8
-// us, 512 x 4096 x 4096 18.4 -> 15.4, 1235 x 6656 x 2005 31.4 -> 28.8, 1500 x
-// 5120 x 5120 49.7 -> 43.1).
+// A tile kernel's time on MI355X:
+//   base + steps * max(lone, step * rounds) * (1 + rowsum) + block * b   microseconds.
+// A chain of K steps takes as long as the CU with the most blocks, `rounds` of
+// them, and what a block does beside it (block4, block1, by the size of a result)
+// counts b times, partly the rounds and partly the mean (`round`): CUs that are
+// done early leave the others the way to memory.  rowsum: where row sums are added
+// up.  Fitted to 2921 products of 65 .. 4096 rows, K and N of 64 .. 11008, each
+// timed with every kernel, so that the kernel it names takes the least time
+// (profiles/tile_kernel_times.csv): 0.4 % above always taking the fastest, in the
+// geometric mean (fitted to two thirds of them, 0.5 % on the rest).  The times
+// themselves are within 10 %.  With the mean in the K steps as well, and
+// coefficients fitted to 150 products of fewer kinds, it was 1.9 %, and 128 x 64
+// tiles were taken too often where K is short and N long (int32 3584 x 320 x 9740
+// 39.7 us, in 128 x 128 tiles 33.8; 1903 x 304 x 8576 19.9 / 17.3), 128 x 256 ones for K
+// up to 1024 (2048 x 768 x 3072 11.7 / 9.9 in 64 x 128).
 struct TileCost {
   TileCfg cfg;
   int bm, bn, trip; // K steps are done in whole trips
-  double lone, step, block, base, round;
+  double lone, step, rowsum, block4, block1, base, round;
 };
 constexpr TileCost kTileCosts[] = {
-    {kD128x128, 128, 128, 1, 0.0, 0.248, 2.67, 2.24, 0.52},
-    {kD128x64, 128, 64, 1, 0.0, 0.203, 0.77, 2.37, 0.43},
-    {kB128x256, 128, 256, 4, 0.0, 0.314, 5.08, 0.22, 1.0},
-    {kB64x256, 64, 256, 4, 0.0, 0.223, 2.24, 2.78, 0.68},
-    {kB64x128, 64, 128, 4, 0.132, 0.163, 0.75, 2.76, 0.64},
+    {kD128x128, 128, 128, 1, 0.018, 0.298, 0.101, 1.989, 2.474, 2.628, 0.012},
+    {kD128x64, 128, 64, 1, 0.069, 0.178, 0.294, 1.006, 1.331, 2.407, 0.003},
+    {kB128x256, 128, 256, 4, 0.022, 0.444, 0.126, 3.496, 3.226, 4.769, 0.0},
+    {kB64x256, 64, 256, 4, 0.009, 0.231, 0.088, 2.381, 2.323, 3.043, 0.346},
+    {kB64x128, 64, 128, 4, 0.027, 0.157, 0.165, 0.756, 0.866, 2.684, 0.331},
 };
-double tile_us(const TileCost &t, int64_t M, int64_t N, int64_t K) {
-  const int64_t blocks = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-  const double whole = (double)((blocks + 255) / 256);
+double tile_us(const TileCost &t, const Sizes &p) {
+  const int64_t blocks = ((p.M + t.bm - 1) / t.bm) * ((p.N + t.bn - 1) / t.bn);
+  const double rounds = (double)((blocks + 255) / 256);
   const double b = std::max(
-      1.0, t.round * whole + (1.0 - t.round) * (double)blocks / 256.0);
-  const double steps = (double)(round_up(K, kGemmBK * t.trip) / kGemmBK);
-  return t.base + steps * std::max(t.lone, t.step * b) + t.block * b;
+      1.0, t.round * rounds + (1.0 - t.round) * (double)blocks / 256.0);
+  const double steps = (double)(round_up(p.K, kGemmBK * t.trip) / kGemmBK);
+  return t.base + steps * std::max(t.lone, t.step * rounds) *
+                      (p.rowsums ? 1.0 + t.rowsum : 1.0) +
+         (p.bytes ? t.block1 : t.block4) * b;
 }
 // Its time, too, where wanted.
 // Override for tests and tuning: OM_MI355X_GEMM_TILE=<TileCfg value>.
-int choose_tile(int64_t M, int64_t N, int64_t K, double *us = nullptr) {
+int choose_tile(const Sizes &p, double *us = nullptr) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
   if (force && force[0]) {
     const int c = atoi(force);
@@ -737,13 +754,13 @@ int choose_tile(int64_t M, int64_t N, int64_t K, double *us = nullptr) {
       return c;
   }
   int best = kD128x128;
-  double least = 0.98 * tile_us(kTileCosts[0], M, N, K); // (ties stay with it)
+  double least = tile_us(kTileCosts[0], p);
   for (const TileCost &t : kTileCosts) {
     // (128 x 256 tiles: K a multiple of 256, the step counts that
     // instantiation is validated at)
-    if (K >= (1 << 24) ? t.trip != 1 : t.cfg == kB128x256 && K % 256 != 0)
+    if (p.K >= (1 << 24) ? t.trip != 1 : t.cfg == kB128x256 && p.K % 256 != 0)
       continue;
-    const double u = tile_us(t, M, N, K);
+    const double u = tile_us(t, p);
     if (u < least) {
       least = u;
       best = t.cfg;
@@ -844,60 +861,60 @@ __global__ __launch_bounds__(256) void k_sum_parts(
 }
 
 // What bounds a product whose tiles cover a part of the CUs is the chain of its
-// K steps, each the time its operands take into one CU: 0.22 us in 128 x 64
-// tiles of k_gemm_i8_dma, 0.28 in 128 x 128 ones, 0.172 in 64 x 128 ones of
-// k_gemm_i8_dma_bs, 0.5 in k_gemm_i8 (u8 rows a little more).  Splitting shortens
-// the chain and costs the launch of k_sum_parts, 2.5 us, and the arrays' way
-// through memory, 1.8 us per million elements.  Taken where that comes out ahead
-// of one piece in the tile chosen for it; more than one block per CU gains nothing.  K of whole steps in the tiles of k_gemm_i8_dma
-// (the others are ahead of them on some shapes and behind on as many: 418 x 7936
-// x 1386 17.1 / 15.8 us, u8 results 517 x 8960 x 576 14.0 / 15.2), other K in
-// those of k_gemm_i8_dma_bs, whose steps do not look for the end of the row
-// (int32 301 x 6384 x 1856 15.4 / 13.8 us, 196 x 5488 x 2688 15.4 / 13.9).
+// K steps, each the time its operands take into one CU: 0.15 us in 64 x 128 tiles
+// of k_gemm_i8_dma_bs, 0.17 in 128 x 64 ones of k_gemm_i8_dma, 0.23 in 128 x 128
+// ones, 0.37 in k_gemm_i8, a third more with row sums.  Splitting shortens the
+// chain and costs the launch of k_sum_parts, 2.5 us, and the arrays' way through
+// memory, 2 us per million elements.  Fitted to 2762 timed splits of 393 products
+// in two to 32 parts (within 4 %, root mean square).  Taken where that comes out
+// ahead of one piece in the tile chosen for it; more than one block per CU gains
+// nothing.  K of whole steps in any of the three, other K in k_gemm_i8_dma_bs, whose
+// steps do not look for the end of the row (int32 301 x 6384 x 1856 15.4 / 13.8 us).
 // Measured in one piece / split: 70 x 8192 x 1024 24.5 / 10.2 us, 118 x 10624 x
-// 1536 31.3 / 12.8, 100 x 4096 x 4096 14.4 / 12.9, 148 x 2304 x 832 9.3 / 8.4; left
-// alone by the rule: 200 x 4096 x 4096 14.3 / 16.3, 128 x 6464 x 9637 21.2 / 21.4.
+// 1536 31.3 / 12.8, 100 x 4096 x 4096 14.4 / 12.9, 148 x 2304 x 832 9.3 / 8.4.
 // The plan is made once per product (GemmArgs::split), after the tests that turn
 // most products away; parts are looked for around the minimum of the model.
 struct SplitForm {
   SplitKernel kernel;
   int64_t tiles, trip;
-  double us_step, us_else; // us_else: beside steps, second launch and arrays
+  double us_step, rowsum, us_else; // us_else: beside steps and arrays
 };
 SplitForm split_form(SplitKernel kernel, int64_t M, int64_t N) {
   const int64_t tm = (M + 127) / 128, t128 = tm * ((N + 127) / 128);
   switch (kernel) {
   case kSplitDma128:
-    return {kernel, t128, 1, 0.28, 2.3};
+    return {kernel, t128, 1, 0.230, 0.31, 6.37};
   case kSplitDma64:
-    return {kernel, tm * ((N + 63) / 64), 1, 0.22, 2.3};
+    return {kernel, tm * ((N + 63) / 64), 1, 0.173, 0.43, 5.81};
   case kSplitBs:
-    return {kernel, ((M + 63) / 64) * ((N + 127) / 128), 4, 0.172, 3.5};
+    return {kernel, ((M + 63) / 64) * ((N + 127) / 128), 4, 0.150, 0.33, 5.85};
   default:
-    return {kernel, t128, 1, 0.5, 3.5};
+    return {kernel, t128, 1, 0.373, 0.29, 6.25};
   }
 }
-bool split_possible(int64_t M, int64_t N, int64_t K, bool any) {
+bool split_possible(const Sizes &p, bool any) {
   // (under 24 steps a second launch is within the model's error, unless they
   // are those of k_gemm_i8)
-  return (K + kGemmBK - 1) / kGemmBK >= (any ? 8 : 24) &&
-         ((M + 127) / 128) * ((N + 127) / 128) <= 128 &&
-         M * N <= ((int64_t)1 << 22) && M * K >= 16 && K < (1 << 24);
+  return (p.K + kGemmBK - 1) / kGemmBK >= (any ? 8 : 24) &&
+         ((p.M + 127) / 128) * ((p.N + 127) / 128) <= 128 &&
+         p.M * p.N <= ((int64_t)1 << 22) && p.M * p.K >= 16 && p.K < (1 << 24);
 }
-// The split of form f that takes less than `least`, which it lowers.
-void try_split(const SplitForm &f, int64_t M, int64_t N, int64_t K,
-    GemmSplit &best, double &least) {
-  const int64_t KT = (K + kGemmBK - 1) / kGemmBK;
-  const double us_part = 1.8e-6 * (double)(M * N);
+// The split of the product in this kernel that takes less than `least`, which it
+// lowers.
+void try_split(SplitKernel kernel, const Sizes &z, GemmSplit &best, double &least) {
+  const SplitForm f = split_form(kernel, z.M, z.N);
+  const int64_t KT = (z.K + kGemmBK - 1) / kGemmBK;
+  const double us_part = 2.02e-6 * (double)(z.M * z.N);
+  const double us_step = f.us_step * (z.rowsums ? 1.0 + f.rowsum : 1.0);
   const int64_t most = 256 / f.tiles < KT / 4 ? 256 / f.tiles : KT / 4;
   // steps * us_step + parts * us_part is least where both are equal
-  const int64_t around = (int64_t)sqrt((double)KT * f.us_step / us_part);
+  const int64_t around = (int64_t)sqrt((double)KT * us_step / us_part);
   const int64_t low = around - 2 < most - 4 ? around - 2 : most - 4;
   for (int64_t p = low < 2 ? 2 : low; p <= most && p <= around + 3; ++p) {
     const int64_t steps = round_up((KT + p - 1) / p, f.trip);
     const int64_t parts = (KT + steps - 1) / steps; // (none without a step)
-    const double us = f.us_else + (double)steps * f.us_step + 2.5 +
-                      us_part * (double)parts;
+    const double us =
+        f.us_else + (double)steps * us_step + us_part * (double)parts;
     if (parts > 1 && us < least) {
       least = us;
       best.parts = (int)parts;
@@ -907,59 +924,47 @@ void try_split(const SplitForm &f, int64_t M, int64_t N, int64_t K,
   }
 }
 // The time of a product over K, a multiple of 16, and how it is split.
-double product_us(int64_t M, int64_t N, int64_t K, bool rowsums, GemmSplit &best) {
+double product_us(const Sizes &p, GemmSplit &best) {
   double least = 0.0;
-  (void)choose_tile(M, N, K, &least);
-  // (row sums of A cost about a seventh of a step)
-  if (rowsums)
-    least += 0.15 * std::max(0.0, least - 3.5);
-  if (!split_possible(M, N, K, false))
+  (void)choose_tile(p, &least);
+  if (!split_possible(p, false))
     return least;
-  double us = 0.98 * least;
-  if (K % kGemmBK != 0) {
-    try_split(split_form(kSplitBs, M, N), M, N, K, best, us);
-  } else {
-    try_split(split_form(kSplitDma128, M, N), M, N, K, best, us);
-    if (N > 64)
-      try_split(split_form(kSplitDma64, M, N), M, N, K, best, us);
+  try_split(kSplitBs, p, best, least);
+  if (p.K % kGemmBK == 0) {
+    try_split(kSplitDma128, p, best, least);
+    if (p.N > 64)
+      try_split(kSplitDma64, p, best, least);
   }
-  return best.parts > 1 ? us : least;
+  return least;
 }
 // And in k_gemm_i8, for any K: tiles of 128 x 128 and of 64 x 128, four blocks of
 // which run on a CU and are dealt out more evenly; the model of kTileCosts, fitted
-// to 44 products timed with both, row sums dearer to the larger tile.  Int32 4099 x
-// 777 x 1001 16.1 us in the larger, 14.4 in the smaller, 1618 x 653 x 311 8.6 / 6.8,
-// u8 1959 x 1891 x 502 17.2 / 12.5; u8 3694 x 278 x 4295 17.5 / 21.3, int32 2290 x 293 x
-// 8977 25.4 / 28.8.
-double any_us(bool low, int64_t M, int64_t N, int64_t K, bool rowsums) {
-  static constexpr TileCost t128 = {
-      kT128x128, 128, 128, 1, 0.434, 0.359, 2.33, 2.62, 0.76};
-  static constexpr TileCost t64 = {
-      kT128x128, 64, 128, 1, 0.266, 0.191, 1.78, 2.62, 0.95};
-  const double us = tile_us(low ? t64 : t128, M, N, K);
-  return us + (rowsums ? (low ? 0.1 : 0.2) * std::max(0.0, us - 3.5) : 0.0);
+// to 662 products of awkward rows timed in both tiles, split and with their rows
+// copied (profiles/awkward_row_times.csv): the choice between these is 0.9 %
+// above always taking the fastest.  Int32 4099 x 777 x 1001 16.1 us in the larger,
+// 14.4 in the smaller, 1618 x 653 x 311 8.6 / 6.8; u8 3694 x 278 x 4295 17.5 / 21.3, u8
+// 575 x 948 x 8448 14.8 / 16.8.
+double any_us(bool low, const Sizes &p) {
+  static constexpr TileCost t128 = {kT128x128, 128, 128, 1, 0.385, 0.335, 0.233,
+      2.701, 3.079, 1.973, 0.402};
+  static constexpr TileCost t64 = {kT128x128, 64, 128, 1, 0.263, 0.188, 0.140,
+      1.502, 1.569, 2.645, 0.496};
+  return tile_us(low ? t64 : t128, p);
 }
-bool any_takes_64_rows(int64_t M, int64_t N, int64_t K, bool rowsums) {
-  return any_us(true, M, N, K, rowsums) < 0.99 * any_us(false, M, N, K, rowsums);
+bool any_takes_64_rows(const Sizes &p) {
+  return any_us(true, p) < any_us(false, p);
 }
-double general_us(int64_t M, int64_t N, int64_t K, bool rowsums, GemmSplit &best) {
-  double least =
-      std::min(any_us(false, M, N, K, rowsums), any_us(true, M, N, K, rowsums));
-  if (split_possible(M, N, K, true)) {
-    // (a long chain is split unless that is clearly worse: 3872 x 10201 x 477 44.4
-    // us in two parts, 48.8 in one piece; a short one where it is ahead: 442 x 1042
-    // x 431 9.9 us in four parts, 9.1 in one piece)
-    double us = K >= 64 * kGemmBK ? 1.15 * least : 0.98 * least - 0.2;
-    try_split(split_form(kSplitAny, M, N), M, N, K, best, us);
-    if (best.parts > 1)
-      least = us;
-  }
+double general_us(const Sizes &p, GemmSplit &best) {
+  double least = std::min(any_us(false, p), any_us(true, p));
+  if (split_possible(p, true))
+    try_split(kSplitAny, p, best, least);
   return least;
 }
 GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   GemmSplit best;
   const bool any = !gemm_fast_path(g.M, g.K, g.A);
-  if (g.X || g.M * g.N <= 0 || !split_possible(g.M, g.N, g.K, any) ||
+  const Sizes p = sizes_of(g);
+  if (g.X || g.M * g.N <= 0 || !split_possible(p, any) ||
       skinny_ok(g.M, g.K, g.A))
     return best;
   if (!any && g.K % 64 == 0 &&
@@ -969,9 +974,9 @@ GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   if (force && force[0])
     return best;
   if (any)
-    (void)general_us(g.M, g.N, g.K, g.b_unsigned || g.b_zp_len > 0, best);
+    (void)general_us(p, best);
   else
-    (void)product_us(g.M, g.N, g.K, g.b_unsigned || g.b_zp_len > 0, best);
+    (void)product_us(p, best);
   return best;
 }
 
@@ -1077,7 +1082,7 @@ hipError_t gemm_launch_cfg(
   if (!gemm_fast_path(g.M, g.K, g.A)) {
     // Any K, any alignment of A (and the forced configurations of the tests
     // when M <= 16); byte loads only for an A of fewer than 16 bytes.
-    const bool low = g.M * g.K >= 16 && any_takes_64_rows(g.M, g.N, g.K, ep.need_rowsum);
+    const bool low = g.M * g.K >= 16 && any_takes_64_rows(sizes_of(g));
     t_last_kernel = low ? "k_gemm_i8 (any K, any alignment; 64x128 tiles)"
                         : "k_gemm_i8 (any K, any alignment)";
     const int tiles_m64 = (int)((g.M + 63) / 64);
@@ -1095,7 +1100,7 @@ hipError_t gemm_launch_cfg(
               A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n128);
     return hipGetLastError();
   }
-  const int cfg = choose_tile(g.M, g.N, g.K);
+  const int cfg = choose_tile(sizes_of(g));
   if (g.K % 64 != 0 && cfg != kB64x256 && cfg != kB64x128)
     return launch_dma<A_MODE, EPI>(st, g, ep, Kpad,
         cfg == kD128x64 || cfg == kD128x128 ? cfg : (int)kD128x128);
@@ -1217,11 +1222,11 @@ __global__ __launch_bounds__(256) void k_pad_rows(const uint8_t *__restrict__ A,
 // time of measuring): f32 154 x 1022 x 2258 11.8 -> 7.4 us, 3711 x 964 x 3580 34.8 ->
 // 28.9, u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone: layer 1674 x 280 x 4123 16.8 /
 // 19.2, int32 4099 x 777 x 1001 14.4 / 18.0, u8 1032 x 487 x 6105 12.2 / 13.2.
-int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
-    bool rowsums) {
+int64_t gemm_padded_k(const GemmArgs &g) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
-  if (M < 1 || K < 1 || N < 1 || (K % 16 == 0 && (((uintptr_t)a) & 15) == 0) ||
-      (force && force[0]))
+  const int64_t M = g.M, K = g.K, N = g.N;
+  if (M < 1 || K < 1 || N < 1 ||
+      (K % 16 == 0 && (((uintptr_t)g.A) & 15) == 0) || (force && force[0]))
     return 0;
   // k_gemm_i8_skinny takes such rows as they are; with many long ones the
   // second line of each piece costs more than the copy (45 x 4981 x 4292 13.1 us,
@@ -1233,13 +1238,15 @@ int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
       N > INT32_MAX)
     return 0;
   GemmSplit s1, s2;
-  double us = product_us(M, N, Kp, rowsums, s1);
-  // (k_gemm_i8_flight, one round of 64 x 128 blocks: 4 us)
+  const Sizes own = sizes_of(g);
+  Sizes padded = own;
+  padded.K = Kp;
+  double us = product_us(padded, s1);
+  // (k_gemm_i8_flight, one round of 64 x 128 blocks)
   if ((Kp == 512 || Kp == 768 || Kp == 1024) &&
       ((M + 63) / 64) * ((N + 127) / 128) <= 256)
-    us = std::min(us, 4.0);
-  us += 3.0 + 5e-7 * (double)(M * K);
-  return general_us(M, N, K, rowsums, s2) > us + std::max(1.6, 0.03 * us) ? Kp : 0;
+    us = std::min(us, 2.4 + 0.002 * (double)Kp);
+  return general_us(own, s2) > us + 3.2 + 4.5e-7 * (double)(M * K) ? Kp : 0;
 }
 
 hipError_t launch_pad_rows(hipStream_t s, const void *a, int64_t M, int64_t K,

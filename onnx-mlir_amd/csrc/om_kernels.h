@@ -213,12 +213,11 @@ hipError_t launch_gemm_batched(hipStream_t s, const GemmArgs &g, const GemmBatch
 // then quantizes with DynamicQuantizeLinear and passes A -- and a block that
 // gives up waiting raises the scratch's flag).
 int gemm_quantizes_rows(int64_t M, int64_t K, int64_t N, const void *x);
-// The row length, if any (0: none), at which the caller should hand `a` over, as
+// The row length, if any (0: none), at which the caller should hand g.A over, as
 // rows made by launch_pad_rows, and pass that length as K.  a_zp: the rows' zero
 // point(s) on the GPU (null: 0), one or one per row; stored_minus_128: rows hold
-// (u8 - 128); rowsums: B carries an offset.
-int64_t gemm_padded_k(int64_t M, int64_t K, int64_t N, const void *a,
-    bool rowsums);
+// (u8 - 128).
+int64_t gemm_padded_k(const GemmArgs &g);
 hipError_t launch_pad_rows(hipStream_t s, const void *a, int64_t M, int64_t K,
     int64_t Kp, const void *a_zp, int64_t a_zp_len, bool stored_minus_128,
     void *out);

@@ -934,8 +934,8 @@ struct Call {
   // Rows of an awkward length or alignment, where that pays: aligned copies whose
   // tail holds the zero point, multiplied over the padded length.
   // stored_minus_128: 8-bit rows that DynamicQuantizeLinear left so.
-  void pad_rows(GemmArgs &g, bool rowsums, bool stored_minus_128) {
-    const int64_t Kp = ok ? gemm_padded_k(g.M, g.K, g.N, g.A, rowsums) : 0;
+  void pad_rows(GemmArgs &g, bool stored_minus_128) {
+    const int64_t Kp = ok ? gemm_padded_k(g) : 0;
     void *const padded = Kp ? scratch_for((size_t)(g.M * Kp)) : nullptr;
     if (!padded)
       return;
@@ -1681,7 +1681,7 @@ void run_matmul(const MatmulSpec &sp) {
     g.narrow = sp.narrow;
   }
   if (b.rank <= 2) {
-    call.pad_rows(g, b_uns || bzl > 0, /*stored_minus_128=*/false);
+    call.pad_rows(g, /*stored_minus_128=*/false);
     if (call.ok)
       call.check(call.gemm(g), sp.op);
     call.finish();
@@ -2173,7 +2173,7 @@ void dyn_quant_matmul_dequant(const char *op, OMTensor *y_t,
     g.relu = relu;
     g.gelu = gelu;
     if (!in_kernel)
-      call.pad_rows(g, g.b_unsigned || bzl > 0, /*stored_minus_128=*/true);
+      call.pad_rows(g, /*stored_minus_128=*/true);
     return call.ok ? call.gemm(g) : hipSuccess;
   };
   const int kind = (call.ok && t_quant_mode == 0 && call.c.dql.grid_blocks >= 0)
