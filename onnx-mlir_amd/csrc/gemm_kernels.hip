@@ -1228,11 +1228,24 @@ int64_t gemm_padded_k(const GemmArgs &g) {
   if (M < 1 || K < 1 || N < 1 ||
       (K % 16 == 0 && (((uintptr_t)g.A) & 15) == 0) || (force && force[0]))
     return 0;
-  // k_gemm_i8_skinny takes such rows as they are; with many long ones the
-  // second line of each piece costs more than the copy (45 x 4981 x 4292 13.1 us,
-  // copied 11.5; layer 37 x 6095 x 612 15.2 / 14.8).
-  if (M <= 64)
-    return M > 32 && K >= 4096 ? round_up(K, 16) : 0;
+  // k_gemm_i8_skinny takes such rows as they are.  Where it reads many bytes at
+  // addresses that are no multiple of 4, or any in more than one round of blocks,
+  // that costs more than the copy's 3 us (893 products timed both ways,
+  // profiles/few_row_times.csv: 0.2 % above always taking the faster; 2.1 % never
+  // copying, 2 % copying 33 rows and more from K = 4096 on).  As they lie / copied:
+  //  - more than 32 rows and 256 blocks of 32 columns: 50 x 1137 x 9152 13.3 / 9.2
+  //    us, 53 x 312 x 10560 9.2 / 7.2;
+  //  - 120 KB in rows that start between such addresses, with up to 32 rows only if
+  //    all do: 43 x 9313 x 1792 (three rows of four) 16.4 / 12.8, 54 x 4604 x 3232 (two
+  //    bytes off) 13.3 / 9.7, but 19 x 2938 x 4032 5.3 / 6.9, 62 x 8552 x 328 (none) 10.4 /
+  //    15.5, 32 x 8022 x 5616 (one of two) 10.7 / 13.0.
+  if (M <= 64) {
+    int64_t odd = 0; // of four rows in turn
+    for (uintptr_t r = 0; r < 4; ++r)
+      odd += (((uintptr_t)g.A + r * (uintptr_t)K) & 3) != 0;
+    const bool many = odd * M * K > 480000 && (M > 32 || odd == 4);
+    return many || (M > 32 && N > 8192) ? round_up(K, 16) : 0;
+  }
   const int64_t Kp = round_up(K, kGemmBK);
   if (Kp >= (1 << 24) || M * (Kp / 16) > UINT32_MAX || M > INT32_MAX ||
       N > INT32_MAX)

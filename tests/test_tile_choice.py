@@ -76,3 +76,35 @@ def _product(rt, oracle, M, K, N, bdt, rng):
 ])
 def test_short_k_and_many_columns(rt, oracle, M, K, N, bdt, kernel):
     assert kernel in _product(rt, oracle, M, K, N, bdt, np.random.default_rng(M))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,offset", [(50, 1137, 9152, 0), (43, 9313, 400, 0), (54, 4604, 330, 2), (24, 5568, 300, 1),
+                                          (33, 315, 8200, 3), (64, 1024, 8200, 1)])
+def test_few_awkward_rows_that_are_copied_first(rt, oracle, M, K, N, offset):
+    """Rows read often at odd addresses, copied to an aligned pitch: results with
+    zero points per tensor and per row, with and without row sums."""
+    rng = np.random.default_rng(M + K)
+    for adt, bdt, per in ((np.uint8, np.int8, False), (np.int8, np.uint8, True)):
+        i, j = np.iinfo(adt), np.iinfo(bdt)
+        a, b = rng.integers(i.min, i.max + 1, (M, K), dtype=adt), rng.integers(j.min, j.max + 1, (K, N), dtype=bdt)
+        az, bz = rng.integers(i.min, i.max + 1, M if per else 1, dtype=adt), rng.integers(j.min, j.max + 1, N if per else 1, dtype=bdt)
+        whole = rt.DeviceArray.from_numpy(np.concatenate([np.full(offset, 77, adt), a.reshape(-1)]))
+        da = rt.DeviceArray.view_of(whole, offset, (M, K))
+        got = rt.MatMulInteger(da, *(rt.DeviceArray.from_numpy(v) for v in (b, az, bz)))
+        rt.synchronize()
+        assert np.array_equal(got.numpy(), oracle.matmul_integer(a, b, az, bz)), (adt, bdt)
+
+
+def test_rows_are_copied_where_that_was_faster():
+    """The rule of gemm_padded_k for up to 64 rows, on the times measured."""
+    rule = re.search(r"odd \* M \* K > (\d+) && \(M > (\d+) \|\| odd == 4\);\s*return many \|\| \(M > 32 && N > (\d+)\)", SOURCE)
+    most, few, columns = (int(v) for v in rule.groups())
+    over = []
+    for r in _table("few_row_times.csv"):
+        M, K, N, offset = (int(r[k]) for k in ("M", "K", "N", "offset"))
+        as_is, copied = float(r["as_they_lie"]), float(r["copied"])
+        odd = sum((offset + i * K) % 4 != 0 for i in range(4))
+        copy = (odd * M * K > most and (M > few or odd == 4)) or (M > 32 and N > columns)
+        over.append((copied if copy else as_is) / min(as_is, copied))
+    assert len(over) > 800 and math.exp(np.mean(np.log(over))) < 1.004  # 1.019 by K >= 4096 alone
