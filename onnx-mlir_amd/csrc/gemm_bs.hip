@@ -359,12 +359,11 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
 }
 
 // 128 x 256 tiles.
-template <int TM, int TN, int D, int NST, int MINB, bool PIPE, int A_MODE,
-    int EPI, bool RS>
-__global__ __launch_bounds__(256, MINB) void k_gemm_i8_bs(
+template <int A_MODE, int EPI, bool RS>
+__global__ __launch_bounds__(256, 2) void k_gemm_i8_bs(
     const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
     int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n) {
-  stream_tile<TM, TN, A_MODE, EPI, RS, false, false>(
+  stream_tile<4, 2, A_MODE, EPI, RS, false, false>(
       A, Bp, M, N, K, Kpad, ep, tiles_m, tiles_n, KSplit{});
 }
 // 64 x 256 and 64 x 128 tiles.
@@ -376,17 +375,18 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma_bs(
       A, Bp, M, N, K, Kpad, ep, tiles_m, tiles_n, ks);
 }
 
+// ragged: the form that looks for the end of the row (only row sums have to); in
+// 64 x 256 tiles nothing is split.
 const char *dma_bs_name(int tn, bool ragged, bool split) {
-  static const char *const names[2][2][2] = {
-      {{"k_gemm_i8_dma_bs (64x128 tiles)",
-           "k_gemm_i8_dma_bs (64x128 tiles, split along K)"},
-          {"k_gemm_i8_dma_bs (64x128 tiles, ragged K)",
-              "k_gemm_i8_dma_bs (64x128 tiles, ragged K, split along K)"}},
-      {{"k_gemm_i8_dma_bs (64x256 tiles)",
-           "k_gemm_i8_dma_bs (64x256 tiles, split along K)"},
-          {"k_gemm_i8_dma_bs (64x256 tiles, ragged K)",
-              "k_gemm_i8_dma_bs (64x256 tiles, ragged K, split along K)"}}};
-  return names[tn - 1][ragged][split];
+  if (tn == 2)
+    return ragged ? "k_gemm_i8_dma_bs (64x256 tiles, ragged K)"
+                  : "k_gemm_i8_dma_bs (64x256 tiles)";
+  static const char *const names[2][2] = {
+      {"k_gemm_i8_dma_bs (64x128 tiles)",
+          "k_gemm_i8_dma_bs (64x128 tiles, split along K)"},
+      {"k_gemm_i8_dma_bs (64x128 tiles, ragged K)",
+          "k_gemm_i8_dma_bs (64x128 tiles, ragged K, split along K)"}};
+  return names[ragged][split];
 }
 
 template <int TN, int A_MODE, int EPI, bool SPLIT>
@@ -394,7 +394,7 @@ void launch_dma_bs(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
   const int Kpad = (int)round_up(g.K, kGemmBK);
   const int tiles_m = (M + 63) / 64, tiles_n = (N + 128 * TN - 1) / (128 * TN);
-  const bool ragged = K % BK != 0;
+  const bool ragged = ep.need_rowsum && K % BK != 0;
   constexpr int MINB = TN == 1 ? 4 : 3;
   note_gemm_kernel(dma_bs_name(TN, ragged, SPLIT));
   auto *const kernel =
@@ -417,8 +417,8 @@ void launch_tile(hipStream_t st, const GemmArgs &g, const EpiParams &ep, BsTile 
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
   const int tiles_m = (M + 127) / 128, tiles_n = (N + 255) / 256;
   note_gemm_kernel("k_gemm_i8_bs (128x256 tiles)");
-  auto *const kernel = ep.need_rowsum ? k_gemm_i8_bs<4, 2, 4, 4, 2, true, A_MODE, EPI, true>
-                                      : k_gemm_i8_bs<4, 2, 4, 4, 2, true, A_MODE, EPI, false>;
+  auto *const kernel = ep.need_rowsum ? k_gemm_i8_bs<A_MODE, EPI, true>
+                                      : k_gemm_i8_bs<A_MODE, EPI, false>;
   kernel<<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
       (const uint8_t *)g.A, g.Bp, M, N, K, (int)round_up(g.K, kGemmBK), ep,
       tiles_m, tiles_n);

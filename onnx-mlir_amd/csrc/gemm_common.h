@@ -247,6 +247,33 @@ bool wreg_pays(int64_t M, int64_t N);
 hipError_t launch_gemm_wreg(hipStream_t st, const GemmArgs &g,
     const EpiParams &ep, int a_mode);
 
+// 16 bytes of a row from v, which was read `back` bytes in front of them (so as not
+// to run past the end of A): the first `len` (0 .. 16) are the row's, the others
+// become those of `fill`.  back < 16, or any number of bytes where len is 0.
+__device__ __forceinline__ v4i row_chunk(v4i v, int back, int len, uint64_t fill) {
+  uint64_t lo = (uint32_t)v.x | ((uint64_t)(uint32_t)v.y << 32);
+  uint64_t hi = (uint32_t)v.z | ((uint64_t)(uint32_t)v.w << 32);
+  const int sh = back * 8;
+  if (sh >= 64) {
+    lo = hi;
+    hi = 0;
+  }
+  const int s1 = sh & 63;
+  if (s1) {
+    lo = (lo >> s1) | (hi << (64 - s1));
+    hi >>= s1;
+  }
+  const uint64_t mlo =
+      len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
+  const uint64_t mhi =
+      len >= 16 ? ~(uint64_t)0
+                : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
+  lo = (lo & mlo) | (fill & ~mlo);
+  hi = (hi & mhi) | (fill & ~mhi);
+  return (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
+      (int)(uint32_t)(hi >> 32)};
+}
+
 // Elements between the arrays of the parts of a product split along K.
 inline int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
 
@@ -263,7 +290,7 @@ hipError_t launch_gemm_bs_split(hipStream_t st, const GemmArgs &g,
 // k_gemm_i8_skinny (gemm_skinny.hip): up to 64 rows.  skinny_quantizes_rows:
 // whether it takes the f32 activation of a fused layer (GemmArgs::X) and
 // quantizes it in every block.
-bool skinny_ok(int64_t M, int64_t K, const void *a);
+bool skinny_ok(int64_t M, int64_t K);
 bool skinny_quantizes_rows(int64_t M, int64_t K, const void *x);
 hipError_t launch_gemm_skinny(hipStream_t st, const GemmArgs &g,
     const EpiParams &ep, int a_mode);

@@ -187,30 +187,8 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
       const int gk = k0 + ((tid + h * THREADS) & 3) * 16;
       const int len = K - gk < 0 ? 0 : K - gk < 16 ? K - gk : 16;
       const uint8_t *const p = arow[h] + k0;
-      // bits to shift down: < 128 whenever the chunk holds a byte of the row
-      const int sh = p < alast ? 0 : (int)(p - alast) * 8;
-      uint64_t lo = (uint32_t)ra[h].x | ((uint64_t)(uint32_t)ra[h].y << 32);
-      uint64_t hi = (uint32_t)ra[h].z | ((uint64_t)(uint32_t)ra[h].w << 32);
-      if (sh >= 64) {
-        lo = hi;
-        hi = 0;
-      }
-      const int s1 = sh & 63;
-      if (s1) {
-        lo = (lo >> s1) | (hi << (64 - s1));
-        hi >>= s1;
-      }
-      const uint64_t fill64 =
-          (uint32_t)kFill | ((uint64_t)(uint32_t)kFill << 32);
-      const uint64_t mlo =
-          len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
-      const uint64_t mhi =
-          len >= 16 ? ~(uint64_t)0
-                    : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
-      lo = (lo & mlo) | (fill64 & ~mlo);
-      hi = (hi & mhi) | (fill64 & ~mhi);
-      ra[h] = (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32),
-          (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+      ra[h] = row_chunk(ra[h], p < alast ? 0 : (int)(p - alast), len,
+          (uint32_t)kFill | ((uint64_t)(uint32_t)kFill << 32));
     }
   };
   // (`tail`: these are the registers of the last K step and that is not whole)
@@ -791,7 +769,7 @@ thread_local bool t_limits_written = false;
 template <int EPI>
 __global__ __launch_bounds__(256) void k_sum_parts(
     const int32_t *__restrict__ in, int parts, int64_t stride, unsigned n,
-    unsigned N, EpiParams ep, bool gelu, bool vector_out) {
+    unsigned N, EpiParams ep, bool vector_out) {
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   const unsigned o = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (o >= n)
@@ -837,7 +815,7 @@ __global__ __launch_bounds__(256) void k_sum_parts(
       r[e] = y[e];
     } else if (EPI == kEpiF32) {
       const float f = relu_f32((float)(int32_t)y[e] * sj[e] + bj[e], ep.floor);
-      r[e] = __float_as_uint(gelu ? gelu_f32(f) : f);
+      r[e] = __float_as_uint(ep.gelu ? gelu_f32(f) : f);
     } else {
       r[e] = requantize(ep, y[e], sj[e], yz);
     }
@@ -965,7 +943,7 @@ GemmSplit split_plan(const GemmArgs &g, int a_mode) {
   const bool any = !gemm_fast_path(g.M, g.K, g.A);
   const Sizes p = sizes_of(g);
   if (g.X || g.M * g.N <= 0 || !split_possible(p, any) ||
-      skinny_ok(g.M, g.K, g.A))
+      skinny_ok(g.M, g.K))
     return best;
   if (!any && g.K % 64 == 0 &&
       (flight_ok(g, a_mode) || (wreg_ok(g) && wreg_pays(g.M, g.N))))
@@ -1025,7 +1003,7 @@ hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
   const unsigned n = (unsigned)(g.M * g.N);
   const bool vec = (((uintptr_t)g.out) & (EPI == kEpiQ8 ? 3 : 15)) == 0;
   k_sum_parts<EPI><<<(n + 1023) / 1024, 256, 0, st>>>(
-      g.parts, p.parts, ks.stride, n, (unsigned)N, ep, g.gelu, vec);
+      g.parts, p.parts, ks.stride, n, (unsigned)N, ep, vec);
   return hipGetLastError();
 }
 
@@ -1073,7 +1051,7 @@ hipError_t gemm_launch_cfg(
   // Up to 64 rows the weight-streaming kernel is ahead of every tile kernel
   // (K=4096 N=11008: M=33 11.6 against 17.2 us, M=48 12.3 / 17.7; K=11008
   // N=4096 M=64: 15.0 / 37.7; K=768 N=3072 M=64: 4.2 / 6.0).
-  if (skinny_ok(g.M, g.K, g.A) && !(force && force[0]))
+  if (skinny_ok(g.M, g.K) && !(force && force[0]))
     return launch_gemm_skinny(st, g, ep, A_MODE);
   if (g.parts && g.split.parts > 1)
     return launch_split<A_MODE, EPI>(st, g, ep, Kpad);
@@ -1183,30 +1161,10 @@ __global__ __launch_bounds__(256) void k_pad_rows(const uint8_t *__restrict__ A,
   const v4i v = *(const v4i_any *)(p < last ? p : last);
   const int left = (int)K - (int)(c * 16);
   const int len = left < 0 ? 0 : left < 16 ? left : 16;
-  uint64_t lo = (uint32_t)v.x | ((uint64_t)(uint32_t)v.y << 32);
-  uint64_t hi = (uint32_t)v.z | ((uint64_t)(uint32_t)v.w << 32);
-  // bits to shift down: < 128 whenever the chunk holds a byte of the row
-  const int sh = p < last ? 0 : (int)(p - last) * 8;
-  if (sh >= 64) {
-    lo = hi;
-    hi = 0;
-  }
-  const int s1 = sh & 63;
-  if (s1) {
-    lo = (lo >> s1) | (hi << (64 - s1));
-    hi >>= s1;
-  }
   const uint64_t fill =
       (uint64_t)(uint8_t)((has_zp ? z : 0) ^ flip) * 0x0101010101010101ull;
-  const uint64_t mlo =
-      len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
-  const uint64_t mhi =
-      len >= 16 ? ~(uint64_t)0
-                : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
-  lo = (lo & mlo) | (fill & ~mlo);
-  hi = (hi & mhi) | (fill & ~mhi);
-  *(v4i *)(out + (uint64_t)i * 16) = (v4i){(int)(uint32_t)lo,
-      (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+  *(v4i *)(out + (uint64_t)i * 16) =
+      row_chunk(v, p < last ? 0 : (int)(p - last), len, fill);
 }
 
 } // namespace

@@ -345,27 +345,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
           const int len = left < 0 ? 0 : left < 16 ? left : 16;
           // bytes the load was moved back by: < 16 where the chunk has any
           const int back = row * K + k0 - (M * K - 16);
-          uint64_t lo = (uint32_t)t.a[j].x | ((uint64_t)(uint32_t)t.a[j].y << 32);
-          uint64_t hi = (uint32_t)t.a[j].z | ((uint64_t)(uint32_t)t.a[j].w << 32);
-          const int sh = back > 0 && len > 0 ? back * 8 : 0;
-          if (sh >= 64) {
-            lo = hi;
-            hi = 0;
-          }
-          const int s1 = sh & 63;
-          if (s1) {
-            lo = (lo >> s1) | (hi << (64 - s1));
-            hi >>= s1;
-          }
-          const uint64_t mlo =
-              len >= 8 ? ~(uint64_t)0 : (((uint64_t)1 << (8 * len)) - 1);
-          const uint64_t mhi =
-              len >= 16 ? ~(uint64_t)0
-                        : (len > 8 ? (((uint64_t)1 << (8 * (len - 8))) - 1) : 0);
-          lo = (lo & mlo) | (kFill & ~mlo);
-          hi = (hi & mhi) | (kFill & ~mhi);
-          t.a[j] = (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32),
-              (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
+          t.a[j] = row_chunk(t.a[j], back > 0 && len > 0 ? back : 0, len, kFill);
         }
       }
 #pragma unroll
@@ -606,8 +586,7 @@ bool skinny_quantizes_rows(int64_t M, int64_t K, const void *x) {
 }
 
 // (K: the offsets of 64 rows and of a column tile's operands stay in 31 bits.)
-bool skinny_ok(int64_t M, int64_t K, const void *a) {
-  (void)a;
+bool skinny_ok(int64_t M, int64_t K) {
   return M >= 1 && M <= 64 && K > 0 && K < (1 << 24) && M * K >= 16;
 }
 
@@ -634,7 +613,7 @@ hipError_t launch_gemm_skinny(hipStream_t st, const GemmArgs &g,
       launch_dq(std::integral_constant<int, 1>{});
     return hipGetLastError();
   }
-  if (!skinny_ok(g.M, g.K, g.A))
+  if (!skinny_ok(g.M, g.K))
     return hipErrorInvalidValue;
   if (a_mode == 0)
     launch_epi<0>(st, g, ep);

@@ -60,15 +60,16 @@ def spills():
 
 
 @pytest.mark.parametrize("kernel,most", [
-    # int8 A, int32 results: the epilogue's, behind the K loop.  68 with the edge
-    # stores by descriptor against 42 with a test per element: whole tiles take the
-    # same time either way (4096 x 768 x 768 7.25 / 7.26 us, 4096 x 3072 x 768 16.2 /
-    # 16.2), cut ones less (4096 x 768 x 1001 9.7 / 10.2)
-    (r"k_gemm_i8_dmaILi128ELi3ELi3ELi0ELi0E", 68),
-    (r"k_gemm_i8_dmaILi(64|128)ELi3ELi3ELi[12]ELi\dE", 0),
-    (r"k_gemm_i8_bsILi4ELi2ELi4ELi4ELi2ELb1ELi\dELi0ELb0E", 9),
-    (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi2E", 0),  # any K, any alignment
+    (r"k_gemm_i8_dmaI", 0),
+    (r"k_gemm_i8_(dma_)?bsI", 0),  # every tile, with and without row sums, split
+    (r"k_gemm_i8_wregI", 0),
+    # any K, any alignment: two blocks of 128 x 128 a CU, or four of 64 x 128, which
+    # leaves 128 registers a lane
+    (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi2E", 0),
+    (r"k_gemm_i8ILi64ELi128ELi2ELi2ELi4E", 11),
+    (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi3E", 20),  # on request only (OM_MI355X_GEMM_TILE=0)
     (r"k_gemm_i8_(skinny|batched|flight)I", 0),
+    (r"k_(pad_rows|sum_parts|copy_in|copy_out|pack_b)", 0),
 ])
 def test_kernels_spill_no_more_registers(spills, kernel, most):
     forms = {n: s for n, s in spills.items() if re.search(kernel, n)}
