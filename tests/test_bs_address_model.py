@@ -1,26 +1,26 @@
-"""Host model of every global and LDS access of k_gemm_i8_bs as it was before A
-was copied in whole lines (gemm_bs.hip; instantiation <TM=4, TN=2, D=4, NST=4,
-PIPE>; the kernel of today: test_bs_line_model.py), of its epilogue's stores
-(gemm_epilogue.h), of k_pad_rows with a byte per thread and of the
-buffer pool's size arithmetic (runtime.hip), checked against the real extents
-of the operands over a grid of shapes; and of the kernel's count of outstanding
-memory operations (its explicit vmcnt waits).  No GPU: this is index arithmetic
-restated for the host, lane by lane.
+"""Host model of the memory accesses of the tile kernels in gemm_bs.hip beside
+those of A (test_bs_line_model.py): weights, results at the edges and inside, parts
+of K; of the copies to an aligned pitch (k_pad_rows) and the chunks that the
+weight-streaming kernel reads at any address; and of the buffer pool's size
+arithmetic (runtime.hip).  No GPU: the index arithmetic restated for the host,
+lane by lane, and checked against the extents of the operands.
 
-Why it exists: a benchmark loop on 4096 x 1040 x 4096 (rows padded to 1088
-bytes, 17 K steps, this instantiation) once ended with an illegal memory
-access that nothing in the suite shows.  The model finds every access of that
-launch in bounds and every wait sufficient (the assertions below hold for it),
-so the cause is not in what is modelled here; the dispatch keeps
-k_gemm_i8_bs to step counts that are multiples of four, rows padded or not (test_dispatch_keeps_bs_to_whole_trips in the GPU suite).
-The model of the waits does find the defect of the other development variant
-that failed on the device, the one with six LDS stages (see the last tests of
-the wait model).
-"""
+Step counts of every kind are among the shapes, 17 above all: an earlier form of
+the streaming kernel ended a benchmark loop on 4096 x 1088 x 4096 with an illegal
+access.  Its addresses were in bounds as well; what went wrong is in
+test_loads_in_flight.py, which holds for the kernels of today that it cannot
+happen, and the loop's waits are in test_bs_line_model.py."""
+import os
+import re
+
 import numpy as np
 import pytest
 
 BK = 64
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SOURCE = open(os.path.join(ROOT, "onnx-mlir_amd", "csrc", "gemm_bs.hip")).read()
+LANE = np.arange(64)
+L32, LH = LANE & 31, LANE >> 5
 
 
 def round_up(a, b):
@@ -28,7 +28,7 @@ def round_up(a, b):
 
 
 # ---------------------------------------------------------------------------
-# the kernel's block -> tile map (XCD interleave, then groups of 8 row tiles)
+# block -> tile (XCD interleave, then groups of 8 row tiles)
 # ---------------------------------------------------------------------------
 def tile_of(pid, nb, tiles_m, tiles_n):
     per = nb >> 3
@@ -53,250 +53,145 @@ def test_every_tile_is_computed_exactly_once(tiles_m, tiles_n):
 
 
 # ---------------------------------------------------------------------------
-# global and LDS addresses
+# weights
 # ---------------------------------------------------------------------------
-def lds_off(r, c):
-    return r * BK + ((c ^ ((r >> 2) & 3)) << 4)
+def buffer_reads(offset, scalar, size):
+    """Which 16-byte loads the device makes: those whose lane offset (with the
+    instruction's own) is below the descriptor's size minus the scalar offset,
+    unsigned."""
+    return offset < (size - scalar) % 2 ** 32
 
 
-def check_bs(M, K, N, es, TM=4, TN=2, D=4, NST=4):
-    """Every address of one launch; es: bytes of an output element."""
-    assert K % BK == 0, "the fast path takes whole K steps only"
-    BM, BN = 32 * TM, 4 * 32 * TN
-    KT = K // BK
-    Npad = round_up(N, 256)
-    tiles_m, tiles_n = (M + BM - 1) // BM, (N + BN - 1) // BN
-    a_bytes, bp_bytes, out_bytes = M * K, Npad * K, M * N * es
-    CA = BM // 64
-    STAGE = BM * BK
-    lane = np.arange(64)
-    l32, lh = lane & 31, lane >> 5
-    crow, cchunk = lane >> 2, (lane & 3) ^ ((lane >> 4) & 3)
-    # steps the prologue and the loop ask for: 0 .. KT - 1 + max(D, NST - 1),
-    # clamped to the last one
-    steps = np.minimum(np.arange(KT + max(D, NST - 1)), KT - 1)
-
-    for tm in range(tiles_m):
-        m0 = tm * BM
-        for wave in range(4):
-            for h in range(CA):
-                # A copies (global_load_lds, 16 bytes a lane)
-                r = (wave * CA + h) * 16 + crow
-                rc = np.where(m0 + r < M, r, M - 1 - m0)
-                assert (rc >= 0).all() and (m0 + rc < M).all()
-                ga = rc * K + cchunk * 16
-                assert ga.max() < 2 ** 32
-                addr = m0 * K + steps[:, None] * BK + ga[None, :]
-                assert addr.min() >= 0 and addr.max() + 16 <= a_bytes, (M, K, N, tm, wave, h)
-                # their LDS side: 1 KiB per copy, lane * 16 within it, in a stage
-                for stage in range(NST):
-                    dst = stage * STAGE + (wave * CA + h) * 1024 + lane * 16
-                    assert dst.max() + 16 <= NST * STAGE
-                    # the copy puts row r's chunk where the operand reads look for it
-                    assert (dst - stage * STAGE == lds_off(r, cchunk)).all()
-    # operand reads of A from LDS
-    for s2 in range(2):
-        for i in range(TM):
-            ra = lds_off(l32, s2 * 2 + lh) + i * 2048
-            assert ra.max() + 16 <= STAGE
-
-    for tn in range(tiles_n):
-        n0 = tn * BN
-        for wave in range(4):
-            ncol0 = n0 + wave * 32 * TN
-            # Bp by buffer loads: descriptor base and range, lane and step offsets
-            base = (ncol0 >> 5) * KT * 2048
-            records = TN * KT * 2048
-            assert base + records <= bp_bytes, (M, K, N, tn, wave)
-            for j in range(TN):
-                boff = j * KT * 2048 + lane * 16
-                for sub in range(2):
-                    off = boff[None, :] + steps[:, None] * 2048 + sub * 1024
-                    assert off.min() >= 0 and off.max() + 16 <= records
-            # the epilogue's per-column operands: clamped to the last column
-            for j in range(TN):
-                n = ncol0 + j * 32 + l32
-                nc = np.where(n < N, n, N - 1)
-                assert (nc >= 0).all() and (nc < N).all()
-
-    # the epilogue's stores
-    for tm in range(tiles_m):
-        for tn in range(tiles_n):
-            for wave in range(4):
-                mrow0, ncol0 = tm * BM, tn * BN + wave * 32 * TN
-                full = (mrow0 + 32 * TM <= M and ncol0 + 32 * TN <= N and
-                        N * (32 * TM + 8) * 4 < 2 ** 31)
-                if full:
-                    # buffer stores: descriptor at the wave tile's first element,
-                    # no range check (0x7FFFFFFF records): lane offset + scalar row offset
-                    base = (mrow0 * N + ncol0) * es
-                    loff = (4 * lh * N + l32) * es
-                    worst = 0
-                    for i in (0, TM - 1):
-                        for r in (0, 15):
-                            rowb = (i * 32 + 8 * (r >> 2) + (r & 3)) * N * es
-                            for j in (0, TN - 1):
-                                voff = loff + j * 32 * es
-                                assert voff.max() + rowb < 2 ** 31
-                                worst = max(worst, int(base + voff.max() + rowb + es))
-                    assert worst <= out_bytes, (M, K, N, tm, tn, wave)
-                else:
-                    # element by element, each guarded by m < M and n < N
-                    m = mrow0 + np.arange(32 * TM)
-                    n = ncol0 + np.arange(32 * TN)
-                    mm, nn = np.meshgrid(m[m < M], n[n < N], indexing="ij")
-                    if mm.size:
-                        assert int((mm * N + nn).max() + 1) * es <= out_bytes
+SHAPES = [(4096, 1024, 4096), (4096, 1088, 4096), (2048, 4096, 11008), (4100, 1088, 4000), (129, 192, 257), (65, 16, 33),
+          (300, 784, 130), (64, 64, 1), (4095, 2048, 8190), (1500, 16, 5120), (90, 4176, 300)]
 
 
-SHAPES = [(4096, 1024, 4096), (4096, 1088, 4096),  # 17 steps: the launch that once died
-          (2048, 4096, 11008), (4096, 3072, 768), (4100, 1088, 4000), (4096, 64, 4096),
-          (4096, 320, 4100), (129, 192, 257), (8192, 11008, 4096), (4095, 2048, 8190)]
-
-
+@pytest.mark.parametrize("TN", [1, 2])
 @pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("part_steps", [0, 4, 12])
+def test_weights_are_read_where_they_lie_and_nowhere_else(TN, M, K, N, part_steps):
+    """Every step that a block asks for, the four that its last trip and its
+    prefetch run past the end among them; part_steps: K split into parts (0: not)."""
+    KTs = round_up(K, BK) // BK
+    bp_bytes = round_up(N, 256) * KTs * BK
+    parts = -(-KTs // part_steps) if part_steps else 1
+    for part in {0, parts - 1}:
+        kfirst = part * part_steps
+        KT = min(part_steps, KTs - kfirst) if part_steps else KTs
+        asked = round_up(KT, 4) + 3
+        for tn in {0, (N - 1) // (128 * TN)}:
+            for wave in range(4):
+                ncol0 = tn * 128 * TN + wave * 32 * TN
+                base = ((ncol0 >> 5) * KTs + kfirst) * 2048
+                size = (TN - 1) * KTs * 2048 + KT * 2048
+                assert base + size <= bp_bytes
+                for step in range(asked):
+                    inside = step < KT
+                    for half in range(2):
+                        for j in range(TN):
+                            lane = j * KTs * 2048 + LANE * 16 + half * 1024
+                            scalar = step * 2048 if inside else 0
+                            read = buffer_reads(lane, scalar, size if inside else 0)
+                            assert read.all() == read.any() == inside
+                            if inside:
+                                at = base + lane + scalar
+                                want = (((ncol0 >> 5) + j) * KTs + kfirst + step) * 2048 + half * 1024 + LANE * 16
+                                assert (at == want).all() and at.max() + 16 <= bp_bytes
+
+
+def test_the_half_step_is_not_in_the_scalar_offset():
+    """An empty descriptor with a scalar offset of 1024 would be read through."""
+    assert buffer_reads(LANE * 16, 1024, 0).all()
+    load = re.search(r"auto load_b = .*?\n  \};", SOURCE, re.S).group(0)
+    assert "offen offset:%4" in load and "bstep" in load and "* 1024" not in load.split("asm volatile")[0]
+
+
+# ---------------------------------------------------------------------------
+# results
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("TM,TN", [(4, 2), (2, 2), (2, 1)])
+@pytest.mark.parametrize("M,N", [(4096, 4096), (4100, 4000), (129, 257), (65, 33), (64, 1), (1, 130), (128, 31), (200, 8190)])
 @pytest.mark.parametrize("es", [1, 4])
-def test_every_access_of_the_shipped_instantiation_is_in_bounds(M, K, N, es):
-    check_bs(M, K, N, es)
+def test_results_are_stored_once_and_inside(TM, TN, M, N, es):
+    """Whole wave tiles by scalar row offsets, cut ones through a descriptor that
+    ends with the tile's last row: the elements that the device does not drop are
+    those of the matrix, each in its place."""
+    BM, BN = 32 * TM, 128 * TN
+    r = np.arange(16)
+    row_of = 8 * (r >> 2) + (r & 3)  # + 4 * lh
+    for tm in {0, (M - 1) // BM}:
+        for tn in {0, (N - 1) // BN}:
+            for wave in range(4):
+                m0, n0 = tm * BM, tn * BN + wave * 32 * TN
+                rows, cols = M - m0, N - n0
+                base = (m0 * N + n0) * es
+                loff = (4 * LH * N + L32) * es
+                if rows <= 0 or cols <= 0:
+                    continue
+                full = rows >= 32 * TM and cols >= 32 * TN
+                nr, nc = min(rows, 32 * TM), min(cols, 32 * TN)
+                size = 0x7FFFFFFF if full else ((nr - 1) * N + nc) * es
+                stored = []
+                for i in range(TM):
+                    for j in range(TN):
+                        lane = np.where(j * 32 + L32 < cols, loff + j * 32 * es, 0x80000000)
+                        for rr in row_of:
+                            rowb = (i * 32 + rr) * N * es
+                            at = lane + rowb
+                            assert at.max() < 2 ** 32
+                            keep = at < size if not full else np.ones(64, bool)
+                            m, n = m0 + i * 32 + rr + 4 * LH, n0 + j * 32 + L32
+                            assert (keep == ((m < M) & (n < N))).all()
+                            assert (base + at[keep] == ((m * N + n) * es)[keep]).all()
+                            stored.append(at[keep])
+                stored = np.concatenate(stored)
+                assert len(stored) == nr * nc == len(np.unique(stored))
+                assert base + stored.max() + es <= M * N * es
 
 
 # ---------------------------------------------------------------------------
-# the count of outstanding memory operations
+# 16-byte chunks at any address
 # ---------------------------------------------------------------------------
-def wait_counts(TM, TN, D, NST, PIPE):
-    CA = (32 * TM) // 64
-    PER_STEP = CA + 2 * TN
-    AHEAD = 1 if PIPE else 0
-    YOUNGER = (NST - 2 - AHEAD) * PER_STEP
-    P0 = (NST - 2) * CA + 2 * D * TN
-    return CA, PER_STEP, AHEAD, YOUNGER, P0
+def chunk(a, M, K, row, k0, fill, length):
+    """row_chunk (gemm_common.h) of the 16 bytes loaded for chunk k0 of `row`: read
+    at their address, or moved back to end with A; the bytes that are not the
+    row's replaced.  `length`: how many are."""
+    at, last = row * K + k0, M * K - 16
+    start = min(at, last)
+    assert 0 <= start and start + 16 <= M * K
+    v = int.from_bytes(a.reshape(-1)[start:start + 16].tobytes(), "little")
+    back = at - start
+    lo, hi = v & (2 ** 64 - 1), v >> 64
+    shift = back * 8 if length > 0 else 0
+    if shift >= 64:
+        lo, hi = hi, 0
+    s1 = shift & 63
+    if s1:
+        lo, hi = ((lo >> s1) | (hi << (64 - s1))) & (2 ** 64 - 1), hi >> s1
+    mlo = 2 ** 64 - 1 if length >= 8 else (1 << (8 * length)) - 1
+    mhi = 2 ** 64 - 1 if length >= 16 else ((1 << (8 * (length - 8))) - 1 if length > 8 else 0)
+    f = int.from_bytes(bytes([fill]) * 8, "little")
+    lo, hi = (lo & mlo) | (f & ~mlo & (2 ** 64 - 1)), (hi & mhi) | (f & ~mhi & (2 ** 64 - 1))
+    return np.frombuffer((lo | hi << 64).to_bytes(16, "little"), np.uint8)
 
 
-def static_asserts_hold(TM, TN, D, NST, PIPE):
-    """The kernel's compile-time conditions on its wait counts (the last one
-    says that step 0 does not use weights that are still on their way: the
-    prologue asks for the rows of NST - 1 steps first and for the weights after
-    them, and the first wait lets the youngest YOUNGER operations stand)."""
-    CA, PER_STEP, AHEAD, YOUNGER, P0 = wait_counts(TM, TN, D, NST, PIPE)
-    return (YOUNGER < 64 and P0 < 64 and NST - 2 - AHEAD >= 0 and D >= NST - 2 and
-            2 * TN * (D - 1) >= YOUNGER)
-
-
-def simulate_waits(KT, TM, TN, D=4, NST=4, PIPE=True):
-    """A wave's vector memory operations in issue order; they complete in
-    order, so `s_waitcnt vmcnt(n)` guarantees all but the youngest n.  Checks
-    that what a step reads has landed when it is read, and that no copy
-    overwrites a stage that some wave may still read."""
-    CA, PER_STEP, AHEAD, YOUNGER, P0 = wait_counts(TM, TN, D, NST, PIPE)
-    ops = []  # (kind, step asked for (before clamping), slot)
-
-    def copy_a(step, stage):
-        for _ in range(CA):
-            ops.append(("a", step, stage))
-
-    def load_b(step, u, sub):
-        for _ in range(TN):
-            ops.append(("b", step, (u, sub)))
-
-    def landed(n_outstanding):
-        return ops[:max(len(ops) - n_outstanding, 0)]
-
-    for p in range(NST - 1):
-        copy_a(p, p)
-    for u in range(D):
-        load_b(u, u, 0)
-        load_b(u, u, 1)
-    if PIPE:
-        done = landed(P0)
-        assert [o for o in done if o[0] == "a" and o[1] == 0] == [("a", 0, 0)] * CA
-    stage = 0
-    for kt in range(KT):
-        u = kt % D
-        done = landed(YOUNGER)
-        # the stage(s) this step reads hold the step's rows and have landed
-        for ahead in range(AHEAD + 1):
-            want, st = kt + ahead, (stage + ahead) % NST
-            last = [o for o in ops if o[0] == "a" and o[2] == st][-CA:]
-            if want < KT:
-                assert all(o[1] == want for o in last), (KT, kt, ahead, last)
-                idx = max(i for i, o in enumerate(ops) if o[0] == "a" and o[2] == st)
-                assert idx < len(done), ("copy not waited for", KT, kt, ahead)
-        # this step's weights (both halves) were asked for D steps ago and have landed
-        for sub in range(2):
-            idx = max(i for i, o in enumerate(ops) if o[0] == "b" and o[2] == (u, sub))
-            assert ops[idx][1] == kt and idx < len(done), ("weights", KT, kt, sub)
-        load_b(kt + D, u, 0)
-        load_b(kt + D, u, 1)
-        # refill the stage that was read in the previous step: every wave has
-        # passed this step's barrier, after it finished those reads
-        target = (stage - 1) % NST
-        assert target not in [(stage + a) % NST for a in range(AHEAD + 1)]
-        copy_a(kt + NST - 1, target)
-        stage = (stage + 1) % NST
-
-
-def model_accepts(TM, TN, D, NST, PIPE):
-    try:
-        for KT in list(range(1, 24)) + [64, 172]:
-            simulate_waits(KT, TM, TN, D=D, NST=NST, PIPE=PIPE)
-    except AssertionError:
-        return False
-    return True
-
-
-def test_shipped_instantiation_waits_for_what_each_step_reads():
-    for KT in list(range(1, 40)) + [64, 172]:
-        simulate_waits(KT, 4, 2, D=4, NST=4, PIPE=True)
-    assert static_asserts_hold(4, 2, 4, 4, True)
-
-
-@pytest.mark.parametrize("NST,D", [(3, 4), (4, 4), (4, 2), (4, 3), (5, 4), (6, 4), (6, 6), (6, 8)])
-def test_compile_time_conditions_reject_what_the_model_rejects(NST, D):
-    """For every tile shape and depth: an instantiation passes the kernel's
-    static_asserts only if the model finds its waits sufficient."""
-    for PIPE in (True, False):
-        if NST - 2 - (1 if PIPE else 0) < 0:
-            continue
-        for TM in (2, 4):
-            for TN in (1, 2, 3, 4):
-                if static_asserts_hold(TM, TN, D, NST, PIPE):
-                    assert model_accepts(TM, TN, D, NST, PIPE), (TM, TN, D, NST, PIPE)
-
-
-def test_six_stage_variant_used_weights_that_had_not_landed():
-    """The development instantiation with six LDS stages (64 x 128 tiles: TM =
-    2, TN = 1, D = 4) that ended in a fault or hang on the device: its first
-    wait lets nine operations stand, and the eight loads of the weights come
-    after the rows in the prologue, so step 0 multiplied with registers whose
-    loads were still in flight.  The kernel now refuses to compile so."""
-    assert not model_accepts(2, 1, 4, 6, True)
-    assert not static_asserts_hold(2, 1, 4, 6, True)
+@pytest.mark.parametrize("M,K", [(65, 1), (70, 3), (129, 15), (66, 17), (200, 64), (65, 1019), (33, 4101), (1, 17), (16, 1), (7, 3),
+                                 (2, 9), (5, 356)])
+def test_padded_rows_hold_the_row_and_its_zero_point(M, K):
+    rng = np.random.default_rng(M + K)
+    a, zp = rng.integers(0, 256, (M, K), dtype=np.uint8), rng.integers(0, 256, M, dtype=np.uint8)
+    Kp = round_up(K, 64)
+    chunks = Kp // 16
+    rows = range(M) if M * chunks < 2000 else [0, 1, M - 2, M - 1]
+    for r in rows:  # thread r * chunks + c
+        got = np.concatenate([chunk(a, M, K, r, c * 16, zp[r], max(0, min(16, K - c * 16))) for c in range(chunks)])
+        assert np.array_equal(got, np.concatenate([a[r], np.full(Kp - K, zp[r], np.uint8)]))
+    assert M * chunks * 16 == M * Kp  # what the runtime asks the pool for
 
 
 # ---------------------------------------------------------------------------
-# k_pad_rows and the pool
+# the pool
 # ---------------------------------------------------------------------------
-@pytest.mark.parametrize("M,K", [(1, 1), (16, 4100), (64, 1001), (33, 15), (64, 65537), (5, 16)])
-def test_pad_rows_stays_inside_both_buffers(M, K):
-    Kp = round_up(K, 16)
-    assert 1 <= M <= 64
-    grid_x = (Kp + 1023) // 1024
-    out_bytes = M * Kp  # what the runtime asks the pool for
-    hi_in = hi_out = 0
-    for r in (0, M - 1):
-        for bx in range(grid_x):
-            c = bx * 256 + np.arange(256)
-            while c.min() < Kp:
-                cc = c[c < Kp]
-                hi_out = max(hi_out, int(r * Kp + cc.max()) + 1)
-                rd = cc[cc < K]
-                if rd.size:
-                    hi_in = max(hi_in, int(r * K + rd.max()) + 1)
-                c = c + grid_x * 256
-    assert hi_in <= M * K and hi_out <= out_bytes
-    assert hi_out == out_bytes  # and every byte of the padded rows is written
-
-
 def test_pool_blocks_are_never_smaller_than_asked_for():
     """Ctx::take: the request rounded up to 256 bytes; an idle block serves it
     if it is the smallest one that is large enough and at most twice as large."""
@@ -314,6 +209,5 @@ def test_pool_blocks_are_never_smaller_than_asked_for():
         assert cap >= want and cap >= need
         if rng.integers(0, 2):
             pool.append(cap)
-    # the sizes of the launch that died: 4096 rows of 1088 bytes, and its packed weights
     for want in (4096 * 1088, 1088 * 4096, 4096 * 4096 * 4):
         assert round_up(want, 256) >= want

@@ -1,8 +1,9 @@
 """Host model of k_gemm_i8_bs and k_gemm_i8_dma_bs, A copied in stages of two K
 steps (onnx-mlir_amd/csrc/gemm_bs.hip): where their copies and operand reads go,
 and whether its explicit waits cover what each step reads.  Index arithmetic
-restated for the CPU; and the kernels themselves on the GPU, forced, at their
-edges."""
+restated for the CPU (weights, results, parts of K: test_bs_address_model.py; the
+registers that loads are still to write: test_loads_in_flight.py); and the kernels
+themselves on the GPU, forced, at their edges."""
 import numpy as np
 import pytest
 
@@ -49,9 +50,14 @@ def test_copies_are_in_bounds_and_lie_where_operands_are_read(TM, M, K):
                 assert len(set((at[g * 16:g * 16 + 16] % 256) // 16)) == 16
 
 
+KTS = [1, 2, 3, 4, 5, 8, 12, 17, 18, 64, 172]
+
+
 @pytest.mark.parametrize("TM,TN", TILES)
-@pytest.mark.parametrize("KT", [4, 8, 12, 64, 172])
+@pytest.mark.parametrize("KT", KTS)
 def test_waits_cover_what_each_step_reads(TM, TN, KT):
+    """One wave's vector memory operations in issue order, over the whole trips of
+    four steps that the loop makes for KT of them."""
     CA, CB = TM, 2 * TN
     ops = []  # (kind, asked for, register set or stage), in issue order
 
@@ -72,15 +78,40 @@ def test_waits_cover_what_each_step_reads(TM, TN, KT):
         if u == 0:
             copy(1)
     landed("a", 0, 0, 3 * CB + CA)
-    for p in range(KT // 2):
+    for p in range(-(-KT // D) * D // 2):
         landed("b", 2 * p, 2 * p % D, young)
-        # overwrites the stage before the last one, which the barrier has freed
-        assert (p + 2) % NST == (p - 2) % NST
         copy(p + 2)
         weights(2 * p + 3)
         landed("b", 2 * p + 1, (2 * p + 1) % D, young)
         landed("a", p + 1, (p + 1) % NST, young)
         weights(2 * p + 4)
+
+
+@pytest.mark.parametrize("KT", KTS)
+def test_no_stage_is_overwritten_while_a_wave_may_read_it(KT):
+    """Barriers, one at the start and one at the top of every odd step: between two
+    of them a wave may be anywhere.  A copy may land as soon as the fastest wave
+    asks for it, and a read may happen as late as the slowest one's next barrier
+    (it waits for its reads before that)."""
+    steps = -(-KT // D) * D
+    passed = {s: 1 + (s + 1) // 2 for s in range(steps)}  # in step s
+    reads, copies = [], [(0, 0), (0, 1)]  # (barriers passed, pair)
+    reads.append((1, 0))  # first operands, behind the first barrier
+    for s in range(steps):
+        p = s // 2
+        if s % 2 == 0:
+            reads += [(passed[s], p), (passed[s], p)]
+            copies.append((passed[s], p + NST - 2))
+        else:
+            reads += [(passed[s], p), (passed[s], p + 1)]
+    for at_copy, pair in copies:
+        for at_read, other in reads:
+            if other % NST != pair % NST:
+                continue
+            if other < pair:  # the stage's earlier contents: read before a barrier that the copy is behind
+                assert at_read < at_copy, (pair, other, at_copy, at_read)
+            elif other == pair:  # its own: read behind a barrier that follows the copy and its wait
+                assert at_read > at_copy or pair == 0, (pair, at_copy, at_read)
 
 
 @pytest.mark.gpu
