@@ -734,8 +734,8 @@ int choose_tile(const Sizes &p, double *us = nullptr) {
   int best = kD128x128;
   double least = tile_us(kTileCosts[0], p);
   for (const TileCost &t : kTileCosts) {
-    // (128 x 256 tiles: K a multiple of 256, the step counts that
-    // instantiation is validated at)
+    // (128 x 256 tiles: K a multiple of 256, whole trips of its loop, the step
+    // counts its times were taken at)
     if (p.K >= (1 << 24) ? t.trip != 1 : t.cfg == kB128x256 && p.K % 256 != 0)
       continue;
     const double u = tile_us(t, p);

@@ -177,11 +177,12 @@ def test_weights_in_registers_kernel_stays_inside_a_ragged_output(rt, oracle, fo
 
 def test_dispatch_keeps_bs_to_whole_trips(rt, oracle):
     """k_gemm_i8_bs runs four K steps per trip of its loop; the dispatch gives it
-    only products whose K is a multiple of 256 (the step counts it is validated
-    at).  4096 x 1088 x 4096 -- 17 steps, the launch that once ended a benchmark
-    loop with an illegal memory access (tests/test_bs_address_model.py) -- takes
-    the 128 x 128 tiles of k_gemm_i8_dma instead and matches the oracle; the
-    same product over K = 1024 still takes k_gemm_i8_bs."""
+    only products whose K is a multiple of 256 (the step counts its times were
+    taken at).  4096 x 1088 x 4096 -- 17 steps, the launch that once ended a
+    benchmark loop with an illegal memory access (why: test_loads_in_flight.py)
+    -- takes the 128 x 128 tiles of k_gemm_i8_dma instead and matches the
+    oracle; the same product over K = 1024 still takes k_gemm_i8_bs.  The 64-row
+    tiles of the same loop take any step count (test_bs_line_model.py)."""
     rng = np.random.default_rng(1088)
     A = rng.integers(0, 256, (4096, 1088), dtype=np.uint8)
     B = rng.integers(-128, 128, (1088, 4096), dtype=np.int8)
