@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n", [1, 15, 4095, 4096, 4097, 16383, 16385, 65535, 65537, 98303, 524288, 524289, 1048576, 1048577,
-                               1300001])
+                               1300001, 2200003])
 def test_sizes_around_chunks_pieces_and_limits(rt, n):
     """Results in chunks of 16 KiB up to 4 MiB, inputs in pieces of 256 KiB up to 2
     MiB, larger ones by the ways for them; lengths that are no whole vectors."""
