@@ -31,7 +31,11 @@
 //   flight; results written through where row pieces are whole lines (8.6 ->
 //   7.5 us, streaming stores 7.9).  Four blocks a CU where 128 registers suffice
 //   (96 x 512x64x512 22.6 -> 20.3 us against three), three for the 128-wide
-//   unaligned form (156 x 441x64x441 39.4 -> 33.7 us against two).
+//   unaligned form (four, with 19 spilled: 88 x 472x472x128 15.9 us, three 13.2).
+//   Rows at any address: one 32-bit offset and one minimum a load; shifts and
+//   masks only in the steps that the end of K lies in (with them, and 64-bit
+//   addresses, in every load: 88 x 472x472x128 19.0 us, so 13.2; 56 x 293x293x80 11.8
+//   / 8.7; 64 x 511x511x64 13.5 / 9.2; aligned rows 88 x 480x480x128 12.4 / 11.5).
 #include "gemm_common.h"
 #include "gemm_epilogue.h"
 
@@ -56,46 +60,76 @@ struct BatchParams {
   bool a_zp_per_matrix, b_zp_per_matrix;
 };
 
-// Bytes at offset `off` of a buffer of `total` bytes, for addresses of any
-// alignment: a load that would run past the buffer's end is moved back to end
-// with it and its bytes shifted down.
-__device__ __forceinline__ uint32_t load4_any(
-    const uint8_t *__restrict__ p, int off, int total) {
-  typedef uint32_t u32_any __attribute__((aligned(1)));
-  const int at = off < total - 4 ? off : total - 4;
-  return *(const u32_any *)(p + at) >> ((off - at) * 8);
+// Results leave the matrix cores as 32 columns by two rows to a store: whole lines
+// only where rows are multiples of 128 bytes.  Otherwise a block puts its tile into
+// LDS, byte o of what goes to `to` at byte (to & 15) + o, and writes it from there in
+// aligned pieces of 16 bytes, written through like whole lines are.
+//
+// `bytes` results of ES bytes each that lie one after the other (a tile as wide as
+// the matrix), `to` a multiple of ES.
+template <int ES>
+__device__ __forceinline__ void tile_out(const uint8_t *lds, char *to, int bytes) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  const int skew = (int)(uintptr_t)to & 15;
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(to - skew, 0, skew + bytes, 0x00020000);
+  const int tid = (int)threadIdx.x;
+  const int first = skew ? 16 : 0, last = (skew + bytes) & ~15; // whole pieces
+  for (int o = first + tid * 16; o < last; o += 256 * 16)
+    __builtin_amdgcn_raw_buffer_store_b128(
+        *(const u4 *)(lds + o), rsrc, o, 0, kAuxThrough);
+  // the ends, one result to a thread: PER threads in front, the next PER behind
+  constexpr int PER = 16 / ES;
+  const int o = tid < PER ? skew + tid * ES
+                          : (last > first ? last : first) + (tid - PER) * ES;
+  if (tid < 2 * PER && o < skew + bytes && (tid >= PER || o < first)) {
+    if constexpr (ES == 4)
+      __builtin_amdgcn_raw_buffer_store_b32(*(const int *)(lds + o), rsrc, o, 0, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b8(lds[o], rsrc, o, 0, 0);
+  }
 }
-__device__ __forceinline__ v4i load16_any(
-    const uint8_t *__restrict__ p, int off, int total) {
-  const int at = off < total - 16 ? off : total - 16;
-  const int sh = (off - at) * 8;
-  const v4i_any raw = *(const v4i_any *)(p + at);
-  uint64_t lo = (uint32_t)raw.x | ((uint64_t)(uint32_t)raw.y << 32);
-  uint64_t hi = (uint32_t)raw.z | ((uint64_t)(uint32_t)raw.w << 32);
-  if (sh >= 64) {
-    lo = hi;
-    hi = 0;
+// BM rows of BN 4-byte results, kRowPitch bytes apart in LDS, that are whole pieces:
+// `tile` and `pitch` are multiples of 16 bytes, and so are `bytes`, those of a row
+// that are there.
+template <int BN>
+constexpr int kRowPitch = BN * 4 + 32;
+template <int BN>
+__device__ __forceinline__ void rows_out(
+    const uint8_t *lds, char *tile, int rows, int bytes, int pitch) {
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  constexpr int PER = BN / 4, AT_ONCE = 256 / PER; // threads of a row; rows
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      tile, 0, (rows - 1) * pitch + bytes, 0x00020000);
+  const int o = (int)threadIdx.x % PER * 16;
+#pragma unroll
+  for (int q0 = 0; q0 < BM; q0 += AT_ONCE) {
+    const int q = q0 + (int)threadIdx.x / PER;
+    __builtin_amdgcn_raw_buffer_store_b128(
+        *(const u4 *)(lds + q * kRowPitch<BN> + o), rsrc,
+        o < bytes ? q * pitch + o : 0x7FFFFFFF, 0, kAuxThrough);
   }
-  const int s1 = sh & 63;
-  if (s1) {
-    lo = (lo >> s1) | (hi << (64 - s1));
-    hi >>= s1;
-  }
-  return (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi,
-      (int)(uint32_t)(hi >> 32)};
 }
 
 // ALIGNED: K % 16 == 0 with A on a 16-byte boundary and N % 4 == 0 with B on a
 // 4-byte one, so that every load is whole and inside its row.
-template <int BN, int EPI, bool ALIGNED>
+// OUT: how results leave, chosen by out_form.
+enum OutForm : int { kOutDirect, kOutTile, kOutRows };
+template <int BN, int EPI, bool ALIGNED, int OUT>
 __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_batched(
     const BatchParams bp, const EpiParams ep) {
   static_assert(BN == 128 || BN == 64, "tile width");
   constexpr int TM = BN == 128 ? 2 : 1; // row tiles of 32 per wave
   constexpr int KPT = BN / 16;          // K rows of B per thread
   constexpr int CG = BN / 4;            // groups of four columns
-  __shared__ __attribute__((aligned(16))) uint8_t sA[2][BM * BK];
-  __shared__ __attribute__((aligned(16))) uint8_t sB[2][BN * BK];
+  // The operands of two steps; at the end, results on their way out.
+  constexpr int ES = EPI == kEpiQ8 ? 1 : 4;
+  constexpr int kOperands = 2 * (BM + BN) * BK;
+  constexpr int kStaged = OUT == kOutDirect ? 0 : BM * kRowPitch<BN> / (4 / ES);
+  __shared__ __attribute__((aligned(16)))
+  uint8_t sm[kOperands > kStaged ? kOperands : kStaged];
+  uint8_t(*const sA)[BM * BK] = (uint8_t(*)[BM * BK])sm;
+  uint8_t(*const sB)[BN * BK] = (uint8_t(*)[BN * BK])(sm + 2 * BM * BK);
   __shared__ int32_t s_rowsum[BM], s_da[BM];
   __shared__ int32_t s_colsum[BN];
 
@@ -158,9 +192,17 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
 #pragma unroll
   for (int i = 0; i < KPT; ++i)
     b_voff[i] = b_col ? b_off + i * N : kOutside;
-  const int64_t a_left = bp.a_total - ai * M * K, b_left = bp.b_total - bi * K * N;
-  const int a_end = a_left < kOutside ? (int)a_left : kOutside;
-  const int b_end = b_left < kOutside ? (int)b_left : kOutside;
+  // Otherwise loads at any address, as 32-bit offsets from a base that lies at most
+  // 15 (3) bytes in front of the matrix, none of which may end behind the last
+  // matrix: those are moved back to end with it (a_last, b_last).  Bytes of the
+  // matrix are among them in the last rows only, of B in the last three (N = 1).
+  const int64_t a_left = bp.a_total - ai * M * K - 16, b_left = bp.b_total - bi * K * N - 4;
+  const int a_back = a_left < 0 ? (int)-a_left : 0, b_back = b_left < 0 ? (int)-b_left : 0;
+  typedef const __attribute__((address_space(1))) uint8_t *glb; // (not flat loads)
+  const glb a_base = (glb)scalar_ptr(Ae - a_back), b_base = (glb)scalar_ptr(Be - b_back);
+  const int a_last = a_left < kOutside ? (int)a_left + a_back : kOutside;
+  const int b_last = b_left < kOutside ? (int)b_left + b_back : kOutside;
+  const int a_any = (a_row ? a_off : ac * 16) + a_back, b_any = b_off + b_back;
 
   int32_t rs = 0, cs[4] = {0, 0, 0, 0};
   // Operands on their way from memory: two K steps, so that a step's loads have
@@ -178,29 +220,38 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
         rb[i] = __builtin_amdgcn_raw_buffer_load_b32(
             brsrc, b_voff[i], k0 * N, 0);
     } else {
-      ra = load16_any(Ae, a_row && k0 + ac * 16 < K ? a_off + k0 : 0, a_end);
+      typedef const __attribute__((address_space(1))) uint32_t u32_any
+          __attribute__((aligned(1)));
+      typedef const __attribute__((address_space(1))) v4i_any v4i_glb;
+      const int a = a_any + k0;
+      ra = *(v4i_glb *)(a_base + lane_offset((uint32_t)(a < a_last ? a : a_last)));
 #pragma unroll
       for (int i = 0; i < KPT; ++i) {
-        const bool in = b_col && k0 + kg * KPT + i < K;
-        rb[i] = load4_any(Be, in ? b_off + (k0 + i) * N : 0, b_end);
+        const int b = b_any + (k0 + i) * N;
+        rb[i] = *(u32_any *)(b_base +
+                                   lane_offset((uint32_t)(b < b_last ? b : b_last)));
       }
     }
   };
-  // Registers to LDS, as int8 and in operand order; bytes past K become 0 in
-  // both operands (rows past M and columns past N are never stored).
-  auto store = [&](int k0, int buf, const v4i &ra, const uint32_t(&rb)[KPT]) {
-    const int gk = k0 + ac * 16;
-    const int len = a_row ? K - gk : 0; // bytes of the chunk inside the row
-    v4i v = ra ^ (v4i){(int)bp.a_flip, (int)bp.a_flip, (int)bp.a_flip,
-                     (int)bp.a_flip};
+  // Registers to LDS, as int8 and in operand order.  In the steps that the last
+  // three rows of B or the end of K lie in, what was moved back is shifted into
+  // place, and bytes past K become 0 in both operands (rows past M and columns past
+  // N are never stored).
+  auto store = [&](int k0, int buf, v4i ra, uint32_t(&rb)[KPT]) {
+    const v4i flip = {(int)bp.a_flip, (int)bp.a_flip, (int)bp.a_flip, (int)bp.a_flip};
+    if (k0 + BK > (ALIGNED ? K : K - 3)) {
+      const int left = K - (k0 + ac * 16), a = a_any + k0;
+      ra = row_chunk(ra, ALIGNED || a < a_last ? 0 : a - a_last,
+          left < 0 ? 0 : left < 16 ? left : 16,
+          (uint64_t)bp.a_flip << 32 | bp.a_flip);
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int keep = len - w * 4;
-      const uint32_t mask = keep >= 4  ? 0xFFFFFFFFu
-                            : keep > 0 ? (1u << (8 * keep)) - 1
-                                       : 0u;
-      v[w] = (int)((uint32_t)v[w] & mask);
+      for (int i = 0; i < KPT; ++i) {
+        const int b = b_any + (k0 + i) * N;
+        const uint32_t r = ALIGNED || b < b_last ? rb[i] : rb[i] >> ((b - b_last) * 8 & 31);
+        rb[i] = k0 + kg * KPT + i < K ? r : bp.b_flip;
+      }
     }
+    const v4i v = ra ^ flip;
     rs += frag_rowsum(v);
     *(v4i *)(&sA[buf][lds_off(ar, ac)]) = v;
     uint32_t o[4][KPT / 4];
@@ -209,7 +260,7 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
       uint32_t r[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        r[i] = k0 + kg * KPT + h * 4 + i < K ? rb[h * 4 + i] ^ bp.b_flip : 0u;
+        r[i] = rb[h * 4 + i] ^ bp.b_flip;
       const uint32_t t0 = __builtin_amdgcn_perm(r[1], r[0], 0x05010400u);
       const uint32_t t1 = __builtin_amdgcn_perm(r[1], r[0], 0x07030602u);
       const uint32_t t2 = __builtin_amdgcn_perm(r[3], r[2], 0x05010400u);
@@ -325,43 +376,105 @@ __global__ __launch_bounds__(256, ALIGNED || BN == 64 ? 4 : 3) void k_gemm_i8_ba
 
   // 32x32 accumulator layout: lane holds column lane % 32; register r holds
   // row 8*(r/4) + 4*(lane/32) + r%4.
-  if (n >= N)
-    return;
   const uint32_t csn = (uint32_t)s_colsum[ct * 32 + l32];
-  // A descriptor over the tile's rows inside the matrix: stores to rows past M
-  // fall outside and are dropped (gemm_batched_ok keeps 64 rows below 2^31
-  // bytes).
-  constexpr int ES = EPI == kEpiQ8 ? 1 : 4;
-  const int rows = M - m0 < BM ? M - m0 : BM;
+  const int rows = M - m0 < BM ? M - m0 : BM, cols = N - n0 < BN ? N - n0 : BN;
   char *const out = (char *)ep.out +
                     (((int64_t)entry * M + m0) * N + n0) * (int64_t)ES;
-  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      out, 0, (int)(((int64_t)rows * N - n0) * ES), 0x00020000);
-  const int voff = ((4 * lh) * N + ct * 32 + l32) * ES;
-  auto rows_out = [&](auto aux) {
+  // f(first, result) for every register, `first` the row of the lanes 0 .. 31
+  auto results = [&](auto f) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int first = rt + i * 32 + 8 * (r >> 2) + (r & 3); // of lane 0
+        const int first = rt + i * 32 + 8 * (r >> 2) + (r & 3);
         const uint32_t da = (uint32_t)s_da[first + 4 * lh];
         const uint32_t y =
             (uint32_t)acc[i][r] + da * csn +
             (uint32_t)db * ((uint32_t)s_rowsum[first + 4 * lh] + (uint32_t)K * da);
-        if (EPI == kEpiI32)
-          __builtin_amdgcn_raw_buffer_store_b32(
-              (int)y, rsrc, voff + first * N * ES, 0, decltype(aux)::value);
-        else
-          __builtin_amdgcn_raw_buffer_store_b8(
-              (unsigned char)requantize(ep, y, sj, yz), rsrc,
-              voff + first * N * ES, 0, decltype(aux)::value);
+        f(first, EPI == kEpiI32 ? y : requantize(ep, y, sj, yz));
       }
     }
   };
-  if (((int64_t)N * ES) % 128 == 0)
-    rows_out(std::integral_constant<int, kAuxThrough>{});
+  auto put = [&](int at, uint32_t v) {
+    if (EPI == kEpiI32)
+      *(uint32_t *)(sm + at) = v;
+    else
+      sm[at] = (uint8_t)v;
+  };
+  const int col = (ct * 32 + l32) * ES;
+  if constexpr (OUT == kOutTile) {
+    // (as wide as the matrix: its results lie one after the other)
+    const int skew = (int)(uintptr_t)out & 15;
+    if (n < N)
+      results([&](int first, uint32_t v) {
+        put(skew + (first + 4 * lh) * N * ES + col, v);
+      });
+    __syncthreads();
+    tile_out<ES>(sm, out, rows * N * ES);
+    return;
+  }
+  if constexpr (OUT == kOutRows) {
+    results([&](int first, uint32_t v) {
+      put((first + 4 * lh) * kRowPitch<BN> + col, v);
+    });
+    __syncthreads();
+    rows_out<BN>(sm, out, rows, cols * 4, N * 4);
+    return;
+  }
+  // A descriptor over the tile's rows inside the matrix: stores to rows past M
+  // fall outside and are dropped (gemm_batched_ok keeps 64 rows below 2^31
+  // bytes).
+  if (n >= N)
+    return;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      out, 0, (int)(((int64_t)rows * N - n0) * ES), 0x00020000);
+  const int voff = ((4 * lh) * N + ct * 32 + l32) * ES;
+  auto direct = [&](auto aux) {
+    results([&](int first, uint32_t v) {
+      if (EPI == kEpiI32)
+        __builtin_amdgcn_raw_buffer_store_b32(
+            (int)v, rsrc, voff + first * N * ES, 0, decltype(aux)::value);
+      else
+        __builtin_amdgcn_raw_buffer_store_b8((unsigned char)v, rsrc,
+            voff + first * N * ES, 0, decltype(aux)::value);
+    });
+  };
+  if (N * ES % 128 == 0)
+    direct(std::integral_constant<int, kAuxThrough>{});
   else
-    rows_out(std::integral_constant<int, 0>{});
+    direct(std::integral_constant<int, 0>{});
+}
+
+// By way of LDS where rows are no whole lines and the grid is more than one round of
+// blocks: up to that the barrier and the second way cost more than the stores (48 x
+// 38x38x80 4.74 us by LDS, 4.57 without).
+//   Tiles as wide as the matrix: 156 x 82x128x82 7.6 -> 6.8 us, 64 x 511x511x64 with 8-bit
+//   results 13.9 -> 9.6, the loads' part of both included.
+//   Rows of whole 16-byte pieces: int32 88 x 472x128x472 28.8 -> 23.4; not 8-bit ones (21.2
+//   -> 23.5), nor other rows, whose ends are stores of their own (64 x 511x64x511 17.2
+//   -> 18.5).
+template <int EPI>
+OutForm out_form(const BatchParams &bp, const EpiParams &ep, int64_t blocks) {
+  constexpr int ES = EPI == kEpiQ8 ? 1 : 4;
+  if (blocks <= 256 || bp.N * ES % 128 == 0)
+    return kOutDirect;
+  if (bp.tiles_n == 1)
+    return kOutTile;
+  return EPI == kEpiI32 && ((((uintptr_t)ep.out) | (uintptr_t)(bp.N * 4)) & 15) == 0
+             ? kOutRows
+             : kOutDirect;
+}
+
+template <int BN, int EPI, bool ALIGNED>
+void launch_form(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
+    unsigned blocks) {
+  const OutForm out = out_form<EPI>(bp, ep, blocks);
+  if (out == kOutTile)
+    k_gemm_i8_batched<BN, EPI, ALIGNED, kOutTile><<<blocks, 256, 0, s>>>(bp, ep);
+  else if (out == kOutDirect)
+    k_gemm_i8_batched<BN, EPI, ALIGNED, kOutDirect><<<blocks, 256, 0, s>>>(bp, ep);
+  else if constexpr (BN == 128 && EPI == kEpiI32) // (more than one tile to a row)
+    k_gemm_i8_batched<BN, EPI, ALIGNED, kOutRows><<<blocks, 256, 0, s>>>(bp, ep);
 }
 
 template <int EPI>
@@ -370,14 +483,14 @@ hipError_t launch_epi(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
   const unsigned blocks = (unsigned)(entries * bp.tiles_m * bp.tiles_n);
   if (bp.N <= 64) {
     if (aligned)
-      k_gemm_i8_batched<64, EPI, true><<<blocks, 256, 0, s>>>(bp, ep);
+      launch_form<64, EPI, true>(s, bp, ep, blocks);
     else
-      k_gemm_i8_batched<64, EPI, false><<<blocks, 256, 0, s>>>(bp, ep);
+      launch_form<64, EPI, false>(s, bp, ep, blocks);
   } else {
     if (aligned)
-      k_gemm_i8_batched<128, EPI, true><<<blocks, 256, 0, s>>>(bp, ep);
+      launch_form<128, EPI, true>(s, bp, ep, blocks);
     else
-      k_gemm_i8_batched<128, EPI, false><<<blocks, 256, 0, s>>>(bp, ep);
+      launch_form<128, EPI, false>(s, bp, ep, blocks);
   }
   return hipGetLastError();
 }
