@@ -93,6 +93,84 @@ struct EpiParams {
   int narrow;
 };
 
+// Whether a launch's arguments are few enough for the short way through the launch
+// call.  Empty kernels of 64 blocks, one after the other, microseconds a launch:
+// structures of 112 bytes 2.8, of 120 bytes 3.5; six pointers 2.9, eight 3.7; a pointer
+// and 104 bytes 2.8; two pointers and 72 bytes 2.9, and 88 bytes 3.7; more, up to 320
+// bytes, 3.5 - 3.7.  (Grid and block sizes that a kernel reads are 256 bytes of arguments
+// behind its own.)
+constexpr bool cheap_arguments(size_t bytes, size_t pointers) {
+  return (bytes + 15) / 16 * 16 + 8 * pointers < 128;
+}
+// EpiParams for kernels of a few microseconds (cheap_arguments), without limits of y.
+// Fields that no two epilogues need share a place:
+//   first   y_scale (kEpiQ8) or bias (kEpiF32)
+//   second  y_zp (kEpiQ8) or x_limits (kEpiF32)
+// and lengths are told apart as 0, 1 and more (2), which is all that kernels ask.
+struct PackedEpi {
+  const void *a_zp, *b_zp;
+  const int32_t *colsum;
+  const float *a_scale, *b_scale;
+  const void *first, *second;
+  void *out;
+  unsigned a_zp_len : 2, b_zp_len : 2, b_scale_len : 2, bias_len : 2;
+  unsigned need_rowsum : 1, relu : 1, gelu : 1, b_unsigned : 1, y_unsigned : 1,
+      narrow : 1;
+};
+inline PackedEpi pack_epi(const EpiParams &e, int epi) {
+  auto length = [](int64_t n) { return n > 1 ? 2u : (unsigned)n; };
+  PackedEpi p = {};
+  p.a_zp = e.a_zp;
+  p.b_zp = e.b_zp;
+  p.colsum = e.colsum;
+  p.a_scale = e.a_scale;
+  p.b_scale = e.b_scale;
+  p.first = epi == kEpiQ8 ? (const void *)e.y_scale : e.bias;
+  p.second = epi == kEpiQ8 ? e.y_zp : e.x_limits;
+  p.out = e.out;
+  p.a_zp_len = length(e.a_zp_len);
+  p.b_zp_len = length(e.b_zp_len);
+  p.b_scale_len = length(e.b_scale_len);
+  p.bias_len = length(e.bias_len);
+  p.need_rowsum = e.need_rowsum;
+  p.relu = e.floor == 0.0f; // (relu_floor: 0 or a NaN)
+  p.gelu = e.gelu;
+  p.b_unsigned = e.b_unsigned;
+  p.y_unsigned = e.y_unsigned;
+  p.narrow = (unsigned)e.narrow;
+  return p;
+}
+static_assert(sizeof(PackedEpi) == 72 && kWrap >= 0 && kWrap < 2 && kSaturate >= 0 &&
+              kSaturate < 2);
+template <int EPI>
+__device__ __forceinline__ EpiParams unpack_epi(const PackedEpi &p) {
+  EpiParams e = {};
+  e.a_zp = p.a_zp;
+  e.b_zp = p.b_zp;
+  e.colsum = p.colsum;
+  e.a_scale = p.a_scale;
+  e.b_scale = p.b_scale;
+  if (EPI == kEpiQ8) {
+    e.y_scale = (const float *)p.first;
+    e.y_zp = p.second;
+  } else if (EPI == kEpiF32) {
+    e.bias = (const float *)p.first;
+    e.x_limits = (const float *)p.second;
+  }
+  e.out = p.out;
+  e.a_zp_len = p.a_zp_len;
+  e.b_zp_len = p.b_zp_len;
+  e.b_scale_len = p.b_scale_len;
+  e.bias_len = p.bias_len;
+  e.need_rowsum = p.need_rowsum;
+  e.floor = p.relu ? 0.0f : __builtin_nanf("");
+  e.gelu = p.gelu;
+  e.b_unsigned = p.b_unsigned;
+  e.y_unsigned = p.y_unsigned;
+  e.narrow = (int)p.narrow;
+  return e;
+}
+
 // Called once by every thread of a block of `nwaves` waves (the waves that are
 // still running, in uniform control flow) with the minimum and maximum of the
 // elements it stored, NaN ignored (+inf / -inf if it stored none).  The block's

@@ -66,11 +66,20 @@ constexpr int kSkinnyDqBytes = 32768;
 // front: layers 13 x 356 x 5568 10.9 -> 3.9 us, 2 x 2380 x 372 10.9 -> 4.1, 15 x
 // 8000 x 871 10.2 (K % 16 == 0, as before); int32 12 x 946 x 734 7.6 -> 3.4, 17 x
 // 4185 x 1633 7.0 -> 7.0.
+struct SkinnyArgs {
+  const void *rows; // A, or X (DQ)
+  const int8_t *Bp;
+  int M, N, K;
+  PackedEpi epi;
+};
+static_assert(cheap_arguments(sizeof(SkinnyArgs), 0));
 template <int A_MODE, int EPI, int DQ, int T, int RT, int CT, bool STG, bool ANY>
-__global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
-    const uint8_t *__restrict__ A, const float *__restrict__ X,
-    const int8_t *__restrict__ Bp, int M, int N, int K, int Kpad,
-    EpiParams ep) {
+__global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(SkinnyArgs args) {
+  const uint8_t *__restrict__ A = DQ ? nullptr : (const uint8_t *)args.rows;
+  const float *__restrict__ X = DQ ? (const float *)args.rows : nullptr;
+  const int8_t *__restrict__ Bp = args.Bp;
+  const int M = args.M, N = args.N, K = args.K;
+  const EpiParams ep = unpack_epi<EPI>(args.epi);
   static_assert(!DQ || (A_MODE == 2 && !STG), "quantized rows");
   static_assert((T == 16 && CT <= 2) || (T == 32 && CT == 1 && !DQ), "tiles");
   static_assert(!ANY || DQ || STG, "rows of any length");
@@ -99,7 +108,7 @@ __global__ __launch_bounds__(WAVES * 64) void k_gemm_i8_skinny(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & (T - 1); // row of A, column of B
   const int lk = lane / T;       // and 16-byte chunk (of each 64 / SUBS bytes)
-  const int KT = Kpad / BK;
+  const int KT = (K + BK - 1) / BK;
   const int per = (KT + WAVES - 1) / WAVES;
   const int kt_begin = wave * per < KT ? wave * per : KT;
   const int kt_end = kt_begin + per < KT ? kt_begin + per : KT;
@@ -508,8 +517,8 @@ void launch_one(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
     if (any_rows(g))
       kernel = k_gemm_i8_skinny<A_MODE, EPI, DQ, T, RT, CT, STG, true>;
   kernel<<<(unsigned)((g.N + T * CT - 1) / (T * CT)), WAVES * 64, 0, st>>>(
-      (const uint8_t *)g.A, g.X, g.Bp, (int)g.M, (int)g.N, (int)g.K,
-      (int)round_up(g.K, kGemmBK), ep);
+      SkinnyArgs{DQ ? (const void *)g.X : g.A, g.Bp, (int)g.M, (int)g.N, (int)g.K,
+          pack_epi(ep, EPI)});
 }
 // Blocks of 16 columns are what fills the device while N / 16 is up to 256.
 constexpr int64_t kOneRound = 256 * 16;
