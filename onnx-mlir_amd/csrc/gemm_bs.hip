@@ -46,7 +46,7 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
 
   int pid = blockIdx.x;
   {
-    const int nb = gridDim.x;
+    const int nb = tiles_m * tiles_n;
     const int per = nb >> 3;
     if (per > 0 && pid < per * 8)
       pid = (pid & 7) * per + (pid >> 3);
@@ -360,19 +360,17 @@ __device__ __forceinline__ void stream_tile(const uint8_t *__restrict__ A,
 
 // 128 x 256 tiles.
 template <int A_MODE, int EPI, bool RS>
-__global__ __launch_bounds__(256, 2) void k_gemm_i8_bs(
-    const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n) {
-  stream_tile<4, 2, A_MODE, EPI, RS, false, false>(
-      A, Bp, M, N, K, Kpad, ep, tiles_m, tiles_n, KSplit{});
+__global__ __launch_bounds__(256, 2) void k_gemm_i8_bs(TileArgs a) {
+  stream_tile<4, 2, A_MODE, EPI, RS, false, false>(a.A, a.Bp, a.M, a.N, a.K,
+      padded_k(a.K), unpack_epi<EPI>(a.epi), tiles_of(a.M, 128), tiles_of(a.N, 256),
+      KSplit{});
 }
 // 64 x 256 and 64 x 128 tiles.
 template <int TN, int MINB, int A_MODE, int EPI, bool RS, bool RAGGED, bool SPLIT>
-__global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma_bs(
-    const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n, KSplit ks) {
-  stream_tile<2, TN, A_MODE, EPI, RS, RAGGED, SPLIT>(
-      A, Bp, M, N, K, Kpad, ep, tiles_m, tiles_n, ks);
+__global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma_bs(TileArgs a) {
+  stream_tile<2, TN, A_MODE, EPI, RS, RAGGED, SPLIT>(a.A, a.Bp, a.M, a.N, a.K,
+      padded_k(a.K), unpack_epi<EPI>(a.epi), tiles_of(a.M, 64),
+      tiles_of(a.N, 128 * TN), KSplit{a.steps, part_stride(a.M, a.N)});
 }
 
 // ragged: the form that looks for the end of the row (only row sums have to); in
@@ -392,7 +390,6 @@ const char *dma_bs_name(int tn, bool ragged, bool split) {
 template <int TN, int A_MODE, int EPI, bool SPLIT>
 void launch_dma_bs(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
-  const int Kpad = (int)round_up(g.K, kGemmBK);
   const int tiles_m = (M + 63) / 64, tiles_n = (N + 128 * TN - 1) / (128 * TN);
   const bool ragged = ep.need_rowsum && K % BK != 0;
   constexpr int MINB = TN == 1 ? 4 : 3;
@@ -402,10 +399,8 @@ void launch_dma_bs(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
           ? (ragged ? k_gemm_i8_dma_bs<TN, MINB, A_MODE, EPI, true, true, SPLIT>
                     : k_gemm_i8_dma_bs<TN, MINB, A_MODE, EPI, true, false, SPLIT>)
           : k_gemm_i8_dma_bs<TN, MINB, A_MODE, EPI, false, false, SPLIT>;
-  const KSplit ks = {g.split.steps, part_stride(g)};
   kernel<<<dim3((unsigned)(tiles_m * tiles_n), SPLIT ? (unsigned)g.split.parts : 1u),
-      256, 0, st>>>((const uint8_t *)g.A, g.Bp, M, N, K, Kpad, ep, tiles_m,
-      tiles_n, SPLIT ? ks : KSplit{});
+      256, 0, st>>>(tile_args(g, ep, EPI));
 }
 
 template <int A_MODE, int EPI>
@@ -414,14 +409,12 @@ void launch_tile(hipStream_t st, const GemmArgs &g, const EpiParams &ep, BsTile 
     return launch_dma_bs<1, A_MODE, EPI, false>(st, g, ep);
   if (tile == kBs64x256)
     return launch_dma_bs<2, A_MODE, EPI, false>(st, g, ep);
-  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int M = (int)g.M, N = (int)g.N;
   const int tiles_m = (M + 127) / 128, tiles_n = (N + 255) / 256;
   note_gemm_kernel("k_gemm_i8_bs (128x256 tiles)");
   auto *const kernel = ep.need_rowsum ? k_gemm_i8_bs<A_MODE, EPI, true>
                                       : k_gemm_i8_bs<A_MODE, EPI, false>;
-  kernel<<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
-      (const uint8_t *)g.A, g.Bp, M, N, K, (int)round_up(g.K, kGemmBK), ep,
-      tiles_m, tiles_n);
+  kernel<<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(tile_args(g, ep, EPI));
 }
 
 template <int A_MODE>

@@ -171,6 +171,26 @@ __device__ __forceinline__ EpiParams unpack_epi(const PackedEpi &p) {
   return e;
 }
 
+template <int EPI>
+__device__ __forceinline__ EpiParams unpack_epi(const EpiParams &e) {
+  return e;
+}
+// What the tile kernels are handed; tiles and K steps follow from the sizes.
+struct TileArgs {
+  const uint8_t *A;
+  const int8_t *Bp;
+  int M, N, K;
+  int steps; // of a part of K (KSplit)
+  PackedEpi epi;
+};
+static_assert(cheap_arguments(sizeof(TileArgs), 0));
+__host__ __device__ constexpr int tiles_of(int n, int tile) {
+  return (int)(((unsigned)n + tile - 1) / tile);
+}
+__host__ __device__ constexpr int padded_k(int K) {
+  return (int)((K > 0 ? (unsigned)K + BK - 1 : BK) / BK * BK);
+}
+
 // Called once by every thread of a block of `nwaves` waves (the waves that are
 // still running, in uniform control flow) with the minimum and maximum of the
 // elements it stored, NaN ignored (+inf / -inf if it stored none).  The block's
@@ -353,7 +373,14 @@ __device__ __forceinline__ v4i row_chunk(v4i v, int back, int len, uint64_t fill
 }
 
 // Elements between the arrays of the parts of a product split along K.
-inline int64_t part_stride(const GemmArgs &g) { return round_up(g.M * g.N, 4); }
+__host__ __device__ constexpr int64_t part_stride(int64_t M, int64_t N) {
+  return (M * N + 3) / 4 * 4;
+}
+inline int64_t part_stride(const GemmArgs &g) { return part_stride(g.M, g.N); }
+inline TileArgs tile_args(const GemmArgs &g, const EpiParams &ep, int epi) {
+  return TileArgs{(const uint8_t *)g.A, g.Bp, (int)g.M, (int)g.N, (int)g.K,
+      g.split.steps, pack_epi(ep, epi)};
+}
 
 // k_gemm_i8_bs and k_gemm_i8_dma_bs (gemm_bs.hip): Bp streamed into registers, K
 // a multiple of 16 (128 x 256 tiles: of 256) and A 16-byte aligned; split: one

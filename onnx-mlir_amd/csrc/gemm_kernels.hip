@@ -52,7 +52,11 @@ using namespace gemm;
 namespace {
 
 // BM x BN block tile, WGM x WGN waves, each wave a (BM/WGM) x (BN/WGN) tile
-// made of 32x32 MFMA tiles.
+// made of 32x32 MFMA tiles.  MINB: blocks that a CU is to hold; of more than two
+// the compiler gets registers for one block fewer, since a fourth block of 64 x
+// 128 brings less than what its 128 registers a lane spill costs (in us, with
+// four / three: 1000 x 1001 x 3000 with row sums 11.9 / 11.3, 300 x 777 x 1001
+// 6.8 / 6.5, 4099 x 777 x 1001 14.5 / 13.7).
 // A_MODE: 0 = int8 as is, 1 = uint8 (XOR 0x80 while staging), 2 = already
 // shifted (stored as u8-128) -- offsets as for uint8, no XOR.
 // A_LOAD: kLoadAligned = K % 64 == 0 and A 16-byte aligned (plain vector
@@ -61,9 +65,15 @@ namespace {
 // = byte loads (an A of fewer than 16 bytes, K = 0).
 template <int BM, int BN, int WGM, int WGN, int MINB, int A_MODE, int EPI,
     int A_LOAD, bool SPLIT = false>
-__global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
-    const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n, KSplit ks = {}) {
+__global__ __launch_bounds__(WGM *WGN * 64, MINB > 2 ? MINB - 1 : MINB)
+void k_gemm_i8(TileArgs args) {
+  const uint8_t *__restrict__ A = args.A;
+  const int8_t *__restrict__ Bp = args.Bp;
+  const int M = args.M, N = args.N, K = args.K;
+  const int Kpad = A_LOAD == kLoadAligned ? K : padded_k(K);
+  const int tiles_m = tiles_of(M, BM), tiles_n = tiles_of(N, BN);
+  const EpiParams ep = unpack_epi<EPI>(args.epi);
+  const KSplit ks = {args.steps, part_stride(M, N)};
   constexpr int THREADS = WGM * WGN * 64;
   constexpr int WTM = BM / WGM, WTN = BN / WGN; // wave tile
   constexpr int TM = WTM / 32, TN = WTN / 32;   // MFMA tiles per wave
@@ -80,7 +90,7 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   // on an XCD share a few A panels and Bp panels.
   int pid = blockIdx.x;
   {
-    const int nb = gridDim.x;
+    const int nb = tiles_m * tiles_n;
     const int per = nb >> 3;
     if (per > 0 && pid < per * 8)
       pid = (pid & 7) * per + (pid >> 3);
@@ -236,23 +246,18 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
                                       16]);
   };
 
-  // Every load and LDS store below is unconditional (steps past the end are
-  // clamped to the last step and their data is never consumed): with no
-  // branch around a load the compiler can wait for exactly the register set
-  // it is about to store and leave the other set's loads in flight.
   const int kfirst = SPLIT ? (int)blockIdx.y * ks.steps : 0; // in steps
   const int KT = SPLIT && ks.steps < KTs - kfirst ? ks.steps : KTs - kfirst;
   auto kclamp = [&](int step) {
     return (kfirst + (step < KT ? step : KT - 1)) * BK;
   };
-  // (The registers of a step past the last one hold that step again, and may
-  // be masked again or not: nobody reads them.)
-  const int ktail =
-      (A_LOAD == kLoadAny && (K & (BK - 1)) != 0 && kfirst + KT == KTs) ? KT - 1 : -1;
+  // The block's last step holds the end of the rows and is not a whole one.
+  const bool tail =
+      A_LOAD == kLoadAny && (K & (BK - 1)) != 0 && kfirst + KT == KTs;
   v4i ra0[CH_A], rb0[CH_B], ra1[CH_A], rb1[CH_B];
   load_global(kclamp(0), ra0, rb0);
   load_global(kclamp(1), ra1, rb1);
-  store_lds(0, ra0, rb0, ktail == 0);
+  store_lds(0, ra0, rb0, tail && KT == 1);
   load_global(kclamp(2), ra0, rb0);
   lds_barrier();
 
@@ -261,15 +266,13 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
   // wave finished reading that one before the last barrier --, refill those
   // registers two steps ahead, then run the MFMAs of both half steps.  RS is
   // whether row sums of A are needed, fixed outside the loop so that the loop
-  // body has no branch.
-  auto k_step = [&](int buf, v4i(&ra)[CH_A], v4i(&rb)[CH_B], int kt,
-                    auto RS) {
+  // body has no branch; `stage` is what the step does for those after it.
+  auto k_step = [&](int buf, auto RS, auto stage) {
     v4i fa0[TM], fb0[TN], fa1[TM], fb1[TN];
     read_frags(buf, 0, fa0, fb0);
     read_frags(buf, 1, fa1, fb1);
     __builtin_amdgcn_sched_barrier(0);
-    store_lds(buf ^ 1, ra, rb, kt + 1 == ktail);
-    load_global(kclamp(kt + 3), ra, rb);
+    stage();
     __builtin_amdgcn_sched_barrier(0);
     const v4i flip = {(int)0x80808080, (int)0x80808080, (int)0x80808080,
         (int)0x80808080};
@@ -302,18 +305,46 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
       for (int j = 0; j < TN; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
             fa1[i], fb1[j], acc[i][j], 0, 0, 0);
-    lds_barrier();
   };
+  // The last two steps stand apart: what stages the last tile may have to mask
+  // it, and what computes the last one stages nothing.  In between every load
+  // and LDS store is unconditional (one load past the end is clamped to the
+  // last step and its data never consumed): with no branch in the loop the
+  // compiler can wait for exactly the register set that it is about to store
+  // and leave the other set's loads in flight.  (With the mask under a branch in
+  // every step, in us: 300 x 777 x 1001 7.2 against 6.5, 1000 x 1001 x 3000 with
+  // row sums 11.7 / 11.3, 5000 x 333 x 2002 17.6 / 17.0, 4099 x 777 x 1001 with
+  // row sums 14.0 / 13.7.)
   auto k_loop = [&](auto RS) {
+    auto stage = [&](int buf, int kt, v4i(&ra)[CH_A], v4i(&rb)[CH_B]) {
+      store_lds(buf ^ 1, ra, rb, false);
+      load_global(kclamp(kt + 3), ra, rb);
+    };
     int kt = 0;
-    while (true) {
-      k_step(0, ra1, rb1, kt, RS);
-      if (++kt >= KT)
+    while (kt < KT - 2) {
+      k_step(0, RS, [&] { stage(0, kt, ra1, rb1); });
+      lds_barrier();
+      ++kt;
+      if (kt >= KT - 2)
         break;
-      k_step(1, ra0, rb0, kt, RS);
-      if (++kt >= KT)
-        break;
+      k_step(1, RS, [&] { stage(1, kt, ra0, rb0); });
+      lds_barrier();
+      ++kt;
     }
+    if (kt < KT - 1) {
+      if (kt & 1) {
+#pragma unroll
+        for (int h = 0; h < CH_A; ++h)
+          ra1[h] = ra0[h];
+#pragma unroll
+        for (int h = 0; h < CH_B; ++h)
+          rb1[h] = rb0[h];
+      }
+      k_step(kt & 1, RS, [&] { store_lds((kt & 1) ^ 1, ra1, rb1, tail); });
+      lds_barrier();
+      ++kt;
+    }
+    k_step(kt & 1, RS, [] {});
   };
   if (need_rs)
     k_loop(std::true_type{});
@@ -356,11 +387,16 @@ __global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(
 // with 8-bit results 24.5 / 25.8).
 template <int BN, int NSTAGE, int MINB, int A_MODE, int EPI, bool RAGGED,
     bool SPLIT = false>
-__global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
-    const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    int K, int Kpad, EpiParams ep, int tiles_m, int tiles_n, KSplit ks = {}) {
+__global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(TileArgs args) {
   // 2 x 2 waves, each a 64 x (BN/2) tile.
-  constexpr int BM = 128, WTM = 64, WTN = BN / 2, TM = 2, TN = WTN / 32;
+  constexpr int BM = 128;
+  const uint8_t *__restrict__ A = args.A;
+  const int8_t *__restrict__ Bp = args.Bp;
+  const int M = args.M, N = args.N, K = args.K, Kpad = padded_k(K);
+  const int tiles_m = tiles_of(M, BM), tiles_n = tiles_of(N, BN);
+  const EpiParams ep = unpack_epi<EPI>(args.epi);
+  const KSplit ks = {args.steps, part_stride(M, N)};
+  constexpr int WTM = 64, WTN = BN / 2, TM = 2, TN = WTN / 32;
   static_assert(BN == 128 || BN == 64, "tile width");
   constexpr int STAGE = (BM + BN) * BK;
   constexpr int CB = BN / 64;      // Bp copies per wave and step
@@ -369,7 +405,7 @@ __global__ __launch_bounds__(256, MINB) void k_gemm_i8_dma(
 
   int pid = blockIdx.x;
   {
-    const int nb = gridDim.x;
+    const int nb = tiles_m * tiles_n;
     const int per = nb >> 3;
     if (per > 0 && pid < per * 8)
       pid = (pid & 7) * per + (pid >> 3);
@@ -766,10 +802,22 @@ thread_local bool t_limits_written = false;
 // after the one before, with the epilogue of a product: 4 consecutive elements
 // of the result per thread.  Bound by the launch and by reading the arrays,
 // which were written a moment ago (at most 256 tiles of 64 KB).
+struct SumArgs {
+  const int32_t *in;
+  int parts;
+  unsigned n, N;
+  bool vector_out;
+  PackedEpi epi;
+};
+static_assert(cheap_arguments(sizeof(SumArgs), 0));
 template <int EPI>
-__global__ __launch_bounds__(256) void k_sum_parts(
-    const int32_t *__restrict__ in, int parts, int64_t stride, unsigned n,
-    unsigned N, EpiParams ep, bool vector_out) {
+__global__ __launch_bounds__(256) void k_sum_parts(SumArgs args) {
+  const int32_t *__restrict__ in = args.in;
+  const int parts = args.parts;
+  const unsigned n = args.n, N = args.N;
+  const int64_t stride = part_stride(1, n);
+  const bool vector_out = args.vector_out;
+  const EpiParams ep = unpack_epi<EPI>(args.epi);
   typedef uint32_t u4 __attribute__((ext_vector_type(4)));
   const unsigned o = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (o >= n)
@@ -915,18 +963,18 @@ double product_us(const Sizes &p, GemmSplit &best) {
   }
   return least;
 }
-// And in k_gemm_i8, for any K: tiles of 128 x 128 and of 64 x 128, four blocks of
+// And in k_gemm_i8, for any K: tiles of 128 x 128 and of 64 x 128, three blocks of
 // which run on a CU and are dealt out more evenly; the model of kTileCosts, fitted
-// to 662 products of awkward rows timed in both tiles, split and with their rows
-// copied (profiles/awkward_row_times.csv): the choice between these is 0.9 %
-// above always taking the fastest.  Int32 4099 x 777 x 1001 16.1 us in the larger,
-// 14.4 in the smaller, 1618 x 653 x 311 8.6 / 6.8; u8 3694 x 278 x 4295 17.5 / 21.3, u8
-// 575 x 948 x 8448 14.8 / 16.8.
+// to 322 products of awkward rows timed in both tiles
+// (profiles/awkward_tile_times.csv): the choice between these is 0.1 % above always
+// taking the fastest.  Int32 4099 x 777 x 1001 14.8 us in the larger, 13.6 in the
+// smaller, 1618 x 653 x 311 8.2 / 5.9; u8 3694 x 278 x 4295 17.6 / 18.4, u8
+// 575 x 948 x 8448 14.2 / 14.6.
 double any_us(bool low, const Sizes &p) {
-  static constexpr TileCost t128 = {kT128x128, 128, 128, 1, 0.385, 0.335, 0.233,
-      2.701, 3.079, 1.973, 0.402};
-  static constexpr TileCost t64 = {kT128x128, 64, 128, 1, 0.263, 0.188, 0.140,
-      1.502, 1.569, 2.645, 0.496};
+  static constexpr TileCost t128 = {kT128x128, 128, 128, 1, 0.393, 0.232, 0.290,
+      2.646, 3.096, 1.674, 0.660};
+  static constexpr TileCost t64 = {kT128x128, 64, 128, 1, 0.268, 0.160, 0.242,
+      1.222, 1.451, 1.973, 0.467};
   return tile_us(low ? t64 : t128, p);
 }
 bool any_takes_64_rows(const Sizes &p) {
@@ -966,12 +1014,9 @@ const char *dma_name(bool narrow, bool ragged) {
 }
 
 template <int A_MODE, int EPI>
-hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
-    int Kpad) {
+hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   const GemmSplit &p = g.split;
-  const uint8_t *A = (const uint8_t *)g.A;
-  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
-  const KSplit ks = {p.steps, part_stride(g)};
+  const int M = (int)g.M, N = (int)g.N;
   EpiParams pe = ep;
   pe.out = g.parts;
   hipError_t e;
@@ -988,14 +1033,11 @@ hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
                              : "k_gemm_i8_dma (128x128 tiles, split along K)";
     if (p.kernel == kSplitAny)
       k_gemm_i8<128, 128, 2, 2, 2, A_MODE, kEpiI32, kLoadAny, true>
-          <<<grid, 256, 0, st>>>(
-              A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+          <<<grid, 256, 0, st>>>(tile_args(g, pe, kEpiI32));
     else if (narrow)
-      k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, false, true><<<grid, 256, 0, st>>>(
-          A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+      k_gemm_i8_dma<64, 3, 3, A_MODE, kEpiI32, false, true><<<grid, 256, 0, st>>>(tile_args(g, pe, kEpiI32));
     else
-      k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, false, true><<<grid, 256, 0, st>>>(
-          A, g.Bp, M, N, K, Kpad, pe, tiles_m, tiles_n, ks);
+      k_gemm_i8_dma<128, 3, 3, A_MODE, kEpiI32, false, true><<<grid, 256, 0, st>>>(tile_args(g, pe, kEpiI32));
     e = hipGetLastError();
   }
   if (e != hipSuccess)
@@ -1003,17 +1045,16 @@ hipError_t launch_split(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
   const unsigned n = (unsigned)(g.M * g.N);
   const bool vec = (((uintptr_t)g.out) & (EPI == kEpiQ8 ? 3 : 15)) == 0;
   k_sum_parts<EPI><<<(n + 1023) / 1024, 256, 0, st>>>(
-      g.parts, p.parts, ks.stride, n, (unsigned)N, ep, vec);
+      SumArgs{g.parts, p.parts, n, (unsigned)N, vec, pack_epi(ep, EPI)});
   return hipGetLastError();
 }
 
 // k_gemm_i8_dma in tiles of 128 columns or, for cfg = kD128x64, of 64.
 template <int A_MODE, int EPI>
 hipError_t launch_dma(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
-    int Kpad, int cfg) {
+    int cfg) {
   const int tiles_m = (int)((g.M + 127) / 128);
-  const uint8_t *A = (const uint8_t *)g.A;
-  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
+  const int N = (int)g.N, K = (int)g.K;
   const bool narrow = cfg == kD128x64, ragged = K % BK != 0;
   const int tiles_n = narrow ? (N + 63) / 64 : (N + 127) / 128;
   t_last_kernel = dma_name(narrow, ragged);
@@ -1022,17 +1063,14 @@ hipError_t launch_dma(hipStream_t st, const GemmArgs &g, const EpiParams &ep,
                        : k_gemm_i8_dma<64, 3, 3, A_MODE, EPI, false>)
              : (ragged ? k_gemm_i8_dma<128, 3, 3, A_MODE, EPI, true>
                        : k_gemm_i8_dma<128, 3, 3, A_MODE, EPI, false>);
-  kernel<<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(
-      A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n, KSplit{});
+  kernel<<<dim3((unsigned)(tiles_m * tiles_n)), 256, 0, st>>>(tile_args(g, ep, EPI));
   return hipGetLastError();
 }
 
 template <int A_MODE, int EPI>
 hipError_t gemm_launch_cfg(
-    hipStream_t st, const GemmArgs &g, const EpiParams &ep, int Kpad) {
+    hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
-  const uint8_t *A = (const uint8_t *)g.A;
-  const int M = (int)g.M, N = (int)g.N, K = (int)g.K;
   if (g.X) {
     // rows quantized inside the kernel (the caller asked gemm_quantizes_rows)
     if (A_MODE != 2 || !gemm_quantizes_rows(g.M, g.K, g.N, g.X))
@@ -1054,7 +1092,7 @@ hipError_t gemm_launch_cfg(
   if (skinny_ok(g.M, g.K) && !(force && force[0]))
     return launch_gemm_skinny(st, g, ep, A_MODE);
   if (g.parts && g.split.parts > 1)
-    return launch_split<A_MODE, EPI>(st, g, ep, Kpad);
+    return launch_split<A_MODE, EPI>(st, g, ep);
   const int tiles_m = (int)((g.M + 127) / 128);
   const int tiles_n128 = (int)((g.N + 127) / 128);
   if (!gemm_fast_path(g.M, g.K, g.A)) {
@@ -1066,21 +1104,18 @@ hipError_t gemm_launch_cfg(
     const int tiles_m64 = (int)((g.M + 63) / 64);
     if (low)
       k_gemm_i8<64, 128, 2, 2, 4, A_MODE, EPI, kLoadAny>
-          <<<dim3((unsigned)(tiles_m64 * tiles_n128)), 256, 0, st>>>(
-              A, g.Bp, M, N, K, Kpad, ep, tiles_m64, tiles_n128);
+          <<<dim3((unsigned)(tiles_m64 * tiles_n128)), 256, 0, st>>>(tile_args(g, ep, EPI));
     else if (g.M * g.K >= 16)
       k_gemm_i8<128, 128, 2, 2, 2, A_MODE, EPI, kLoadAny>
-          <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(
-              A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n128);
+          <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(tile_args(g, ep, EPI));
     else
       k_gemm_i8<128, 128, 2, 2, 2, A_MODE, EPI, kLoadBytes>
-          <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(
-              A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n128);
+          <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(tile_args(g, ep, EPI));
     return hipGetLastError();
   }
   const int cfg = choose_tile(sizes_of(g));
   if (g.K % 64 != 0 && cfg != kB64x256 && cfg != kB64x128)
-    return launch_dma<A_MODE, EPI>(st, g, ep, Kpad,
+    return launch_dma<A_MODE, EPI>(st, g, ep,
         cfg == kD128x64 || cfg == kD128x128 ? cfg : (int)kD128x128);
   // One round of blocks with everything requested at once: small problems,
   // where a pipelined K loop would pay the memory latency step after step
@@ -1108,20 +1143,19 @@ hipError_t gemm_launch_cfg(
                         : cfg == kB64x256 ? kBs64x256
                                           : kBs64x128;
     if (!bs_ok(g, tile)) // (forced, on a K this kernel does not take)
-      return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x128);
+      return launch_dma<A_MODE, EPI>(st, g, ep, kD128x128);
     return launch_gemm_bs(st, g, ep, A_MODE, tile);
   }
   case kD128x64:
-    return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x64);
+    return launch_dma<A_MODE, EPI>(st, g, ep, kD128x64);
   case kW128x384: // (forced, on a shape that kernel does not take)
   case kFlight:
   case kD128x128:
-    return launch_dma<A_MODE, EPI>(st, g, ep, Kpad, kD128x128);
+    return launch_dma<A_MODE, EPI>(st, g, ep, kD128x128);
   default:
     t_last_kernel = "k_gemm_i8 (128x128 tiles through registers)";
     k_gemm_i8<128, 128, 2, 2, 3, A_MODE, EPI, kLoadAligned>
-        <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(
-            A, g.Bp, M, N, K, Kpad, ep, tiles_m, tiles_n128);
+        <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(tile_args(g, ep, EPI));
     break;
   }
   return hipGetLastError();
@@ -1129,14 +1163,14 @@ hipError_t gemm_launch_cfg(
 
 template <int A_MODE>
 hipError_t gemm_launch_epi(
-    hipStream_t st, const GemmArgs &g, const EpiParams &ep, int Kpad) {
+    hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   switch (g.epi) {
   case kEpiI32:
-    return gemm_launch_cfg<A_MODE, kEpiI32>(st, g, ep, Kpad);
+    return gemm_launch_cfg<A_MODE, kEpiI32>(st, g, ep);
   case kEpiF32:
-    return gemm_launch_cfg<A_MODE, kEpiF32>(st, g, ep, Kpad);
+    return gemm_launch_cfg<A_MODE, kEpiF32>(st, g, ep);
   default:
-    return gemm_launch_cfg<A_MODE, kEpiQ8>(st, g, ep, Kpad);
+    return gemm_launch_cfg<A_MODE, kEpiQ8>(st, g, ep);
   }
 }
 
@@ -1275,7 +1309,6 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
   if (g.M > INT32_MAX || g.N > INT32_MAX || g.K > INT32_MAX ||
       g.M * g.N > ((int64_t)1 << 40))
     return hipErrorInvalidValue;
-  const int Kpad = (int)round_up(g.K > 0 ? g.K : 1, kGemmBK);
   EpiParams ep;
   ep.a_zp = g.a_zp;
   ep.a_zp_len = g.a_zp ? g.a_zp_len : 0;
@@ -1308,13 +1341,13 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs &g) {
   hipError_t e;
   switch (a_mode) {
   case 0:
-    e = gemm_launch_epi<0>(s, g, ep, Kpad);
+    e = gemm_launch_epi<0>(s, g, ep);
     break;
   case 1:
-    e = gemm_launch_epi<1>(s, g, ep, Kpad);
+    e = gemm_launch_epi<1>(s, g, ep);
     break;
   default:
-    e = gemm_launch_epi<2>(s, g, ep, Kpad);
+    e = gemm_launch_epi<2>(s, g, ep);
     break;
   }
   if (e == hipSuccess && g.y_limits && !t_limits_written)

@@ -109,11 +109,24 @@ constexpr int wreg_younger(int s, int pf, int fix_ops, int fix_read, int fix_wri
 
 // LIM: minimum and maximum of the (f32) results are kept per lane while they
 // are stored and reduced over the grid when the block ends (EpiParams::limits).
+// LIM: minimum and maximum of the results are asked for.
+template <bool LIM>
+struct WregArgs {
+  const uint8_t *A;
+  const int8_t *Bp;
+  int M, N;
+  std::conditional_t<LIM, EpiParams, PackedEpi> epi;
+};
+static_assert(cheap_arguments(sizeof(WregArgs<false>), 0));
 template <int KH, int WAVES, int NR, int A_MODE, int EPI, bool STREAM, int ACT,
     bool LIM = false>
-__global__ __launch_bounds__(WAVES * 64, 1) void k_gemm_i8_wreg(
-    const uint8_t *__restrict__ A, const int8_t *__restrict__ Bp, int M, int N,
-    EpiParams ep, int regions_m, int regions_n, int bp_tiles) {
+__global__ __launch_bounds__(WAVES * 64, 1) void k_gemm_i8_wreg(WregArgs<LIM> args) {
+  const uint8_t *__restrict__ A = args.A;
+  const int8_t *__restrict__ Bp = args.Bp;
+  const int M = args.M, N = args.N;
+  const EpiParams ep = unpack_epi<EPI>(args.epi);
+  const int regions_m = tiles_of(M, 32 * NR), regions_n = tiles_of(N, 32 * WAVES);
+  const int bp_tiles = tiles_of(N, kGemmBN) * (kGemmBN / 32);
   constexpr int K = 32 * KH;
   constexpr int CPR = K / 16;           // 16-byte chunks per row of A
   constexpr int CPT = KH / WAVES;       // copy instructions per wave and tile
@@ -166,7 +179,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void k_gemm_i8_wreg(
   // panels of A and of Bp.
   int pid = blockIdx.x;
   {
-    const int nb = gridDim.x;
+    const int nb = regions_m * regions_n;
     const int per = nb >> 3;
     if (per > 0 && pid < per * 8)
       pid = (pid & 7) * per + (pid >> 3);
@@ -621,7 +634,6 @@ hipError_t wreg_launch(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
   const int regions_m = (int)((g.M + 32 * kWregNR - 1) / (32 * kWregNR));
   const int ntiles = (int)((g.N + 31) / 32);
   const int regions_n = (ntiles + kWregWaves - 1) / kWregWaves;
-  const int bp_tiles = (int)(round_up(g.N, kGemmBN) / 32);
   // Minimum and maximum of the results (EpiParams::limits) are taken in the
   // kernel for the f32 results of a fused layer (its activations arrive
   // stored minus 128: A_MODE 2); elsewhere a pass over y takes them.
@@ -629,13 +641,13 @@ hipError_t wreg_launch(hipStream_t st, const GemmArgs &g, const EpiParams &ep) {
     if (ep.limits.out != nullptr) {
       k_gemm_i8_wreg<kWregKH, kWregWaves, kWregNR, A_MODE, EPI, true, ACT, true>
           <<<dim3((unsigned)(regions_m * regions_n)), dim3(kWregWaves * 64), 0, st>>>(
-              (const uint8_t *)g.A, g.Bp, M, N, ep, regions_m, regions_n, bp_tiles);
+              WregArgs<true>{(const uint8_t *)g.A, g.Bp, M, N, ep});
       return hipGetLastError();
     }
   }
   k_gemm_i8_wreg<kWregKH, kWregWaves, kWregNR, A_MODE, EPI, true, ACT>
       <<<dim3((unsigned)(regions_m * regions_n)), dim3(kWregWaves * 64), 0, st>>>(
-          (const uint8_t *)g.A, g.Bp, M, N, ep, regions_m, regions_n, bp_tiles);
+          WregArgs<false>{(const uint8_t *)g.A, g.Bp, M, N, pack_epi(ep, EPI)});
   return hipGetLastError();
 }
 

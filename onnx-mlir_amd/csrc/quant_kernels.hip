@@ -1749,12 +1749,30 @@ constexpr int64_t kGridPrefixMost = (int64_t)192 << 20;
 // PREFIX: tensors beyond kGridMaxPerThread.  The first `prefix` float4 are only reduced, the
 // ones after them (NV per thread of the grid) are kept and quantized as above;
 // the launcher quantizes the prefix with a launch of its own.
+struct DqlGridArgs { // (one structure: see cheap_arguments in gemm_common.h)
+  const float *x;
+  uint8_t *y;
+  int64_t n, prefix;
+  float *scale_out;
+  uint8_t *zp_out;
+  unsigned long long *slots;
+  unsigned *failed;
+  uint32_t flip;
+  unsigned blocks, epoch, spin_limit;
+};
+static_assert(sizeof(DqlGridArgs) <= 112);
 template <int NV, bool PREFIX>
-__global__ __launch_bounds__(kGridThreads) void k_dql_grid(
-    const float *__restrict__ x, int64_t n, int64_t prefix, uint8_t *__restrict__ y,
-    float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, uint32_t flip,
-    unsigned long long *slots, unsigned epoch, unsigned *failed,
-    unsigned spin_limit) {
+__global__ __launch_bounds__(kGridThreads) void k_dql_grid(DqlGridArgs args) {
+  const float *__restrict__ x = args.x;
+  uint8_t *__restrict__ y = args.y;
+  int64_t n = args.n;
+  const int64_t prefix = args.prefix;
+  float *__restrict__ scale_out = args.scale_out;
+  uint8_t *__restrict__ zp_out = args.zp_out;
+  unsigned long long *const slots = args.slots;
+  unsigned *const failed = args.failed;
+  const uint32_t flip = args.flip;
+  const unsigned nblocks = args.blocks, epoch = args.epoch, spin_limit = args.spin_limit;
   constexpr int kWaves = kGridThreads / 64;
   __shared__ float s_lo[kWaves], s_hi[kWaves];
   __shared__ int s_ok;
@@ -1766,7 +1784,7 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
     constexpr int kMU = 3;
     const f4a *__restrict__ x4 = (const f4a *)x;
     for (int64_t base = (int64_t)blockIdx.x * (kGridThreads * kMU); base < prefix;
-         base += (int64_t)gridDim.x * (kGridThreads * kMU)) {
+         base += (int64_t)nblocks * (kGridThreads * kMU)) {
       f4a q[kMU];
 #pragma unroll
       for (int j = 0; j < kMU; ++j) {
@@ -1792,7 +1810,7 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
   // last whole float4 is not read (zeros, which are neutral: the range that
   // DynamicQuantizeLinear takes always includes 0) and not written, and no
   // register holds an address or an index.
-  const unsigned total = gridDim.x * kGridThreads;
+  const unsigned total = nblocks * kGridThreads;
   const unsigned gtid = blockIdx.x * kGridThreads + threadIdx.x;
   const unsigned xbytes = (unsigned)(nvec * 16);
   // (The scalar offset is kept within the descriptor's size, from which the
@@ -1871,7 +1889,7 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
   bool ok = true;
   lo = __builtin_inff();
   hi = -__builtin_inff();
-  for (unsigned i = threadIdx.x; i < gridDim.x; i += kGridThreads) {
+  for (unsigned i = threadIdx.x; i < nblocks; i += kGridThreads) {
     u64x2 w = {0, 0};
     bool got = false;
     for (unsigned spin = 0; spin < spin_limit; ++spin) {
@@ -1890,8 +1908,8 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_grid(
     hi = __builtin_fmaxf(hi, __uint_as_float((unsigned)w.y));
   }
   // only the waves that had a slot to poll take part in the fold
-  const unsigned pollers = gridDim.x < (unsigned)kGridThreads
-                               ? (gridDim.x + 63) / 64
+  const unsigned pollers = nblocks < (unsigned)kGridThreads
+                               ? (nblocks + 63) / 64
                                : (unsigned)kWaves;
   if ((threadIdx.x >> 6) < pollers) {
     lo = wave_min(lo);
@@ -1955,7 +1973,7 @@ constexpr int kGridReported = 32;
 __global__ __launch_bounds__(kGridThreads) void k_dql_repair(
     const float *__restrict__ x, int64_t n, uint8_t *__restrict__ y,
     float *__restrict__ scale_out, uint8_t *__restrict__ zp_out, uint32_t flip,
-    const unsigned *failed, unsigned epoch) {
+    const unsigned *failed, unsigned epoch, unsigned blocks) {
   if (*failed != epoch)
     return;
   constexpr int kWaves = kGridThreads / 64, kUnroll = 8;
@@ -2003,7 +2021,7 @@ __global__ __launch_bounds__(kGridThreads) void k_dql_repair(
   }
   const float recip = 1.0f / scale;
   for (int64_t i = (int64_t)blockIdx.x * kGridThreads + threadIdx.x; i < nvec;
-       i += (int64_t)gridDim.x * kGridThreads)
+       i += (int64_t)blocks * kGridThreads)
     ((uint32_t *)y)[i] =
         quant_four<false, true, false>(x4[i], scale, recip, zpf, flip);
   if (blockIdx.x == 0 && te < n)
@@ -2546,9 +2564,7 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
       ((((uintptr_t)y) & 3) == 0)) {
     const int64_t total = (int64_t)scratch.grid_blocks * kGridThreads;
     const int64_t nvec = n >> 2;
-    void (*fn_launch)(const float *, int64_t, int64_t, uint8_t *, float *, uint8_t *,
-        uint32_t, unsigned long long *, unsigned, unsigned *, unsigned) =
-        nullptr;
+    void (*fn_launch)(DqlGridArgs) = nullptr;
     // Up to two float4 per thread of the whole grid the launch takes only as
     // many blocks as that needs: the fewer blocks, the shorter the exchange
     // (64 Ki elements: 16 blocks 5.4 us, 4 blocks of 4 float4 per thread 7.0,
@@ -2580,8 +2596,8 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
         const bool repaired = nvec > kGridReported * total;
         unsigned *const failed = repaired ? ex.repaired : ex.failed;
         hipLaunchKernelGGL(fn_launch, dim3((unsigned)blocks),
-            dim3(kGridThreads), 0, s, x, n, prefix, y, scale, zp, flip, ex.slots,
-            ex.epoch, failed, ex.spin_limit);
+            dim3(kGridThreads), 0, s, DqlGridArgs{x, y, n, prefix, scale, zp, ex.slots,
+            failed, flip, (unsigned)blocks, ex.epoch, ex.spin_limit});
         hipError_t e = hipGetLastError();
         const bool launched = e == hipSuccess;
         // (If a block gave up, the front is quantized with parameters that were
@@ -2591,7 +2607,7 @@ hipError_t launch_dynamic_quantize(hipStream_t s, DqlScratch &scratch,
               s, x, 1, 1, prefix * 4, scale, zp, y, flip);
         if (e == hipSuccess && repaired) {
           k_dql_repair<<<scratch.grid_blocks, kGridThreads, 0, s>>>(
-              x, n, y, scale, zp, flip, failed, ex.epoch);
+              x, n, y, scale, zp, flip, failed, ex.epoch, scratch.grid_blocks);
           e = hipGetLastError();
         }
         dql_exchange_end(s, launched);

@@ -20,7 +20,8 @@ def kernels():
 
 
 @pytest.mark.parametrize("name", ["k_gemm_i8_skinnyI", "k_gemm_i8_batched_flatI", "k_quant_flatI", "k_quant_tiledI", "k_quant_lastaxisI",
-                                  "k_quant_gatherI", "k_dequant8_flatI", "k_dequant8_gatherI", "k_dql_small"])
+                                  "k_quant_gatherI", "k_dequant8_flatI", "k_dequant8_gatherI", "k_dql_small",
+                                  "k_gemm_i8I", "k_gemm_i8_dmaI", "k_gemm_i8_bsI", "k_gemm_i8_dma_bsI", "k_sum_partsI", "k_dql_gridI", "k_dql_repair"])
 def test_short_kernels_are_cheap_to_launch(kernels, name):
     forms = [k for k in kernels if name in k[".name"]]
     assert forms
