@@ -36,6 +36,7 @@
 //   masks only in the steps that the end of K lies in (with them, and 64-bit
 //   addresses, in every load: 88 x 472x472x128 19.0 us, so 13.2; 56 x 293x293x80 11.8
 //   / 8.7; 64 x 511x511x64 13.5 / 9.2; aligned rows 88 x 480x480x128 12.4 / 11.5).
+#include "gemm_batched_out.h"
 #include "gemm_common.h"
 #include "gemm_epilogue.h"
 
@@ -108,19 +109,15 @@ __device__ __forceinline__ BatchParams expand(const FlatBatch &f, const PackedEp
 template <int ES>
 __device__ __forceinline__ void tile_out(const uint8_t *lds, char *to, int bytes) {
   typedef unsigned u4 __attribute__((ext_vector_type(4)));
-  const int skew = (int)(uintptr_t)to & 15;
+  const TilePieces p = tile_pieces((int)(uintptr_t)to & 15, bytes);
   const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc(to - skew, 0, skew + bytes, 0x00020000);
+      __builtin_amdgcn_make_buffer_rsrc(to - p.skew, 0, p.end, 0x00020000);
   const int tid = (int)threadIdx.x;
-  const int first = skew ? 16 : 0, last = (skew + bytes) & ~15; // whole pieces
-  for (int o = first + tid * 16; o < last; o += 256 * 16)
+  for (int o = p.first + tid * 16; o < p.last; o += 256 * 16)
     __builtin_amdgcn_raw_buffer_store_b128(
         *(const u4 *)(lds + o), rsrc, o, 0, kAuxThrough);
-  // the ends, one result to a thread: PER threads in front, the next PER behind
-  constexpr int PER = 16 / ES;
-  const int o = tid < PER ? skew + tid * ES
-                          : (last > first ? last : first) + (tid - PER) * ES;
-  if (tid < 2 * PER && o < skew + bytes && (tid >= PER || o < first)) {
+  const int o = tile_end<ES>(p, tid);
+  if (o >= 0) {
     if constexpr (ES == 4)
       __builtin_amdgcn_raw_buffer_store_b32(*(const int *)(lds + o), rsrc, o, 0, 0);
     else
@@ -151,8 +148,7 @@ __device__ __forceinline__ void rows_out(
 
 // ALIGNED: K % 16 == 0 with A on a 16-byte boundary and N % 4 == 0 with B on a
 // 4-byte one, so that every load is whole and inside its row.
-// OUT: how results leave, chosen by out_form.
-enum OutForm : int { kOutDirect, kOutTile, kOutRows };
+// OUT: how results leave, chosen by out_form (gemm_batched_out.h).
 template <int BN, int EPI, bool ALIGNED, int OUT>
 __device__ __forceinline__ void batched_tile(
     const BatchParams &bp, const EpiParams &ep) {
@@ -496,26 +492,6 @@ __global__ __launch_bounds__(256, (kBlocksPerCu<BN, ALIGNED>)) void k_gemm_i8_ba
   batched_tile<BN, EPI, ALIGNED, OUT>(expand(fb, pe, BN), unpack_epi<EPI>(pe));
 }
 
-// By way of LDS where rows are no whole lines and the grid is more than one round of
-// blocks: up to that the barrier and the second way cost more than the stores (48 x
-// 38x38x80 4.74 us by LDS, 4.57 without).
-//   Tiles as wide as the matrix: 156 x 82x128x82 7.6 -> 6.8 us, 64 x 511x511x64 with 8-bit
-//   results 13.9 -> 9.6, the loads' part of both included.
-//   Rows of whole 16-byte pieces: int32 88 x 472x128x472 28.8 -> 23.4; not 8-bit ones (21.2
-//   -> 23.5), nor other rows, whose ends are stores of their own (64 x 511x64x511 17.2
-//   -> 18.5).
-template <int EPI>
-OutForm out_form(const BatchParams &bp, const EpiParams &ep, int64_t blocks) {
-  constexpr int ES = EPI == kEpiQ8 ? 1 : 4;
-  if (blocks <= 256 || bp.N * ES % 128 == 0)
-    return kOutDirect;
-  if (bp.tiles_n == 1)
-    return kOutTile;
-  return EPI == kEpiI32 && ((((uintptr_t)ep.out) | (uintptr_t)(bp.N * 4)) & 15) == 0
-             ? kOutRows
-             : kOutDirect;
-}
-
 template <int BN, int EPI, bool ALIGNED, int OUT>
 void launch_out(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
     const FlatBatch *flat) {
@@ -531,7 +507,8 @@ void launch_out(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
 template <int BN, int EPI, bool ALIGNED>
 void launch_form(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
     const FlatBatch *flat) {
-  const OutForm out = out_form<EPI>(bp, ep, bp.blocks);
+  const OutForm out = out_form(
+      EPI == kEpiQ8 ? 1 : 4, bp.N, bp.tiles_n, (uint64_t)(uintptr_t)ep.out, bp.blocks);
   if (out == kOutTile)
     launch_out<BN, EPI, ALIGNED, kOutTile>(s, bp, ep, flat);
   else if (out == kOutDirect)

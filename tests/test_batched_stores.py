@@ -1,23 +1,66 @@
 """How k_gemm_i8_batched reads and writes rows of any length (gemm_batched.hip):
 a grid of more than one round of blocks, operands and results at odd addresses up
 to the last byte of their buffers, results next to memory that must stay as it is;
-and the pieces in which a tile leaves LDS, restated for the CPU."""
+and the pieces in which a tile leaves LDS (gemm_batched_out.h, built for the host)."""
+import ctypes
+import os
+import subprocess
+
 import numpy as np
 import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "onnx-mlir_amd", "csrc")
+DIRECT, TILE, ROWS = 0, 1, 2  # OutForm
+
+
+@pytest.fixture(scope="module")
+def out(tmp_path_factory):
+    """What a launch and a block ask gemm_batched_out.h."""
+    folder = tmp_path_factory.mktemp("out")
+    (folder / "out.cpp").write_text("""
+#include "gemm_batched_out.h"
+using namespace om::gemm;
+extern "C" {
+int form(int result, int N, int tiles_n, uint64_t out, int64_t blocks) { return out_form(result, N, tiles_n, out, blocks); }
+int first(int skew, int bytes) { return tile_pieces(skew, bytes).first; }
+int last(int skew, int bytes) { return tile_pieces(skew, bytes).last; }
+int end1(int skew, int bytes, int tid) { return tile_end<1>(tile_pieces(skew, bytes), tid); }
+int end4(int skew, int bytes, int tid) { return tile_end<4>(tile_pieces(skew, bytes), tid); }
+}
+""")
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, "-o", str(folder / "out.so"), str(folder / "out.cpp")])
+    lib = ctypes.CDLL(str(folder / "out.so"))
+    lib.form.argtypes = [ctypes.c_int] * 3 + [ctypes.c_uint64, ctypes.c_int64]
+    return lib
+
+
+def test_how_results_leave(out):
+    """One by one up to 256 blocks, where rows are whole lines, where the first result
+    does not start on a multiple of its size."""
+    at = 1 << 40
+    for N in (1, 7, 33, 63, 100, 127):
+        tiles_n = 1
+        assert out.form(4, N, tiles_n, at, 257) == TILE and out.form(4, N, tiles_n, at, 256) == DIRECT
+        for off in range(1, 16):
+            assert out.form(4, N, tiles_n, at + off, 300) == (DIRECT if off % 4 else TILE), off
+            assert out.form(1, N, tiles_n, at + off, 300) == TILE
+    assert out.form(4, 64, 1, at, 300) == out.form(1, 128, 1, at, 300) == out.form(4, 160, 2, at, 300) == DIRECT
+    assert [out.form(4, N, 2, at, 300) for N in (132, 133, 134, 196)] == [ROWS, DIRECT, DIRECT, ROWS]
+    assert all(out.form(4, 132, 2, at + off, 300) == DIRECT for off in range(1, 16)) and out.form(1, 132, 2, at, 300) == DIRECT
 
 
 @pytest.mark.parametrize("es", [1, 4])
 @pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 64 * 7, 64 * 127, 64 * 100 + 1])
-def test_a_tile_leaves_in_pieces_that_cover_it_once(es, count):
-    """tile_out: aligned pieces of 16 bytes and single results at the two ends."""
-    size, per = count * es, 16 // es
-    for skew in range(0, 16, es):
-        first, last = 16 if skew else 0, (skew + size) & ~15
-        written = [(o, 16) for t in range(256) for o in range(first + t * 16, last, 256 * 16)]
-        for t in range(2 * per):
-            o = skew + t * es if t < per else max(first, last) + (t - per) * es
-            if o < skew + size and (t >= per or o < first):
-                written.append((o, es))
+def test_a_tile_leaves_in_pieces_that_cover_it_once(out, es, count):
+    """tile_out: aligned pieces of 16 bytes and single results at the two ends, from
+    every address that out_form lets through."""
+    size = count * es
+    for skew in range(16):
+        if out.form(es, 63, 1, (1 << 40) + skew, 300) != TILE:
+            continue
+        written = [(o, 16) for t in range(256) for o in range(out.first(skew, size) + t * 16, out.last(skew, size), 256 * 16)]
+        ends = [(out.end1 if es == 1 else out.end4)(skew, size, t) for t in range(256)]
+        written += [(o, es) for o in ends if o >= 0]
         covered = np.zeros(skew + size + 16, int)
         for o, n in written:
             covered[o:o + n] += 1
@@ -65,3 +108,21 @@ def test_many_entries_at_any_address(rt, oracle, count, M, K, N, a_off, b_off, y
             got = whole.numpy()
             assert np.array_equal(got[32 + y_off:32 + y_off + acc.size].reshape(acc.shape), want), (adt, dtype)
             assert (got[:32 + y_off] == 90).all() and (got[32 + y_off + acc.size:] == 90).all(), (adt, dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count,M,K,N", [(300, 5, 16, 7), (260, 64, 63, 100), (130, 65, 32, 132)])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_int32_results_that_start_between_words(rt, oracle, count, M, K, N, off):
+    rng = np.random.default_rng(M + off)
+    a, b = rng.integers(0, 256, (count, M, K), dtype=np.uint8), rng.integers(-128, 128, (count, K, N), dtype=np.int8)
+    want = np.matmul(a.astype(np.int32), b.astype(np.int32))
+    whole = rt.DeviceArray.from_numpy(np.full(want.nbytes + 64, 90, np.uint8))
+    y = rt.DeviceArray.view_of(whole, 32 + off, (want.nbytes,))
+    y.shape, y.dtype, y.size = want.shape, want.dtype, want.size
+    rt.MatMulInteger(rt.DeviceArray.from_numpy(a), rt.DeviceArray.from_numpy(b), None, None, out=y)
+    rt.synchronize()
+    assert rt.last_gemm_kernel() == "k_gemm_i8_batched"
+    got = whole.numpy()
+    assert np.array_equal(got[32 + off:][:want.nbytes].view(np.int32).reshape(want.shape), want)
+    assert (got[:32 + off] == 90).all() and (got[32 + off + want.nbytes:] == 90).all()
