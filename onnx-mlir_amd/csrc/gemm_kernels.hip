@@ -306,40 +306,39 @@ void k_gemm_i8(TileArgs args) {
         acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(
             fa1[i], fb1[j], acc[i][j], 0, 0, 0);
   };
-  // The last two steps stand apart: what stages the last tile may have to mask
-  // it, and what computes the last one stages nothing.  In between every load
-  // and LDS store is unconditional (one load past the end is clamped to the
-  // last step and its data never consumed): with no branch in the loop the
-  // compiler can wait for exactly the register set that it is about to store
-  // and leave the other set's loads in flight.  (With the mask under a branch in
-  // every step, in us: 300 x 777 x 1001 7.2 against 6.5, 1000 x 1001 x 3000 with
-  // row sums 11.7 / 11.3, 5000 x 333 x 2002 17.6 / 17.0, 4099 x 777 x 1001 with
-  // row sums 14.0 / 13.7.)
+  // The last two or three steps stand apart: what stages the last tile may have to
+  // mask it, and what computes the last one stages nothing.  In the loop every load
+  // and LDS store is unconditional (one load past the end is clamped to the last
+  // step and its data never consumed), and the loop has one way out, behind an odd
+  // step: so the compiler waits for exactly the register set that it is about to
+  // store and leaves the other set's loads in flight.  (With a way out between its
+  // two steps, the second waited for the loads of the first as well, in us: f32 109 x
+  // 10959 x 224 59.0 against 39.6, 320 x 10002 x 3584 54.4 / 39.5, int32 4099 x 777 x 1001
+  // with row sums 14.0 / 13.4.  With the mask under a branch in every step, and four
+  // blocks of 64 x 128 a CU: 49.0, 45.9, 14.8.)
   auto k_loop = [&](auto RS) {
-    auto stage = [&](int buf, int kt, v4i(&ra)[CH_A], v4i(&rb)[CH_B]) {
-      store_lds(buf ^ 1, ra, rb, false);
-      load_global(kclamp(kt + 3), ra, rb);
+    auto whole = [&](int buf, int kt, v4i(&ra)[CH_A], v4i(&rb)[CH_B]) {
+      k_step(buf, RS, [&] {
+        store_lds(buf ^ 1, ra, rb, false);
+        load_global(kclamp(kt + 3), ra, rb);
+      });
+      lds_barrier();
     };
     int kt = 0;
-    while (kt < KT - 2) {
-      k_step(0, RS, [&] { stage(0, kt, ra1, rb1); });
-      lds_barrier();
-      ++kt;
-      if (kt >= KT - 2)
-        break;
-      k_step(1, RS, [&] { stage(1, kt, ra0, rb0); });
-      lds_barrier();
-      ++kt;
+    for (; kt < KT - 3; kt += 2) {
+      whole(0, kt, ra1, rb1);
+      whole(1, kt + 1, ra0, rb0);
     }
-    if (kt < KT - 1) {
-      if (kt & 1) {
+    if (kt == KT - 3) {
+      whole(0, kt++, ra1, rb1);
 #pragma unroll
-        for (int h = 0; h < CH_A; ++h)
-          ra1[h] = ra0[h];
+      for (int h = 0; h < CH_A; ++h)
+        ra1[h] = ra0[h];
 #pragma unroll
-        for (int h = 0; h < CH_B; ++h)
-          rb1[h] = rb0[h];
-      }
+      for (int h = 0; h < CH_B; ++h)
+        rb1[h] = rb0[h];
+    }
+    if (kt == KT - 2) {
       k_step(kt & 1, RS, [&] { store_lds((kt & 1) ^ 1, ra1, rb1, tail); });
       lds_barrier();
       ++kt;

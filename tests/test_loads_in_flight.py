@@ -166,6 +166,56 @@ def test_empty_descriptors_come_with_an_offset_of_zero(kernels):
         assert loads and 2 * sum("offset:1024" in t for t in loads) == len(loads), (name, loads[:4])
 
 
+def loops_of(body):
+    """The loops (strongly connected parts of the branches) as lists of instructions."""
+    at = {ins.address: i for i, ins in enumerate(body)}
+    nexts = [([at[ins.target]] if ins.target is not None else []) +
+             ([i + 1] if ins.op not in ("s_branch", "s_endpgm") and i + 1 < len(body) else []) for i, ins in enumerate(body)]
+    order, low, stack, found = {}, {}, [], []
+    for root in range(len(body)):
+        walk = [] if root in order else [(root, iter(nexts[root]))]
+        if walk:
+            order[root] = low[root] = len(order)
+            stack.append(root)
+        while walk:
+            i, rest = walk[-1]
+            for j in rest:
+                if j not in order:
+                    order[j] = low[j] = len(order)
+                    stack.append(j)
+                    walk.append((j, iter(nexts[j])))
+                    break
+                if j in low:
+                    low[i] = min(low[i], order[j])
+            else:
+                walk.pop()
+                if walk:
+                    low[walk[-1][0]] = min(low[walk[-1][0]], low[i])
+                if low[i] == order[i]:
+                    part = sorted(stack[stack.index(i):])
+                    del stack[stack.index(i):]
+                    for j in part:
+                        del low[j]
+                    if len(part) > 1:
+                        found.append([body[j] for j in part])
+    return found
+
+
+def test_the_k_loop_waits_for_one_set_of_loads(kernels):
+    """k_gemm_i8 keeps the operands of two steps on their way: in its loop nothing waits
+    for the loads of the step before (with a way out in front of the odd step it did in
+    every second step, 109 x 10959 x 224 49 -> 59 us)."""
+    forms = {n: body for n, body in kernels.items() if re.search(r"k_gemm_i8ILi\d+ELi128E.*Li[12]ELb[01]EEE", n)}
+    assert len(forms) > 20
+    for name, body in forms.items():
+        loops = [part for part in loops_of(body) if any("mfma" in ins.op for ins in part)]
+        assert len(loops) == 2, name  # with and without row sums
+        for part in loops:
+            loads = sum(ins.op == "global_load_dwordx4" for ins in part)
+            waits = [ins.waits[0] for ins in part if ins.waits[0] is not None]
+            assert loads == 2 * (3 if "ILi64E" in name else 4) and min(waits) >= loads // 2, (name, loads, waits)
+
+
 @pytest.mark.parametrize("wait,touch,seen", [
     ("s_waitcnt vmcnt(0)", "v_mov_b32_e32 v4, 0", False),
     ("s_waitcnt vmcnt(1)", "v_mov_b32_e32 v4, 0", False),    # one younger load may stand
