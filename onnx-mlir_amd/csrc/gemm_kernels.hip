@@ -888,10 +888,11 @@ __global__ __launch_bounds__(256) void k_sum_parts(SumArgs args) {
 // What bounds a product whose tiles cover a part of the CUs is the chain of its
 // K steps, each the time its operands take into one CU: 0.15 us in 64 x 128 tiles
 // of k_gemm_i8_dma_bs, 0.17 in 128 x 64 ones of k_gemm_i8_dma, 0.23 in 128 x 128
-// ones, 0.37 in k_gemm_i8, a third more with row sums.  Splitting shortens the
-// chain and costs the launch of k_sum_parts, 2.5 us, and the arrays' way through
+// ones, 0.28 in k_gemm_i8, a third to a half more with row sums.  Splitting shortens
+// the chain and costs the launch of k_sum_parts, 2.5 us, and the arrays' way through
 // memory, 2 us per million elements.  Fitted to 2762 timed splits of 393 products
-// in two to 32 parts (within 4 %, root mean square).  Taken where that comes out
+// in two to 32 parts (within 4 %, root mean square; those in k_gemm_i8 to 1994
+// of 510 products in its present form, within 5 %).  Taken where that comes out
 // ahead of one piece in the tile chosen for it; more than one block per CU gains
 // nothing.  K of whole steps in any of the three, other K in k_gemm_i8_dma_bs, whose
 // steps do not look for the end of the row (int32 301 x 6384 x 1856 15.4 / 13.8 us).
@@ -914,7 +915,7 @@ SplitForm split_form(SplitKernel kernel, int64_t M, int64_t N) {
   case kSplitBs:
     return {kernel, ((M + 63) / 64) * ((N + 127) / 128), 4, 0.150, 0.33, 5.85};
   default:
-    return {kernel, t128, 1, 0.373, 0.29, 6.25};
+    return {kernel, t128, 1, 0.279, 0.52, 6.68};
   }
 }
 bool split_possible(const Sizes &p, bool any) {
@@ -963,17 +964,21 @@ double product_us(const Sizes &p, GemmSplit &best) {
   return least;
 }
 // And in k_gemm_i8, for any K: tiles of 128 x 128 and of 64 x 128, three blocks of
-// which run on a CU and are dealt out more evenly; the model of kTileCosts, fitted
-// to 322 products of awkward rows timed in both tiles
-// (profiles/awkward_tile_times.csv): the choice between these is 0.1 % above always
-// taking the fastest.  Int32 4099 x 777 x 1001 14.8 us in the larger, 13.6 in the
-// smaller, 1618 x 653 x 311 8.2 / 5.9; u8 3694 x 278 x 4295 17.6 / 18.4, u8
-// 575 x 948 x 8448 14.2 / 14.6.
+// which run on a CU and are dealt out more evenly; the model of kTileCosts.  Its
+// times are compared with those of other ways, so that they, kSplitAny's and the
+// copy's (gemm_padded_k) are fitted together, to the times themselves and to the
+// choice: to two thirds of 1294 products of awkward rows of up to 8.3e10
+// multiply-adds, each timed in both tiles, with its rows copied and in up to ten
+// splits (profiles/awkward_row_times.csv).  What is chosen takes 0.6 % longer than the
+// fastest way in the geometric mean, on the third that was left out as on the rest, and
+// 0.5 % above 26 us; the times are within 8 %, root mean square.  (Fitted to the choice
+// between the two tiles alone, and to products of up to 26 us, long ones were thought
+// 11 % too fast and left where they lie: 2.1 %, above 26 us 9 %.)
 double any_us(bool low, const Sizes &p) {
-  static constexpr TileCost t128 = {kT128x128, 128, 128, 1, 0.393, 0.232, 0.290,
-      2.646, 3.096, 1.674, 0.660};
-  static constexpr TileCost t64 = {kT128x128, 64, 128, 1, 0.268, 0.160, 0.242,
-      1.222, 1.451, 1.973, 0.467};
+  static constexpr TileCost t128 = {kT128x128, 128, 128, 1, 0.527, 0.350, 0.239,
+      2.419, 2.531, 1.932, 0.390};
+  static constexpr TileCost t64 = {kT128x128, 64, 128, 1, 0.219, 0.198, 0.214,
+      1.126, 1.180, 2.398, 0.305};
   return tile_us(low ? t64 : t128, p);
 }
 bool any_takes_64_rows(const Sizes &p) {
@@ -1208,11 +1213,11 @@ __global__ __launch_bounds__(256) void k_pad_rows(const uint8_t *__restrict__ A,
 // this says (0: not), the tail of each row filled with its zero point, and
 // multiplies with that K: (a - a_zp) is zero there, so the products, the row sums
 // and the K * (a offset) * (b offset) term of the zero-point algebra are those of
-// the original rows, bit for bit.  Where the copy -- 3 us and two ways through
-// memory -- costs clearly less than it saves (128 x 128 tiles of k_gemm_i8 at the
-// time of measuring): f32 154 x 1022 x 2258 11.8 -> 7.4 us, 3711 x 964 x 3580 34.8 ->
-// 28.9, u8 1260 x 3993 x 5876 50.7 -> 43.6; left alone: layer 1674 x 280 x 4123 16.8 /
-// 19.2, int32 4099 x 777 x 1001 14.4 / 18.0, u8 1032 x 487 x 6105 12.2 / 13.2.
+// the original rows, bit for bit.  Where the copy -- 2.9 us and two ways through
+// memory, by the fit of any_us -- costs less than it saves: int32 1178 x 4084 x 8832
+// 74.5 us as it lies, 58.5 copied, f32 with row sums 4095 x 2749 x 2584 59.1 / 49.2, u8
+// 1905 x 7689 x 1664 49.4 / 41.7; left alone: int32 with row sums 4099 x 777 x 1001 13.6 /
+// 17.3, u8 575 x 948 x 8448 13.7 / 15.2.
 int64_t gemm_padded_k(const GemmArgs &g) {
   const char *force = getenv("OM_MI355X_GEMM_TILE");
   const int64_t M = g.M, K = g.K, N = g.N;
@@ -1250,7 +1255,7 @@ int64_t gemm_padded_k(const GemmArgs &g) {
   if ((Kp == 512 || Kp == 768 || Kp == 1024) &&
       ((M + 63) / 64) * ((N + 127) / 128) <= 256)
     us = std::min(us, 2.4 + 0.002 * (double)Kp);
-  return general_us(own, s2) > us + 3.2 + 4.5e-7 * (double)(M * K) ? Kp : 0;
+  return general_us(own, s2) > us + 2.9 + 3.6e-7 * (double)(M * K) ? Kp : 0;
 }
 
 hipError_t launch_pad_rows(hipStream_t s, const void *a, int64_t M, int64_t K,

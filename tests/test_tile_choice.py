@@ -1,15 +1,18 @@
 """Which kernel a product takes: the modelled times (gemm_kernels.hip) against the
 times that were measured (profiles/*.csv), and the choice on the GPU."""
 import csv
+import ctypes
 import math
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-SOURCE = open(os.path.join(ROOT, "onnx-mlir_amd", "csrc", "gemm_kernels.hip")).read()
+CSRC = os.path.join(ROOT, "onnx-mlir_amd", "csrc")
+SOURCE = open(os.path.join(CSRC, "gemm_kernels.hip")).read()
 
 
 def _coefficients(pattern):
@@ -58,6 +61,73 @@ def test_tiles_of_awkward_rows():
         small, large = float(r["any_64x128"]), float(r["any_128x128"])
         over.append((small if _us(t64, *sizes) < _us(t128, *sizes) else large) / min(small, large))
     assert len(over) > 500 and math.exp(np.mean(np.log(over))) < 1.012
+
+
+@pytest.fixture(scope="module")
+def plan(rt, tmp_path_factory):
+    """(copied, parts, steps of a part) as the runtime library decides for rows of any
+    length: what it asks before it launches a product."""
+    folder = tmp_path_factory.mktemp("plan")
+    (folder / "plan.cpp").write_text("""
+#include "om_kernels.h"
+extern "C" void plan(int64_t M, int64_t K, int64_t N, int bytes, int rowsums, int64_t *out) {
+  om::GemmArgs g = {};
+  g.A = (const void *)((uintptr_t)1 << 40); // (never read)
+  g.a_unsigned = true;
+  g.b_unsigned = rowsums;
+  g.M = M, g.K = K, g.N = N;
+  g.epi = bytes ? om::kEpiQ8 : om::kEpiI32;
+  out[0] = om::gemm_padded_k(g) != 0;
+  om::gemm_plan_split(g);
+  out[1] = g.split.parts;
+  out[2] = g.split.steps;
+}
+""")
+    subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", CSRC, "-I", os.path.join(ROOT, "include"),
+                           "-I", "/opt/rocm/include", "-o", str(folder / "plan.so"), str(folder / "plan.cpp"), rt.LIB_PATH,
+                           "-Wl,--allow-shlib-undefined", "-Wl,-rpath," + os.path.dirname(rt.LIB_PATH)])
+    lib = ctypes.CDLL(str(folder / "plan.so"))
+    lib.plan.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p]
+
+    def ask(M, K, N, bytes_, rowsums):
+        out = (ctypes.c_int64 * 3)()
+        lib.plan(M, K, N, bytes_, rowsums, out)
+        return bool(out[0]), out[1], out[2]
+    return ask
+
+
+def test_the_way_of_awkward_rows_is_the_fastest_measured(plan):
+    """Copied first, split along K or in one piece of either tile: the library's choice
+    between all of them, on their times."""
+    t128, = _coefficients(r"static constexpr TileCost t128 = (\{.*?\});")
+    t64, = _coefficients(r"static constexpr TileCost t64 = (\{.*?\});")
+    over, longer = [], []
+    for r in _table("awkward_row_times.csv"):
+        sizes = int(r["M"]), int(r["K"]), int(r["N"]), r["results"] == "u8", r["rowsums"] == "1"
+        steps = -(-sizes[1] // 64)
+        # (parts of so many steps -> time; asked for n, there may be fewer)
+        splits = {-(-steps // -(-steps // int(n[6:]))): float(t) for n, t in r.items() if n.startswith("split_") and t}
+        ways = [float(r[n]) for n in ("any_64x128", "any_128x128", "rows_copied")] + list(splits.values())
+        copied, parts, _ = plan(*sizes)
+        if copied:
+            taken = ways[2]
+        elif parts > 1:  # (between the parts that were timed)
+            taken = float(np.interp(math.log(parts), *zip(*((math.log(p), splits[p]) for p in sorted(splits)))))
+        else:
+            taken = ways[0] if _us(t64, *sizes) < _us(t128, *sizes) else ways[1]
+        over.append(taken / min(ways))
+        if min(ways) > 26:
+            longer.append(over[-1])
+    assert len(over) > 1200 and len(longer) > 150
+    assert math.exp(np.mean(np.log(over))) < 1.008, math.exp(np.mean(np.log(over)))
+    assert math.exp(np.mean(np.log(longer))) < 1.007, math.exp(np.mean(np.log(longer)))
+    assert sum(o > 1.1 for o in over) < 0.02 * len(over)
+
+
+@pytest.mark.parametrize("M,K,N,bytes_,rowsums", [(1178, 4084, 8832, False, False), (4095, 2749, 2584, False, True), (3882, 826, 10618, False, True),
+                                                  (1905, 7689, 1664, True, False), (1092, 4017, 9663, False, False)])
+def test_long_products_of_awkward_rows_are_copied_first(plan, M, K, N, bytes_, rowsums):
+    assert plan(M, K, N, bytes_, rowsums)[0]
 
 
 def _product(rt, oracle, M, K, N, bdt, rng):
