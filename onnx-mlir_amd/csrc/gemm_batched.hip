@@ -100,13 +100,13 @@ __device__ __forceinline__ BatchParams expand(const FlatBatch &f, const PackedEp
 }
 
 // Results leave the matrix cores as 32 columns by two rows to a store: whole lines
-// only where rows are multiples of 128 bytes.  Otherwise a block puts its tile into
-// LDS, byte o of what goes to `to` at byte (to & 15) + o, and writes it from there in
-// aligned pieces of 16 bytes, written through like whole lines are.
+// only where rows are multiples of 128 bytes.  Otherwise, by the rule of out_form, a
+// block puts its tile into LDS, byte o of what goes to `to` at byte (to & 15) + o, and
+// writes it from there in aligned pieces of 16 bytes, written through like whole lines
+// are.
 //
-// `bytes` results of ES bytes each that lie one after the other (a tile as wide as
-// the matrix), `to` a multiple of ES.
-template <int ES>
+// `bytes` bytes of int32 results that lie one after the other (a tile as wide as the
+// matrix), `to` a multiple of 4.
 __device__ __forceinline__ void tile_out(const uint8_t *lds, char *to, int bytes) {
   typedef unsigned u4 __attribute__((ext_vector_type(4)));
   const TilePieces p = tile_pieces((int)(uintptr_t)to & 15, bytes);
@@ -116,13 +116,9 @@ __device__ __forceinline__ void tile_out(const uint8_t *lds, char *to, int bytes
   for (int o = p.first + tid * 16; o < p.last; o += 256 * 16)
     __builtin_amdgcn_raw_buffer_store_b128(
         *(const u4 *)(lds + o), rsrc, o, 0, kAuxThrough);
-  const int o = tile_end<ES>(p, tid);
-  if (o >= 0) {
-    if constexpr (ES == 4)
-      __builtin_amdgcn_raw_buffer_store_b32(*(const int *)(lds + o), rsrc, o, 0, 0);
-    else
-      __builtin_amdgcn_raw_buffer_store_b8(lds[o], rsrc, o, 0, 0);
-  }
+  const int o = tile_end(p, tid);
+  if (o >= 0)
+    __builtin_amdgcn_raw_buffer_store_b32(*(const int *)(lds + o), rsrc, o, 0, 0);
 }
 // BM rows of BN 4-byte results, kRowPitch bytes apart in LDS, that are whole pieces:
 // `tile` and `pitch` are multiples of 16 bytes, and so are `bytes`, those of a row
@@ -159,7 +155,8 @@ __device__ __forceinline__ void batched_tile(
   // The operands of two steps; at the end, results on their way out.
   constexpr int ES = EPI == kEpiQ8 ? 1 : 4;
   constexpr int kOperands = 2 * (BM + BN) * BK;
-  constexpr int kStaged = OUT == kOutDirect ? 0 : BM * kRowPitch<BN> / (4 / ES);
+  constexpr int kStaged = OUT == kOutDirect ? 0 : BM * kRowPitch<BN>;
+  static_assert(OUT == kOutDirect || EPI == kEpiI32, "results by way of LDS");
   __shared__ __attribute__((aligned(16)))
   uint8_t sm[kOperands > kStaged ? kOperands : kStaged];
   uint8_t(*const sA)[BM * BK] = (uint8_t(*)[BM * BK])sm;
@@ -429,22 +426,17 @@ __device__ __forceinline__ void batched_tile(
       }
     }
   };
-  auto put = [&](int at, uint32_t v) {
-    if (EPI == kEpiI32)
-      *(uint32_t *)(sm + at) = v;
-    else
-      sm[at] = (uint8_t)v;
-  };
-  const int col = (ct * 32 + l32) * ES;
+  auto put = [&](int at, uint32_t v) { *(uint32_t *)(sm + at) = v; };
+  const int col = (ct * 32 + l32) * 4;
   if constexpr (OUT == kOutTile) {
     // (as wide as the matrix: its results lie one after the other)
     const int skew = (int)(uintptr_t)out & 15;
     if (n < N)
       results([&](int first, uint32_t v) {
-        put(skew + (first + 4 * lh) * N * ES + col, v);
+        put(skew + (first + 4 * lh) * N * 4 + col, v);
       });
     __syncthreads();
-    tile_out<ES>(sm, out, rows * N * ES);
+    tile_out(sm, out, rows * N * 4);
     return;
   }
   if constexpr (OUT == kOutRows) {
@@ -507,14 +499,16 @@ void launch_out(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
 template <int BN, int EPI, bool ALIGNED>
 void launch_form(hipStream_t s, const BatchParams &bp, const EpiParams &ep,
     const FlatBatch *flat) {
-  const OutForm out = out_form(
-      EPI == kEpiQ8 ? 1 : 4, bp.N, bp.tiles_n, (uint64_t)(uintptr_t)ep.out, bp.blocks);
-  if (out == kOutTile)
-    launch_out<BN, EPI, ALIGNED, kOutTile>(s, bp, ep, flat);
-  else if (out == kOutDirect)
-    launch_out<BN, EPI, ALIGNED, kOutDirect>(s, bp, ep, flat);
-  else if constexpr (BN == 128 && EPI == kEpiI32) // (more than one tile to a row)
-    launch_out<BN, EPI, ALIGNED, kOutRows>(s, bp, ep, flat);
+  const OutForm out = out_form(EPI == kEpiI32, bp.M, bp.N, bp.tiles_m, bp.tiles_n,
+      (uint64_t)(uintptr_t)ep.out, bp.blocks);
+  if constexpr (EPI == kEpiI32) {
+    if (out == kOutTile)
+      return launch_out<BN, EPI, ALIGNED, kOutTile>(s, bp, ep, flat);
+    if constexpr (BN == 128) // (more than one tile to a row)
+      if (out == kOutRows)
+        return launch_out<BN, EPI, ALIGNED, kOutRows>(s, bp, ep, flat);
+  }
+  launch_out<BN, EPI, ALIGNED, kOutDirect>(s, bp, ep, flat);
 }
 
 template <int EPI>

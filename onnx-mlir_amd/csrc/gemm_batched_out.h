@@ -10,26 +10,33 @@ namespace gemm {
 
 enum OutForm : int { kOutDirect, kOutTile, kOutRows };
 
-// By way of LDS where rows are no whole lines and the grid is more than one round of
-// blocks: up to that the barrier and the second way cost more than the stores (48 x
-// 38x38x80 4.74 us by LDS, 4.57 without).
-//   Tiles as wide as the matrix: 156 x 82x128x82 7.6 -> 6.8 us, 64 x 511x511x64 with 8-bit
-//   results 13.9 -> 9.6, the loads' part of both included.
-//   Rows of whole 16-byte pieces: int32 88 x 472x128x472 28.8 -> 23.4; not 8-bit ones (21.2
-//   -> 23.5), nor other rows, whose ends are stores of their own (64 x 511x64x511 17.2
-//   -> 18.5).
-// result: bytes of one; out: where the first goes.  Results that do not start on a
-// multiple of their size are stored one by one: pieces of 16 bytes would end inside
-// them.
-constexpr OutForm out_form(int result, int N, int tiles_n, uint64_t out, int64_t blocks) {
-  if (blocks <= 256 || (int64_t)N * result % 128 == 0 || out % (uint64_t)result != 0)
+// int32 results go by way of LDS where rows are no whole lines, in tiles as wide as the
+// matrix and in rows of whole 16-byte pieces (not in other rows, whose ends are stores
+// of their own: 64 x 511x64x511 17.2 us, 18.5 by LDS).  Timed both ways for 600 products
+// (us, direct / by LDS):
+//   more than one block a CU: what a block writes then stands beside another's loads
+//   (472x128x472 in 256 blocks 4.98 / 5.00, 320 5.72 / 5.50, 512 6.76 / 6.07; 64x64x100 in 256
+//   4.28 / 4.36, 320 4.84 / 4.69, 768 7.67 / 6.05);
+//   6 KB of results to a tile, for the barrier and the second way: below 2 KB 5 % slower
+//   in the geometric mean, 2 to 6 KB 1.5 %, 6 to 8 KB 2 % faster, 8 to 20 KB 4 %;
+//   up to 48 MB in all: up to 32 MB, the size of the L2s, 5 % faster, 32 to 48 MB 2 %, above 1 to
+//   4 % slower (148 x 173x32x572 14.1 / 15.1).
+// 8-bit results do not: 2 % slower in the geometric mean of 173 products, up to 19 %.
+// Results that do not start on a multiple of 4 are stored one by one: pieces of 16 bytes
+// would end inside them.
+// tiles_m, tiles_n: of a matrix; out: where the first result goes.
+constexpr OutForm out_form(bool int32, int64_t M, int64_t N, int tiles_m, int tiles_n,
+    uint64_t out, int64_t blocks) {
+  const int64_t tiles = (int64_t)tiles_m * tiles_n, bytes = M * N * 4;
+  if (!int32 || N % 32 == 0 || out % 4 != 0 || blocks <= 256 ||
+      bytes < 6 * 1024 * tiles || blocks / tiles * bytes > 48000000)
     return kOutDirect;
   if (tiles_n == 1)
     return kOutTile;
-  return result == 4 && out % 16 == 0 && N % 4 == 0 ? kOutRows : kOutDirect;
+  return out % 16 == 0 && N % 4 == 0 ? kOutRows : kOutDirect;
 }
 
-// The pieces of `bytes` bytes of results that lie one after the other from `skew`
+// The pieces of `bytes` bytes of int32 results that lie one after the other from `skew`
 // bytes behind a multiple of 16 on, as offsets from that multiple: aligned ones of 16
 // bytes from `first` up to `last`, and single results in front and behind, one to a
 // thread.
@@ -39,14 +46,12 @@ struct TilePieces {
 constexpr TilePieces tile_pieces(int skew, int bytes) {
   return {skew, skew ? 16 : 0, (skew + bytes) & ~15, skew + bytes};
 }
-// The single result of ES bytes that thread `tid` writes: 16 / ES threads in front,
-// the next 16 / ES behind; negative: none.
-template <int ES>
+// The single result that thread `tid` writes: four threads in front, the next four
+// behind; negative: none.
 constexpr int tile_end(const TilePieces &p, int tid) {
-  constexpr int PER = 16 / ES;
-  const int o = tid < PER ? p.skew + tid * ES
-                          : (p.last > p.first ? p.last : p.first) + (tid - PER) * ES;
-  return tid < 2 * PER && o < p.end && (tid >= PER || o < p.first) ? o : -1;
+  const int o = tid < 4 ? p.skew + tid * 4
+                        : (p.last > p.first ? p.last : p.first) + (tid - 4) * 4;
+  return tid < 8 && o < p.end && (tid >= 4 || o < p.first) ? o : -1;
 }
 
 } // namespace gemm

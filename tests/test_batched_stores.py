@@ -21,51 +21,54 @@ def out(tmp_path_factory):
 #include "gemm_batched_out.h"
 using namespace om::gemm;
 extern "C" {
-int form(int result, int N, int tiles_n, uint64_t out, int64_t blocks) { return out_form(result, N, tiles_n, out, blocks); }
+int form(bool int32, int64_t M, int64_t N, uint64_t out, int64_t entries) {
+  const int tiles_m = (int)((M + 63) / 64), tiles_n = (int)((N + 127) / 128);
+  return out_form(int32, M, N, tiles_m, tiles_n, out, entries * tiles_m * tiles_n);
+}
 int first(int skew, int bytes) { return tile_pieces(skew, bytes).first; }
 int last(int skew, int bytes) { return tile_pieces(skew, bytes).last; }
-int end1(int skew, int bytes, int tid) { return tile_end<1>(tile_pieces(skew, bytes), tid); }
-int end4(int skew, int bytes, int tid) { return tile_end<4>(tile_pieces(skew, bytes), tid); }
+int end(int skew, int bytes, int tid) { return tile_end(tile_pieces(skew, bytes), tid); }
 }
 """)
     subprocess.check_call(["g++", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, "-o", str(folder / "out.so"), str(folder / "out.cpp")])
     lib = ctypes.CDLL(str(folder / "out.so"))
-    lib.form.argtypes = [ctypes.c_int] * 3 + [ctypes.c_uint64, ctypes.c_int64]
+    lib.form.argtypes = [ctypes.c_bool, ctypes.c_int64, ctypes.c_int64, ctypes.c_uint64, ctypes.c_int64]
     return lib
 
 
 def test_how_results_leave(out):
     """One by one up to 256 blocks, where rows are whole lines, where the first result
-    does not start on a multiple of its size."""
+    does not start on a multiple of four, in tiles of few results and above 48 MB."""
     at = 1 << 40
-    for N in (1, 7, 33, 63, 100, 127):
-        tiles_n = 1
-        assert out.form(4, N, tiles_n, at, 257) == TILE and out.form(4, N, tiles_n, at, 256) == DIRECT
+    for N in (33, 63, 100, 127):
+        assert out.form(True, 64, N, at, 257) == TILE and out.form(True, 64, N, at, 256) == DIRECT
+        assert out.form(True, 65, N, at, 300) == (TILE if 65 * N * 4 >= 2 * 6144 else DIRECT)
         for off in range(1, 16):
-            assert out.form(4, N, tiles_n, at + off, 300) == (DIRECT if off % 4 else TILE), off
-            assert out.form(1, N, tiles_n, at + off, 300) == TILE
-    assert out.form(4, 64, 1, at, 300) == out.form(1, 128, 1, at, 300) == out.form(4, 160, 2, at, 300) == DIRECT
-    assert [out.form(4, N, 2, at, 300) for N in (132, 133, 134, 196)] == [ROWS, DIRECT, DIRECT, ROWS]
-    assert all(out.form(4, 132, 2, at + off, 300) == DIRECT for off in range(1, 16)) and out.form(1, 132, 2, at, 300) == DIRECT
+            assert out.form(True, 64, N, at + off, 300) == (DIRECT if off % 4 else TILE), off
+            assert out.form(False, 64, N, at + off, 300) == DIRECT
+    assert out.form(True, 64, 64, at, 300) == out.form(True, 64, 160, at, 300) == DIRECT
+    assert [out.form(True, 64, N, at, 300) for N in (132, 133, 134, 196)] == [ROWS, DIRECT, DIRECT, ROWS]
+    assert all(out.form(True, 64, 132, at + off, 300) == DIRECT for off in range(1, 16)) and out.form(False, 64, 132, at, 300) == DIRECT
+    assert [out.form(True, M, 48, at, 300) for M in (31, 32)] == [DIRECT, TILE]
+    assert [out.form(True, M, 196, at, 300) for M in (15, 16)] == [DIRECT, ROWS]
+    assert [out.form(True, 64, 100, at, n) for n in (48000000 // 25600, 48000000 // 25600 + 1)] == [TILE, DIRECT]
 
 
-@pytest.mark.parametrize("es", [1, 4])
 @pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 64 * 7, 64 * 127, 64 * 100 + 1])
-def test_a_tile_leaves_in_pieces_that_cover_it_once(out, es, count):
+def test_a_tile_leaves_in_pieces_that_cover_it_once(out, count):
     """tile_out: aligned pieces of 16 bytes and single results at the two ends, from
     every address that out_form lets through."""
-    size = count * es
+    size = count * 4
     for skew in range(16):
-        if out.form(es, 63, 1, (1 << 40) + skew, 300) != TILE:
+        if out.form(True, 64, 63, (1 << 40) + skew, 300) != TILE:
             continue
         written = [(o, 16) for t in range(256) for o in range(out.first(skew, size) + t * 16, out.last(skew, size), 256 * 16)]
-        ends = [(out.end1 if es == 1 else out.end4)(skew, size, t) for t in range(256)]
-        written += [(o, es) for o in ends if o >= 0]
+        written += [(o, 4) for o in (out.end(skew, size, t) for t in range(256)) if o >= 0]
         covered = np.zeros(skew + size + 16, int)
         for o, n in written:
             covered[o:o + n] += 1
         assert (covered[skew:skew + size] == 1).all() and covered.sum() == size, skew
-    assert 15 + 64 * 128 * es <= 64 * (128 * 4 + 32) // (4 // es)  # the LDS it lies in
+    assert 15 + 64 * 128 * 4 <= 64 * (128 * 4 + 32)  # the LDS it lies in
 
 
 @pytest.mark.gpu
