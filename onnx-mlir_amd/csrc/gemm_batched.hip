@@ -9,7 +9,7 @@
 // k_gemm_i8_batched
 //   Bound: the int32 results (32 x 12 heads of 128x64x128: 25 MB out, 6 MB in;
 //   4.5 us at the 5.66 TB/s the device stores at) and, with one K step, the
-//   chain load -> LDS -> MFMA -> store of a block.  Measured 7.0 us = 4.5 TB/s.
+//   chain load -> LDS -> MFMA -> store of a block.  Measured 6.1 us = 5.1 TB/s.
 //   Why one launch: packing B and multiplying, matrix by matrix, is three
 //   launches of 1.3 to 3.5 us an entry, whatever the entry's size (the same
 //   product: 3.5 ms).
@@ -548,8 +548,11 @@ bool gemm_batched_ok(const GemmArgs &g, const GemmBatch &b) {
 
 // One launch against packing each matrix of B and multiplying entry by entry,
 // both by a cost model in microseconds, fitted to 3600 products (1 to 32 entries,
-// 1 to 2048 rows, K 32 to 11008, N 32 to 4096, odd sizes among them): its choice is
-// more than 4 % behind the other for 21 of them, at most 15 %.
+// 1 to 2048 rows, K 32 to 11008, N 32 to 4096, odd sizes among them) when loads at any
+// address and launches took longer.  Of 500 timed both ways with the kernels as they
+// are, its choice is more than 4 % behind for 13, all but one of them one to three
+// entries (1 x 10x4516x38 27.0 us for 10.6), and 0.9 % in the geometric mean; with 1.15
+// for rows at any address, which is what long chains show, 1.6 %.
 //   One launch: the chain of a block's K steps, or where there are more blocks
 //   than the device holds what the CUs have to do in sum.  It does not split K, so
 //   few entries with a long K are a few blocks: 1 x 8192 x 128 70 us against 14

@@ -52,11 +52,10 @@ using namespace gemm;
 namespace {
 
 // BM x BN block tile, WGM x WGN waves, each wave a (BM/WGM) x (BN/WGN) tile
-// made of 32x32 MFMA tiles.  MINB: blocks that a CU is to hold; of more than two
-// the compiler gets registers for one block fewer, since a fourth block of 64 x
-// 128 brings less than what its 128 registers a lane spill costs (in us, with
-// four / three: 1000 x 1001 x 3000 with row sums 11.9 / 11.3, 300 x 777 x 1001
-// 6.8 / 6.5, 4099 x 777 x 1001 14.5 / 13.7).
+// made of 32x32 MFMA tiles.  MINB: blocks that a CU is to hold.  Three of 64 x 128,
+// without spilled registers; a fourth, which spills 4 of its 128 registers a lane, is
+// 0.3 % slower in the geometric mean of 1002 products (in us, four / three: int32 4099 x
+// 777 x 1001 with row sums 15.4 / 13.9, 2717 x 88 x 2204 8.0 / 9.3).
 // A_MODE: 0 = int8 as is, 1 = uint8 (XOR 0x80 while staging), 2 = already
 // shifted (stored as u8-128) -- offsets as for uint8, no XOR.
 // A_LOAD: kLoadAligned = K % 64 == 0 and A 16-byte aligned (plain vector
@@ -65,8 +64,7 @@ namespace {
 // = byte loads (an A of fewer than 16 bytes, K = 0).
 template <int BM, int BN, int WGM, int WGN, int MINB, int A_MODE, int EPI,
     int A_LOAD, bool SPLIT = false>
-__global__ __launch_bounds__(WGM *WGN * 64, MINB > 2 ? MINB - 1 : MINB)
-void k_gemm_i8(TileArgs args) {
+__global__ __launch_bounds__(WGM *WGN * 64, MINB) void k_gemm_i8(TileArgs args) {
   const uint8_t *__restrict__ A = args.A;
   const int8_t *__restrict__ Bp = args.Bp;
   const int M = args.M, N = args.N, K = args.K;
@@ -891,8 +889,9 @@ __global__ __launch_bounds__(256) void k_sum_parts(SumArgs args) {
 // ones, 0.28 in k_gemm_i8, a third to a half more with row sums.  Splitting shortens
 // the chain and costs the launch of k_sum_parts, 2.5 us, and the arrays' way through
 // memory, 2 us per million elements.  Fitted to 2762 timed splits of 393 products
-// in two to 32 parts (within 4 %, root mean square; those in k_gemm_i8 to 1994
-// of 510 products in its present form, within 5 %).  Taken where that comes out
+// in two to 32 parts (within 4 %, root mean square, and within 6 % of 2991 of 200
+// products since launches take less; those in k_gemm_i8 to 1994 of 510 products,
+// within 5 %).  Taken where that comes out
 // ahead of one piece in the tile chosen for it; more than one block per CU gains
 // nothing.  K of whole steps in any of the three, other K in k_gemm_i8_dma_bs, whose
 // steps do not look for the end of the row (int32 301 x 6384 x 1856 15.4 / 13.8 us).
@@ -1107,7 +1106,7 @@ hipError_t gemm_launch_cfg(
                         : "k_gemm_i8 (any K, any alignment)";
     const int tiles_m64 = (int)((g.M + 63) / 64);
     if (low)
-      k_gemm_i8<64, 128, 2, 2, 4, A_MODE, EPI, kLoadAny>
+      k_gemm_i8<64, 128, 2, 2, 3, A_MODE, EPI, kLoadAny>
           <<<dim3((unsigned)(tiles_m64 * tiles_n128)), 256, 0, st>>>(tile_args(g, ep, EPI));
     else if (g.M * g.K >= 16)
       k_gemm_i8<128, 128, 2, 2, 2, A_MODE, EPI, kLoadAny>
@@ -1158,7 +1157,7 @@ hipError_t gemm_launch_cfg(
     return launch_dma<A_MODE, EPI>(st, g, ep, kD128x128);
   default:
     t_last_kernel = "k_gemm_i8 (128x128 tiles through registers)";
-    k_gemm_i8<128, 128, 2, 2, 3, A_MODE, EPI, kLoadAligned>
+    k_gemm_i8<128, 128, 2, 2, 2, A_MODE, EPI, kLoadAligned>
         <<<dim3((unsigned)(tiles_m * tiles_n128)), 256, 0, st>>>(tile_args(g, ep, EPI));
     break;
   }

@@ -63,15 +63,15 @@ def spills():
     (r"k_gemm_i8_dmaI", 0),
     (r"k_gemm_i8_(dma_)?bsI", 0),  # every tile, with and without row sums, split
     (r"k_gemm_i8_wregI", 0),
-    # any K, any alignment: two blocks of 128 x 128 a CU, or four of 64 x 128, which
-    # leaves 128 registers a lane
+    # any K, any alignment: two blocks of 128 x 128 a CU, or three of 64 x 128
     (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi2E", 0),
-    (r"k_gemm_i8ILi64ELi128ELi2ELi2ELi4E", 11),
-    (r"k_gemm_i8ILi128ELi128ELi2ELi2ELi3E", 20),  # on request only (OM_MI355X_GEMM_TILE=0)
-    (r"k_gemm_i8_(skinny|batched|flight)I", 0),
+    (r"k_gemm_i8ILi64ELi128ELi2ELi2ELi3E", 0),
+    (r"k_gemm_i8_(skinny|batched|batched_flat|flight)I", 0),
     (r"k_(pad_rows|sum_parts|copy_in|copy_out|pack_b)", 0),
 ])
 def test_kernels_spill_no_more_registers(spills, kernel, most):
     forms = {n: s for n, s in spills.items() if re.search(kernel, n)}
+    for name in re.search(r"\((.*)\)I", kernel).group(1).split("|") if "(skinny" in kernel else ():
+        assert any("k_gemm_i8_" + name + "I" in n for n in forms), name
     assert forms, sorted(spills)
     assert max(forms.values()) <= most, {n: s for n, s in forms.items() if s > most}
