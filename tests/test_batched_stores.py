@@ -129,3 +129,25 @@ def test_int32_results_that_start_between_words(rt, oracle, count, M, K, N, off)
     got = whole.numpy()
     assert np.array_equal(got[32 + off:][:want.nbytes].view(np.int32).reshape(want.shape), want)
     assert (got[:32 + off] == 90).all() and (got[32 + off + want.nbytes:] == 90).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,form", [(64, 63, 100, TILE), (40, 48, 62, TILE), (65, 33, 132, ROWS), (66, 130, 196, ROWS), (9, 65, 33, DIRECT)])
+@pytest.mark.parametrize("alead,blead", [((10, 1, 3), (10, 9, 1)), ((270,), (270,)), ((1,), (270,))])
+@pytest.mark.parametrize("adt,bdt", [(np.uint8, np.int8), (np.int8, np.uint8)])
+def test_every_way_out_with_zero_points_of_every_row_and_column(rt, out, M, K, N, form, alead, blead, adt, bdt):
+    """270 entries: in batch dimensions that do not merge (the general form of the
+    arguments) and in one, each matrix of B with one of A or all with the same, int8
+    and uint8 on either side."""
+    rng = np.random.default_rng(M + K + N)
+    i, j = np.iinfo(adt), np.iinfo(bdt)
+    a, b = rng.integers(i.min, i.max + 1, alead + (M, K), dtype=adt), rng.integers(j.min, j.max + 1, blead + (K, N), dtype=bdt)
+    az, bz = rng.integers(i.min, i.max + 1, alead + (M, 1), dtype=adt), rng.integers(j.min, j.max + 1, blead + (1, N), dtype=bdt)
+    for azp, bzp in ((az, bz), (az.reshape(-1)[:1].reshape(()), bz), (None, None)):
+        want = np.matmul(a.astype(np.int32) - (0 if azp is None else azp.astype(np.int32)), b.astype(np.int32) - (0 if bzp is None else bzp.astype(np.int32)))
+        y = rt.DeviceArray(want.shape, np.int32)
+        assert out.form(True, M, N, y.ptr, 270) == form
+        rt.MatMulInteger(*(None if v is None else rt.DeviceArray.from_numpy(v) for v in (a, b, azp, bzp)), out=y)
+        rt.synchronize()
+        assert rt.last_gemm_kernel() == "k_gemm_i8_batched"
+        assert np.array_equal(y.numpy(), want), (azp is None, bzp is None)

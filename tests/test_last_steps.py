@@ -12,13 +12,9 @@ def rt():
     return om_mi355x
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("K", [17, 64, 65, 128, 130, 192, 200, 256, 257, 320, 321])
-@pytest.mark.parametrize("M", [67, 129])
-def test_counts_of_k_steps(rt, M, K):
+def _check(rt, M, K, N, kernel):
     """A at an odd address, with and without row sums.  Whole numbers: exact."""
     rng = np.random.default_rng(M * K)
-    N = 70
     for bdt in (np.int8, np.uint8):
         i = np.iinfo(bdt)
         a, b = rng.integers(0, 256, (M, K), dtype=np.uint8), rng.integers(i.min, i.max + 1, (K, N), dtype=bdt)
@@ -27,5 +23,26 @@ def test_counts_of_k_steps(rt, M, K):
         got = rt.MatMulInteger(rt.DeviceArray.view_of(whole, 1, (M, K)), rt.DeviceArray.from_numpy(b),
                                rt.DeviceArray.from_numpy(az), None if bz is None else rt.DeviceArray.from_numpy(bz))
         rt.synchronize()
-        want = (a.astype(np.int64) - 77) @ (b.astype(np.int64) - (0 if bz is None else 131))
-        assert np.array_equal(got.numpy(), want), rt.last_gemm_kernel()
+        assert rt.last_gemm_kernel() == "k_gemm_i8 (any K, any alignment" + kernel, rt.last_gemm_kernel()
+        # (float64 holds sums of 2^16 products of 16 bits exactly)
+        want = (a.astype(np.float64) - 77) @ (b.astype(np.float64) - (0 if bz is None else 131))
+        assert np.array_equal(got.numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [17, 64, 65, 128, 130, 192, 200, 256, 257, 320, 321])
+@pytest.mark.parametrize("M", [67, 129])
+def test_counts_of_k_steps(rt, M, K):
+    _check(rt, M, K, 70, "; 64x128 tiles)")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [64, 65, 130, 190, 250, 300, 321, 400])
+def test_counts_of_k_steps_in_tiles_of_128_rows(rt, K):
+    _check(rt, 1366, K, 4429, ")")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [1473, 1537, 1601, 1665, 2049, 1793])  # a last part of 4, 5, 1, 2, 3 and 4 steps
+def test_counts_of_k_steps_of_the_last_part(rt, K):
+    _check(rt, 67, K, 70, "; split along K)")
