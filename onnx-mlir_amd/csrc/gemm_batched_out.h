@@ -12,15 +12,17 @@ enum OutForm : int { kOutDirect, kOutTile, kOutRows };
 
 // int32 results go by way of LDS where rows are no whole lines, in tiles as wide as the
 // matrix and in rows of whole 16-byte pieces (not in other rows, whose ends are stores
-// of their own: 64 x 511x64x511 17.2 us, 18.5 by LDS).  Timed both ways for 600 products
-// (us, direct / by LDS):
+// of their own: 64 x 511x64x511 17.2 us, 18.5 by LDS).  707 products timed both ways
+// (profiles/batched_way_out_times.csv; us, direct / by LDS):
 //   more than one block a CU: what a block writes then stands beside another's loads
 //   (472x128x472 in 256 blocks 4.98 / 5.00, 320 5.72 / 5.50, 512 6.76 / 6.07; 64x64x100 in 256
 //   4.28 / 4.36, 320 4.84 / 4.69, 768 7.67 / 6.05);
 //   6 KB of results to a tile, for the barrier and the second way: below 2 KB 5 % slower
-//   in the geometric mean, 2 to 6 KB 1.5 %, 6 to 8 KB 2 % faster, 8 to 20 KB 4 %;
-//   up to 48 MB in all: up to 32 MB, the size of the L2s, 5 % faster, 32 to 48 MB 2 %, above 1 to
-//   4 % slower (148 x 173x32x572 14.1 / 15.1).
+//   in the geometric mean, 2 to 6 KB 1.5 %, 6 to 8 KB 2 % faster, 8 to 20 KB 3 %, more 6 %;
+//   up to 48 MB in all: up to 32 MB, the size of the L2s, 5 % faster, 32 to 48 MB 3 %; 48 to
+//   75 MB 4 % slower (148 x 173x32x572 14.1 / 15.1).  Above that it depends on what the last-
+//   level cache holds of the results that a program goes through: with three in turn 6 %
+//   faster (0.68 to 1.10) to 110 MB, 18 % slower (0.70 to 1.54) beyond.
 // 8-bit results do not: 2 % slower in the geometric mean of 173 products, up to 19 %.
 // Results that do not start on a multiple of 4 are stored one by one: pieces of 16 bytes
 // would end inside them.

@@ -2,7 +2,9 @@
 a grid of more than one round of blocks, operands and results at odd addresses up
 to the last byte of their buffers, results next to memory that must stay as it is;
 and the pieces in which a tile leaves LDS (gemm_batched_out.h, built for the host)."""
+import csv
 import ctypes
+import math
 import os
 import subprocess
 
@@ -52,6 +54,21 @@ def test_how_results_leave(out):
     assert [out.form(True, M, 48, at, 300) for M in (31, 32)] == [DIRECT, TILE]
     assert [out.form(True, M, 196, at, 300) for M in (15, 16)] == [DIRECT, ROWS]
     assert [out.form(True, 64, 100, at, n) for n in (48000000 // 25600, 48000000 // 25600 + 1)] == [TILE, DIRECT]
+
+
+def test_the_way_out_is_the_faster_one_measured(out):
+    """Up to 75 MB, where it does not depend on what the last-level cache holds."""
+    over, never = [], []
+    with open(os.path.join(os.path.dirname(os.path.dirname(CSRC)), "profiles", "batched_way_out_times.csv")) as f:
+        for r in csv.DictReader(line for line in f if not line.startswith("#")):
+            E, M, N, direct, lds = int(r["entries"]), int(r["M"]), int(r["N"]), float(r["direct"]), float(r["by_lds"])
+            if E * M * N * 4 > 75e6:
+                continue
+            form = out.form(r["results"] == "i32", M, N, 1 << 40, E)
+            over.append((direct if form == DIRECT else lds) / min(direct, lds))
+            never.append(direct / min(direct, lds))
+    assert len(over) > 700
+    assert math.exp(np.mean(np.log(over))) < 1.01 < math.exp(np.mean(np.log(never))), (over, never)
 
 
 @pytest.mark.parametrize("count", [1, 2, 3, 4, 5, 15, 16, 17, 31, 33, 64 * 7, 64 * 127, 64 * 100 + 1])
